@@ -5,7 +5,7 @@
 //   box around the group; a counting sort puts every particle in its cell,
 //   ordered by host index inside a cell, and the occupied cells are
 //   compacted into a list of cell centres;
-// * one thread per pixel marches its ray (pinhole camera,
+// * one wavefront per pixel marches its ray (pinhole camera,
 //   geometry/pinhole_camera.hpp:33-65). At every step the distance bound is
 //   the minimum over all occupied cells of the rounded-box distance
 //   |max(q, 0)| + min(max_k q_k, 0) - grid_diameter, q = |x - centre| -
@@ -29,6 +29,7 @@
 #include <cmath>
 #include <limits>
 #include <stdexcept>
+#include <type_traits>
 #include <vector>
 
 namespace prtcl_amd {
@@ -205,39 +206,31 @@ __global__ void k_tr_scan_add(uint32_t *out, int64_t n, const uint32_t *bsum) {
 }
 
 __global__ void k_tr_place(const int64_t *lin_of, int64_t n, const uint32_t *start,
-                           uint32_t *cursor, int64_t *ent) {
+                           uint32_t *cursor, uint32_t *ent) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kTB + threadIdx.x;
   if (i >= n)
     return;
   const int64_t lin = lin_of[i];
   if (lin >= 0)
-    ent[start[lin] + atomicAdd(&cursor[lin], 1u)] = i;
+    ent[start[lin] + atomicAdd(&cursor[lin], 1u)] = static_cast<uint32_t>(i);
 }
 
-// host order inside every cell (insertion sort of the cell's entries)
-__global__ void k_tr_sort_cells(const uint32_t *start, int64_t ncells, int64_t *ent) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * kTB + threadIdx.x;
-  if (c >= ncells)
-    return;
-  const uint32_t b = start[c], e = start[c + 1];
-  for (uint32_t k = b + 1; k < e; ++k) {
-    const int64_t v = ent[k];
-    uint32_t j = k;
-    while (j > b && ent[j - 1] > v) {
-      ent[j] = ent[j - 1];
-      --j;
-    }
-    ent[j] = v;
-  }
-}
-
-__global__ void k_tr_pack(const double *x, const int64_t *ent, int64_t n, double *ex) {
+// positions packed by cell, in host order inside every cell: the particle at
+// (unordered) entry k goes to its cell's start plus the number of the cell's
+// entries with a smaller host index
+__global__ void k_tr_pack(const double *x, const int64_t *lin_of, const uint32_t *start,
+                          const uint32_t *ent, int64_t n, double *ex) {
   const int64_t k = static_cast<int64_t>(blockIdx.x) * kTB + threadIdx.x;
   if (k >= n)
     return;
-  const int64_t i = ent[k];
+  const uint32_t i = ent[k];
+  const int64_t c = lin_of[i];
+  const uint32_t b = start[c], e = start[c + 1];
+  uint32_t r = b;
+  for (uint32_t m = b; m < e; ++m)
+    r += ent[m] < i ? 1u : 0u;
   for (int d = 0; d < 3; ++d)
-    ex[3 * k + d] = x[3 * i + d];
+    ex[3 * static_cast<int64_t>(r) + d] = x[3 * static_cast<int64_t>(i) + d];
 }
 
 __global__ void k_tr_flags(const uint32_t *count, int64_t ncells, uint32_t *flag) {
@@ -282,10 +275,11 @@ __global__ void k_tr_gplace(const uint32_t *gidx, const double *centres, int64_t
     gcent[3 * pos + d] = centres[3 * k + d];
 }
 
-// the non-empty groups: box (centre, half extents) containing the boxes of
-// half extent gd around the centres of all its cells, and the cell range
+// the non-empty groups: box (centre relative to the cell box's origin, half
+// extents) containing the boxes of half extent gd around the centres of all
+// its cells, and the cell range
 __global__ void k_tr_glist(const uint32_t *gcount, const uint32_t *gocc, const uint32_t *gstart,
-                           int64_t ng, CellBox B, double half, double *gbox, uint32_t *grange) {
+                           int64_t ng, CellBox B, double half, float *gbox, uint32_t *grange) {
   const int64_t g = static_cast<int64_t>(blockIdx.x) * kTB + threadIdx.x;
   if (g >= ng || gcount[g] == 0)
     return;
@@ -297,8 +291,8 @@ __global__ void k_tr_glist(const uint32_t *gcount, const uint32_t *gocc, const u
     const double c0 = static_cast<double>(o[k] + kGroup * gc[k]);
     const double lo = B.gd * c0 + half - B.gd;
     const double hi = B.gd * (c0 + (kGroup - 1)) + half + B.gd;
-    gbox[6 * j + k] = 0.5 * (lo + hi);
-    gbox[6 * j + 3 + k] = 0.5 * (hi - lo);
+    gbox[6 * j + k] = static_cast<float>(0.5 * (lo + hi) - B.gd * static_cast<double>(o[k]));
+    gbox[6 * j + 3 + k] = static_cast<float>(0.5 * (hi - lo));
   }
   grange[2 * j] = gstart[g];
   grange[2 * j + 1] = gstart[g + 1];
@@ -316,136 +310,366 @@ __device__ inline double box_sdf(const double *x, const double *c, const double 
   return (sqrt(dot3(qm, qm)) + std_min(mc, 0.0)) - gd;
 }
 
-// minimum of the cell distances of group g into sdf (cells of half extent gd)
-__device__ inline void group_min(const double *x, const uint32_t *grange, const double *gcent,
-                                 int64_t g, double gd, double *sdf) {
-  const double e[3] = {gd, gd, gd};
-  for (uint32_t c = grange[2 * g]; c < grange[2 * g + 1]; ++c)
-    *sdf = std_min(*sdf, box_sdf(x, gcent + 3 * static_cast<int64_t>(c), e, gd));
+// FP32 estimate of box_sdf for a point and a centre relative to the same
+// origin; within the march's margin of the exact value
+__device__ inline float box_sdf_f32(const float *x, const float *c, const float *e, float gd) {
+  const float q0 = fabsf(x[0] - c[0]) - e[0], q1 = fabsf(x[1] - c[1]) - e[1],
+              q2 = fabsf(x[2] - c[2]) - e[2];
+  const float m0 = fmaxf(q0, 0.0f), m1 = fmaxf(q1, 0.0f), m2 = fmaxf(q2, 0.0f);
+  return sqrtf(m0 * m0 + m1 * m1 + m2 * m2) + fminf(fmaxf(q0, fmaxf(q1, q2)), 0.0f) - gd;
 }
 
-__global__ __launch_bounds__(kTB) void k_tr_march(TraceParams P, const double *gbox,
-                                                  const uint32_t *grange, const double *gcent,
-                                                  int64_t ngroups, const uint32_t *start,
-                                                  const double *ex, CellBox B, double *image,
-                                                  double *par) {
-  const int64_t pid = static_cast<int64_t>(blockIdx.x) * kTB + threadIdx.x;
-  if (pid >= P.width * P.height)
-    return;
-  const int64_t ix = pid % P.width, iy = pid / P.width;
+__device__ inline float wave_min_all(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    v = fminf(v, __shfl_xor(v, o, 64));
+  return v;
+}
 
-  // pinhole_camera.hpp:53-62
-  double d[3];
-  {
-    const double px = (P.sox + static_cast<double>(ix)) * P.pixel_size;
-    const double py = (P.soy + static_cast<double>(iy)) * P.pixel_size;
-    double dir0[3];
-    for (int k = 0; k < 3; ++k) {
-      const double pp = ((P.O[k] + px * P.hh[k]) + py * P.v[k]) - P.f * P.p[k];
-      dir0[k] = P.O[k] - pp;
-    }
-    normalized3(dir0, d);
-  }
+__device__ inline double wave_std_min_all(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    v = std_min(v, __shfl_xor(v, o, 64));
+  return v;
+}
 
-  double t = 0, normal[3] = {0, 0, 0};
-  bool done = false;  // broke out of the march
-  for (int64_t step = 0; step < P.max_steps && !done; ++step) {
-    double rx[3];
-    for (int k = 0; k < 3; ++k)
-      rx[k] = P.O[k] + t * d[k];
-    // the minimum over every occupied cell of the reference, exactly: a
-    // group's box contains its cells' boxes, so its distance bounds theirs
-    // from below, and a group whose bound exceeds the minimum found so far
-    // (beyond a margin far above the rounding of either) cannot lower it.
-    // The group with the smallest bound is evaluated first.
-    double sdf = DBL_MAX;
-    int64_t first = -1;
-    double best_lb = DBL_MAX;
-    for (int64_t g = 0; g < ngroups; ++g) {
-      const double lb = box_sdf(rx, gbox + 6 * g, gbox + 6 * g + 3, P.gd);
-      if (lb < best_lb) {
-        best_lb = lb;
-        first = g;
+// orders a wavefront's own LDS writes before its later reads
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// particles listed at once by the march (one more round of 64 may be appended
+// before a list that is too long is emptied)
+constexpr int kNearCap = 448;
+constexpr int kMarchWaves = kTB / 64;
+
+// a / b, correctly rounded, with y = 1 / b correctly rounded: Markstein's
+// iteration (IBM J. Res. Dev. 34, 1990), twice, so that the first quotient
+// need not be faithful. For operands whose quotient is far from the range's
+// ends, as distances over h and kernel sums over h^3 are.
+struct Divisor {
+  double b, y;
+};
+__device__ inline double divide(double a, const Divisor &d) {
+  double q = a * d.y;
+  q = fma(fma(-d.b, q, a), d.y, q);
+  return fma(fma(-d.b, q, a), d.y, q);
+}
+
+// One wavefront per pixel. A ray of one lane would be a serial chain of up to
+// 300 steps, each over every group, the cells of the near ones and up to
+// 27 cells of particles, and the slowest ray would decide the time; here
+// the 64 lanes share each step's groups, cells and particles. Near the surface
+// the bound is divided by the particle count, so a ray that hits takes a
+// hundred or more short steps; what bounds the kernel is the FP64 issue of
+// those. Per such step:
+//  * The particles within reach plus a skin are listed in LDS once, in the
+//    reference's order (cells x outermost, then host order), and the list
+//    serves every step that stays in the cell and within the skin. Values are
+//    computed 64 at a time and subtracted one after the other, in order.
+//  * The gradient is summed once, at the last step that summed particles: only
+//    there does it reach the image.
+//  * sdf = max(cell distance, phi): one cell's distance bounds the minimum over
+//    the cells from above, so a phi above it needs no search. The last search's
+//    cell gives that bound.
+// The minimum over all cells is exact where it is needed: groups and cells are
+// filtered by an FP32 distance with a margin of 32 roundings of the largest
+// coordinate, and every cell that the filter leaves is evaluated in FP64. The
+// minimum does not depend on the order.
+// 400 x 300 pixels of 125,000 particles: 80.4 ms with one lane per pixel,
+// 26.6 ms with one wavefront and a search, a walk over 27 cells and a gradient
+// in every step, 10.3 ms now.
+__global__ __launch_bounds__(kTB) void k_tr_march(
+    TraceParams P, const float *__restrict__ gbox, const uint32_t *__restrict__ grange,
+    const double *__restrict__ gcent, int64_t ngroups, const uint32_t *__restrict__ start,
+    const double *__restrict__ ex, CellBox B, double *image, double *par) {
+  __shared__ uint32_t s_idx[kMarchWaves][kNearCap + 64];
+  __shared__ double s_val[kMarchWaves][4][64];
+  const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  const uint64_t below = (1ull << lane) - 1ull;
+  uint32_t *idx = s_idx[wv];
+  const float gdf = static_cast<float>(P.gd);
+  const float ef[3] = {gdf, gdf, gdf};
+  const double e3[3] = {P.gd, P.gd, P.gd};
+  const double org[3] = {P.gd * B.ox, P.gd * B.oy, P.gd * B.oz};
+  const double ext = P.gd * (B.nx > B.ny ? (B.nx > B.nz ? B.nx : B.nz)
+                                         : (B.ny > B.nz ? B.ny : B.nz));
+  const Divisor by_half{P.half, 1.0 / P.half}, by_h3{P.h3, 1.0 / P.h3}, by_h4{P.h4, 1.0 / P.h4};
+  // w > 0 needs r < 2 half: a particle beyond reach + skin has none anywhere
+  // within skin of the point that the list was made for
+  const double skin = 0.25 * P.half;
+  const double reach2 = (2 * P.half + skin) * (2 * P.half + skin) * (1 + 1e-9);
+  const double skin2 = skin * skin * (1 - 1e-9);
+
+  for (int64_t pid = static_cast<int64_t>(blockIdx.x) * kMarchWaves + wv;
+       pid < P.width * P.height; pid += static_cast<int64_t>(gridDim.x) * kMarchWaves) {
+    const int64_t ix = pid % P.width, iy = pid / P.width;
+
+    // pinhole_camera.hpp:53-62
+    double d[3];
+    {
+      const double px = (P.sox + static_cast<double>(ix)) * P.pixel_size;
+      const double py = (P.soy + static_cast<double>(iy)) * P.pixel_size;
+      double dir0[3];
+      for (int k = 0; k < 3; ++k) {
+        const double pp = ((P.O[k] + px * P.hh[k]) + py * P.v[k]) - P.f * P.p[k];
+        dir0[k] = P.O[k] - pp;
       }
+      normalized3(dir0, d);
     }
-    if (first >= 0)
-      group_min(rx, grange, gcent, first, P.gd, &sdf);
-    for (int64_t g = 0; g < ngroups; ++g) {
-      if (g == first)
-        continue;
-      const double lb = box_sdf(rx, gbox + 6 * g, gbox + 6 * g + 3, P.gd);
-      if (lb > sdf + 1e-9 * (fabs(sdf) + P.gd))
-        continue;
-      group_min(rx, grange, gcent, g, P.gd, &sdf);
-    }
-    if (sdf < P.gd) {
-      int32_t rc[3];
-      for (int k = 0; k < 3; ++k)
-        rc[k] = static_cast<int32_t>(floor(rx[k] / P.gd));
-      double phi = P.phi0, grad[3] = {0, 0, 0};
-      int64_t count = 0;
-      for (int cx = -1; cx <= 1; ++cx)
-        for (int cy = -1; cy <= 1; ++cy)
-          for (int cz = -1; cz <= 1; ++cz) {
-            int64_t lin;
-            if (!cell_index(B, rc[0] + cx, rc[1] + cy, rc[2] + cz, &lin))
-              continue;
-            for (uint32_t e = start[lin]; e < start[lin + 1]; ++e) {
-              double dv[3];
-              for (int k = 0; k < 3; ++k)
-                dv[k] = rx[k] - ex[3 * static_cast<int64_t>(e) + k];
-              const double r = sqrt(dot3(dv, dv));
-              const double w = evalq(P.alpha, fabs(r) / P.half) / P.h3;
-              if (w > 0) {
-                double g[3] = {0, 0, 0};
-                if (!(r < P.grad_eps)) {
-                  const double dr =
-                      -copysign(evaldq(P.alpha, fabs(r) / P.half) / P.h4, r);
-                  const double s = dr / r;
-                  for (int k = 0; k < 3; ++k)
-                    g[k] = s * dv[k];
-                }
-                phi -= w;
-                for (int k = 0; k < 3; ++k)
-                  grad[k] -= g[k];
-                ++count;
-              }
-            }
+
+    double rx[3];           // the ray's point
+    int32_t rc[3];          // its cell, where the particles are summed
+    double sdf;             // least distance of the cells evaluated so far
+    int64_t best_cell = -1; // the cell that gave it
+    float xf[3], margin;
+
+    // exact minimum over the cells [c0, c1) that the filter leaves into sdf
+    // (a comparison with NaN leaves a cell in)
+    auto group_cells = [&](uint32_t c0, uint32_t c1) {
+      for (uint32_t c = c0; c < c1; c += 64) {
+        const bool in = c + lane < c1;
+        const double *cp = gcent + 3 * static_cast<int64_t>(in ? c + lane : c0);
+        const double cc[3] = {cp[0], cp[1], cp[2]};
+        const float cf[3] = {static_cast<float>(cc[0] - org[0]),
+                             static_cast<float>(cc[1] - org[1]),
+                             static_cast<float>(cc[2] - org[2])};
+        const float lb = box_sdf_f32(xf, cf, ef, gdf);
+        float bound = wave_min_all(in ? lb : 3.0e38f);
+        bound = fminf(bound, static_cast<float>(sdf)) + 2.0f * margin;
+        const bool keep = in && !(lb > bound);
+        if (__ballot(keep) == 0ull)
+          continue;
+        double v = DBL_MAX;
+        if (keep)
+          v = std_min(v, box_sdf(rx, cc, e3, P.gd));
+        const double m = wave_std_min_all(v);
+        if (m < sdf) {
+          sdf = m;
+          best_cell = c + __ffsll(static_cast<long long>(__ballot(v == m))) - 1;
+        }
+      }
+    };
+    // the minimum over every occupied cell
+    auto search = [&]() {
+      double far = 0;
+      for (int k = 0; k < 3; ++k) {
+        xf[k] = static_cast<float>(rx[k] - org[k]);
+        far = fmax(far, fabs(rx[k] - org[k]));
+      }
+      // 32 roundings of the largest term of either distance
+      margin = 2e-6f * static_cast<float>(far + ext + P.gd);
+      sdf = DBL_MAX;
+      best_cell = -1;
+      if (ngroups <= 0)
+        return;
+      // the group with the smallest estimate first
+      float best = 3.0e38f;
+      int64_t at = -1;
+      for (int64_t g0 = 0; g0 < ngroups; g0 += 64) {
+        const int64_t g = g0 + lane;
+        const float lb =
+            g < ngroups ? box_sdf_f32(xf, gbox + 6 * g, gbox + 6 * g + 3, gdf) : 3.0e38f;
+        if (g < ngroups && (lb < best || at < 0)) {
+          best = lb;
+          at = g;
+        }
+      }
+      const float m = wave_min_all(best);
+      const uint64_t who = __ballot(at >= 0 && best == m);
+      // NaN estimates (a ray point that is not finite): any group
+      const int64_t first = __shfl(at, who ? __ffsll(static_cast<long long>(who)) - 1 : 0, 64);
+      group_cells(grange[2 * first], grange[2 * first + 1]);
+      for (int64_t g0 = 0; g0 < ngroups; g0 += 64) {
+        const int64_t g = g0 + lane;
+        const bool in = g < ngroups && g != first;
+        const float lb =
+            in ? box_sdf_f32(xf, gbox + 6 * g, gbox + 6 * g + 3, gdf) : 3.0e38f;
+        uint64_t left = __ballot(in && !(lb > static_cast<float>(sdf) + 2.0f * margin));
+        while (left) {
+          const int l = __ffsll(static_cast<long long>(left)) - 1;
+          left &= left - 1;
+          // the bound may have come down since the ballot
+          if (__shfl(lb, l, 64) > static_cast<float>(sdf) + 2.0f * margin)
+            continue;
+          group_cells(grange[2 * (g0 + l)], grange[2 * (g0 + l) + 1]);
+        }
+      }
+    };
+
+    int n = 0;                 // listed particles
+    bool listed = false;       // the list serves the cell lc around lx
+    int32_t lc[3] = {0, 0, 0};
+    double lx[3] = {0, 0, 0};
+    double acc[4];             // phi, and minus the gradient's sum
+    int64_t count = 0;
+    // subtracts the values of the listed particles in list order
+    auto sum_list = [&](auto grad_tag) {
+      constexpr bool kGrad = decltype(grad_tag)::value;
+      constexpr int kVals = kGrad ? 4 : 1;
+      wave_lds_sync();
+      for (int m = 0; m < n; m += 64) {
+        double w = 0, g[3] = {0, 0, 0};
+        if (m + lane < n) {
+          const double *xp = ex + 3 * static_cast<int64_t>(idx[m + lane]);
+          double dv[3];
+          for (int k = 0; k < 3; ++k)
+            dv[k] = rx[k] - xp[k];
+          const double r = sqrt(dot3(dv, dv));
+          const double q = divide(fabs(r), by_half);
+          w = divide(evalq(P.alpha, q), by_h3);
+          if (kGrad && w > 0 && !(r < P.grad_eps)) {
+            const double dr = -copysign(divide(evaldq(P.alpha, q), by_h4), r);
+            const double s = dr / r;
+            for (int k = 0; k < 3; ++k)
+              g[k] = s * dv[k];
           }
-      if (count > 0) {
-        const double s = P.L * static_cast<double>(count);
-        phi /= s;
-        for (int k = 0; k < 3; ++k)
-          normal[k] = grad[k] / s;
-        sdf = std_max(sdf, phi);
-      } else {
-        sdf = std_max(sdf, P.gd / 4);
+        }
+        const uint64_t hit = __ballot(w > 0);
+        const int nh = __popcll(hit);
+        if (w > 0) {
+          const int at = __popcll(hit & below);
+          s_val[wv][0][at] = w;
+          if (kGrad)
+            for (int k = 0; k < 3; ++k)
+              s_val[wv][1 + k][at] = g[k];
+        }
+        wave_lds_sync();
+        for (int k = 0; k < nh; ++k)
+          for (int v = 0; v < kVals; ++v)
+            acc[v] -= s_val[wv][v][k];
+        count += nh;
+        wave_lds_sync();
       }
+    };
+    // phi and the particle count (kGrad: the gradient too) at rx
+    auto sum_particles = [&](auto grad_tag) {
+      acc[0] = P.phi0;
+      acc[1] = acc[2] = acc[3] = 0;
+      count = 0;
+      if (listed && rc[0] == lc[0] && rc[1] == lc[1] && rc[2] == lc[2]) {
+        double m[3];
+        for (int k = 0; k < 3; ++k)
+          m[k] = rx[k] - lx[k];
+        if (dot3(m, m) <= skin2) {
+          sum_list(grad_tag);
+          return;
+        }
+      }
+      for (int k = 0; k < 3; ++k) {
+        lc[k] = rc[k];
+        lx[k] = rx[k];
+      }
+      listed = true;
+      n = 0;
+      // lane c < 27: the entries of cell c of the stencil
+      uint32_t cb = 0, ce = 0;
+      if (lane < 27) {
+        int64_t lin;
+        if (cell_index(B, rc[0] + lane / 9 - 1, rc[1] + lane / 3 % 3 - 1, rc[2] + lane % 3 - 1,
+                       &lin)) {
+          cb = start[lin];
+          ce = start[lin + 1];
+        }
+      }
+      uint64_t cells = __ballot(ce > cb);
+      while (cells) {
+        const int c = __ffsll(static_cast<long long>(cells)) - 1;
+        cells &= cells - 1;
+        const uint32_t b = __shfl(cb, c, 64), e = __shfl(ce, c, 64);
+        for (uint32_t p0 = b; p0 < e; p0 += 64) {
+          const uint32_t p = p0 + lane;
+          bool ok = false;
+          if (p < e) {
+            const double *xp = ex + 3 * static_cast<int64_t>(p);
+            double dv[3];
+            for (int k = 0; k < 3; ++k)
+              dv[k] = rx[k] - xp[k];
+            ok = !(dot3(dv, dv) > reach2);
+          }
+          const uint64_t hit = __ballot(ok);
+          if (ok)
+            idx[n + __popcll(hit & below)] = p;
+          n += __popcll(hit);
+          if (n > kNearCap) {  // crowded: summed as it goes, not kept
+            sum_list(grad_tag);
+            n = 0;
+            listed = false;
+          }
+        }
+      }
+      sum_list(grad_tag);
+    };
+
+    double t = 0, t_sum = -1;  // t_sum: the last step that summed particles
+    bool done = false;         // broke out of the march
+    for (int64_t step = 0; step < P.max_steps && !done; ++step) {
+      for (int k = 0; k < 3; ++k)
+        rx[k] = P.O[k] + t * d[k];
+      bool exact = false;
+      if (best_cell >= 0) {
+        const double *cp = gcent + 3 * best_cell;
+        const double cc[3] = {cp[0], cp[1], cp[2]};
+        sdf = box_sdf(rx, cc, e3, P.gd);
+      }
+      if (best_cell < 0 || !(sdf < P.gd)) {
+        search();
+        exact = true;
+      }
+      if (sdf < P.gd) {
+        for (int k = 0; k < 3; ++k)
+          rc[k] = static_cast<int32_t>(floor(rx[k] / P.gd));
+        sum_particles(std::false_type{});
+        double phi = P.gd / 4;
+        if (count > 0) {
+          phi = acc[0] / (P.L * static_cast<double>(count));
+          t_sum = t;
+        }
+        if (!exact && !(sdf <= phi))
+          search();
+        sdf = std_max(sdf, phi);
+      }
+      if (sdf < 1e-6) {
+        done = true;
+        break;
+      }
+      t += sdf;
+      if (t >= P.max_parameter)
+        done = true;
     }
-    if (sdf < 1e-6) {
-      done = true;
-      break;
+    if (!done)
+      t = P.max_parameter;  // ran out of steps
+    double pix;
+    if (t == P.max_parameter) {
+      pix = 0;
+    } else if (t > P.max_parameter) {
+      pix = 0.3;
+    } else {
+      double normal[3] = {0, 0, 0};
+      if (t_sum >= 0) {
+        for (int k = 0; k < 3; ++k) {
+          rx[k] = P.O[k] + t_sum * d[k];
+          rc[k] = static_cast<int32_t>(floor(rx[k] / P.gd));
+        }
+        sum_particles(std::true_type{});
+        const double s = P.L * static_cast<double>(count);
+        for (int k = 0; k < 3; ++k)
+          normal[k] = acc[1 + k] / s;
+      }
+      double dn[3], nn[3];
+      normalized3(d, dn);
+      normalized3(normal, nn);
+      pix = -dot3(dn, nn);
     }
-    t += sdf;
-    if (t >= P.max_parameter)
-      done = true;
+    if (lane == 0) {
+      image[pid] = pix;
+      if (par)
+        par[pid] = t;
+    }
   }
-  if (!done)
-    t = P.max_parameter;  // ran out of steps
-  double pix;
-  if (t == P.max_parameter) {
-    pix = 0;
-  } else if (t > P.max_parameter) {
-    pix = 0.3;
-  } else {
-    double dn[3], nn[3];
-    normalized3(d, dn);
-    normalized3(normal, nn);
-    pix = -dot3(dn, nn);
-  }
-  image[pid] = pix;
-  if (par)
-    par[pid] = t;
 }
 
 struct Dev {
@@ -574,7 +798,7 @@ void trace_scene(SceneBase &sc, CtxResources &res, int group, const prtcl_hip_ca
   Dev occ(sizeof(uint32_t) * static_cast<size_t>(ncells + 1));
   Dev flag(sizeof(uint32_t) * static_cast<size_t>(ncells + 1));
   Dev lin_of(sizeof(int64_t) * static_cast<size_t>(n > 0 ? n : 1));
-  Dev ent(sizeof(int64_t) * static_cast<size_t>(n > 0 ? n : 1));
+  Dev ent(sizeof(uint32_t) * static_cast<size_t>(n > 0 ? n : 1));
   Dev ex(sizeof(double) * static_cast<size_t>(n3 > 0 ? n3 : 1));
   PRTCL_HIP_CHECK(hipMemsetAsync(count.p, 0, sizeof(uint32_t) * (ncells + 1), st));
   PRTCL_HIP_CHECK(hipMemsetAsync(cursor.p, 0, sizeof(uint32_t) * (ncells + 1), st));
@@ -589,11 +813,10 @@ void trace_scene(SceneBase &sc, CtxResources &res, int group, const prtcl_hip_ca
   PRTCL_HIP_CHECK(hipStreamSynchronize(st));
   if (placed > 0) {
     hipLaunchKernelGGL(k_tr_place, dim3(blocks(n)), dim3(kTB), 0, st, lin_of.as<const int64_t>(),
-                       n, startb.as<const uint32_t>(), cursor.as<uint32_t>(), ent.as<int64_t>());
-    hipLaunchKernelGGL(k_tr_sort_cells, dim3(blocks(ncells)), dim3(kTB), 0, st,
-                       startb.as<const uint32_t>(), ncells, ent.as<int64_t>());
+                       n, startb.as<const uint32_t>(), cursor.as<uint32_t>(), ent.as<uint32_t>());
     hipLaunchKernelGGL(k_tr_pack, dim3(blocks(placed)), dim3(kTB), 0, st, x.as<const double>(),
-                       ent.as<const int64_t>(), static_cast<int64_t>(placed), ex.as<double>());
+                       lin_of.as<const int64_t>(), startb.as<const uint32_t>(),
+                       ent.as<const uint32_t>(), static_cast<int64_t>(placed), ex.as<double>());
   }
   hipLaunchKernelGGL(k_tr_flags, dim3(blocks(ncells)), dim3(kTB), 0, st,
                      count.as<const uint32_t>(), ncells, flag.as<uint32_t>());
@@ -638,17 +861,19 @@ void trace_scene(SceneBase &sc, CtxResources &res, int group, const prtcl_hip_ca
   PRTCL_HIP_CHECK(hipMemcpyAsync(&ngroups, gocc.as<uint32_t>() + ng, sizeof(ngroups),
                                  hipMemcpyDeviceToHost, st));
   PRTCL_HIP_CHECK(hipStreamSynchronize(st));
-  Dev gbox(sizeof(double) * 6 * static_cast<size_t>(ngroups > 0 ? ngroups : 1));
+  Dev gbox(sizeof(float) * 6 * static_cast<size_t>(ngroups > 0 ? ngroups : 1));
   Dev grange(sizeof(uint32_t) * 2 * static_cast<size_t>(ngroups > 0 ? ngroups : 1));
   hipLaunchKernelGGL(k_tr_glist, dim3(blocks(ng)), dim3(kTB), 0, st, gcount.as<const uint32_t>(),
                      gocc.as<const uint32_t>(), gstart.as<const uint32_t>(), ng, B, P.half,
-                     gbox.as<double>(), grange.as<uint32_t>());
+                     gbox.as<float>(), grange.as<uint32_t>());
 
   const int64_t npx = cam.width * cam.height;
   Dev img(sizeof(double) * static_cast<size_t>(npx));
   Dev par(sizeof(double) * static_cast<size_t>(npx));
-  hipLaunchKernelGGL(k_tr_march, dim3(blocks(npx)), dim3(kTB), 0, st, P,
-                     gbox.as<const double>(), grange.as<const uint32_t>(),
+  // large sensors: each wavefront takes several pixels (2^32 threads at most)
+  const int64_t mb = std::min<int64_t>((npx + kMarchWaves - 1) / kMarchWaves, int64_t(1) << 22);
+  hipLaunchKernelGGL(k_tr_march, dim3(static_cast<unsigned>(mb)), dim3(kTB), 0, st, P,
+                     gbox.as<const float>(), grange.as<const uint32_t>(),
                      gcent.as<const double>(), static_cast<int64_t>(ngroups),
                      startb.as<const uint32_t>(), ex.as<const double>(), B, img.as<double>(),
                      par.as<double>());

@@ -154,6 +154,8 @@ void launch(const char *name, void (*k)(P...), dim3 g, dim3 b, size_t, hipStream
 #define __builtin_amdgcn_wave_barrier() \
   ((void)::emu::wave_op(::emu::kOpBallot, 0u, 0, 64, __LINE__, __FILE__))
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
+// used on values that are uniform over the wavefront
+#define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_rsqf(x) (1.0f / std::sqrt(static_cast<float>(x)))
 #define __builtin_amdgcn_rcpf(x) (1.0f / static_cast<float>(x))
 

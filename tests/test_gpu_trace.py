@@ -70,3 +70,22 @@ def test_trace_of_an_empty_group(hip_ctx):
     with pytest.raises(hip.HipError):
         s.trace(hip.camera((0, -1, 0), (0, 1, 0), (0, 0, 1), 1.0, 0, 12), "fluid")
     s.destroy()
+
+
+@pytest.mark.parametrize("n,spread,size", [(1, 0.0, (1, 1)), (70, 0.02, (7, 5)),
+                                           (2000, 0.06, (9, 13)), (700, 0.9, (33, 3))],
+                         ids=["one", "few", "crowded", "scattered"])
+def test_trace_of_uneven_clouds(hip_ctx, n, spread, size):
+    """One particle, cells with more particles than one wavefront and than the
+    march lists at once, and groups that hold few cells each; odd sensors."""
+    from prtcl_amd import hip
+    rng = np.random.default_rng(n)
+    x = (0.3 + spread * rng.random((n, 3))).astype(np.float32)
+    sc = scenes.Scene(name="cloud", spacing=0.025, fluid_x=x, fluid_v=np.zeros_like(x),
+                      fluid_m=np.ones(n, np.float32), time_of_birth=np.zeros(n, np.float32),
+                      boundary_x=np.zeros((0, 3), np.float32), smoothing_scale=0.025)
+    print(f"case: cloud of {n}, trace", flush=True)
+    s = hip.HipScene(hip_ctx, sc)
+    c = 0.3 + 0.5 * spread
+    _compare(s, "fluid", ((c, c - 1.0, c + 0.1), (0, 1, -0.1), (0, 0, 1), 1.0, *size))
+    s.destroy()
