@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "fused.hpp"
+#include "scan8.hpp"
 
 namespace prtcl_amd {
 
@@ -129,18 +130,6 @@ __device__ __forceinline__ void grid_walk(const SceneView<T> &S, int i, const ve
         fn(j);
     }
   });
-}
-
-// Calls fn(j) for every fluid neighbour j != i of particle i, from the list
-// (global slots) or over the grid for a particle whose list overflowed.
-template <class T, class Fn>
-__device__ __forceinline__ void walk(const SceneView<T> &S, const NbrList &L, int i,
-                                     const vec4_t<T> &xi, Fn &&fn) {
-  const uint32_t info = L.info[i];
-  if (!(info & kListOverflow))
-    list_visit(L, Spans::of(L.blk[i / kBlock]), static_cast<size_t>(S.nf), i, info, fn);
-  else
-    grid_walk(S, i, xi, fn);
 }
 
 // the three x-runs of slab s (rows dz = s - 1, dy = -1..1) of a cell, in
@@ -284,39 +273,30 @@ __device__ __forceinline__ double first_iteration(const SceneView<T> &S, int i,
 // the candidates are read from global memory (through L2) and both phases
 // run once over all 27 cells.
 // ---------------------------------------------------------------------------
-template <class T, bool kWithSource, bool kStage>
-__device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrList &L,
-                                             vec4_t<T> *vout, unsigned lb) {
-  constexpr uint32_t kCap = slab_cap<T>();
-  __shared__ vec4_t<T> sx[kStage ? kCap + kRunPad : 1];
-  // rows kNbrCap + 1 .. kNbrCap + 8 take the writes of a lane past its cap
-  __shared__ uint16_t lst[kNbrCap + 9][kBlock];
-  __shared__ BlockRanges sR;
-  const unsigned t = threadIdx.x;
-  const int i = static_cast<int>(lb * kBlock + t);
-  const bool valid = i < S.nf;
-  const uint32_t cell = valid ? S.fcell[i] : 0u;
-  block_spans(S.grid, S.fstart, valid, cell, sR);
-  if (t < 6)
-    reinterpret_cast<uint32_t *>(L.blk + lb)[t] = t < 3 ? sR.base[t] : sR.len[t - 3];
-  const Spans R = Spans::of(sR);
-  const uint32_t smax = R.max_len();
-  const bool staged = kStage && smax <= kCap;
-  const bool encodable = smax <= 0x10000u;
+// the pair sums of the setup pass for one particle (or one lane's share)
+template <class T, bool kWithSource>
+struct SetupSums {
+  const SceneView<T> &S;
+  const FastSpline<T> K;
+  vec4_t<T> xi;
+  T dtg0, dtg1, dtg2, vs0, vs1, vs2;
+  // density, G_f, sum |gradW|^2 and the velocity-divergence sum of the source
+  // term; density and G_b of the boundary
+  T rho = 0, gf0 = 0, gf1 = 0, gf2 = 0, s2 = 0, dsum = 0;
+  T rhob = 0, gb0 = 0, gb1 = 0, gb2 = 0;
+  bool near_boundary = false;
 
-  const FastSpline<T> K = fast_spline(S);
-  const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
-  const vec4_t<T> xi = valid ? S.xm[i] : zero4;
-  const vec4_t<T> vi = valid ? S.v[i] : zero4;
-  const T Hi = fade_step(S, vi.w);
-  const T dtg0 = S.dt * S.g0, dtg1 = S.dt * S.g1, dtg2 = S.dt * S.g2;
-  const T vs0 = vi.x + dtg0 * Hi, vs1 = vi.y + dtg1 * Hi, vs2 = vi.z + dtg2 * Hi;
-  // density (self term W(0) = 4 alpha / h^3), G_f, sum |gradW|^2 and the
-  // velocity-divergence sum of the source term
-  T rho = xi.w * K.aw * T(4), gf0 = 0, gf1 = 0, gf2 = 0, s2 = 0, dsum = 0;
-  // pair sums of neighbour (x_j, m_j) = pj with velocity vj (read only
-  // with kWithSource)
-  auto pair2 = [&](const vec4_t<T> &pj, const vec4_t<T> &vj) {
+  __device__ __forceinline__ SetupSums(const SceneView<T> &view, const vec4_t<T> &x,
+                                       const vec4_t<T> &vi)
+      : S(view), K(fast_spline(view)), xi(x) {
+    const T Hi = fade_step(S, vi.w);
+    dtg0 = S.dt * S.g0, dtg1 = S.dt * S.g1, dtg2 = S.dt * S.g2;
+    vs0 = vi.x + dtg0 * Hi, vs1 = vi.y + dtg1 * Hi, vs2 = vi.z + dtg2 * Hi;
+  }
+  // density self term W(0) = 4 alpha / h^3
+  __device__ __forceinline__ T self() const { return xi.w * K.aw * T(4); }
+  // neighbour (x_j, m_j) = pj with velocity vj (read only with kWithSource)
+  __device__ __forceinline__ void pair(const vec4_t<T> &pj, const vec4_t<T> &vj) {
     const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
     T w, f;
     K.eval(d0 * d0 + d1 * d1 + d2 * d2, w, f);
@@ -333,9 +313,103 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
       const T u2 = vs2 - (vj.z + dtg2 * Hj);
       dsum += pj.w * (u0 * g0 + u1 * g1 + u2 * g2);
     }
-  };
-  auto load_v = [&](uint32_t j) { return kWithSource ? S.v[j] : zero4; };
-  auto pair = [&](const vec4_t<T> &pj, uint32_t j) { pair2(pj, load_v(j)); };
+  }
+  __device__ __forceinline__ vec4_t<T> load_v(uint32_t j) const {
+    return kWithSource ? S.v[j] : make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  }
+  // the boundary particles of slots [b, e)
+  __device__ __forceinline__ void boundary(uint32_t b, uint32_t e) {
+    for (uint32_t j = b; j < e; j += 4) {
+      vec4_t<T> pk[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        pk[u] = S.bxV[min(j + u, e - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const vec4_t<T> pj = pk[u];
+        const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
+        const T r2 = sqdist_exact(d0, d1, d2);
+        if (j + u >= e || !(r2 < S.thr2))
+          continue;
+        near_boundary = true;
+        T w, f;
+        K.eval(r2, w, f);
+        rhob += pj.w * w;
+        gb0 += pj.w * (f * d0);
+        gb1 += pj.w * (f * d1);
+        gb2 += pj.w * (f * d2);
+      }
+    }
+  }
+  // the particle's fields from the complete sums; returns its aprde term of
+  // IISPH iteration 1 (S.first_iter)
+  __device__ __forceinline__ double finish(int i, T birth, vec4_t<T> *vout) {
+    const T rho0 = S.rho0;
+    rho += rho0 * rhob;
+    const T irho = T(1) / rho;
+    const T irho2 = irho * irho;
+    const T k14 = T(1.4) * rho0;
+    const T c0 = -(gf0 + k14 * gb0) * irho2;
+    const T c1 = -(gf1 + k14 * gb1) * irho2;
+    const T c2 = -(gf2 + k14 * gb2) * irho2;
+    const T gs0 = gf0 + rho0 * gb0, gs1 = gf1 + rho0 * gb1, gs2 = gf2 + rho0 * gb2;
+    const T fac = S.dt * S.dt * rho0 * irho;
+    const T AA = fac * ((c0 * gs0 + c1 * gs1 + c2 * gs2) - xi.w * irho2 * s2);
+    S.rho[i] = rho;
+    S.c[i] = make4<vec4_t<T>>(c0, c1, c2, T(0));
+    S.G[i] = make4<vec4_t<T>>(gs0, gs1, gs2, T(0));
+    S.AA[i] = AA;
+    S.p[i] = T(0);
+    S.pr[i] = T(0);
+    S.xq[i] = make4<vec4_t<T>>(xi.x, xi.y, xi.z, T(0));
+    S.xa[S.xa_x(static_cast<size_t>(i))] = xi;
+    if (kWithSource) {
+      const T src = (rho0 - rho) -
+                    S.dt * rho0 * irho * (dsum + rho0 * (vs0 * gb0 + vs1 * gb1 + vs2 * gb2));
+      S.s[i] = src;
+      vout[i] = make4<vec4_t<T>>(vs0, vs1, vs2, birth);
+      if (S.first_iter)
+        return first_iteration(S, i, xi, rho, src, AA);
+    } else {
+      S.vd[i] = make4<vec4_t<T>>(gb0, gb1, gb2, T(0));  // G_b for the source pass
+    }
+    return 0.0;
+  }
+};
+
+template <class T, bool kStage>
+struct SetupShared {
+  vec4_t<T> sx[kStage ? slab_cap<T>() + kRunPad : 1];
+  // rows kNbrCap + 1 .. kNbrCap + 8 take the writes of a lane past its cap
+  uint16_t lst[kNbrCap + 9][kBlock];
+  BlockRanges sR;
+};
+
+template <class T, bool kWithSource, bool kStage>
+__device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrList &L,
+                                             vec4_t<T> *vout, unsigned lb,
+                                             SetupShared<T, kStage> &sh) {
+  constexpr uint32_t kCap = slab_cap<T>();
+  auto &sx = sh.sx;
+  auto &lst = sh.lst;
+  BlockRanges &sR = sh.sR;
+  const unsigned t = threadIdx.x;
+  const int i = static_cast<int>(lb * kBlock + t);
+  const bool valid = i < S.nf;
+  const uint32_t cell = valid ? S.fcell[i] : 0u;
+  block_spans(S.grid, S.fstart, valid, cell, sR);
+  if (t < 6)
+    reinterpret_cast<uint32_t *>(L.blk + lb)[t] = t < 3 ? sR.base[t] : sR.len[t - 3];
+  const Spans R = Spans::of(sR);
+  const uint32_t smax = R.max_len();
+  const bool staged = kStage && smax <= kCap;
+  const bool encodable = smax <= 0x10000u;
+
+  const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  const vec4_t<T> xi = valid ? S.xm[i] : zero4;
+  const vec4_t<T> vi = valid ? S.v[i] : zero4;
+  SetupSums<T, kWithSource> q(S, xi, vi);
+  q.rho = q.self();
   uint32_t cnt = 0;
   uint32_t cs[3] = {0u, 0u, 0u};  // entries per slab
   // candidate test of the slab-s runs, positions from global memory
@@ -405,7 +479,7 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
 #pragma unroll 4
           for (uint32_t e = c0; e < cnt; ++e) {
             const uint32_t u = lst[e][t];
-            pair(sx[u], base + u);
+            q.pair(sx[u], q.load_v(base + u));
           }
         }
       }
@@ -434,100 +508,49 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
         for (int k = 0; k < 4; ++k) {
           const uint32_t j = slot(e + k);
           px[k] = S.xm[j];
-          pv[k] = load_v(j);
+          pv[k] = q.load_v(j);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-          pair2(px[k], pv[k]);
+          q.pair(px[k], pv[k]);
       }
       for (; e < cnt; ++e) {
         const uint32_t j = slot(e);
-        pair2(S.xm[j], load_v(j));
+        q.pair(S.xm[j], q.load_v(j));
       }
     }
   }
   // the rest is per particle; with S.first_iter the block then sums the
   // aprde terms of IISPH iteration 1 (every thread takes part)
   auto finish = [&]() -> double {
-  const size_t nn = static_cast<size_t>(S.nf);
-  uint32_t info;
-  if (over) {
-    // more neighbours than the list holds: all pair sums again over the grid
-    rho = xi.w * K.aw * T(4);
-    gf0 = gf1 = gf2 = s2 = dsum = T(0);
-    grid_walk(S, i, xi, [&](uint32_t j) { pair(S.xm[j], j); });
-    info = kListOverflow;
-  } else {
-    // chunks of 8 entries, one 16-byte store per lane (1 KB per wavefront)
-    for (uint32_t g = 0; g * kChunk < cnt; ++g) {
-      uint32_t w[4];
+    const size_t nn = static_cast<size_t>(S.nf);
+    uint32_t info;
+    if (over) {
+      // more neighbours than the list holds: all pair sums again over the grid
+      q.rho = q.self();
+      q.gf0 = q.gf1 = q.gf2 = q.s2 = q.dsum = T(0);
+      grid_walk(S, i, xi, [&](uint32_t j) { q.pair(S.xm[j], q.load_v(j)); });
+      info = kListOverflow;
+    } else {
+      // chunks of 8 entries, one 16-byte store per lane (1 KB per wavefront)
+      for (uint32_t g = 0; g * kChunk < cnt; ++g) {
+        uint32_t w[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t e0 = g * kChunk + 2 * k;
-        const uint32_t lo = e0 < cnt ? lst[e0][t] : 0u;
-        const uint32_t hi = e0 + 1 < cnt ? lst[e0 + 1][t] : 0u;
-        w[k] = lo | (hi << 16);
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t e0 = g * kChunk + 2 * k;
+          const uint32_t lo = e0 < cnt ? lst[e0][t] : 0u;
+          const uint32_t hi = e0 + 1 < cnt ? lst[e0 + 1][t] : 0u;
+          w[k] = lo | (hi << 16);
+        }
+        reinterpret_cast<uint4 *>(L.idx)[static_cast<size_t>(g) * nn + static_cast<size_t>(i)] =
+            make_uint4(w[0], w[1], w[2], w[3]);
       }
-      reinterpret_cast<uint4 *>(L.idx)[static_cast<size_t>(g) * nn + static_cast<size_t>(i)] =
-          make_uint4(w[0], w[1], w[2], w[3]);
+      info = cs[0] | (cs[1] << 8) | (cs[2] << 16);
     }
-    info = cs[0] | (cs[1] << 8) | (cs[2] << 16);
-  }
-  L.info[i] = info;
-  T rhob = 0, gb0 = 0, gb1 = 0, gb2 = 0;
-  runs(S.grid, cell, S.bstart, [&](uint32_t b, uint32_t e) {
-    for (uint32_t j = b; j < e; j += 4) {
-      vec4_t<T> pk[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        pk[u] = S.bxV[min(j + u, e - 1)];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const vec4_t<T> pj = pk[u];
-        const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
-        const T r2 = sqdist_exact(d0, d1, d2);
-        if (j + u >= e || !(r2 < S.thr2))
-          continue;
-        T w, f;
-        K.eval(r2, w, f);
-        rhob += pj.w * w;
-        gb0 += pj.w * (f * d0);
-        gb1 += pj.w * (f * d1);
-        gb2 += pj.w * (f * d2);
-      }
-    }
-  });
-  const T rho0 = S.rho0;
-  rho += rho0 * rhob;
-  const T irho = T(1) / rho;
-  const T irho2 = irho * irho;
-  const T k14 = T(1.4) * rho0;
-  const T c0 = -(gf0 + k14 * gb0) * irho2;
-  const T c1 = -(gf1 + k14 * gb1) * irho2;
-  const T c2 = -(gf2 + k14 * gb2) * irho2;
-  const T gs0 = gf0 + rho0 * gb0, gs1 = gf1 + rho0 * gb1, gs2 = gf2 + rho0 * gb2;
-  const T fac = S.dt * S.dt * rho0 * irho;
-  const T AA = fac * ((c0 * gs0 + c1 * gs1 + c2 * gs2) - xi.w * irho2 * s2);
-  S.rho[i] = rho;
-  S.c[i] = make4<vec4_t<T>>(c0, c1, c2, T(0));
-  S.G[i] = make4<vec4_t<T>>(gs0, gs1, gs2, T(0));
-  S.AA[i] = AA;
-  S.p[i] = T(0);
-  S.pr[i] = T(0);
-  S.xq[i] = make4<vec4_t<T>>(xi.x, xi.y, xi.z, T(0));
-  S.xa[S.xa_x(static_cast<size_t>(i))] = xi;
-  if (kWithSource) {
-    const T src = (rho0 - rho) -
-                  S.dt * rho0 * irho * (dsum + rho0 * (vs0 * gb0 + vs1 * gb1 + vs2 * gb2));
-    S.s[i] = src;
-    vout[i] = make4<vec4_t<T>>(vs0, vs1, vs2, vi.w);
-    if (S.first_iter)
-      return first_iteration(S, i, xi, rho, src, AA);
-  } else {
-    S.vd[i] = make4<vec4_t<T>>(gb0, gb1, gb2, T(0));  // G_b for the source pass
-  }
-  return 0.0;
+    runs(S.grid, cell, S.bstart, [&](uint32_t b, uint32_t e) { q.boundary(b, e); });
+    L.info[i] = info | (q.near_boundary && !over ? kListBoundary : 0u);
+    return q.finish(i, vi.w, vout);
   };
   const double term = valid ? finish() : 0.0;
   if (kWithSource && S.first_iter) {
@@ -537,43 +560,177 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
   }
 }
 
-template <class T, bool kWithSource, bool kStage>
-__global__ __launch_bounds__(kBlock) void k_setup(SceneView<T> S, NbrList L,
-                                                  vec4_t<T> *vout, SolveBegin B) {
-  k_setup_body<T, kWithSource, kStage>(S, L, vout, xcd_block(blockIdx.x, gridDim.x));
+// The setup pass with 8 lanes per particle (scenes of up to kSplitMax
+// particles, which do not fill the chip with one): the lanes share the
+// candidates (scan8), the accepted neighbours and the boundary runs, and their
+// sums are added in a fixed tree. Bound by its chain of dependent loads: run
+// bounds, candidates of three slabs, neighbours. Measured, one lane -> eight:
+// 2,048 particles 42 -> 12.5 us, 8,000: 42 -> 13.1, 59,000: 41 -> 27, 125,000:
+// 50 -> 46, 250,000: 78 -> 82, 1M: 230 -> 294 (the lanes' idle slots cost more
+// than the shorter chain gives).
+template <class T, bool kWithSource>
+__device__ __forceinline__ void k_setup8_body(const SceneView<T> &S, const NbrList &L,
+                                              vec4_t<T> *vout, unsigned lb,
+                                              Scan8Shared &sh) {
+  const unsigned sub = threadIdx.x % kScanLanes, p = threadIdx.x / kScanLanes;
+  const int i = static_cast<int>(lb * kScanParts + p);
+  const bool valid = i < S.nf;
+  const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  const vec4_t<T> xi = valid ? S.xm[i] : zero4;
+  const vec4_t<T> vi = valid ? S.v[i] : zero4;
+  const uint32_t cell = valid ? S.fcell[i] : 0u;
+  const Scan8 c = scan8<T, false>(S, L, lb, sh, i, valid, cell, xi);
+  SetupSums<T, kWithSource> q(S, xi, vi);
+  if (valid && !c.over) {
+    const Spans R = Spans::of(sh.R);
+    const uint32_t c0 = c.cs0, c01 = c.cs0 + c.cs1;
+    const uint32_t d1 = R.b1 - R.b0, d2 = R.b2 - R.b1;
+    for (uint32_t e0 = sub; e0 < c.cnt; e0 += 4u * kScanLanes) {
+      vec4_t<T> px[4], pv[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t e = e0 + static_cast<uint32_t>(k) * kScanLanes;
+        if (e < c.cnt) {
+          const uint32_t j =
+              R.b0 + sh.lst[p][e] + (e >= c0 ? d1 : 0u) + (e >= c01 ? d2 : 0u);
+          px[k] = S.xm[j];
+          pv[k] = q.load_v(j);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (e0 + static_cast<uint32_t>(k) * kScanLanes < c.cnt)
+          q.pair(px[k], pv[k]);
+    }
+  } else if (valid && sub == 0) {
+    grid_walk(S, i, xi, [&](uint32_t j) { q.pair(S.xm[j], q.load_v(j)); });
+  }
+  if (valid && S.nb > 0) {
+    uint32_t b, e;
+    run_bounds(S.grid, cell, S.bstart, static_cast<int>(sub), &b, &e);
+    q.boundary(b, e);
+    if (sub == 0) {
+      run_bounds(S.grid, cell, S.bstart, 8, &b, &e);
+      q.boundary(b, e);
+    }
+  }
+  for (T *v : {&q.rho, &q.gf0, &q.gf1, &q.gf2, &q.s2, &q.rhob, &q.gb0, &q.gb1, &q.gb2})
+    *v = lanes_sum<kScanLanes>(*v);
+  if (kWithSource)
+    q.dsum = lanes_sum<kScanLanes>(q.dsum);
+  const uint64_t near = __ballot(q.near_boundary) >> ((threadIdx.x % kWave) & ~7u);
+  double term = 0.0;
+  if (valid) {
+    scan8_write(L, sh, static_cast<size_t>(S.nf), i, c, (near & 0xFFu) != 0u);
+    if (sub == 0) {
+      q.rho += q.self();
+      term = q.finish(i, vi.w, vout);
+    }
+  }
+  if (kWithSource && S.first_iter) {
+    const double bs = particle_sum<kScanLanes>(term);
+    if (threadIdx.x == 0)
+      S.partials[lb] = bs;
+  }
+}
+
+template <class T, bool kWithSource>
+__global__ __launch_bounds__(kBlock) void k_setup8(SceneView<T> S, NbrList L, vec4_t<T> *vout,
+                                                   SolveBegin B) {
+  __shared__ Scan8Shared sh;
+  k_setup8_body<T, kWithSource>(S, L, vout, xcd_block(blockIdx.x, gridDim.x), sh);
   // no thread of the setup reads the control block
   if (B.seq != 0u && blockIdx.x == 0 && threadIdx.x == 0)
     begin_solve(S.ctl, B);
 }
 
+template <class T, bool kWithSource, bool kStage>
+__global__ __launch_bounds__(kBlock) void k_setup(SceneView<T> S, NbrList L,
+                                                  vec4_t<T> *vout, SolveBegin B) {
+  __shared__ SetupShared<T, kStage> sh;
+  k_setup_body<T, kWithSource, kStage>(S, L, vout, xcd_block(blockIdx.x, gridDim.x), sh);
+  // no thread of the setup reads the control block
+  if (B.seq != 0u && blockIdx.x == 0 && threadIdx.x == 0)
+    begin_solve(S.ctl, B);
+}
+
+// does run r of particle i's boundary cells hold a particle within the radius
+template <class T>
+__device__ __forceinline__ bool boundary_in_run(const SceneView<T> &S, uint32_t cell,
+                                                const vec4_t<T> &xi, int r) {
+  uint32_t b, e;
+  run_bounds(S.grid, cell, S.bstart, r, &b, &e);
+  bool any = false;
+  for (uint32_t j = b; j < e; ++j) {
+    const vec4_t<T> pj = S.bxV[j];
+    any = any || sqdist_exact(xi.x - pj.x, xi.y - pj.y, xi.z - pj.z) < S.thr2;
+  }
+  return any;
+}
+
+// The list of the procedures (8 lanes per particle). A procedure that walks
+// it visits the particles of a grid walk in the same order, without the
+// seven eighths of the candidates that the predicate rejects. Bound by the
+// vector issue of the tests and appends.
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_build_list(SceneView<T> S, NbrList L) {
+  __shared__ Scan8Shared sh;
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>(lb * kScanParts + threadIdx.x / kScanLanes);
+  const unsigned sub = threadIdx.x % kScanLanes;
+  const bool valid = i < S.nf;
+  const vec4_t<T> xi =
+      valid ? S.xm[i] : make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  const uint32_t cell = valid ? S.fcell[i] : 0u;
+  const Scan8 c = scan8<T, true>(S, L, lb, sh, i, valid, cell, xi);
+  bool near = false;
+  if (valid && S.nb > 0)
+    near = boundary_in_run(S, cell, xi, static_cast<int>(sub)) ||
+           (sub == 0 && boundary_in_run(S, cell, xi, 8));
+  const uint64_t m = __ballot(near) >> ((threadIdx.x % kWave) & ~7u);
+  if (valid)
+    scan8_write(L, sh, static_cast<size_t>(S.nf), i, c, (m & 0xFFu) != 0u);
+}
+
 // explicit viscosity (viscosity.hpp:171-240) over the list, then
 // v* = v + dt (g + a_visc) H   (gravity.hpp:133, symplectic_euler.hpp:172-200)
-template <class T>
+template <class T, int kLanes>
 __device__ __forceinline__ void k_viscosity_list_body(const SceneView<T> &S, const NbrList &L,
                                                       vec4_t<T> *vout, unsigned lb) {
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
-  if (i >= S.nf)
-    return;
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
+  const bool valid = i < S.nf;
   const FastSpline<T> K = fast_spline(S);
-  const vec4_t<T> xi = S.xm[i], vi = S.v[i];
-  const T rhoi = S.rho[i];
+  const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  const vec4_t<T> xi = valid ? S.xm[i] : zero4, vi = valid ? S.v[i] : zero4;
+  const T rhoi = valid ? S.rho[i] : T(1);
+  const uint32_t info = valid ? L.info[i] : 0u;
   const T cf = T(10) * S.mu_f / rhoi;
   T a0 = 0, a1 = 0, a2 = 0;
-  auto pair = [&](uint32_t j) {
-    const vec4_t<T> pj = S.xm[j];
+  struct Rec {
+    vec4_t<T> x, v;
+    T rho;
+  };
+  auto pair = [&](const Rec &q) {
+    const vec4_t<T> &pj = q.x, &vj = q.v;
     const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
     const T r2 = d0 * d0 + d1 * d1 + d2 * d2;
-    const vec4_t<T> vj = S.v[j];
-    const T s = cf * (pj.w / S.rho[j]) *
+    const T s = cf * (pj.w / q.rho) *
                 ((vi.x - vj.x) * d0 + (vi.y - vj.y) * d1 + (vi.z - vj.z) * d2) /
                 (r2 + S.hh001) * K.gradf(r2);
     a0 += s * d0;
     a1 += s * d1;
     a2 += s * d2;
   };
-  walk(S, L, i, xi, pair);
+  auto load = [&](uint32_t j) { return Rec{S.xm[j], S.v[j], S.rho[j]}; };
+  if (valid && !(info & kListOverflow))
+    list_gather_lanes<kLanes, 4>(L, pass_spans<kLanes>(L, S.nf, lb), static_cast<size_t>(S.nf), i, info, sub,
+                                 load, pair);
+  else if (valid && sub == 0)
+    grid_walk(S, i, xi, [&](uint32_t j) { pair(load(j)); });
   const T cb = T(10) * S.mu_b / rhoi * S.rho0 / rhoi;
-  runs(S.grid, S.fcell[i], S.bstart, [&](uint32_t b, uint32_t e) {
+  auto wall = [&](uint32_t b, uint32_t e) {
     for (uint32_t j = b; j < e; ++j) {
       const vec4_t<T> pj = S.bxV[j];
       const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
@@ -587,7 +744,23 @@ __device__ __forceinline__ void k_viscosity_list_body(const SceneView<T> &S, con
       a1 += s * d1;
       a2 += s * d2;
     }
-  });
+  };
+  if (list_has_boundary(info)) {
+    if (kLanes == 1) {
+      runs(S.grid, S.fcell[i], S.bstart, wall);
+    } else {
+      for (uint32_t r = sub; r < 9u; r += kLanes) {
+        uint32_t b, e;
+        run_bounds(S.grid, S.fcell[i], S.bstart, static_cast<int>(r), &b, &e);
+        wall(b, e);
+      }
+    }
+  }
+  a0 = lanes_sum<kLanes>(a0);
+  a1 = lanes_sum<kLanes>(a1);
+  a2 = lanes_sum<kLanes>(a2);
+  if (!valid || sub != 0)
+    return;
   const T H = fade_step(S, vi.w);
   T g0, g1, g2;
   step_gravity(S, xi.x, xi.y, xi.z, g0, g1, g2);
@@ -595,10 +768,10 @@ __device__ __forceinline__ void k_viscosity_list_body(const SceneView<T> &S, con
                              vi.z + S.dt * (g2 + a2) * H, vi.w);
 }
 
-template <class T>
+template <class T, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_viscosity_list(SceneView<T> S, NbrList L,
                                                            vec4_t<T> *vout) {
-  k_viscosity_list_body(S, L, vout, xcd_block(blockIdx.x, gridDim.x));
+  k_viscosity_list_body<T, kLanes>(S, L, vout, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // v* = v + dt a_axial(x) H (gravity.hpp:189-215, symplectic_euler.hpp:172-200)
@@ -623,24 +796,36 @@ __global__ __launch_bounds__(kBlock) void k_gravity_v(SceneView<T> S, vec4_t<T> 
 }
 
 // source term s from the integrated velocities (explicit-viscosity path)
-template <class T>
+template <class T, int kLanes>
 __device__ __forceinline__ void k_source_list_body(const SceneView<T> &S, const NbrList &L,
                                                    unsigned lb) {
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
+  const bool valid = i < S.nf;
+  const FastSpline<T> K = fast_spline(S);
+  const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  const vec4_t<T> xi = valid ? S.xm[i] : zero4, vi = valid ? S.v[i] : zero4;
+  const vec4_t<T> gb = valid ? S.vd[i] : zero4;
+  const uint32_t info = valid ? L.info[i] : 0u;
+  T dsum = 0;
+  struct Rec {
+    vec4_t<T> x, v;
+  };
+  auto pair = [&](const Rec &q) {
+    const T d0 = xi.x - q.x.x, d1 = xi.y - q.x.y, d2 = xi.z - q.x.z;
+    const T f = K.gradf(d0 * d0 + d1 * d1 + d2 * d2);
+    dsum += q.x.w * f * ((vi.x - q.v.x) * d0 + (vi.y - q.v.y) * d1 + (vi.z - q.v.z) * d2);
+  };
+  auto load = [&](uint32_t j) { return Rec{S.xm[j], S.v[j]}; };
+  if (valid && !(info & kListOverflow))
+    list_gather_lanes<kLanes, 4>(L, pass_spans<kLanes>(L, S.nf, lb), static_cast<size_t>(S.nf), i, info, sub,
+                                 load, pair);
+  else if (valid && sub == 0)
+    grid_walk(S, i, xi, [&](uint32_t j) { pair(load(j)); });
+  dsum = lanes_sum<kLanes>(dsum);
   double term = 0.0;
-  if (i < S.nf) {
-    const FastSpline<T> K = fast_spline(S);
-    const vec4_t<T> xi = S.xm[i], vi = S.v[i], gb = S.vd[i];
+  if (valid && sub == 0) {
     const T rhoi = S.rho[i];
-    T dsum = 0;
-    auto pair = [&](uint32_t j) {
-      const vec4_t<T> pj = S.xm[j];
-      const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
-      const T f = K.gradf(d0 * d0 + d1 * d1 + d2 * d2);
-      const vec4_t<T> vj = S.v[j];
-      dsum += pj.w * f * ((vi.x - vj.x) * d0 + (vi.y - vj.y) * d1 + (vi.z - vj.z) * d2);
-    };
-    walk(S, L, i, xi, pair);
     const T rho0 = S.rho0;
     const T src = (rho0 - rhoi) -
                   S.dt * rho0 / rhoi * (dsum + rho0 * (vi.x * gb.x + vi.y * gb.y + vi.z * gb.z));
@@ -649,15 +834,15 @@ __device__ __forceinline__ void k_source_list_body(const SceneView<T> &S, const 
       term = first_iteration(S, i, xi, rhoi, src, S.AA[i]);
   }
   if (S.first_iter) {  // IISPH iteration 1: the block's aprde partial
-    const double bs = block_sum<kBlock>(term);
+    const double bs = particle_sum<kLanes>(term);
     if (threadIdx.x == 0)
       S.partials[lb] = bs;
   }
 }
 
-template <class T>
+template <class T, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_source_list(SceneView<T> S, NbrList L) {
-  k_source_list_body(S, L, xcd_block(blockIdx.x, gridDim.x));
+  k_source_list_body<T, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Walk of the list entries of particle i (all threads of the block call it).
@@ -665,11 +850,11 @@ __global__ __launch_bounds__(kBlock) void k_source_list(SceneView<T> S, NbrList 
 // then use(lds(u)) for the neighbour at LDS index u. Otherwise
 // use(load(j)) over the whole list with global slots, a chunk of 8 gathers
 // in flight.
-template <bool kStage, uint32_t kCap, int kGroup = 8, class Stage, class Lds, class Load,
-          class Use>
+template <bool kStage, uint32_t kCap, int kLanes, int kGroup = 8, class Stage, class Lds,
+          class Load, class Use>
 __device__ __forceinline__ void list_walk(const NbrList &L, const Spans &R, size_t n, int i,
-                                          uint32_t info, Stage &&stage, Lds &&lds, Load &&load,
-                                          Use &&use) {
+                                          uint32_t info, uint32_t sub, Stage &&stage, Lds &&lds,
+                                          Load &&load, Use &&use) {
   const uint32_t live = (info & kListOverflow) ? 0u : info;
   if (kStage && R.max_len() <= kCap) {
     uint32_t e = 0;
@@ -693,21 +878,22 @@ __device__ __forceinline__ void list_walk(const NbrList &L, const Spans &R, size
       e += c;
     }
   } else {
-    list_gather<kGroup>(L, R, n, i, live, load, use);
+    list_gather_lanes<kLanes, kGroup>(L, R, n, i, live, sub, load, use);
   }
 }
 
 // IISPH pressure acceleration over the list: a_i = p_i c_i - sum m_j pr_j gradW
-template <class T, bool kStage>
+template <class T, bool kStage, int kLanes>
 __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const NbrList &L,
                                                   unsigned lb) {
   if (S.ctl->done)
     return;
   constexpr uint32_t kCap = slab_cap<T>();
   __shared__ vec4_t<T> sq[kStage ? kCap : 1];
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
   const bool valid = i < S.nf;
-  const Spans R = Spans::of(L.blk[lb]);
+  const Spans R = pass_spans<kLanes>(L, S.nf, lb);
   const FastSpline<T> K = fast_spline(S);
   const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
   const vec4_t<T> xi = valid ? S.xm[i] : zero4;
@@ -723,27 +909,30 @@ __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const N
     a1 += s * d1;
     a2 += s * d2;
   };
-  list_walk<kStage, kCap>(
-      L, R, static_cast<size_t>(S.nf), i, info, [&](int s) { stage_span(R, s, S.xq, sq); },
+  list_walk<kStage, kCap, kLanes>(
+      L, R, static_cast<size_t>(S.nf), i, info, sub, [&](int s) { stage_span(R, s, S.xq, sq); },
       [&](uint32_t u) { return sq[u]; }, [&](uint32_t j) { return S.xq[j]; }, pair);
-  if (!valid)
-    return;
-  if (info & kListOverflow)
+  if (valid && sub == 0 && (info & kListOverflow))
     grid_walk(S, i, xi, [&](uint32_t j) { pair(S.xq[j]); });
+  a0 = lanes_sum<kLanes>(a0);
+  a1 = lanes_sum<kLanes>(a1);
+  a2 = lanes_sum<kLanes>(a2);
+  if (!valid || sub != 0)
+    return;
   const vec4_t<T> ai = make4<vec4_t<T>>(pi * ci.x - K.ag3 * a0, pi * ci.y - K.ag3 * a1,
                                         pi * ci.z - K.ag3 * a2, T(0));
   // the pressure pass gathers it from here; the integration copies it to a
   S.xa[S.xa_a(static_cast<size_t>(i))] = ai;
 }
 
-template <class T, bool kStage>
+template <class T, bool kStage, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_accel_list(SceneView<T> S, NbrList L) {
-  k_accel_list_body<T, kStage>(S, L, xcd_block(blockIdx.x, gridDim.x));
+  k_accel_list_body<T, kStage, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // IISPH relaxed Jacobi update over the list, FP64 aprde reduction and the
 // device-side convergence decision (example.lua:409-421)
-template <class T, bool kStage>
+template <class T, bool kStage, int kLanes>
 __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, const NbrList &L,
                                                      unsigned lb) {
   if (S.ctl->done)
@@ -754,9 +943,10 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
   };
   __shared__ vec4_t<T> sx[kStage ? kCap : 1];
   __shared__ vec4_t<T> sa[kStage ? kCap : 1];
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
   const bool valid = i < S.nf;
-  const Spans R = Spans::of(L.blk[lb]);
+  const Spans R = pass_spans<kLanes>(L, S.nf, lb);
   const FastSpline<T> K = fast_spline(S);
   const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
   const vec4_t<T> xi = valid ? S.xm[i] : zero4;
@@ -772,8 +962,8 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
     sum += q.x.w * K.gradf_unscaled(d0 * d0 + d1 * d1 + d2 * d2) *
            (q.a.x * d0 + q.a.y * d1 + q.a.z * d2);
   };
-  list_walk<kStage, kCap, 4>(
-      L, R, static_cast<size_t>(S.nf), i, info,
+  list_walk<kStage, kCap, kLanes, 4>(
+      L, R, static_cast<size_t>(S.nf), i, info, sub,
       [&](int s) {
         stage_span(R, s, S.xm, sx);
         stage_span_fn(R, s, [&](size_t g) { return S.xa[S.xa_a(g)]; }, sa);
@@ -781,12 +971,13 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
       [&](uint32_t u) { return XA{sx[u], sa[u]}; },
       [&](uint32_t j) { return XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]}; },
       pair);
+  if (valid && sub == 0 && (info & kListOverflow))
+    grid_walk(S, i, xi, [&](uint32_t j) {
+      pair(XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]});
+    });
+  sum = lanes_sum<kLanes>(sum);
   double term = 0.0;
-  if (valid) {
-    if (info & kListOverflow)
-      grid_walk(S, i, xi, [&](uint32_t j) {
-        pair(XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]});
-      });
+  if (valid && sub == 0) {
     const T Ap = S.dt * S.dt * S.rho0 / rhoi *
                  ((ai.x * gs.x + ai.y * gs.y + ai.z * gs.z) - K.ag3 * sum);
     const T rcp = (fabs(AA) > T(1e-9)) ? T(1) / AA : T(0);
@@ -798,24 +989,32 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
     S.xq[i] = make4<vec4_t<T>>(xi.x, xi.y, xi.z, xi.w * pn / (rhoi * rhoi));
     term = static_cast<double>((Ap - si) / S.rho0 * ((T(1e-9) < pn) ? T(1) : T(0)));
   }
-  const double bs = block_sum<kBlock>(term);
+  const double bs = particle_sum<kLanes>(term);
   if (threadIdx.x == 0)
     S.partials[lb] = bs;
 }
 
-template <class T, bool kStage>
+template <class T, bool kStage, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_pressure_list(SceneView<T> S, NbrList L) {
-  k_pressure_list_body<T, kStage>(S, L, xcd_block(blockIdx.x, gridDim.x));
+  k_pressure_list_body<T, kStage, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Sum of the block partials in block order (FP64, fixed tree) and the
 // convergence decision of example.lua:418-419: stop when it >= min_it and
-// aprde / nprde < tol, or at max_it.
+// aprde / nprde < tol, or at max_it. half: the partials are of half the
+// particles of a list pass's block (k_setup8) and are added in pairs first.
 __device__ __forceinline__ void k_pressure_finalize_body(Ctl *c, const double *partials,
-                                                        unsigned nparts) {
+                                                        unsigned nparts, bool half = false) {
   if (c->done)
     return;
-  const double acc = block_sum<kBlock>(strided_sum<kBlock>(partials, nparts));
+  double part = 0.0;
+  if (half) {
+    for (unsigned k = 2u * threadIdx.x; k < nparts; k += 2u * kBlock)
+      part += partials[k] + (k + 1u < nparts ? partials[k + 1u] : 0.0);
+  } else {
+    part = strided_sum<kBlock>(partials, nparts);
+  }
+  const double acc = block_sum<kBlock>(part);
   if (threadIdx.x == 0) {
     c->aprde = acc;
     const int it = c->iters + 1;
@@ -831,8 +1030,8 @@ __device__ __forceinline__ void k_pressure_finalize_body(Ctl *c, const double *p
 }
 
 __global__ __launch_bounds__(kBlock) void k_pressure_finalize(Ctl *c, const double *partials,
-                                                              unsigned nparts) {
-  k_pressure_finalize_body(c, partials, nparts);
+                                                              unsigned nparts, bool half) {
+  k_pressure_finalize_body(c, partials, nparts, half);
 }
 
 template <class T>
@@ -908,79 +1107,102 @@ __global__ __launch_bounds__(kBlock) void k_speed_finalize(Ctl *c, const double 
   k_speed_finalize_body<T>(c, partials, nparts, seq);
 }
 
-// ---- batched wrappers (prtcl_hip_step over several scenes)
+// ---- batched wrappers (prtcl_hip_step over several scenes): the setup and list
+// passes take the body that the block's scene takes alone (split_scene)
+// the two setup bodies share their LDS, so the large scenes' blocks keep
+// their five per CU
 template <class T, bool kStage>
-__global__ __launch_bounds__(kBlock) void k_setup_b(const BatchEntry<T> *tab,
-                                                    const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  k_setup_body<T, true, kStage>(E.S, NbrList{E.nidx, E.ninfo, E.nblk}, E.vtmp,
-                                u & kBatchLocalMask);
+union SetupPool {
+  SetupShared<T, kStage> setup;
+  Scan8Shared scan;
+};
+
+// this block's entry E, list L and local block lb in the units of its pass (kF
+// blocks for each block of a split scene); returns from the kernel for a block
+// past the scene's particles
+#define BATCH_PASS_ENTRY(kF, total)                                                       \
+  unsigned part;                                                                          \
+  const uint32_t u = batch_block(B, kF, &part);                                           \
+  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];                                     \
+  const bool split = split_scene(E.S.nf);                                                 \
+  const unsigned lb = (u & kBatchLocalMask) * (split ? (kF) : 1u) + part;                 \
+  if (lb >= total(E.S.nf))                                                                \
+    return;                                                                               \
+  const NbrList L{E.nidx, E.ninfo, E.nblk, E.nshift}
+
+constexpr unsigned kSetupParts = kBlock / kScanParts;  // setup blocks per block of a split scene
+constexpr unsigned kListParts = kListLanes;
+
+template <class T, bool kWithSource, bool kStage>
+__global__ __launch_bounds__(kBlock) void k_setup_b(const BatchEntry<T> *tab, BatchBlocks B) {
+  __shared__ SetupPool<T, kStage> sh;
+  BATCH_PASS_ENTRY(kSetupParts, setup_blocks);
+  if (split)
+    k_setup8_body<T, kWithSource>(E.S, L, E.vtmp, lb, sh.scan);
+  else
+    k_setup_body<T, kWithSource, kStage>(E.S, L, E.vtmp, lb, sh.setup);
 }
 
-// scenes with explicit viscosity or axial gravity: the setup without the
-// source term, then v* (explicit viscosity and gravity, or the axial gravity
+// scenes with explicit viscosity or axial gravity: after the setup without the
+// source term, v* (explicit viscosity and gravity, or the axial gravity
 // alone) into vtmp, then the source term and iteration 1 from v* (the three
 // launches of FusedOps::setup for such a scene)
-template <class T, bool kStage>
-__global__ __launch_bounds__(kBlock) void k_setup_nosrc_b(const BatchEntry<T> *tab,
-                                                          const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  k_setup_body<T, false, kStage>(E.S, NbrList{E.nidx, E.ninfo, E.nblk}, E.vtmp,
-                                 u & kBatchLocalMask);
-}
-
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_vstar_b(const BatchEntry<T> *tab,
-                                                    const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  if (E.explicit_visc)
-    k_viscosity_list_body(E.S, NbrList{E.nidx, E.ninfo, E.nblk}, E.vtmp, u & kBatchLocalMask);
+__global__ __launch_bounds__(kBlock) void k_vstar_b(const BatchEntry<T> *tab, BatchBlocks B) {
+  BATCH_PASS_ENTRY(kListParts, list_blocks);
+  if (!E.explicit_visc)
+    k_gravity_v_body(E.S, E.vtmp, lb);  // blocks past the particles find none
+  else if (split)
+    k_viscosity_list_body<T, kListLanes>(E.S, L, E.vtmp, lb);
   else
-    k_gravity_v_body(E.S, E.vtmp, u & kBatchLocalMask);
+    k_viscosity_list_body<T, 1>(E.S, L, E.vtmp, lb);
 }
 
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_source_b(const BatchEntry<T> *tab,
-                                                     const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
+__global__ __launch_bounds__(kBlock) void k_source_b(const BatchEntry<T> *tab, BatchBlocks B) {
+  BATCH_PASS_ENTRY(kListParts, list_blocks);
   SceneView<T> S2 = E.S;
   S2.v = E.vtmp;  // the integrated velocities
-  k_source_list_body(S2, NbrList{E.nidx, E.ninfo, E.nblk}, u & kBatchLocalMask);
+  if (split)
+    k_source_list_body<T, kListLanes>(S2, L, lb);
+  else
+    k_source_list_body<T, 1>(S2, L, lb);
 }
 
 template <class T, bool kStage>
-__global__ __launch_bounds__(kBlock) void k_accel_b(const BatchEntry<T> *tab,
-                                                    const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  k_accel_list_body<T, kStage>(E.S, NbrList{E.nidx, E.ninfo, E.nblk}, u & kBatchLocalMask);
+__global__ __launch_bounds__(kBlock) void k_accel_b(const BatchEntry<T> *tab, BatchBlocks B) {
+  BATCH_PASS_ENTRY(kListParts, list_blocks);
+  if (split)
+    k_accel_list_body<T, false, kListLanes>(E.S, L, lb);
+  else
+    k_accel_list_body<T, kStage, 1>(E.S, L, lb);
 }
 
 template <class T, bool kStage>
-__global__ __launch_bounds__(kBlock) void k_pressure_b(const BatchEntry<T> *tab,
-                                                       const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  k_pressure_list_body<T, kStage>(E.S, NbrList{E.nidx, E.ninfo, E.nblk}, u & kBatchLocalMask);
+__global__ __launch_bounds__(kBlock) void k_pressure_b(const BatchEntry<T> *tab, BatchBlocks B) {
+  BATCH_PASS_ENTRY(kListParts, list_blocks);
+  if (split)
+    k_pressure_list_body<T, false, kListLanes>(E.S, L, lb);
+  else
+    k_pressure_list_body<T, kStage, 1>(E.S, L, lb);
 }
 
 // one block per scene
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_pressure_finalize_b(const BatchEntry<T> *tab) {
   const BatchEntry<T> &E = tab[blockIdx.x];
-  k_pressure_finalize_body(E.S.ctl, E.S.partials, E.nblocks);
+  k_pressure_finalize_body(E.S.ctl, E.S.partials, list_blocks(E.S.nf));
 }
 
 // iteration 1's convergence step for the scenes whose solve it could end
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_first_finalize_b(const BatchEntry<T> *tab) {
   const BatchEntry<T> &E = tab[blockIdx.x];
+  // partials of the setup, or of the source pass of the three-launch setup
   if (!E.first_preset)
-    k_pressure_finalize_body(E.S.ctl, E.S.partials, E.nblocks);
+    k_pressure_finalize_body(E.S.ctl, E.S.partials,
+                             E.split_setup ? list_blocks(E.S.nf) : setup_blocks(E.S.nf),
+                             !E.split_setup && split_scene(E.S.nf));
 }
 
 // guarded: each scene's integration only once its solve (E.seq) is done;
@@ -988,7 +1210,7 @@ __global__ __launch_bounds__(kBlock) void k_first_finalize_b(const BatchEntry<T>
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_integrate_b(const BatchEntry<T> *tab,
                                                         const uint32_t *pmap, int guarded) {
-  const uint32_t u = pmap[blockIdx.x];
+  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   if (E.viscous)
     return;
@@ -1007,57 +1229,81 @@ __global__ __launch_bounds__(kBlock) void k_speed_finalize_b(const BatchEntry<T>
 }  // namespace
 
 template <class T>
+void FusedOps<T>::build_list(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
+  if (S.nf > 0)
+    hipLaunchKernelGGL(k_build_list<T>, dim3(grid_blocks(S.nf, kScanParts)), dim3(kBlock), 0, st,
+                       S, L);
+}
+
+template <class T>
 void FusedOps<T>::setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
                         bool explicit_viscosity, vec4_t<T> *vtmp, bool lds,
                         const SolveBegin &B) {
   if (S.nf <= 0)
     return;
-  const dim3 gr(grid_blocks(S.nf)), bl(kBlock);
+  const dim3 gr(setup_blocks(S.nf)), bl(kBlock);
+  const bool split = split_scene(S.nf);
   // the one-pass setup folds a uniform g into every neighbour's velocity;
   // explicit viscosity or a position-dependent (axial) gravity need the
   // integrated velocities first
   if (!explicit_viscosity && !S.axial) {
-    if (lds)
+    if (split)
+      hipLaunchKernelGGL((k_setup8<T, true>), gr, bl, 0, st, S, L, vtmp, B);
+    else if (lds)
       hipLaunchKernelGGL((k_setup<T, true, true>), gr, bl, 0, st, S, L, vtmp, B);
     else
       hipLaunchKernelGGL((k_setup<T, true, false>), gr, bl, 0, st, S, L, vtmp, B);
     return;
   }
-  if (lds)
+  if (split)
+    hipLaunchKernelGGL((k_setup8<T, false>), gr, bl, 0, st, S, L, vtmp, B);
+  else if (lds)
     hipLaunchKernelGGL((k_setup<T, false, true>), gr, bl, 0, st, S, L, vtmp, B);
   else
     hipLaunchKernelGGL((k_setup<T, false, false>), gr, bl, 0, st, S, L, vtmp, B);
-  if (explicit_viscosity)
-    hipLaunchKernelGGL(k_viscosity_list<T>, gr, bl, 0, st, S, L, vtmp);
+  const dim3 gl(list_blocks(S.nf));
+  if (!explicit_viscosity)
+    hipLaunchKernelGGL(k_gravity_v<T>, dim3(grid_blocks(S.nf)), bl, 0, st, S, vtmp);
+  else if (split)
+    hipLaunchKernelGGL((k_viscosity_list<T, kListLanes>), gl, bl, 0, st, S, L, vtmp);
   else
-    hipLaunchKernelGGL(k_gravity_v<T>, gr, bl, 0, st, S, vtmp);
+    hipLaunchKernelGGL((k_viscosity_list<T, 1>), gl, bl, 0, st, S, L, vtmp);
   // the integrated velocities replace v once every thread has read the old ones
   SceneView<T> S2 = S;
   S2.v = vtmp;
-  hipLaunchKernelGGL(k_source_list<T>, gr, bl, 0, st, S2, L);
+  if (split)
+    hipLaunchKernelGGL((k_source_list<T, kListLanes>), gl, bl, 0, st, S2, L);
+  else
+    hipLaunchKernelGGL((k_source_list<T, 1>), gl, bl, 0, st, S2, L);
 }
 
 template <class T>
 void FusedOps<T>::accel(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool lds) {
   if (S.nf <= 0)
     return;
-  const dim3 gr(grid_blocks(S.nf)), bl(kBlock);
-  if (lds)
-    hipLaunchKernelGGL((k_accel_list<T, true>), gr, bl, 0, st, S, L);
+  const dim3 gr(list_blocks(S.nf)), bl(kBlock);
+  if (split_scene(S.nf))
+    hipLaunchKernelGGL((k_accel_list<T, false, kListLanes>), gr, bl, 0, st, S, L);
+  else if (lds)
+    hipLaunchKernelGGL((k_accel_list<T, true, 1>), gr, bl, 0, st, S, L);
   else
-    hipLaunchKernelGGL((k_accel_list<T, false>), gr, bl, 0, st, S, L);
+    hipLaunchKernelGGL((k_accel_list<T, false, 1>), gr, bl, 0, st, S, L);
 }
 
 template <class T>
 void FusedOps<T>::pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool lds) {
   if (S.nf <= 0)
     return;
-  const unsigned nb = grid_blocks(S.nf);
-  if (lds)
-    hipLaunchKernelGGL((k_pressure_list<T, true>), dim3(nb), dim3(kBlock), 0, st, S, L);
+  const unsigned nb = list_blocks(S.nf);
+  if (split_scene(S.nf))
+    hipLaunchKernelGGL((k_pressure_list<T, false, kListLanes>), dim3(nb), dim3(kBlock), 0, st, S,
+                       L);
+  else if (lds)
+    hipLaunchKernelGGL((k_pressure_list<T, true, 1>), dim3(nb), dim3(kBlock), 0, st, S, L);
   else
-    hipLaunchKernelGGL((k_pressure_list<T, false>), dim3(nb), dim3(kBlock), 0, st, S, L);
-  hipLaunchKernelGGL(k_pressure_finalize, dim3(1), dim3(kBlock), 0, st, S.ctl, S.partials, nb);
+    hipLaunchKernelGGL((k_pressure_list<T, false, 1>), dim3(nb), dim3(kBlock), 0, st, S, L);
+  hipLaunchKernelGGL(k_pressure_finalize, dim3(1), dim3(kBlock), 0, st, S.ctl, S.partials, nb,
+                     false);
 }
 
 // a = the acceleration of the last pressure-acceleration pass
@@ -1069,10 +1315,14 @@ __global__ __launch_bounds__(kBlock) void k_copy_accel(SceneView<T> S) {
 }
 
 template <class T>
-void FusedOps<T>::finish_first_iteration(hipStream_t st, const SceneView<T> &S) {
+void FusedOps<T>::finish_first_iteration(hipStream_t st, const SceneView<T> &S,
+                                         bool explicit_viscosity) {
+  // written by the setup, or by the source pass of the three-launch setup
+  const bool three = explicit_viscosity || S.axial;
   if (S.nf > 0)
     hipLaunchKernelGGL(k_pressure_finalize, dim3(1), dim3(kBlock), 0, st, S.ctl, S.partials,
-                       grid_blocks(S.nf));
+                       three ? list_blocks(S.nf) : setup_blocks(S.nf),
+                       !three && split_scene(S.nf));
 }
 
 template <class T>
@@ -1099,50 +1349,49 @@ void FusedOps<T>::integrate(hipStream_t st, const SceneView<T> &S, unsigned seq)
 }
 
 template <class T>
-void FusedOps<T>::setup_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *pmap,
-                              unsigned npblocks, bool lds) {
-  if (npblocks == 0)
-    return;
-  if (lds)
-    hipLaunchKernelGGL((k_setup_b<T, true>), dim3(npblocks), dim3(kBlock), 0, st, tab, pmap);
-  else
-    hipLaunchKernelGGL((k_setup_b<T, false>), dim3(npblocks), dim3(kBlock), 0, st, tab, pmap);
+void FusedOps<T>::setup_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
+                              bool lds) {
+  const dim3 bl(kBlock);
+  const BatchBlocks B1 = B.group(0), B3 = B.group(1);
+  if (const unsigned n = B1.launch(kSetupParts)) {
+    if (lds)
+      hipLaunchKernelGGL((k_setup_b<T, true, true>), dim3(n), bl, 0, st, tab, B1);
+    else
+      hipLaunchKernelGGL((k_setup_b<T, true, false>), dim3(n), bl, 0, st, tab, B1);
+  }
+  if (const unsigned n = B3.launch(kSetupParts)) {
+    if (lds)
+      hipLaunchKernelGGL((k_setup_b<T, false, true>), dim3(n), bl, 0, st, tab, B3);
+    else
+      hipLaunchKernelGGL((k_setup_b<T, false, false>), dim3(n), bl, 0, st, tab, B3);
+    const dim3 gl(B3.launch(kListParts));
+    hipLaunchKernelGGL(k_vstar_b<T>, gl, bl, 0, st, tab, B3);
+    hipLaunchKernelGGL(k_source_b<T>, gl, bl, 0, st, tab, B3);
+  }
 }
 
 template <class T>
-void FusedOps<T>::setup_split_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                                    unsigned nblocks, bool lds) {
-  if (nblocks == 0)
+void FusedOps<T>::accel_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
+                              bool lds) {
+  const unsigned n = B.launch(kListParts);
+  if (n == 0)
     return;
-  const dim3 gr(nblocks), bl(kBlock);
   if (lds)
-    hipLaunchKernelGGL((k_setup_nosrc_b<T, true>), gr, bl, 0, st, tab, map);
+    hipLaunchKernelGGL((k_accel_b<T, true>), dim3(n), dim3(kBlock), 0, st, tab, B);
   else
-    hipLaunchKernelGGL((k_setup_nosrc_b<T, false>), gr, bl, 0, st, tab, map);
-  hipLaunchKernelGGL(k_vstar_b<T>, gr, bl, 0, st, tab, map);
-  hipLaunchKernelGGL(k_source_b<T>, gr, bl, 0, st, tab, map);
+    hipLaunchKernelGGL((k_accel_b<T, false>), dim3(n), dim3(kBlock), 0, st, tab, B);
 }
 
 template <class T>
-void FusedOps<T>::accel_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *pmap,
-                              unsigned npblocks, bool lds) {
-  if (npblocks == 0)
+void FusedOps<T>::pressure_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
+                                 unsigned nscenes, bool lds) {
+  const unsigned n = B.launch(kListParts);
+  if (n == 0)
     return;
   if (lds)
-    hipLaunchKernelGGL((k_accel_b<T, true>), dim3(npblocks), dim3(kBlock), 0, st, tab, pmap);
+    hipLaunchKernelGGL((k_pressure_b<T, true>), dim3(n), dim3(kBlock), 0, st, tab, B);
   else
-    hipLaunchKernelGGL((k_accel_b<T, false>), dim3(npblocks), dim3(kBlock), 0, st, tab, pmap);
-}
-
-template <class T>
-void FusedOps<T>::pressure_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *pmap,
-                                 unsigned npblocks, unsigned nscenes, bool lds) {
-  if (npblocks == 0)
-    return;
-  if (lds)
-    hipLaunchKernelGGL((k_pressure_b<T, true>), dim3(npblocks), dim3(kBlock), 0, st, tab, pmap);
-  else
-    hipLaunchKernelGGL((k_pressure_b<T, false>), dim3(npblocks), dim3(kBlock), 0, st, tab, pmap);
+    hipLaunchKernelGGL((k_pressure_b<T, false>), dim3(n), dim3(kBlock), 0, st, tab, B);
   hipLaunchKernelGGL(k_pressure_finalize_b<T>, dim3(nscenes), dim3(kBlock), 0, st, tab);
 }
 

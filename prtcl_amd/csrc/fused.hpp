@@ -99,6 +99,9 @@ struct ScheduleTuner {
 
 template <class T>
 struct FusedOps {
+  // the neighbour list alone, for the procedures: every particle includes
+  // itself, at its place in slot order
+  static void build_list(hipStream_t st, const SceneView<T> &S, const NbrList &L);
   // density, neighbour list, IISPH c / AA / s, integrated velocity into vtmp
   // B.seq != 0: the first kernel also begins solve B (one launch fewer)
   static void setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
@@ -110,7 +113,8 @@ struct FusedOps {
   // the convergence step of IISPH iteration 1, whose pressures and aprde
   // partials the setup (with S.first_iter) has written (batched: for the
   // scenes without first_preset)
-  static void finish_first_iteration(hipStream_t st, const SceneView<T> &S);
+  static void finish_first_iteration(hipStream_t st, const SceneView<T> &S,
+                                     bool explicit_viscosity);
   static void finish_first_iteration_batch(hipStream_t st, const BatchEntry<T> *tab,
                                            unsigned nscenes);
   // v += dt a H, x += dt v, with a from S.xa, also stored to S.a; seq > 0:
@@ -119,17 +123,13 @@ struct FusedOps {
   static void integrate(hipStream_t st, const SceneView<T> &S, unsigned seq = 0);
   // S.a from S.xa (before a procedure kernel reads the acceleration)
   static void copy_accel(hipStream_t st, const SceneView<T> &S);
-  // the same passes over every scene of a batch (pmap: block map)
-  static void setup_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *pmap,
-                          unsigned npblocks, bool lds);
-  // the three setup launches of scenes with explicit viscosity (entry flag
-  // explicit_visc) or axial gravity, over the blocks of `map`
-  static void setup_split_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                                unsigned nblocks, bool lds);
-  static void accel_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *pmap,
-                          unsigned npblocks, bool lds);
-  static void pressure_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *pmap,
-                             unsigned npblocks, unsigned nscenes, bool lds);
+  // the same passes over every scene of a batch; group 0 of B are the scenes with
+  // the one-launch setup, group 1 those with the three-launch setup (entry
+  // flag explicit_visc: explicit viscosity, else axial gravity)
+  static void setup_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B, bool lds);
+  static void accel_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B, bool lds);
+  static void pressure_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
+                             unsigned nscenes, bool lds);
   // guarded: each scene as integrate() with seq = its solve's sequence
   static void integrate_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *pmap,
                               unsigned npblocks, unsigned nscenes, bool guarded = false);

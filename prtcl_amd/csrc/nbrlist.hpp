@@ -25,6 +25,12 @@
 namespace prtcl_amd {
 
 constexpr uint32_t kListOverflow = 1u << 31;
+// set where a boundary particle is within the radius, so later passes skip
+// the boundary walk of the others (an overflowed particle always walks)
+constexpr uint32_t kListBoundary = 1u << 24;
+__device__ __forceinline__ bool list_has_boundary(uint32_t info) {
+  return (info & (kListBoundary | kListOverflow)) != 0u;
+}
 // LDS bytes of one staged field array of one span (the real4 fields of 1536
 // particles in FP32, 768 in FP64); a block whose span is larger reads the
 // neighbours' fields from global memory instead
@@ -41,10 +47,15 @@ struct BlockRanges {
   uint32_t spare[2];
 };
 
+// slots per span table: a block's 256, or the 32 of a block that searches with
+// 8 lanes per particle (scan8.hpp)
+constexpr uint32_t kSpanShiftBlock = 8, kSpanShiftScan = 5;
+
 struct NbrList {
   uint16_t *idx;
   uint32_t *info;
-  BlockRanges *blk;  // one per block of kBlock slots
+  BlockRanges *blk;  // one per 1 << shift slots
+  uint32_t shift;
 };
 
 // The span table of one block in registers (selected by slab without
@@ -60,6 +71,11 @@ struct Spans {
     return l0 > l1 ? (l0 > l2 ? l0 : l2) : (l1 > l2 ? l1 : l2);
   }
 };
+
+// the span table of particle i's list
+__device__ __forceinline__ Spans list_spans(const NbrList &L, int i) {
+  return Spans::of(L.blk[i >> L.shift]);
+}
 
 // Cooperative copy of the span of slab s into LDS: dst[u] = src[base + u]
 // (all threads of the block call it).
@@ -174,6 +190,152 @@ __device__ __forceinline__ void list_gather(const NbrList &L, const Spans &R, si
           use(v[k]);
     }
   }
+}
+
+// ---- several lanes per particle (small scenes)
+//
+// A small scene does not fill the chip with one lane per particle (65,536
+// particles are one wavefront per SIMD), and a pass takes as long as one lane's
+// chain of list chunks and gathers. Up to kSplitMax particles each pass gives a
+// particle kListLanes lanes: lane l takes chunks l, l + kListLanes, ... (a mean
+// list of 30 entries is four chunks, one per lane) and the lanes' sums are added
+// in a fixed tree. Measured per launch, one lane -> four, accel pass: 2,048
+// particles 5.9 -> 3.7 us, 8,000: 6.3 -> 3.9, 59,000: 5.5 -> 5.2, 125,000: 7.2 ->
+// 7.3, 250,000: 13.6 -> 13.6; pressure pass 8.1 -> 4.7, 8.3 -> 4.9, 8.0 -> 7.1,
+// 10.0 -> 10.4, 20.7 -> 21.3. The rule depends on the scene alone, so that a
+// scene's results are the same alone and in a batch; a batch fills the chip, and
+// tthere the lanes' idle slots cost: with the line at 65,536, 16 scenes of
+// 2,000 to 200,000 particles took 11.83 ms instead of 11.60 ms for 10 steps. Below
+// 16,384 a batch's share of the work is too small to show.
+constexpr int kSplitMax = 16384;
+constexpr int kListLanes = 4;
+__host__ __device__ inline bool split_scene(int nf) { return nf <= kSplitMax; }
+// threads of a list pass
+__host__ __device__ inline long list_threads(int nf) {
+  return split_scene(nf) ? static_cast<long>(nf) * kListLanes : nf;
+}
+// blocks of a list pass and of the setup pass (scan8.hpp where split)
+__host__ __device__ inline unsigned list_blocks(int nf) { return grid_blocks(list_threads(nf)); }
+__host__ __device__ inline unsigned setup_blocks(int nf) {
+  return split_scene(nf) ? grid_blocks(nf, 1 << kSpanShiftScan) : grid_blocks(nf);
+}
+__host__ __device__ inline uint32_t list_shift(int nf) {
+  return split_scene(nf) ? kSpanShiftScan : kSpanShiftBlock;
+}
+
+// The blocks of 256 particles of a batch's scenes: words (scene, local block)
+// in four runs, two groups (0, 1: one, 2, 3: the other) of one-lane scenes and
+// of split scenes. A list or setup pass launches `factor` blocks for each block
+// of a split scene; each run is spread over the XCDs in contiguous parts.
+struct BatchBlocks {
+  const uint32_t *map;
+  unsigned n[4];
+  __host__ unsigned launch(unsigned factor) const {
+    return n[0] + n[2] + factor * (n[1] + n[3]);
+  }
+  __host__ BatchBlocks group(int g) const {
+    return BatchBlocks{map + (g ? n[0] + n[1] : 0u),
+                       {g ? 0u : n[0], g ? 0u : n[1], g ? n[2] : 0u, g ? n[3] : 0u}};
+  }
+};
+// the word of this block and its part (0 .. factor - 1) of a split scene's block
+__device__ __forceinline__ uint32_t batch_block(const BatchBlocks &B, unsigned factor,
+                                                unsigned *part) {
+  unsigned x = blockIdx.x;
+  const uint32_t *m = B.map;
+  uint32_t word = 0;
+  *part = 0;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const unsigned f = (s & 1) ? factor : 1u;
+    const unsigned cnt = f * B.n[s];
+    if (x < cnt) {
+      const unsigned l = xcd_block(x, cnt);
+      *part = l % f;
+      word = m[l / f];
+      break;
+    }
+    x -= cnt;
+    m += B.n[s];
+  }
+  return word;
+}
+
+// the span table of a wavefront of a fused list pass with kLanes lanes per
+// particle (block lb of the pass), uniform over the wavefront: one lane per
+// particle goes with a table per block, four with a table per 32 particles
+template <int kLanes>
+__device__ __forceinline__ Spans pass_spans(const NbrList &L, int nf, unsigned lb) {
+  if (kLanes == 1)
+    return Spans::of(L.blk[lb]);
+  static_assert(kWave / kListLanes <= (1 << kSpanShiftScan), "one table per wavefront");
+  const int first = __builtin_amdgcn_readfirstlane(
+      static_cast<int>((lb * kBlock + (threadIdx.x & ~63u)) / kLanes));
+  return Spans::of(L.blk[first < nf ? first >> kSpanShiftScan : 0]);
+}
+
+// list_gather for lane `sub` of kLanes lanes of particle i
+template <int kLanes, int kGroup, class Load, class Use>
+__device__ __forceinline__ void list_gather_lanes(const NbrList &L, const Spans &R, size_t n, int i,
+                                                  uint32_t info, uint32_t sub, Load &&load,
+                                                  Use &&use) {
+  if (kLanes == 1) {
+    list_gather<kGroup>(L, R, n, i, info, load, use);
+    return;
+  }
+  const uint32_t c0 = info & 0xFFu;
+  const uint32_t c01 = c0 + ((info >> 8) & 0xFFu);
+  const uint32_t c = c01 + ((info >> 16) & 0xFFu);
+  const uint32_t d1 = R.b1 - R.b0, d2 = R.b2 - R.b1;
+  using V = decltype(load(0u));
+  for (uint32_t g = sub; g * kChunk < c; g += kLanes) {
+    const uint4 q = list_chunk(L, n, i, g);
+#pragma unroll
+    for (int h = 0; h < static_cast<int>(kChunk); h += kGroup) {
+      V v[kGroup];
+#pragma unroll
+      for (int k = 0; k < kGroup; ++k) {
+        const uint32_t e = g * kChunk + h + k;
+        if (e < c)
+          v[k] = load(R.b0 + chunk_entry(q, h + k) + (e >= c0 ? d1 : 0u) + (e >= c01 ? d2 : 0u));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < kGroup; ++k)
+        if (g * kChunk + h + k < c)
+          use(v[k]);
+    }
+  }
+}
+
+// the sum over a particle's kLanes lanes, in every one of them (all lanes of
+// the wavefront call it)
+template <int kLanes, class T>
+__device__ __forceinline__ T lanes_sum(T v) {
+#pragma unroll
+  for (int o = 1; o < kLanes; o <<= 1)
+    v += __shfl_xor(v, o, kWave);
+  return v;
+}
+
+// The sum over a block of a value that the first of every kLanes lanes holds
+// (valid in thread 0; all threads of the block call it, once per kernel). With
+// several lanes neighbouring particles are added first, so that the sums of two
+// blocks of 32 particles (8 lanes) add up to exactly the sum of the block of 64
+// (4 lanes) that they make.
+template <int kLanes>
+__device__ __forceinline__ double particle_sum(double v) {
+  if (kLanes == 1)
+    return block_sum<kBlock>(v);
+  static_assert(kBlock / kWave == 4, "four wavefronts per block");
+  __shared__ double ws[kBlock / kWave];
+#pragma unroll
+  for (int o = kLanes; o < kWave; o <<= 1)
+    v += __shfl_xor(v, o, kWave);
+  if (threadIdx.x % kWave == 0)
+    ws[threadIdx.x / kWave] = v;
+  __syncthreads();
+  return (ws[0] + ws[1]) + (ws[2] + ws[3]);
 }
 
 }  // namespace prtcl_amd

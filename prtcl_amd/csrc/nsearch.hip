@@ -368,7 +368,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_state(V *__restrict__ xd, con
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cell_keys_b(const BatchEntry<T> *tab,
                                                         const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
+  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   k_cell_keys_body<T>(E.S.grid, E.S.xm, E.S.nf, E.S.fcell, E.count, E.rank,
                       u & kBatchLocalMask);
@@ -411,7 +411,7 @@ __global__ __launch_bounds__(kScanBS) void k_scan_down_b(const BatchEntry<T> *ta
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_scatter_b(const BatchEntry<T> *tab,
                                                       const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
+  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   k_scatter_body(E.S.grid, E.S.fcell, E.rank, E.start, E.S.nf, E.perm, u & kBatchLocalMask);
 }
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter_b(const BatchEntry<T> *tab,
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_stable_rank_b(const BatchEntry<T> *tab,
                                                           const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
+  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   k_stable_rank_body(E.S.grid, E.S.fcell, E.start, E.perm, E.S.nf, E.rank,
                      u & kBatchLocalMask);
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(kBlock) void k_stable_rank_b(const BatchEntry<T> *t
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_place_state_b(const BatchEntry<T> *tab,
                                                           const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
+  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   k_place_state_body<vec4_t<T>>(E.S.grid, E.S.fcell, E.start, E.perm, E.S.nf, E.x_dst, E.S.xm,
                                 E.v_dst, E.S.v, E.id_dst,
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(kBlock) void k_place_state_b(const BatchEntry<T> *t
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_gather_state_b(const BatchEntry<T> *tab,
                                                            const uint32_t *pmap) {
-  const uint32_t u = pmap[blockIdx.x];
+  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   k_gather_state_body<vec4_t<T>>(E.x_dst, E.S.xm, E.v_dst, E.S.v, E.id_dst,
                                  reinterpret_cast<const uint32_t *>(E.S.id), E.cell_dst,

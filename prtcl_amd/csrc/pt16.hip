@@ -61,7 +61,7 @@ __device__ __forceinline__ void fluid_pairs_list(const SceneView<T> &S, const Nb
     return;
   }
   fn(static_cast<uint32_t>(i), T(0), T(0), T(0), T(0), xv, kSelfEntry);
-  list_visit_indexed(L, Spans::of(L.blk[lb]), static_cast<size_t>(S.nf), i, info,
+  list_visit_indexed(L, list_spans(L, i), static_cast<size_t>(S.nf), i, info,
                      [&](uint32_t e, uint32_t j) {
                        const vec4_t<T> pj = S.xm[j];
                        const T d0 = xv.x - pj.x, d1 = xv.y - pj.y, d2 = xv.z - pj.z;
@@ -185,7 +185,7 @@ __device__ __forceinline__ void pt16_omega_rhs_body(const SceneView<T> &S, const
     exact();
   } else {
     const size_t n = static_cast<size_t>(S.nf);
-    list_visit_indexed(L, Spans::of(L.blk[lb]), n, i, L.info[i], [&](uint32_t e, uint32_t j) {
+    list_visit_indexed(L, list_spans(L, i), n, i, L.info[i], [&](uint32_t e, uint32_t j) {
       const vec4_t<T> wj = S.om[j];
       const T c = S.pcoef[coef_index(n, i, e)];
       a0 += c * (wi.x - wj.x);
@@ -309,7 +309,7 @@ __device__ __forceinline__ T product_s_list(const SceneView<T> &S, const NbrList
   }
   out -= (xv.w * S.K.w(T(0))) * wi;
   const size_t n = static_cast<size_t>(S.nf);
-  const Spans R = Spans::of(L.blk[lb]);
+  const Spans R = list_spans(L, i);
   const uint32_t c0 = info & 0xFFu;
   const uint32_t c01 = c0 + ((info >> 8) & 0xFFu);
   const uint32_t c = list_count(info);
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(kBlock) void k_pt16_cg_apply(SceneView<T> S, int wh
 // number cg_seq + s with the tolerance and cap of its system.
 template <class T>
 __device__ __forceinline__ NbrList pt16_list(const BatchEntry<T> &E) {
-  return NbrList{E.nidx, E.ninfo, E.nblk};
+  return NbrList{E.nidx, E.ninfo, E.nblk, E.nshift};
 }
 
 #define PT16_BATCH_ENTRY                              \

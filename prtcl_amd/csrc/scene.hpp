@@ -250,6 +250,7 @@ struct BatchEntry {
   uint16_t *nidx;             // neighbour list of the scene (NbrList)
   uint32_t *ninfo;
   BlockRanges *nblk;
+  uint32_t nshift;
   vec4_t<T> *vtmp;            // integrated velocity written by the setup pass
   uint32_t *count, *start;    // fluid grid counts / starts
   uint32_t *rank, *perm;      // sort buffers (result in rank)

@@ -415,6 +415,7 @@ class SceneImpl final : public SceneBase {
     PRTCL_HIP_CHECK(hipGetLastError());
     PRTCL_HIP_CHECK(hipStreamSynchronize(st));
     if (field == PRTCL_HIP_F_POSITION) {
+      proc_list_valid_ = false;
       // host-side bounding box for the grid domain
       const T *hp = static_cast<const T *>(host);
       double lo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, hi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
@@ -544,6 +545,7 @@ class SceneImpl final : public SceneBase {
                                      res_->stream));
       PRTCL_HIP_CHECK(hipStreamSynchronize(res_->stream));
     }
+    proc_list_valid_ = false;
     if (group == PRTCL_HIP_FLUID)
       fgrid_dirty_ = true;
     else
@@ -689,6 +691,7 @@ class SceneImpl final : public SceneBase {
 
   void build_boundary_grid() {
     hipStream_t st = res_->stream;
+    proc_list_valid_ = false;
     const uint32_t *pm = GridOps<T>::sort_group(st, gd_, P_.bxV, nb_, P_.bcell, G_.count,
                                                 G_.bstart, P_.brank, P_.bperm, G_.scan_tmp);
     if (nb_ > 0) {
@@ -704,6 +707,7 @@ class SceneImpl final : public SceneBase {
   // carries over between steps (x, m, v, t_birth, id)
   void build_fluid_grid(bool all) {
     hipStream_t st = res_->stream;
+    proc_list_valid_ = false;
     if (!all) {
       // the step's sort: only the carried state moves, placed by the
       // stable-rank pass itself (x -> xq, v -> tmpV4, id -> tmpI, cell ->
@@ -885,7 +889,21 @@ class SceneImpl final : public SceneBase {
     return S;
   }
 
-  NbrList nbr_list() const { return NbrList{P_.nidx, P_.ninfo, P_.nblk}; }
+  // the fused step's list
+  NbrList nbr_list() const { return NbrList{P_.nidx, P_.ninfo, P_.nblk, list_shift(nf_)}; }
+
+  // The list of the procedures: the neighbours (the particle itself included)
+  // that a walk over the grid would visit now, in its order. Built by the first
+  // procedure that needs it and kept until the positions, the slots or the
+  // grid change; the fused step writes its own list to the same memory.
+  NbrList proc_list() {
+    const NbrList L{P_.nidx, P_.ninfo, P_.nblk, kSpanShiftScan};
+    if (!proc_list_valid_) {
+      FusedOps<T>::build_list(res_->stream, view(), L);
+      proc_list_valid_ = true;
+    }
+    return L;
+  }
 
   void require_grid() {
     if (!grid_built_)
@@ -905,7 +923,7 @@ class SceneImpl final : public SceneBase {
         }
         SphOps<T>::volume(st, view());
         break;
-      case PRTCL_HIP_P_DENSITY_COMPUTE_DENSITY: require_grid(); SphOps<T>::density(st, view()); break;
+      case PRTCL_HIP_P_DENSITY_COMPUTE_DENSITY: require_grid(); SphOps<T>::density(st, view(), proc_list()); break;
       case PRTCL_HIP_P_GRAVITY_INITIALIZE_ACCELERATION: SphOps<T>::gravity(st, view()); break;
       case PRTCL_HIP_P_GRAVITY_INITIALIZE_AXIAL_ACCELERATION:
         SphOps<T>::gravity_axial(st, view());
@@ -913,24 +931,25 @@ class SceneImpl final : public SceneBase {
       case PRTCL_HIP_P_GRAVITY_ACCUMULATE_ACCELERATION:
         SphOps<T>::gravity_accumulate(st, view());
         break;
-      case PRTCL_HIP_P_VISCOSITY_ACCUMULATE_ACCELERATION: require_grid(); SphOps<T>::viscosity(st, view()); break;
+      case PRTCL_HIP_P_VISCOSITY_ACCUMULATE_ACCELERATION: require_grid(); SphOps<T>::viscosity(st, view(), proc_list()); break;
       case PRTCL_HIP_P_SE_INTEGRATE_VELOCITY_WITH_HARD_FADE: SphOps<T>::integrate_v(st, view()); break;
       case PRTCL_HIP_P_SE_INTEGRATE_POSITION:
         SphOps<T>::integrate_x(st, view());
+        proc_list_valid_ = false;
         steps_enqueued_ += nf_ > 0 ? 1u : 0u;
         break;
       case PRTCL_HIP_P_IISPH_SETUP:
         require_grid();
-        SphOps<T>::iisph_setup(st, view());
+        SphOps<T>::iisph_setup(st, view(), proc_list());
         ctl_op(kCtlSetNprde, 0, nf_);
         break;
       case PRTCL_HIP_P_IISPH_ITERATION_PRESSURE_ACCELERATION:
         require_grid();
-        SphOps<T>::iisph_accel(st, view(), false);
+        SphOps<T>::iisph_accel(st, view(), proc_list(), false);
         break;
       case PRTCL_HIP_P_IISPH_ITERATION_PRESSURE:
         require_grid();
-        SphOps<T>::iisph_pressure(st, view(), false);
+        SphOps<T>::iisph_pressure(st, view(), proc_list(), false);
         break;
       case PRTCL_HIP_P_WKBB18_COMPUTE_DIAGONAL:
       case PRTCL_HIP_P_WKBB18_ACCUMULATE_ACCELERATION:
@@ -1198,13 +1217,14 @@ class SceneImpl final : public SceneBase {
              static_cast<int>(seq), nprde);
     const SceneView<T> S = view();
     const NbrList L = nbr_list();
+    const NbrList PL = fused || nf_ == 0 ? L : proc_list();
     Profiler &pf = res_->prof;
     tprof_.on = tune;
     // iterations enqueued so far (the iteration taken by the setup counts)
     int enq = 0;
     if (first) {
       if (!preset)
-        FusedOps<T>::finish_first_iteration(st, S);
+        FusedOps<T>::finish_first_iteration(st, S, desc.explicit_viscosity != 0);
       enq = 1;
     }
     // one IISPH iteration (pressure acceleration, pressure, finalize) replayed
@@ -1232,7 +1252,7 @@ class SceneImpl final : public SceneBase {
         if (fused)
           FusedOps<T>::accel(st, S, L, sc.accel_lds);
         else
-          SphOps<T>::iisph_accel(st, S, true);
+          SphOps<T>::iisph_accel(st, S, PL, true);
         tprof_.end(st, q);
         pf.end(st, r);
         r = pf.begin(st, kStagePressure, enq + k);
@@ -1240,7 +1260,7 @@ class SceneImpl final : public SceneBase {
         if (fused)
           FusedOps<T>::pressure(st, S, L, sc.pressure_lds);
         else
-          SphOps<T>::iisph_pressure(st, S, true);
+          SphOps<T>::iisph_pressure(st, S, PL, true);
         tprof_.end(st, q);
         pf.end(st, r);
       }
@@ -1359,7 +1379,7 @@ class SceneImpl final : public SceneBase {
       } else {
         const SceneView<T> S = view();
         r = pf.begin(st, kStageDensity);
-        SphOps<T>::density(st, S);
+        SphOps<T>::density(st, S, proc_list());
         pf.end(st, r);
         r = pf.begin(st, kStageGravityIntegrateV);
         if (desc.axial_gravity)  // example.lua:390-391
@@ -1369,14 +1389,14 @@ class SceneImpl final : public SceneBase {
         pf.end(st, r);
         if (desc.explicit_viscosity) {
           r = pf.begin(st, kStageViscosity);
-          SphOps<T>::viscosity(st, S);
+          SphOps<T>::viscosity(st, S, proc_list());
           pf.end(st, r);
         }
         r = pf.begin(st, kStageGravityIntegrateV);
         SphOps<T>::integrate_v(st, S);
         pf.end(st, r);
         r = pf.begin(st, kStageSetup);
-        SphOps<T>::iisph_setup(st, S);
+        SphOps<T>::iisph_setup(st, S, proc_list());
         pf.end(st, r);
       }
       int it = 0;
@@ -1449,6 +1469,7 @@ class SceneImpl final : public SceneBase {
         }
         r = pf.begin(st, kStageIntegrateX);
         SphOps<T>::integrate_x(st, S);
+        proc_list_valid_ = false;
         steps_enqueued_ += nf_ > 0 ? 1u : 0u;
         pf.end(st, r);
       }
@@ -1523,18 +1544,22 @@ class SceneImpl final : public SceneBase {
         SphOps<T>::volume(st, sc->view());
       }
     }
-    // block maps: logical block b of the batch (scene order, then local
-    // block) is dispatched as hardware block xcd(b), as in the single-scene
-    // kernels, so each XCD takes a contiguous run of cell-ordered particles
-    // (plist1 / plist3: the blocks of scenes with the one-launch and with
-    // the three-launch setup)
-    std::vector<uint32_t> plist, tlist, plist1, plist3;
+    // block map: the blocks of the scenes with the one-launch setup, then of
+    // those with the three-launch setup, each the one-lane scenes before the
+    // split ones (BatchBlocks). The kernels spread it over the XCDs as the
+    // single-scene kernels do, so each XCD takes a contiguous run of
+    // cell-ordered particles.
+    std::vector<uint32_t> plist, tlist;
+    BatchBlocks blocks{};
+    for (int run = 0; run < 4; ++run) {
+      const size_t before = plist.size();
+      for (unsigned k = 0; k < ns; ++k)
+        if (v[k]->split_setup() == (run >= 2) && split_scene(v[k]->nf_) == ((run & 1) != 0))
+          for (unsigned b = 0; b < grid_blocks(v[k]->nf_); ++b)
+            plist.push_back((k << kBatchLocalBits) | b);
+      blocks.n[run] = static_cast<unsigned>(plist.size() - before);
+    }
     for (unsigned k = 0; k < ns; ++k) {
-      const unsigned nb = grid_blocks(v[k]->nf_);
-      for (unsigned b = 0; b < nb; ++b) {
-        plist.push_back((k << kBatchLocalBits) | b);
-        (v[k]->split_setup() ? plist3 : plist1).push_back((k << kBatchLocalBits) | b);
-      }
       const unsigned nt = scan_tiles(v[k]->gd_.ncells);
       for (unsigned b = 0; b < nt; ++b)
         tlist.push_back((k << kBatchLocalBits) | b);
@@ -1573,22 +1598,16 @@ class SceneImpl final : public SceneBase {
     const unsigned nvn = nvg > 0 ? static_cast<unsigned>(vlist_n.size()) : 0u;
     const unsigned nps = static_cast<unsigned>(psc.size());
     const unsigned npb = static_cast<unsigned>(ptlist.size());
-    // the setup's own block maps only when some scene has the three-launch
-    // setup (else pmap serves)
-    const unsigned np3 = static_cast<unsigned>(plist3.size());
-    const unsigned np1 = np3 > 0 ? static_cast<unsigned>(plist1.size()) : 0u;
     // pinned / device table layout: [sort | setup | solve] entries, the
-    // WKBB18 entries, pmap, tmap, vmap, the setup maps, the WKBB18 split
-    // maps, the pt16 entries and map
+    // WKBB18 entries, pmap, tmap, vmap, the WKBB18 split maps, the pt16
+    // entries and map
     auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
     const size_t tab_bytes = align(sizeof(BatchEntry<T>) * ns);
     const size_t off_visc = 3 * tab_bytes;
     const size_t off_pmap = off_visc + align(sizeof(BatchEntry<T>) * nvs);
     const size_t off_tmap = off_pmap + align(sizeof(uint32_t) * np);
     const size_t off_vmap = off_tmap + align(sizeof(uint32_t) * nt);
-    const size_t off_s1map = off_vmap + align(sizeof(uint32_t) * nvb);
-    const size_t off_s3map = off_s1map + align(sizeof(uint32_t) * np1);
-    const size_t off_vnmap = off_s3map + align(sizeof(uint32_t) * np3);
+    const size_t off_vnmap = off_vmap + align(sizeof(uint32_t) * nvb);
     const size_t off_vgmap = off_vnmap + align(sizeof(uint32_t) * nvn);
     const size_t off_pt = off_vgmap + align(sizeof(uint32_t) * nvg);
     const size_t off_ptmap = off_pt + align(sizeof(BatchEntry<T>) * nps);
@@ -1610,17 +1629,11 @@ class SceneImpl final : public SceneBase {
     uint32_t *tmap = reinterpret_cast<uint32_t *>(hb + off_tmap);
     uint32_t *vmap = reinterpret_cast<uint32_t *>(hb + off_vmap);
     for (unsigned b = 0; b < np; ++b)
-      pmap[b] = plist[xcd_of(b, np)];
+      pmap[b] = plist[b];
     for (unsigned b = 0; b < nt; ++b)
       tmap[b] = tlist[b];
     for (unsigned b = 0; b < nvb; ++b)
       vmap[b] = vlist[xcd_of(b, nvb)];
-    uint32_t *s1map = reinterpret_cast<uint32_t *>(hb + off_s1map);
-    uint32_t *s3map = reinterpret_cast<uint32_t *>(hb + off_s3map);
-    for (unsigned b = 0; b < np1; ++b)
-      s1map[b] = plist1[xcd_of(b, np1)];
-    for (unsigned b = 0; b < np3; ++b)
-      s3map[b] = plist3[xcd_of(b, np3)];
     uint32_t *vnmap = reinterpret_cast<uint32_t *>(hb + off_vnmap);
     uint32_t *vgmap = reinterpret_cast<uint32_t *>(hb + off_vgmap);
     for (unsigned b = 0; b < nvn; ++b)
@@ -1645,6 +1658,7 @@ class SceneImpl final : public SceneBase {
       E.nidx = s.P_.nidx;
       E.ninfo = s.P_.ninfo;
       E.nblk = s.P_.nblk;
+      E.nshift = list_shift(s.nf_);
       E.count = s.G_.count;
       E.start = s.G_.fstart;
       E.rank = s.P_.frank;
@@ -1663,6 +1677,7 @@ class SceneImpl final : public SceneBase {
       std::swap(s.P_.fcell, s.P_.frank);
       s.fgrid_dirty_ = false;
       s.grid_built_ = true;
+      s.proc_list_valid_ = false;
       s.steps_since_permute_ += 1;
       if (s.desc.permute_every > 0 && s.steps_since_permute_ >= s.desc.permute_every) {
         permute[k] = 1;
@@ -1740,10 +1755,9 @@ class SceneImpl final : public SceneBase {
     const auto *d_tmap = reinterpret_cast<const uint32_t *>(db + off_tmap);
     const auto *d_visc = reinterpret_cast<const BatchEntry<T> *>(db + off_visc);
     const auto *d_vmap = reinterpret_cast<const uint32_t *>(db + off_vmap);
-    const auto *d_s1map = reinterpret_cast<const uint32_t *>(db + off_s1map);
-    const auto *d_s3map = reinterpret_cast<const uint32_t *>(db + off_s3map);
     const auto *d_pt = reinterpret_cast<const BatchEntry<T> *>(db + off_pt);
     const auto *d_ptmap = reinterpret_cast<const uint32_t *>(db + off_ptmap);
+    blocks.map = d_pmap;
     BatchMaps vm;
     vm.all = reinterpret_cast<const uint32_t *>(db + off_vmap);
     vm.n_all = nvb;
@@ -1774,12 +1788,7 @@ class SceneImpl final : public SceneBase {
     tp.on = tune;
     r = pf.begin(st, kStageSetup);
     int q = tp.begin(st, kStageSetup);
-    if (np3 == 0) {
-      FusedOps<T>::setup_batch(st, d_setup, d_pmap, np, sc.setup_lds);
-    } else {
-      FusedOps<T>::setup_batch(st, d_setup, d_s1map, np1, sc.setup_lds);
-      FusedOps<T>::setup_split_batch(st, d_setup, d_s3map, np3, sc.setup_lds);
-    }
+    FusedOps<T>::setup_batch(st, d_setup, blocks, sc.setup_lds);
     tp.end(st, q);
     pf.end(st, r);
     hipLaunchKernelGGL(k_begin_solve_b<T>, dim3(grid_blocks(ns, 64)), dim3(64), 0, st, d_solve,
@@ -1800,14 +1809,14 @@ class SceneImpl final : public SceneBase {
     int enq = fold_first ? 1 : 0;  // iterations enqueued (iteration 1 by the setup)
     const bool graph = !sc.eager && !pf.on && !tune;
     const std::string key =
-        graph ? graph_key(kGraphBatchIteration | sizeof(T), d_solve, d_pmap, np, ns, sc)
+        graph ? graph_key(kGraphBatchIteration | sizeof(T), d_solve, blocks, ns, sc)
               : std::string();
     auto enqueue = [&](int n) {
       if (graph) {
         for (int j = 0; j < n; ++j)
           res->batch_graphs[sizeof(T) == 8 ? 1 : 0].launch(st, key, [&] {
-            FusedOps<T>::accel_batch(st, d_solve, d_pmap, np, sc.accel_lds);
-            FusedOps<T>::pressure_batch(st, d_solve, d_pmap, np, ns, sc.pressure_lds);
+            FusedOps<T>::accel_batch(st, d_solve, blocks, sc.accel_lds);
+            FusedOps<T>::pressure_batch(st, d_solve, blocks, ns, sc.pressure_lds);
           });
         enq += n;
         return;
@@ -1815,12 +1824,12 @@ class SceneImpl final : public SceneBase {
       for (int j = 0; j < n; ++j) {
         int q1 = pf.begin(st, kStagePressureAccel, enq + j);
         int q2 = tp.begin(st, kStagePressureAccel, enq + j);
-        FusedOps<T>::accel_batch(st, d_solve, d_pmap, np, sc.accel_lds);
+        FusedOps<T>::accel_batch(st, d_solve, blocks, sc.accel_lds);
         tp.end(st, q2);
         pf.end(st, q1);
         q1 = pf.begin(st, kStagePressure, enq + j);
         q2 = tp.begin(st, kStagePressure, enq + j);
-        FusedOps<T>::pressure_batch(st, d_solve, d_pmap, np, ns, sc.pressure_lds);
+        FusedOps<T>::pressure_batch(st, d_solve, blocks, ns, sc.pressure_lds);
         tp.end(st, q2);
         pf.end(st, q1);
       }
@@ -2249,7 +2258,7 @@ class SceneImpl final : public SceneBase {
     A.take(P.fperm, f);
     A.take(P.nidx, static_cast<size_t>(kNbrCap) * f);
     A.take(P.ninfo, f);
-    A.take(P.nblk, grid_blocks(static_cast<long>(f)));
+    A.take(P.nblk, grid_blocks(static_cast<long>(f), 1 << kSpanShiftScan));
     A.take(P.bxV, b);
     A.take(P.btmpV4, b);
     A.take(P.bid, b);
@@ -2258,7 +2267,9 @@ class SceneImpl final : public SceneBase {
     A.take(P.bcell, b);
     A.take(P.brank, b);
     A.take(P.bperm, b);
-    A.take(P.partials, grid_blocks(static_cast<long>(std::max(f, b))) + 1);
+    // one per block of the largest launch that writes them
+    A.take(P.partials, std::max({grid_blocks(static_cast<long>(std::max(f, b))),
+                                 setup_blocks(nf), list_blocks(nf)}) + 1);
     A.take(P.cg_part, 3 * static_cast<size_t>(grid_blocks(static_cast<long>(f))) + 3);
     A.take(P.ctl, 1);
     const size_t nv = pcg ? f : 1;
@@ -2377,6 +2388,7 @@ class SceneImpl final : public SceneBase {
   GridDims gd_{};
   BBox bb_f_, bb_b_;
   bool grid_built_ = false, bgrid_dirty_ = true, fgrid_dirty_ = true;
+  bool proc_list_valid_ = false;  // proc_list() holds for the present positions
   double clock_ = 0;
   int steps_since_permute_ = 0;
   ScheduleTuner tuner_;

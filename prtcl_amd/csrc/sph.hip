@@ -1,9 +1,18 @@
 // SPH procedure kernels of the reference schemes, one thread per particle in
-// cell order, each gathering over the 9 x-runs of the 27-cell neighbourhood
-// (3 contiguous cells per run). The per-pair arithmetic follows the
-// generated reference code operation by operation (expression trees cited
-// per kernel), FP32 without FMA contraction, so individual pair terms equal
-// the CPU's; only the order in which neighbours are summed differs.
+// cell order. The fluid neighbours come from the list that the first procedure
+// after a change of the positions builds (FusedOps::build_list: the particles
+// of a walk over the 27 cells, in its order, the particle itself included);
+// boundary neighbours, and those of a particle whose list overflowed, are
+// gathered over the 9 x-runs of the 27 cells (3 contiguous cells per run). The
+// per-pair arithmetic follows the generated reference code operation by
+// operation (expression trees cited per kernel), FP32 without FMA
+// contraction, so individual pair terms equal the CPU's; only the order in
+// which neighbours are summed differs.
+//
+// A procedure is bound by the latency of its gathers (list chunk, then the
+// neighbours' fields, groups of four in flight). 64,000 particles, two steps of 13
+// procedures that read neighbours: 2.64 ms with a walk over the grid in each
+// (216 candidates, 68-93 us a procedure), 1.54 ms with the list.
 #include "sph.hpp"
 
 namespace prtcl_amd {
@@ -54,6 +63,44 @@ __device__ __forceinline__ void for_neighbors(const SceneView<T> &S, const vec4_
   });
 }
 
+// Visits the fluid neighbours of particle i from the list, or over the grid
+// for a particle whose list overflowed: fn(d0, d1, d2, r2, pj, f) with
+// d = xi - xj and f = load(j), the neighbour's further fields, gathered ahead of
+// the arithmetic with its position.
+template <class T, class Load, class Fn>
+__device__ __forceinline__ void fluid_neighbors(const SceneView<T> &S, const NbrList &L, int i,
+                                                uint32_t info, const vec4_t<T> &xi, Load &&load,
+                                                Fn &&fn) {
+  struct Rec {
+    vec4_t<T> x;
+    decltype(load(0u)) f;
+  };
+  if (!(info & kListOverflow)) {
+    list_gather<4>(
+        L, list_spans(L, i), static_cast<size_t>(S.nf), i, info,
+        [&](uint32_t j) { return Rec{S.xm[j], load(j)}; },
+        [&](const Rec &q) {
+          const T d0 = xi.x - q.x.x, d1 = xi.y - q.x.y, d2 = xi.z - q.x.z;
+          fn(d0, d1, d2, sqdist_exact(d0, d1, d2), q.x, q.f);
+        });
+  } else {
+    for_neighbors(S, xi, S.fcell[i], S.fstart, S.xm,
+                  [&](uint32_t j, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
+                    fn(d0, d1, d2, r2, pj, load(j));
+                  });
+  }
+}
+
+struct Nothing {};
+
+// the boundary neighbours, over the grid; a particle with none is told by its list
+template <class T, class Fn>
+__device__ __forceinline__ void boundary_neighbors(const SceneView<T> &S, int i, uint32_t info,
+                                                   const vec4_t<T> &xi, Fn &&fn) {
+  if (list_has_boundary(info))
+    for_neighbors(S, xi, S.fcell[i], S.bstart, S.bxV, fn);
+}
+
 template <class T>
 __device__ __forceinline__ T step_l(T eps, T x) {  // unit_step_l (eigen.hpp:306-314)
   return (eps < x) ? T(1) : T(0);
@@ -76,17 +123,20 @@ __global__ __launch_bounds__(kBlock) void k_volume(SceneView<T> S) {
 
 // ---- density.compute_density (density.hpp:160-215)
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_density(SceneView<T> S) {
+__global__ __launch_bounds__(kBlock) void k_density(SceneView<T> S, NbrList L) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   if (i >= S.nf)
     return;
   const vec4_t<T> xi = S.xm[i];
-  const uint32_t ci = S.fcell[i];
+  const uint32_t info = L.info[i];
   T rho = 0;
-  for_neighbors(S, xi, ci, S.fstart, S.xm,
-                [&](uint32_t, T, T, T, T r2, const vec4_t<T> &pj) { rho += pj.w * S.K.w(r2); });
-  for_neighbors(S, xi, ci, S.bstart, S.bxV, [&](uint32_t, T, T, T, T r2, const vec4_t<T> &pj) {
+  fluid_neighbors(S, L, i, info, xi, [](uint32_t) { return Nothing{}; },
+                  [&](T, T, T, T r2, const vec4_t<T> &pj, const Nothing &) {
+                    rho += pj.w * S.K.w(r2);
+                  });
+  boundary_neighbors(S, i, info, xi, [&](uint32_t, T, T, T, T r2, const vec4_t<T> &pj) {
     rho += (pj.w * S.rho0) * S.K.w(r2);
   });
   S.rho[i] = rho;
@@ -125,28 +175,33 @@ __global__ __launch_bounds__(kBlock) void k_gravity_axial(SceneView<T> S) {
 
 // ---- viscosity.accumulate_acceleration (viscosity.hpp:171-240)
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_viscosity(SceneView<T> S) {
+__global__ __launch_bounds__(kBlock) void k_viscosity(SceneView<T> S, NbrList L) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   if (i >= S.nf)
     return;
   const vec4_t<T> xi = S.xm[i], vi = S.v[i];
   const T rhoi = S.rho[i];
-  const uint32_t ci = S.fcell[i];
+  const uint32_t info = L.info[i];
   vec4_t<T> ai = S.a[i];
-  for_neighbors(S, xi, ci, S.fstart, S.xm,
-                [&](uint32_t j, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
-                  const vec4_t<T> vj = S.v[j];
+  struct VR {
+    vec4_t<T> v;
+    T rho;
+  };
+  fluid_neighbors(S, L, i, info, xi, [&](uint32_t j) { return VR{S.v[j], S.rho[j]}; },
+                [&](T d0, T d1, T d2, T r2, const vec4_t<T> &pj, const VR &q) {
+                  const vec4_t<T> vj = q.v;
                   const T f = S.K.gradf(r2);
                   const T g0 = f * d0, g1 = f * d1, g2 = f * d2;
-                  const T s = (((T(10) * (S.mu_f / rhoi)) * (pj.w / S.rho[j])) *
+                  const T s = (((T(10) * (S.mu_f / rhoi)) * (pj.w / q.rho)) *
                                dot3_exact(vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, d0, d1, d2)) /
                               (r2 + S.hh001);
                   ai.x += s * g0;
                   ai.y += s * g1;
                   ai.z += s * g2;
                 });
-  for_neighbors(S, xi, ci, S.bstart, S.bxV,
+  boundary_neighbors(S, i, info, xi,
                 [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
                   const T f = S.K.gradf(r2);
                   const T g0 = f * d0, g1 = f * d1, g2 = f * d2;
@@ -229,24 +284,25 @@ __global__ __launch_bounds__(kBlock) void k_integrate_x(SceneView<T> S) {
 
 // ---- iisph.setup pass 1 (iisph.hpp:197-249): helper c
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_iisph_c(SceneView<T> S) {
+__global__ __launch_bounds__(kBlock) void k_iisph_c(SceneView<T> S, NbrList L) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   if (i >= S.nf)
     return;
   const vec4_t<T> xi = S.xm[i];
   const T rhoi = S.rho[i];
-  const uint32_t ci = S.fcell[i];
+  const uint32_t info = L.info[i];
   T c0 = 0, c1 = 0, c2 = 0;
-  for_neighbors(S, xi, ci, S.fstart, S.xm,
-                [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
+  fluid_neighbors(S, L, i, info, xi, [](uint32_t) { return Nothing{}; },
+                [&](T d0, T d1, T d2, T r2, const vec4_t<T> &pj, const Nothing &) {
                   const T f = S.K.gradf(r2);
                   const T s = pj.w / (rhoi * rhoi);
                   c0 -= s * (f * d0);
                   c1 -= s * (f * d1);
                   c2 -= s * (f * d2);
                 });
-  for_neighbors(S, xi, ci, S.bstart, S.bxV,
+  boundary_neighbors(S, i, info, xi,
                 [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
                   const T f = S.K.gradf(r2);
                   const T s = ((T(0.7) * T(2)) * S.rho0) * (pj.w / (rhoi * rhoi));
@@ -259,26 +315,26 @@ __global__ __launch_bounds__(kBlock) void k_iisph_c(SceneView<T> S) {
 
 // ---- iisph.setup pass 2 (iisph.hpp:252-354): p = 0, source s, diagonal AA
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_iisph_s_aa(SceneView<T> S) {
+__global__ __launch_bounds__(kBlock) void k_iisph_s_aa(SceneView<T> S, NbrList L) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   if (i >= S.nf)
     return;
   const vec4_t<T> xi = S.xm[i], vi = S.v[i], ci = S.c[i];
   const T rhoi = S.rho[i];
   const T mi = xi.w;
-  const uint32_t cell = S.fcell[i];
+  const uint32_t info = L.info[i];
   T s = 0, AA = 0;
-  for_neighbors(S, xi, cell, S.fstart, S.xm,
-                [&](uint32_t j, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
-                  const vec4_t<T> vj = S.v[j];
+  fluid_neighbors(S, L, i, info, xi, [&](uint32_t j) { return S.v[j]; },
+                [&](T d0, T d1, T d2, T r2, const vec4_t<T> &pj, const vec4_t<T> &vj) {
                   const T f = S.K.gradf(r2);
                   const T g0 = f * d0, g1 = f * d1, g2 = f * d2;
                   s += pj.w * dot3_exact(vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, g0, g1, g2);
                   AA += pj.w * dot3_exact(ci.x, ci.y, ci.z, g0, g1, g2);
                   AA -= (pj.w * (mi / (rhoi * rhoi))) * dot3_exact(g0, g1, g2, g0, g1, g2);
                 });
-  for_neighbors(S, xi, cell, S.bstart, S.bxV,
+  boundary_neighbors(S, i, info, xi,
                 [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
                   const T f = S.K.gradf(r2);
                   const T g0 = f * d0, g1 = f * d1, g2 = f * d2;
@@ -295,27 +351,31 @@ __global__ __launch_bounds__(kBlock) void k_iisph_s_aa(SceneView<T> S) {
 
 // ---- iisph.iteration_pressure_acceleration (iisph.hpp:358-423)
 template <class T, bool kSolve>
-__global__ __launch_bounds__(kBlock) void k_iisph_accel(SceneView<T> S) {
+__global__ __launch_bounds__(kBlock) void k_iisph_accel(SceneView<T> S, NbrList L) {
 #pragma clang fp contract(off)
   if (kSolve && S.ctl->done)
     return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   if (i >= S.nf)
     return;
   const vec4_t<T> xi = S.xm[i];
   const T rhoi = S.rho[i], pi = S.p[i];
-  const uint32_t cell = S.fcell[i];
+  const uint32_t info = L.info[i];
   T a0 = 0, a1 = 0, a2 = 0;
-  for_neighbors(S, xi, cell, S.fstart, S.xm,
-                [&](uint32_t j, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
-                  const T rhoj = S.rho[j];
+  struct PR {
+    T p, rho;
+  };
+  fluid_neighbors(S, L, i, info, xi, [&](uint32_t j) { return PR{S.p[j], S.rho[j]}; },
+                [&](T d0, T d1, T d2, T r2, const vec4_t<T> &pj, const PR &q) {
+                  const T rhoj = q.rho;
                   const T f = S.K.gradf(r2);
-                  const T s = pj.w * ((pi / (rhoi * rhoi)) + (S.p[j] / (rhoj * rhoj)));
+                  const T s = pj.w * ((pi / (rhoi * rhoi)) + (q.p / (rhoj * rhoj)));
                   a0 -= s * (f * d0);
                   a1 -= s * (f * d1);
                   a2 -= s * (f * d2);
                 });
-  for_neighbors(S, xi, cell, S.bstart, S.bxV,
+  boundary_neighbors(S, i, info, xi,
                 [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
                   const T f = S.K.gradf(r2);
                   const T s = ((T(0.7) * S.rho0) * pj.w) * ((T(2) * pi) / (rhoi * rhoi));
@@ -331,25 +391,25 @@ __global__ __launch_bounds__(kBlock) void k_iisph_accel(SceneView<T> S) {
 //      block order and takes the convergence decision of example.lua:418-419
 //      on the device when kSolve.
 template <class T, bool kSolve>
-__global__ __launch_bounds__(kBlock) void k_iisph_pressure(SceneView<T> S) {
+__global__ __launch_bounds__(kBlock) void k_iisph_pressure(SceneView<T> S, NbrList L) {
 #pragma clang fp contract(off)
   if (kSolve && S.ctl->done)
     return;
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   double term = 0.0;
   if (i < S.nf) {
     const vec4_t<T> xi = S.xm[i], ai = S.a[i];
     const T rhoi = S.rho[i];
-    const uint32_t cell = S.fcell[i];
+    const uint32_t info = L.info[i];
     T Ap = 0;
-    for_neighbors(S, xi, cell, S.fstart, S.xm,
-                  [&](uint32_t j, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
-                    const vec4_t<T> aj = S.a[j];
+    fluid_neighbors(S, L, i, info, xi, [&](uint32_t j) { return S.a[j]; },
+                  [&](T d0, T d1, T d2, T r2, const vec4_t<T> &pj, const vec4_t<T> &aj) {
                     const T f = S.K.gradf(r2);
                     Ap += pj.w * dot3_exact(ai.x - aj.x, ai.y - aj.y, ai.z - aj.z, f * d0,
                                             f * d1, f * d2);
                   });
-    for_neighbors(S, xi, cell, S.bstart, S.bxV,
+    boundary_neighbors(S, i, info, xi,
                   [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
                     const T f = S.K.gradf(r2);
                     Ap += (S.rho0 * pj.w) * dot3_exact(ai.x, ai.y, ai.z, f * d0, f * d1, f * d2);
@@ -366,7 +426,7 @@ __global__ __launch_bounds__(kBlock) void k_iisph_pressure(SceneView<T> S) {
   }
   const double bs = block_sum<kBlock>(term);
   if (threadIdx.x == 0)
-    S.partials[blockIdx.x] = bs;
+    S.partials[lb] = bs;
 }
 
 // aprde = sum of the block partials in block order (FP64); kSolve also takes
@@ -494,13 +554,13 @@ void SphOps<T>::volume(hipStream_t st, const SceneView<T> &S) {
     hipLaunchKernelGGL(k_volume<T>, dim3(grid_blocks(S.nb)), dim3(kBlock), 0, st, S);
 }
 
-#define PRTCL_FLUID_LAUNCH(kern)                                                     \
+#define PRTCL_FLUID_LAUNCH(kern, ...)                                                \
   if (S.nf > 0)                                                                      \
-  hipLaunchKernelGGL(kern, dim3(grid_blocks(S.nf)), dim3(kBlock), 0, st, S)
+  hipLaunchKernelGGL(kern, dim3(grid_blocks(S.nf)), dim3(kBlock), 0, st, S, ##__VA_ARGS__)
 
 template <class T>
-void SphOps<T>::density(hipStream_t st, const SceneView<T> &S) {
-  PRTCL_FLUID_LAUNCH(k_density<T>);
+void SphOps<T>::density(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
+  PRTCL_FLUID_LAUNCH(k_density<T>, L);
 }
 template <class T>
 void SphOps<T>::gravity(hipStream_t st, const SceneView<T> &S) {
@@ -515,8 +575,8 @@ void SphOps<T>::gravity_axial(hipStream_t st, const SceneView<T> &S) {
   PRTCL_FLUID_LAUNCH(k_gravity_axial<T>);
 }
 template <class T>
-void SphOps<T>::viscosity(hipStream_t st, const SceneView<T> &S) {
-  PRTCL_FLUID_LAUNCH(k_viscosity<T>);
+void SphOps<T>::viscosity(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
+  PRTCL_FLUID_LAUNCH(k_viscosity<T>, L);
 }
 template <class T>
 void SphOps<T>::integrate_v(hipStream_t st, const SceneView<T> &S) {
@@ -548,29 +608,31 @@ void SphOps<T>::integrate_x(hipStream_t st, const SceneView<T> &S) {
   hipLaunchKernelGGL(k_speed_finalize<T>, dim3(1), dim3(kBlock), 0, st, S.ctl, S.partials, nb);
 }
 template <class T>
-void SphOps<T>::iisph_setup(hipStream_t st, const SceneView<T> &S) {
-  PRTCL_FLUID_LAUNCH(k_iisph_c<T>);
-  PRTCL_FLUID_LAUNCH(k_iisph_s_aa<T>);
+void SphOps<T>::iisph_setup(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
+  PRTCL_FLUID_LAUNCH(k_iisph_c<T>, L);
+  PRTCL_FLUID_LAUNCH(k_iisph_s_aa<T>, L);
 }
 template <class T>
-void SphOps<T>::iisph_accel(hipStream_t st, const SceneView<T> &S, bool solve) {
+void SphOps<T>::iisph_accel(hipStream_t st, const SceneView<T> &S, const NbrList &L,
+                            bool solve) {
   if (solve) {
-    PRTCL_FLUID_LAUNCH((k_iisph_accel<T, true>));
+    PRTCL_FLUID_LAUNCH((k_iisph_accel<T, true>), L);
   } else {
-    PRTCL_FLUID_LAUNCH((k_iisph_accel<T, false>));
+    PRTCL_FLUID_LAUNCH((k_iisph_accel<T, false>), L);
   }
 }
 template <class T>
-void SphOps<T>::iisph_pressure(hipStream_t st, const SceneView<T> &S, bool solve) {
+void SphOps<T>::iisph_pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L,
+                               bool solve) {
   if (S.nf <= 0)
     return;
   const unsigned nb = grid_blocks(S.nf);
   if (solve) {
-    hipLaunchKernelGGL((k_iisph_pressure<T, true>), dim3(nb), dim3(kBlock), 0, st, S);
+    hipLaunchKernelGGL((k_iisph_pressure<T, true>), dim3(nb), dim3(kBlock), 0, st, S, L);
     hipLaunchKernelGGL(k_pressure_finalize<true>, dim3(1), dim3(kBlock), 0, st, S.ctl,
                        S.partials, nb);
   } else {
-    hipLaunchKernelGGL((k_iisph_pressure<T, false>), dim3(nb), dim3(kBlock), 0, st, S);
+    hipLaunchKernelGGL((k_iisph_pressure<T, false>), dim3(nb), dim3(kBlock), 0, st, S, L);
     hipLaunchKernelGGL(k_pressure_finalize<false>, dim3(1), dim3(kBlock), 0, st, S.ctl,
                        S.partials, nb);
   }

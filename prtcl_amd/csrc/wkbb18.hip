@@ -187,7 +187,7 @@ __device__ __forceinline__ void corr_body(const SceneView<T> &S, const NbrList &
   };
   const uint32_t info = kList ? L.info[i] : kListOverflow;
   if (kList && !(info & kListOverflow)) {
-    list_visit(L, Spans::of(L.blk[i / kBlock]), static_cast<size_t>(S.nf), i, info,
+    list_visit(L, list_spans(L, i), static_cast<size_t>(S.nf), i, info,
                [&](uint32_t j) {
                  const vec4_t<T> pj = S.xm[j];
                  const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void k_diag_list(SceneView<T> S, NbrList L)
   };
   const uint32_t info = L.info[i];
   if (!(info & kListOverflow)) {
-    list_visit(L, Spans::of(L.blk[i / kBlock]), n, i, info, fluid);
+    list_visit(L, list_spans(L, i), n, i, info, fluid);
   } else {
     nbrs_exact(S, xi, S.fcell[i], S.fstart, S.xm,
                [&](uint32_t j, T, T, T, T, const vec4_t<T> &) {
@@ -526,7 +526,7 @@ __device__ __forceinline__ void product_list(const SceneView<T> &S, const NbrLis
   auto use = [&](const XW &q) { pair(xq, wi, q.x, q.w, l0, l1, l2); };
   const uint32_t info = L.info[i];
   if (!(info & kListOverflow)) {
-    list_gather<4>(L, Spans::of(L.blk[i / kBlock]), n, i, info,
+    list_gather<4>(L, list_spans(L, i), n, i, info,
                    [&](uint32_t j) {
                      return XW{S.cxp[2 * static_cast<size_t>(j)], w[static_cast<size_t>(ws) * j]};
                    },
@@ -631,7 +631,7 @@ __device__ __forceinline__ void diag_setup_list_body(const SceneView<T> &S, cons
     };
     const uint32_t info = L.info[i];
     if (!(info & kListOverflow)) {
-      list_gather<4>(L, Spans::of(L.blk[i / kBlock]), n, i, info,
+      list_gather<4>(L, list_spans(L, i), n, i, info,
                      [&](uint32_t j) { return P{S.xm[j], S.rho[j], S.v[j]}; }, both);
     } else {
       nbrs_exact(S, xi, S.fcell[i], S.fstart, S.xm,
@@ -846,7 +846,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_apply(SceneView<T> S) {
 // beta in its vector kernels, otherwise its one-block kernels do.
 template <class T>
 __device__ __forceinline__ NbrList entry_list(const BatchEntry<T> &E) {
-  return NbrList{E.nidx, E.ninfo, E.nblk};
+  return NbrList{E.nidx, E.ninfo, E.nblk, E.nshift};
 }
 
 template <class T, bool kGC>

@@ -1,0 +1,110 @@
+"""The passes that give a particle several lanes (scenes of up to 16,384
+particles) and the procedures' list, at the sizes where they change: groups of
+32 and 64 particles with remainders, and the line between one lane and several.
+Bars: density is one pair sum in another order (2e-5 of the field's scale, as for
+the single procedures), position after one step as for whole steps (1e-5)."""
+
+import numpy as np
+import pytest
+
+from prtcl_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+SPLIT = 16384  # kSplitMax
+
+
+def _block(n, seed=4):
+    """n particles of a jittered block in a box, moving."""
+    s = 0.025
+    side = int(np.ceil(n ** (1 / 3)))
+    box = scenes.box_boundary(side + 4, side + 4, side + 4, s)
+    fx = scenes.fluid_block((side, side, side), (1, 1, 1), s, 1e-3, scenes.stream_base(seed, n))
+    v = np.random.default_rng(n).uniform(-0.2, 0.2, (n, 3))
+    sc = scenes._finish(f"block{n}", s, fx[:n], box, 1, v=v)
+    sc.permute_every = 0
+    return sc
+
+
+def _close(gpu, ref, rtol, what):
+    scale = float(np.max(np.abs(ref)))
+    err = float(np.max(np.abs(np.asarray(gpu, np.float64) - ref))) / scale
+    assert err <= rtol, f"{what}: {err:.3e} > {rtol:.1e}"
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 65, 255, 257, 1025, SPLIT, SPLIT + 1])
+def test_step_sizes_vs_oracle(hip_ctx, oracle_lib, n):
+    from prtcl_amd import hip
+    sc = _block(n)
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    g = hip.HipScene(hip_ctx, sc)
+    o.prepare()
+    g.prepare()
+    o.step()
+    g.step(1)
+    _close(g.download("fluid", "density"), o.get("fluid", "density"), 2e-5, "density")
+    _close(g.download("fluid", "position"), o.get("fluid", "position"), 1e-5, "position")
+    g.destroy()
+
+
+def test_batch_of_both_kinds_equals_alone(hip_ctx):
+    """One launch over scenes with several lanes per particle and one beyond the
+    line, whose blocks differ in size: each as it is alone."""
+    from prtcl_amd import hip
+    out = []
+    for together in (True, False):
+        hs = [hip.HipScene(hip_ctx, _block(n)) for n in (300, SPLIT + 1, 33, SPLIT)]
+        for h in hs:
+            h.prepare()
+        for _ in range(2):
+            if together:
+                hip_ctx.step(hs, 1)
+            else:
+                for h in hs:
+                    h.step(1)
+        out.append([(h.step_info(), h.download("fluid", "velocity"),
+                     h.download("fluid", "pressure")) for h in hs])
+        for h in hs:
+            h.destroy()
+    for (ia, va, pa), (ib, vb, pb) in zip(*out):
+        assert ia == ib
+        np.testing.assert_array_equal(va, vb)
+        np.testing.assert_array_equal(pa, pb)
+
+
+@pytest.mark.parametrize("spacing", [1.0, 0.6], ids=["list", "overflow"])
+def test_procedures_follow_the_positions(hip_ctx, oracle_lib, spacing):
+    """A procedure between two changes of the positions reads a list that an
+    earlier one built; after an upload, an update or an integration it must see
+    the new positions (lists that overflow walk the grid)."""
+    from prtcl_amd import hip
+    s = 0.025
+    fx = scenes.fluid_block((9, 9, 9), (3, 3, 3), spacing * s, 1e-4, scenes.stream_base(9, 0))
+    sc = scenes._finish("moving", s, fx, scenes.box_boundary(15, 15, 15, s), 1)
+    sc.permute_every = 0
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    g = hip.HipScene(hip_ctx, sc)
+    o.prepare()
+    g.prepare()
+
+    def same(what):
+        for x in (o, g):
+            x.run("density.compute_density")
+        _close(g.download("fluid", "density"), o.get("fluid", "density"), 2e-5, what)
+
+    same("first")
+    moved = fx[:, [1, 2, 0]] + np.float32(0.3 * s)
+    g.upload("fluid", "position", moved)
+    g.run("neighborhood.update")
+    o.set("fluid", "position", moved)
+    o.update()
+    same("after an upload")
+    v = np.random.default_rng(1).uniform(-5, 5, fx.shape).astype(np.float32)
+    g.upload("fluid", "velocity", v)
+    o.set("fluid", "velocity", v)
+    for x in (o, g):
+        x.run("symplectic_euler.integrate_position")
+    g.run("neighborhood.update")
+    o.update()
+    same("after an integration")
+    g.destroy()
