@@ -204,7 +204,7 @@ __device__ __forceinline__ void list_gather(const NbrList &L, const Spans &R, si
 // 7.3, 250,000: 13.6 -> 13.6; pressure pass 8.1 -> 4.7, 8.3 -> 4.9, 8.0 -> 7.1,
 // 10.0 -> 10.4, 20.7 -> 21.3. The rule depends on the scene alone, so that a
 // scene's results are the same alone and in a batch; a batch fills the chip, and
-// tthere the lanes' idle slots cost: with the line at 65,536, 16 scenes of
+// there the lanes' idle slots cost: with the line at 65,536, 16 scenes of
 // 2,000 to 200,000 particles took 11.83 ms instead of 11.60 ms for 10 steps. Below
 // 16,384 a batch's share of the work is too small to show.
 constexpr int kSplitMax = 16384;

@@ -27,35 +27,31 @@ struct Pt16Ops {
   // target velocity gradient += cross_product_matrix(0.5 w) (pt16.hpp:521-535)
   static void spin(hipStream_t st, const SceneView<T> &S);
   // which = 0: vorticity diffusion (system diagonal pt16_same_density, guess
-  // and result in vorticity[dim]); which = 1: velocity reconstruction
-  // (diagonal pt16_density, guess and result in velocity[dim])
+  // and result in the vorticity); which = 1: velocity reconstruction
+  // (diagonal pt16_density, guess and result in the velocity). part: room for
+  // 9 partials per list block, and for 3 per list block and 6 per block
   static void cg_setup(hipStream_t st, const SceneView<T> &S, const NbrList *L, int which,
-                       int dim, double *part, double tol, int max_k, unsigned seq);
+                       double *part, double tol, int max_k, unsigned seq);
   // split: the alpha and beta reductions in one-block kernels of their own
   // (always so above kFusedCgBlocks blocks); the results do not depend on it
   static void cg_iteration(hipStream_t st, const SceneView<T> &S, const NbrList *L, int which,
                            double *part, bool split);
-  static void cg_apply(hipStream_t st, const SceneView<T> &S, int which, int dim);
-  // the same over every pt16 scene of a batch (list forms; map: block map of
-  // the scenes' blocks); each table entry carries the scene's xi, CG
-  // partials, the tolerance and cap of both systems, the sequence number of
-  // the step's first solve (solve s = 0..5 runs under cg_seq + s) and the
-  // fold choice. any_split: some scene takes alpha and beta from the
-  // one-block kernels
-  static void setup_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                          unsigned nblocks);
-  static void omega_rhs_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                              unsigned nblocks);
-  static void spin_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                         unsigned nblocks);
-  static void vrec_rhs_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                             unsigned nblocks);
-  static void cg_setup_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                             unsigned nblocks, unsigned nscenes, int which, int dim, int solve);
-  static void cg_iteration_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                                 unsigned nblocks, unsigned nscenes, int which, bool any_split);
-  static void cg_apply_batch(hipStream_t st, const BatchEntry<T> *tab, const uint32_t *map,
-                             unsigned nblocks, int which, int dim);
+  static void cg_apply(hipStream_t st, const SceneView<T> &S, int which);
+  // the same over every pt16 scene of a batch (list forms); each table entry
+  // carries the scene's xi, CG partials, the tolerance and cap of both systems,
+  // the sequence number of the step's first solve (the second runs under the
+  // next) and the fold choice. any_split: some scene takes alpha and beta from
+  // the one-block kernels
+  static void setup_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B);
+  static void omega_rhs_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B);
+  static void spin_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B);
+  static void vrec_rhs_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B);
+  static void cg_setup_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
+                             unsigned nscenes, int which);
+  static void cg_iteration_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
+                                 unsigned nscenes, int which, bool any_split);
+  static void cg_apply_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
+                             int which);
 };
 
 }  // namespace prtcl_amd

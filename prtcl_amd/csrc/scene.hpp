@@ -58,6 +58,11 @@ struct Ctl {
   int cg_iter, cg_done, cg_max_k;
   int cg_iter_next;  // cg_iter + 1, set beside alpha (read while cg_iter is written)
   double cg_tol;
+  // three scalar systems solved side by side (cg_ctl.hpp)
+  struct Cg3 {
+    double thr[3], ry[3], ry_prev[3], alpha[3], beta[3];
+    int iter[3], iter_next[3], done[3];
+  } c3;
   // end-of-step report: steps finished (integrations of the position) and
   // how many of them produced a non-finite position or speed; published to
   // host_mirror[3] as (step_count << 32) | nonfinite_steps
@@ -77,8 +82,9 @@ __device__ __forceinline__ bool integrate_now(const Ctl *c, unsigned seq) {
 }
 
 // host_mirror words: [0] IISPH progress, [1] its aprde / nprde, [2] CG
-// progress, [3] end-of-step report
+// progress, [3] end-of-step report, [4] see kMirrorCg3
 constexpr int kMirrorStep = 3;
+constexpr int kMirrorCg3 = 4;  // iterations of the third component of a pt16 solve
 
 // Counts the finished step (one thread; after the integration kernel of the
 // step): folds the non-finite flag of the step into the running count,
@@ -183,10 +189,10 @@ struct SceneView {
   T *gc;  // gradient correction L (3x3 column-major per fluid particle)
   // pt16 (scenes with implicit viscosity 3; empty otherwise): vorticity, the
   // right-hand sides of its two systems, the target velocity gradient (3x3
-  // column-major), pt16_density, pt16_same_density and the scalar PCG vectors
+  // column-major), pt16_density and pt16_same_density; its PCG vectors are
+  // those of WKBB18 (p in the first half of cxp)
   V4 *om, *orhs, *vrhs;
   T *tvg, *prho, *psrho;
-  T *scx, *scr, *scp, *scq, *scy;
   // list form of the pt16 products (fused steps): m_j W_ij of list entry e of
   // particle i at pcoef[((e / 4) * nf + i) * 4 + e % 4], written once per step
   T *pcoef;

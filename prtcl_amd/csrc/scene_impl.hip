@@ -867,11 +867,6 @@ class SceneImpl final : public SceneBase {
     S.tvg = P_.tvg;
     S.prho = P_.prho;
     S.psrho = P_.psrho;
-    S.scx = P_.scx;
-    S.scr = P_.scr;
-    S.scp = P_.scp;
-    S.scq = P_.scq;
-    S.scy = P_.scy;
     S.pcoef = P_.pcoef;
     S.id = P_.id;
     S.fcell = P_.fcell;
@@ -1065,10 +1060,18 @@ class SceneImpl final : public SceneBase {
     return p;
   }
 
+  // iterations of the third component of the last pt16 solve (published with its
+  // progress, before the host saw it done)
+  int last_component_iters() const {
+    return nf_ > 0 ? static_cast<int>(__atomic_load_n(&mirror_host_[kMirrorCg3], __ATOMIC_ACQUIRE))
+                   : 0;
+  }
+
   // pt16.setup / solve_vorticity_diffusion / vorticity_preservation /
   // solve_velocity_reconstruction (pt16.hpp:213-760); each solve is one scalar
-  // PCG per vector component with tolerance pt16_maximum_error and cap
-  // pt16_maximum_iterations, pt16_iterations = the last component's count
+  // PCG per vector component, the three side by side, with tolerance
+  // pt16_maximum_error and cap pt16_maximum_iterations, pt16_iterations = the
+  // last component's count
   // with `fused` the fluid sums and the CG products use the step's
   // neighbour list (the pair coefficients are written by the set-up)
   void run_pt16(int proc, bool fused = false) {
@@ -1082,28 +1085,26 @@ class SceneImpl final : public SceneBase {
     const T xi = static_cast<T>(pt16_xi_);
     const bool split = tuner_.current().cg_split;
     auto solve = [&](int which) {
-      for (int dim = 0; dim < 3; ++dim) {
-        const unsigned seq = ++seq_;
-        const int max_k = std::max(0, pt16_max_k_);
-        int r = pf.begin(st, kStagePcgVector);
-        Pt16Ops<T>::cg_setup(st, S, pl, which, dim, P_.cg_part, pt16_tol_, max_k, seq);
-        pf.end(st, r);
-        const Progress p = cg_loop(seq, max_k, predicted_pt16_[which], [&](int tag) {
-          const int rp = pf.begin(st, kStagePcgSpmv, tag);
-          Pt16Ops<T>::cg_iteration(st, S, pl, which, P_.cg_part, split);
-          pf.end(st, rp);
-        });
-        r = pf.begin(st, kStagePcgVector);
-        Pt16Ops<T>::cg_apply(st, S, which, dim);
-        pf.end(st, r);
-        PRTCL_HIP_CHECK(hipGetLastError());
-        if (pf.on) {
-          PRTCL_HIP_CHECK(hipStreamSynchronize(st));
-          pf.resolve(p.iters);
-        }
-        predicted_pt16_[which] = std::max(1, p.iters);
-        pt16_iters_ = p.iters;
+      const unsigned seq = ++seq_;
+      const int max_k = std::max(0, pt16_max_k_);
+      int r = pf.begin(st, kStagePcgVector);
+      Pt16Ops<T>::cg_setup(st, S, pl, which, P_.cg_part, pt16_tol_, max_k, seq);
+      pf.end(st, r);
+      const Progress p = cg_loop(seq, max_k, predicted_pt16_[which], [&](int tag) {
+        const int rp = pf.begin(st, kStagePcgSpmv, tag);
+        Pt16Ops<T>::cg_iteration(st, S, pl, which, P_.cg_part, split);
+        pf.end(st, rp);
+      });
+      r = pf.begin(st, kStagePcgVector);
+      Pt16Ops<T>::cg_apply(st, S, which);
+      pf.end(st, r);
+      PRTCL_HIP_CHECK(hipGetLastError());
+      if (pf.on) {
+        PRTCL_HIP_CHECK(hipStreamSynchronize(st));
+        pf.resolve(p.iters);
       }
+      predicted_pt16_[which] = std::max(1, p.iters);
+      pt16_iters_ = last_component_iters();
     };
     int r = pf.begin(st, kStagePt16Setup);
     switch (proc) {
@@ -1573,11 +1574,7 @@ class SceneImpl final : public SceneBase {
       if (!v[k]->desc.implicit_viscosity)
         continue;
       if (v[k]->desc.implicit_viscosity == 3) {
-        const unsigned kp = static_cast<unsigned>(psc.size());
         psc.push_back(k);
-        const unsigned nb = grid_blocks(v[k]->nf_);
-        for (unsigned b = 0; b < nb; ++b)
-          ptlist.push_back((kp << kBatchLocalBits) | b);
         continue;
       }
       const unsigned kv = static_cast<unsigned>(vsc.size());
@@ -1589,6 +1586,15 @@ class SceneImpl final : public SceneBase {
         (gc ? vlist_g : vlist_n).push_back((kv << kBatchLocalBits) | b);
       }
     }
+    // the pt16 scenes' blocks (entries of their own table), one-lane scenes first
+    BatchBlocks pblocks{};
+    for (int run = 0; run < 2; ++run)
+      for (unsigned kp = 0; kp < psc.size(); ++kp)
+        if (split_scene(v[psc[kp]]->nf_) == (run == 1))
+          for (unsigned b = 0; b < grid_blocks(v[psc[kp]]->nf_); ++b) {
+            ptlist.push_back((kp << kBatchLocalBits) | b);
+            ++pblocks.n[run];
+          }
     const unsigned np = static_cast<unsigned>(plist.size());
     const unsigned nt = static_cast<unsigned>(tlist.size());
     const unsigned nvs = static_cast<unsigned>(vsc.size());
@@ -1643,7 +1649,7 @@ class SceneImpl final : public SceneBase {
     auto *t_pt = reinterpret_cast<BatchEntry<T> *>(hb + off_pt);
     uint32_t *ptmap = reinterpret_cast<uint32_t *>(hb + off_ptmap);
     for (unsigned b = 0; b < npb; ++b)
-      ptmap[b] = ptlist[xcd_of(b, npb)];
+      ptmap[b] = ptlist[b];
     // the pointer swaps of build_fluid_grid() and of the setup pass are done
     // on the host while the three tables are filled
     std::vector<char> permute(ns, 0);
@@ -1721,9 +1727,8 @@ class SceneImpl final : public SceneBase {
       any_split = any_split || !E.cg_fold;
       t_visc[kv] = E;
     }
-    // pt16 after the IISPH solve: six scalar CG solves (vorticity and
-    // velocity components) under six consecutive sequence numbers, as
-    // run_pt16 takes them
+    // pt16 after the IISPH solve: two solves (vorticity, velocity) under two
+    // consecutive sequence numbers, as run_pt16 takes them
     bool pt_any_split = false;
     std::vector<unsigned> pt_seq0(nps);
     for (unsigned kp = 0; kp < nps; ++kp) {
@@ -1736,7 +1741,7 @@ class SceneImpl final : public SceneBase {
       E.pt16_tol[1] = s.desc.pt16_velocity_maximum_error;
       E.pt16_max_k[1] = std::max(0, static_cast<int>(s.desc.pt16_velocity_maximum_iterations));
       pt_seq0[kp] = s.seq_ + 1;
-      s.seq_ += 6;
+      s.seq_ += 2;
       E.cg_seq = pt_seq0[kp];
       E.cg_fold = !cg_split && E.nblocks <= kFusedCgBlocks ? 1 : 0;
       pt_any_split = pt_any_split || !E.cg_fold;
@@ -1756,7 +1761,7 @@ class SceneImpl final : public SceneBase {
     const auto *d_visc = reinterpret_cast<const BatchEntry<T> *>(db + off_visc);
     const auto *d_vmap = reinterpret_cast<const uint32_t *>(db + off_vmap);
     const auto *d_pt = reinterpret_cast<const BatchEntry<T> *>(db + off_pt);
-    const auto *d_ptmap = reinterpret_cast<const uint32_t *>(db + off_ptmap);
+    pblocks.map = reinterpret_cast<const uint32_t *>(db + off_ptmap);
     blocks.map = d_pmap;
     BatchMaps vm;
     vm.all = reinterpret_cast<const uint32_t *>(db + off_vmap);
@@ -1993,52 +1998,50 @@ class SceneImpl final : public SceneBase {
     // spin, velocity reconstruction (three solves, which write the
     // velocity), integrate x
     std::vector<Progress> ptp(nps);
-    std::vector<int> pt_last(nps * 2, 0);
     if (nps > 0) {
       r = pf.begin(st, kStageGravityIntegrateV);
-      SphOps<T>::integrate_v_batch(st, d_pt, d_ptmap, npb, true);
+      SphOps<T>::integrate_v_batch(st, d_pt, pblocks.map, npb, true);
       pf.end(st, r);
       r = pf.begin(st, kStagePt16Setup);
-      Pt16Ops<T>::setup_batch(st, d_pt, d_ptmap, npb);
-      Pt16Ops<T>::omega_rhs_batch(st, d_pt, d_ptmap, npb);
+      Pt16Ops<T>::setup_batch(st, d_pt, pblocks);
+      Pt16Ops<T>::omega_rhs_batch(st, d_pt, pblocks);
       pf.end(st, r);
       for (int which = 0; which < 2; ++which) {
         if (which == 1) {
-          Pt16Ops<T>::spin_batch(st, d_pt, d_ptmap, npb);
+          Pt16Ops<T>::spin_batch(st, d_pt, pblocks);
           r = pf.begin(st, kStagePt16Setup);
-          Pt16Ops<T>::vrec_rhs_batch(st, d_pt, d_ptmap, npb);
+          Pt16Ops<T>::vrec_rhs_batch(st, d_pt, pblocks);
           pf.end(st, r);
         }
         int cap = 1, pred = 1;
+        std::vector<unsigned> seqs_s(nps);
         for (unsigned kp = 0; kp < nps; ++kp) {
           const SceneImpl &s = *v[psc[kp]];
           const int mk = which == 0 ? s.desc.pt16_vorticity_maximum_iterations
                                     : s.desc.pt16_velocity_maximum_iterations;
           cap = std::max(cap, std::max(0, mk) + 1);
           pred = std::max(pred, std::min(std::max(1, s.predicted_pt16_[which]), 16));
+          seqs_s[kp] = pt_seq0[kp] + static_cast<unsigned>(which);
         }
-        for (int dim = 0; dim < 3; ++dim) {
-          const int solve = 3 * which + dim;
-          std::vector<unsigned> seqs_s(nps);
-          for (unsigned kp = 0; kp < nps; ++kp)
-            seqs_s[kp] = pt_seq0[kp] + static_cast<unsigned>(solve);
-          r = pf.begin(st, kStagePcgVector);
-          Pt16Ops<T>::cg_setup_batch(st, d_pt, d_ptmap, npb, nps, which, dim, solve);
-          pf.end(st, r);
-          ptp = cg_loop_batch(psc, seqs_s, pred, cap, [&](int tag) {
-            const int q1 = pf.begin(st, kStagePcgSpmv, tag);
-            Pt16Ops<T>::cg_iteration_batch(st, d_pt, d_ptmap, npb, nps, which, pt_any_split);
-            pf.end(st, q1);
-          });
-          r = pf.begin(st, kStagePcgVector);
-          Pt16Ops<T>::cg_apply_batch(st, d_pt, d_ptmap, npb, which, dim);
-          pf.end(st, r);
-          for (unsigned kp = 0; kp < nps; ++kp)
-            pt_last[2 * kp + which] = ptp[kp].iters;
+        r = pf.begin(st, kStagePcgVector);
+        Pt16Ops<T>::cg_setup_batch(st, d_pt, pblocks, nps, which);
+        pf.end(st, r);
+        ptp = cg_loop_batch(psc, seqs_s, pred, cap, [&](int tag) {
+          const int q1 = pf.begin(st, kStagePcgSpmv, tag);
+          Pt16Ops<T>::cg_iteration_batch(st, d_pt, pblocks, nps, which, pt_any_split);
+          pf.end(st, q1);
+        });
+        r = pf.begin(st, kStagePcgVector);
+        Pt16Ops<T>::cg_apply_batch(st, d_pt, pblocks, which);
+        pf.end(st, r);
+        for (unsigned kp = 0; kp < nps; ++kp) {
+          SceneImpl &s = *v[psc[kp]];
+          s.predicted_pt16_[which] = std::max(1, ptp[kp].iters);
+          s.pt16_iters_ = s.last_component_iters();
         }
       }
       r = pf.begin(st, kStageIntegrateX);
-      SphOps<T>::integrate_x_batch(st, d_pt, d_ptmap, npb, nps);
+      SphOps<T>::integrate_x_batch(st, d_pt, pblocks.map, npb, nps);
       pf.end(st, r);
     }
     if (fixed)  // the last kernel reading the tables is enqueued
@@ -2050,13 +2053,9 @@ class SceneImpl final : public SceneBase {
       s.predicted_cg_ = std::max(1, cgp[kv].iters);
       s.last_wkbb_ = cgp[kv].iters;
     }
-    // as run_pt16 leaves them: the predictions from each system's last
-    // component, the velocity system's settings and last count
+    // as run_pt16 leaves them: the velocity system's settings
     for (unsigned kp = 0; kp < nps; ++kp) {
       SceneImpl &s = *v[psc[kp]];
-      s.predicted_pt16_[0] = std::max(1, pt_last[2 * kp]);
-      s.predicted_pt16_[1] = std::max(1, pt_last[2 * kp + 1]);
-      s.pt16_iters_ = pt_last[2 * kp + 1];
       s.pt16_tol_ = s.desc.pt16_velocity_maximum_error;
       s.pt16_max_k_ = s.desc.pt16_velocity_maximum_iterations;
     }
@@ -2216,7 +2215,7 @@ class SceneImpl final : public SceneBase {
     V4 *xm, *v, *a, *c, *G, *vd, *tmpV4, *xq, *xa;
     T *rho, *p, *pr, *s, *AA, *Ap, *tmpT, *sp, *tmpSp, *gc;
     V4 *om, *orhs, *vrhs;
-    T *tvg, *prho, *psrho, *pone, *odiag, *vdiag, *scx, *scr, *scp, *scq, *scy, *pcoef;
+    T *tvg, *prho, *psrho, *pone, *odiag, *vdiag, *pcoef;
     int32_t *id, *tmpI;
     uint32_t *fcell, *frank, *fperm, *ninfo;
     uint16_t *nidx;
@@ -2270,7 +2269,10 @@ class SceneImpl final : public SceneBase {
     // one per block of the largest launch that writes them
     A.take(P.partials, std::max({grid_blocks(static_cast<long>(std::max(f, b))),
                                  setup_blocks(nf), list_blocks(nf)}) + 1);
-    A.take(P.cg_part, 3 * static_cast<size_t>(grid_blocks(static_cast<long>(f))) + 3);
+    // WKBB18: 3 per block; pt16: 9 per list block in the set-up, 3 per list
+    // block and 6 per block in an iteration
+    A.take(P.cg_part, pt16 ? 9 * static_cast<size_t>(std::max(list_blocks(nf), 1u))
+                           : 3 * static_cast<size_t>(grid_blocks(static_cast<long>(f))) + 3);
     A.take(P.ctl, 1);
     const size_t nv = pcg ? f : 1;
     for (V4 **q : {&P.cgx, &P.cgr, &P.cgq, &P.cgy, &P.cgb})
@@ -2281,8 +2283,7 @@ class SceneImpl final : public SceneBase {
       A.take(*q, np);
     A.take(P.tvg, 9 * np);
     A.take(P.pcoef, pt16 ? static_cast<size_t>(kNbrCap) * f : 1);
-    for (T **q : {&P.prho, &P.psrho, &P.pone, &P.odiag, &P.vdiag, &P.scx, &P.scr, &P.scp,
-                  &P.scq, &P.scy})
+    for (T **q : {&P.prho, &P.psrho, &P.pone, &P.odiag, &P.vdiag})
       A.take(*q, np);
   }
 
@@ -2295,7 +2296,7 @@ class SceneImpl final : public SceneBase {
       f(reinterpret_cast<void **>(q));
     for (T **q : {&P_.rho, &P_.p, &P_.pr, &P_.s, &P_.AA, &P_.Ap, &P_.tmpT, &P_.sp, &P_.tmpSp,
                   &P_.gc, &P_.tvg, &P_.prho, &P_.psrho, &P_.pone, &P_.odiag, &P_.vdiag,
-                  &P_.scx, &P_.scr, &P_.scp, &P_.scq, &P_.scy, &P_.pcoef})
+                  &P_.pcoef})
       f(reinterpret_cast<void **>(q));
     for (int32_t **q : {&P_.id, &P_.tmpI, &P_.bid, &P_.btmpI, &P_.permd})
       f(reinterpret_cast<void **>(q));
@@ -2339,7 +2340,7 @@ class SceneImpl final : public SceneBase {
       Arena::rebase(*q, base);
     for (T **q : {&P_.rho, &P_.p, &P_.pr, &P_.s, &P_.AA, &P_.Ap, &P_.tmpT, &P_.sp, &P_.tmpSp,
                   &P_.gc, &P_.tvg, &P_.prho, &P_.psrho, &P_.pone, &P_.odiag, &P_.vdiag,
-                  &P_.scx, &P_.scr, &P_.scp, &P_.scq, &P_.scy, &P_.pcoef})
+                  &P_.pcoef})
       Arena::rebase(*q, base);
     for (int32_t **q : {&P_.id, &P_.tmpI, &P_.bid, &P_.btmpI, &P_.permd})
       Arena::rebase(*q, base);
@@ -2367,6 +2368,7 @@ class SceneImpl final : public SceneBase {
                                   4 * std::max<size_t>(1, size_t(nf_) + size_t(nb_)),
                                   hipHostMallocDefault));
     mirror_host_[0] = mirror_host_[1] = mirror_host_[2] = mirror_host_[kMirrorStep] = 0;
+    mirror_host_[kMirrorCg3] = 0;
     PRTCL_HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void **>(&mirror_dev_),
                                             mirror_host_, 0));
     ctl_op(kCtlInit);

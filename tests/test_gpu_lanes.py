@@ -14,14 +14,14 @@ pytestmark = pytest.mark.gpu
 SPLIT = 16384  # kSplitMax
 
 
-def _block(n, seed=4):
+def _block(n, seed=4, **kw):
     """n particles of a jittered block in a box, moving."""
     s = 0.025
     side = int(np.ceil(n ** (1 / 3)))
     box = scenes.box_boundary(side + 4, side + 4, side + 4, s)
     fx = scenes.fluid_block((side, side, side), (1, 1, 1), s, 1e-3, scenes.stream_base(seed, n))
     v = np.random.default_rng(n).uniform(-0.2, 0.2, (n, 3))
-    sc = scenes._finish(f"block{n}", s, fx[:n], box, 1, v=v)
+    sc = scenes._finish(f"block{n}", s, fx[:n], box, 1, v=v, **kw)
     sc.permute_every = 0
     return sc
 
@@ -43,6 +43,27 @@ def test_step_sizes_vs_oracle(hip_ctx, oracle_lib, n):
     o.step()
     g.step(1)
     _close(g.download("fluid", "density"), o.get("fluid", "density"), 2e-5, "density")
+    _close(g.download("fluid", "position"), o.get("fluid", "position"), 1e-5, "position")
+    g.destroy()
+
+
+@pytest.mark.parametrize("n", [31, 33, 65, 257])
+@pytest.mark.parametrize("iv", [1, 2, 3], ids=["wkbb18", "wkbb18_gc", "pt16"])
+def test_viscous_step_sizes_vs_oracle(hip_ctx, oracle_lib, iv, n):
+    """The CG of implicit viscosity with several lanes per particle (pt16: its three
+    components side by side). Both sides stop at a relative residual of 1e-4, if
+    need be one iteration apart: velocity to ten times that."""
+    from prtcl_amd import hip
+    sc = _block(n, implicit_viscosity=iv, fluid_viscosity=10.0, boundary_viscosity=10.0,
+                wkbb18_maximum_error=1e-4, pt16_vorticity_maximum_error=1e-4,
+                pt16_velocity_maximum_error=1e-4)
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    g = hip.HipScene(hip_ctx, sc)
+    o.prepare()
+    g.prepare()
+    o.step()
+    g.step(1)
+    _close(g.download("fluid", "velocity"), o.get("fluid", "velocity"), 1e-3, "velocity")
     _close(g.download("fluid", "position"), o.get("fluid", "position"), 1e-5, "position")
     g.destroy()
 
