@@ -1015,7 +1015,7 @@ class SceneImpl final : public SceneBase {
       Wkbb18Ops<T>::iteration_product(st, S, pl, gc, P_.cg_part);
       pf.end(st, rp);
       rp = pf.begin(st, kStagePcgVector, tag);
-      Wkbb18Ops<T>::iteration_vectors(st, S, P_.cg_part, split);
+      Wkbb18Ops<T>::iteration_vectors(st, S, pl, P_.cg_part, split);
       pf.end(st, rp);
     });
     r = pf.begin(st, kStagePcgVector);
@@ -1566,10 +1566,9 @@ class SceneImpl final : public SceneBase {
         tlist.push_back((k << kBatchLocalBits) | b);
     }
     // the scenes whose step ends with WKBB18 or pt16, with tables and block
-    // maps of their own: the WKBB18 scenes all together and, apart, those
-    // without and with the gradient correction; the pt16 scenes
+    // maps of their own
     std::vector<unsigned> vsc, psc;  // WKBB18 scenes, pt16 scenes
-    std::vector<uint32_t> vlist, vlist_n, vlist_g, ptlist;
+    std::vector<uint32_t> vlist, ptlist;
     for (unsigned k = 0; k < ns; ++k) {
       if (!v[k]->desc.implicit_viscosity)
         continue;
@@ -1577,15 +1576,21 @@ class SceneImpl final : public SceneBase {
         psc.push_back(k);
         continue;
       }
-      const unsigned kv = static_cast<unsigned>(vsc.size());
       vsc.push_back(k);
-      const unsigned nb = grid_blocks(v[k]->nf_);
-      const bool gc = v[k]->desc.implicit_viscosity == 2;
-      for (unsigned b = 0; b < nb; ++b) {
-        vlist.push_back((kv << kBatchLocalBits) | b);
-        (gc ? vlist_g : vlist_n).push_back((kv << kBatchLocalBits) | b);
-      }
     }
+    // the WKBB18 scenes' blocks (entries of their own table): those without, then
+    // those with the gradient correction
+    BatchBlocks vblocks{};
+    for (int run = 0; run < 4; ++run)
+      for (unsigned kv = 0; kv < vsc.size(); ++kv) {
+        const SceneImpl &s = *v[vsc[kv]];
+        if ((s.desc.implicit_viscosity == 2) == (run >= 2) &&
+            split_scene(s.nf_) == ((run & 1) != 0))
+          for (unsigned b = 0; b < grid_blocks(s.nf_); ++b) {
+            vlist.push_back((kv << kBatchLocalBits) | b);
+            ++vblocks.n[run];
+          }
+      }
     // the pt16 scenes' blocks (entries of their own table), one-lane scenes first
     BatchBlocks pblocks{};
     for (int run = 0; run < 2; ++run)
@@ -1599,23 +1604,18 @@ class SceneImpl final : public SceneBase {
     const unsigned nt = static_cast<unsigned>(tlist.size());
     const unsigned nvs = static_cast<unsigned>(vsc.size());
     const unsigned nvb = static_cast<unsigned>(vlist.size());
-    // the split maps only when some WKBB18 scene has the gradient correction
-    const unsigned nvg = static_cast<unsigned>(vlist_g.size());
-    const unsigned nvn = nvg > 0 ? static_cast<unsigned>(vlist_n.size()) : 0u;
+    const bool any_gc = vblocks.n[2] + vblocks.n[3] > 0;
     const unsigned nps = static_cast<unsigned>(psc.size());
     const unsigned npb = static_cast<unsigned>(ptlist.size());
     // pinned / device table layout: [sort | setup | solve] entries, the
-    // WKBB18 entries, pmap, tmap, vmap, the WKBB18 split maps, the pt16
-    // entries and map
+    // WKBB18 entries, pmap, tmap, vmap, the pt16 entries and map
     auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
     const size_t tab_bytes = align(sizeof(BatchEntry<T>) * ns);
     const size_t off_visc = 3 * tab_bytes;
     const size_t off_pmap = off_visc + align(sizeof(BatchEntry<T>) * nvs);
     const size_t off_tmap = off_pmap + align(sizeof(uint32_t) * np);
     const size_t off_vmap = off_tmap + align(sizeof(uint32_t) * nt);
-    const size_t off_vnmap = off_vmap + align(sizeof(uint32_t) * nvb);
-    const size_t off_vgmap = off_vnmap + align(sizeof(uint32_t) * nvn);
-    const size_t off_pt = off_vgmap + align(sizeof(uint32_t) * nvg);
+    const size_t off_pt = off_vmap + align(sizeof(uint32_t) * nvb);
     const size_t off_ptmap = off_pt + align(sizeof(BatchEntry<T>) * nps);
     const size_t total = off_ptmap + align(sizeof(uint32_t) * npb);
     if (fixed && total > fixed->bytes)
@@ -1639,13 +1639,7 @@ class SceneImpl final : public SceneBase {
     for (unsigned b = 0; b < nt; ++b)
       tmap[b] = tlist[b];
     for (unsigned b = 0; b < nvb; ++b)
-      vmap[b] = vlist[xcd_of(b, nvb)];
-    uint32_t *vnmap = reinterpret_cast<uint32_t *>(hb + off_vnmap);
-    uint32_t *vgmap = reinterpret_cast<uint32_t *>(hb + off_vgmap);
-    for (unsigned b = 0; b < nvn; ++b)
-      vnmap[b] = vlist_n[xcd_of(b, nvn)];
-    for (unsigned b = 0; b < nvg; ++b)
-      vgmap[b] = vlist_g[xcd_of(b, nvg)];
+      vmap[b] = vlist[b];
     auto *t_pt = reinterpret_cast<BatchEntry<T> *>(hb + off_pt);
     uint32_t *ptmap = reinterpret_cast<uint32_t *>(hb + off_ptmap);
     for (unsigned b = 0; b < npb; ++b)
@@ -1763,20 +1757,7 @@ class SceneImpl final : public SceneBase {
     const auto *d_pt = reinterpret_cast<const BatchEntry<T> *>(db + off_pt);
     pblocks.map = reinterpret_cast<const uint32_t *>(db + off_ptmap);
     blocks.map = d_pmap;
-    BatchMaps vm;
-    vm.all = reinterpret_cast<const uint32_t *>(db + off_vmap);
-    vm.n_all = nvb;
-    if (nvg > 0) {
-      vm.plain = reinterpret_cast<const uint32_t *>(db + off_vnmap);
-      vm.n_plain = nvn;
-      vm.gc = reinterpret_cast<const uint32_t *>(db + off_vgmap);
-      vm.n_gc = nvg;
-    } else {
-      vm.plain = vm.all;
-      vm.n_plain = nvb;
-      vm.gc = nullptr;
-      vm.n_gc = 0;
-    }
+    vblocks.map = d_vmap;
 
     int r = pf.begin(st, kStageSort);
     GridOps<T>::sort_batch(st, d_sort, d_pmap, np, d_tmap, nt, ns);
@@ -1964,13 +1945,13 @@ class SceneImpl final : public SceneBase {
       r = pf.begin(st, kStageGravityIntegrateV);
       SphOps<T>::integrate_v_batch(st, d_visc, d_vmap, nvb, true);
       pf.end(st, r);
-      if (nvg > 0) {  // the step's gradient correction (x and rho are final)
+      if (any_gc) {  // the step's gradient correction (x and rho are final)
         r = pf.begin(st, kStageCorrection);
-        Wkbb18Ops<T>::correction_batch(st, d_visc, vm);
+        Wkbb18Ops<T>::correction_batch(st, d_visc, vblocks);
         pf.end(st, r);
       }
       r = pf.begin(st, kStageWkbb18DiagSetup);
-      Wkbb18Ops<T>::diagonal_setup_batch(st, d_visc, vm, nvs);
+      Wkbb18Ops<T>::diagonal_setup_batch(st, d_visc, vblocks, nvs);
       pf.end(st, r);
       int cap = 1, pred = 1;
       for (unsigned kv = 0; kv < nvs; ++kv) {
@@ -1980,11 +1961,11 @@ class SceneImpl final : public SceneBase {
       }
       cgp = cg_loop_batch(vsc, cg_seqs, pred, cap, [&](int tag) {
         const int q1 = pf.begin(st, kStagePcgSpmv, tag);
-        Wkbb18Ops<T>::iteration_batch(st, d_visc, vm, nvs, any_split);
+        Wkbb18Ops<T>::iteration_batch(st, d_visc, vblocks, nvs, any_split);
         pf.end(st, q1);
       });
       r = pf.begin(st, kStagePcgVector);
-      Wkbb18Ops<T>::apply_batch(st, d_visc, vm);
+      Wkbb18Ops<T>::apply_batch(st, d_visc, vblocks);
       pf.end(st, r);
       r = pf.begin(st, kStageGravityIntegrateV);
       SphOps<T>::integrate_v_batch(st, d_visc, d_vmap, nvb, false);
@@ -2074,14 +2055,6 @@ class SceneImpl final : public SceneBase {
     }
     PRTCL_HIP_CHECK(hipGetLastError());
     return status;
-  }
-
-  // hardware block b of n -> logical block (the XCD remap of the fused kernels)
-  static unsigned xcd_of(unsigned b, unsigned n) {
-    constexpr unsigned kXcd = 8;
-    const unsigned per = n / kXcd, rem = n % kXcd;
-    const unsigned x = b % kXcd, k = b / kXcd;
-    return x * per + (x < rem ? x : rem) + k;
   }
 
   // ------------------------------------------------------------ residency
@@ -2269,10 +2242,10 @@ class SceneImpl final : public SceneBase {
     // one per block of the largest launch that writes them
     A.take(P.partials, std::max({grid_blocks(static_cast<long>(std::max(f, b))),
                                  setup_blocks(nf), list_blocks(nf)}) + 1);
-    // WKBB18: 3 per block; pt16: 9 per list block in the set-up, 3 per list
+    // WKBB18: 3 per list block; pt16: 9 per list block in the set-up, 3 per list
     // block and 6 per block in an iteration
     A.take(P.cg_part, pt16 ? 9 * static_cast<size_t>(std::max(list_blocks(nf), 1u))
-                           : 3 * static_cast<size_t>(grid_blocks(static_cast<long>(f))) + 3);
+                           : 3 * static_cast<size_t>(std::max(list_blocks(nf), 1u)));
     A.take(P.ctl, 1);
     const size_t nv = pcg ? f : 1;
     for (V4 **q : {&P.cgx, &P.cgr, &P.cgq, &P.cgy, &P.cgb})

@@ -482,7 +482,7 @@ __global__ __launch_bounds__(kBlock) void k_speed_finalize(Ctl *c, const double 
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_integrate_v_b(const BatchEntry<T> *tab,
                                                           const uint32_t *map, int from_xa) {
-  const uint32_t u = map[blockIdx.x];
+  const uint32_t u = map[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   const SceneView<T> &S = E.S;
   const int i = static_cast<int>((u & kBatchLocalMask) * kBlock + threadIdx.x);
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(kBlock) void k_integrate_v_b(const BatchEntry<T> *t
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_integrate_x_b(const BatchEntry<T> *tab,
                                                           const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
+  const uint32_t u = map[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
   integrate_x_body(E.S, u & kBatchLocalMask);
 }

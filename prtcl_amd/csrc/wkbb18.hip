@@ -18,6 +18,7 @@
 #include "wkbb18.hpp"
 #include "cg_ctl.hpp"
 #include "exact_walk.hpp"
+#include "scan8.hpp"
 
 namespace prtcl_amd {
 
@@ -165,46 +166,53 @@ __global__ __launch_bounds__(kBlock) void k_corr_identity(SceneView<T> S) {
 // ---- correction.compute_gradient_correction (correction.hpp:161-217):
 // L_i = pinv(sum_f (m_j / rho_i) gradW_ij (x_j - x_i)^T), exact walk in the
 // reference's FP32 operation order, or over the step's neighbour list
-template <class T, bool kList>
+template <class T, bool kList, int kLanes>
 __device__ __forceinline__ void corr_body(const SceneView<T> &S, const NbrList &L,
                                           unsigned lb) {
 #pragma clang fp contract(off)
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
-  if (i >= S.nf)
-    return;
-  const vec4_t<T> xi = S.xm[i];
-  const T rhoi = S.rho[i];
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
+  const bool valid = i < S.nf;
   T M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  auto add = [&](const vec4_t<T> &pj, T f, T d0, T d1, T d2) {
-    const T g[3] = {f * d0, f * d1, f * d2};
-    const T e[3] = {pj.x - xi.x, pj.y - xi.y, pj.z - xi.z};
-    const T k = pj.w / rhoi;
+  if (valid) {
+    const vec4_t<T> xi = S.xm[i];
+    const T rhoi = S.rho[i];
+    auto add = [&](const vec4_t<T> &pj, T f, T d0, T d1, T d2) {
+      const T g[3] = {f * d0, f * d1, f * d2};
+      const T e[3] = {pj.x - xi.x, pj.y - xi.y, pj.z - xi.z};
+      const T k = pj.w / rhoi;
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
+      for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int r = 0; r < 3; ++r)
-        M[r + 3 * c] += k * (g[r] * e[c]);
-  };
-  const uint32_t info = kList ? L.info[i] : kListOverflow;
-  if (kList && !(info & kListOverflow)) {
-    list_visit(L, list_spans(L, i), static_cast<size_t>(S.nf), i, info,
-               [&](uint32_t j) {
-                 const vec4_t<T> pj = S.xm[j];
-                 const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
-                 add(pj, S.K.gradf(sqdist_exact(d0, d1, d2)), d0, d1, d2);
-               });
-  } else {
-    nbrs_exact(S, xi, S.fcell[i], S.fstart, S.xm,
-               [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
-                 add(pj, S.K.gradf(r2), d0, d1, d2);
-               });
+        for (int r = 0; r < 3; ++r)
+          M[r + 3 * c] += k * (g[r] * e[c]);
+    };
+    const uint32_t info = kList ? L.info[i] : kListOverflow;
+    if (kList && !(info & kListOverflow)) {
+      list_gather_lanes<kLanes, 8>(
+          L, pass_spans<kLanes>(L, S.nf, lb), static_cast<size_t>(S.nf), i, info, sub,
+          [&](uint32_t j) { return S.xm[j]; },
+          [&](const vec4_t<T> &pj) {
+            const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
+            add(pj, S.K.gradf(sqdist_exact(d0, d1, d2)), d0, d1, d2);
+          });
+    } else if (sub == 0) {
+      nbrs_exact(S, xi, S.fcell[i], S.fstart, S.xm,
+                 [&](uint32_t, T d0, T d1, T d2, T r2, const vec4_t<T> &pj) {
+                   add(pj, S.K.gradf(r2), d0, d1, d2);
+                 });
+    }
   }
-  pinv3(M, S.gc + 9 * static_cast<size_t>(i));
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+    M[k] = lanes_sum<kLanes>(M[k]);
+  if (valid && sub == 0)
+    pinv3(M, S.gc + 9 * static_cast<size_t>(i));
 }
 
-template <class T, bool kList>
+template <class T, bool kList, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_corr(SceneView<T> S, NbrList L) {
-  corr_body<T, kList>(S, L, xcd_block(blockIdx.x, gridDim.x));
+  corr_body<T, kList, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // L_i g with Eigen's fixed-size product order per row: l0 g0 + (l1 g1 + l2 g2)
@@ -353,48 +361,35 @@ __device__ __forceinline__ T gradf_fast(const SceneView<T> &S, T r2) {
   return r2 < S.K.eps * S.K.eps ? T(0) : ag3 * (u * u - t * t) * rinv;
 }
 
-// with kGC: M = I - dt L_i (D + B), and the product applies L_i to the summed
-// vector (equal in real arithmetic to applying it per pair)
-template <class T, bool kGC>
-__global__ __launch_bounds__(kBlock) void k_diag_list(SceneView<T> S, NbrList L) {
-  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
-  if (i >= S.nf)
+// the boundary neighbours of particle i in a fused step, runs sub, sub + kLanes,
+// ... of its cells (nothing for a particle whose list tells it has none):
+// fn(d0, d1, d2, pj)
+template <int kLanes, class T, class Fn>
+__device__ __forceinline__ void boundary_lanes(const SceneView<T> &S, int i, uint32_t info,
+                                               uint32_t sub, const vec4_t<T> &xi, Fn &&fn) {
+  if (!list_has_boundary(info))
     return;
-  const vec4_t<T> xi = S.xm[i];
-  const T rhoi = S.rho[i];
-  const size_t n = static_cast<size_t>(S.nf);
-  T D[6] = {0, 0, 0, 0, 0, 0};  // symmetric: xx yy zz xy xz yz
-  auto add = [&](T k, T d0, T d1, T d2) {
-    D[0] += k * d0 * d0;
-    D[1] += k * d1 * d1;
-    D[2] += k * d2 * d2;
-    D[3] += k * d0 * d1;
-    D[4] += k * d0 * d2;
-    D[5] += k * d1 * d2;
-  };
-  const T cf = T(10) * S.mu_f / rhoi;
-  auto fluid = [&](uint32_t j) {
-    const vec4_t<T> pj = S.xm[j];
-    const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
-    const T r2 = d0 * d0 + d1 * d1 + d2 * d2;
-    add(cf * pj.w / S.rho[j] * gradf_fast(S, r2) / (r2 + S.hh001), d0, d1, d2);
-  };
-  const uint32_t info = L.info[i];
-  if (!(info & kListOverflow)) {
-    list_visit(L, list_spans(L, i), n, i, info, fluid);
-  } else {
-    nbrs_exact(S, xi, S.fcell[i], S.fstart, S.xm,
-               [&](uint32_t j, T, T, T, T, const vec4_t<T> &) {
-                 if (j != static_cast<uint32_t>(i))
-                   fluid(j);
-               });
+  const uint32_t cell = S.fcell[i];
+  for (uint32_t r = sub; r < 9u; r += kLanes) {
+    uint32_t b, e;
+    run_bounds(S.grid, cell, S.bstart, static_cast<int>(r), &b, &e);
+    for (uint32_t j = b; j < e; ++j) {
+      const vec4_t<T> pj = S.bxV[j];
+      const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
+      if (sqdist_exact(d0, d1, d2) < S.thr2)
+        fn(d0, d1, d2, pj);
+    }
   }
-  T B[6] = {0, 0, 0, 0, 0, 0};
+}
+
+// the symmetric boundary matrix B_i = sum_b k_ib gradW_ib x_ib^T (xx yy zz xy xz
+// yz), this lane's share
+template <int kLanes, class T>
+__device__ __forceinline__ void boundary_matrix(const SceneView<T> &S, int i, uint32_t info,
+                                                uint32_t sub, const vec4_t<T> &xi, T rhoi,
+                                                T B[6]) {
   const T cb = T(10) * S.mu_b / rhoi * S.rho0 / rhoi;
-  nbrs_exact(S, xi, S.fcell[i], S.bstart, S.bxV, [&](uint32_t, T d0, T d1, T d2, T r2e,
-                                                       const vec4_t<T> &pj) {
-    (void)r2e;
+  boundary_lanes<kLanes>(S, i, info, sub, xi, [&](T d0, T d1, T d2, const vec4_t<T> &pj) {
     const T r2 = d0 * d0 + d1 * d1 + d2 * d2;
     const T k = cb * pj.w * gradf_fast(S, r2) / (r2 + S.hh001);
     B[0] += k * d0 * d0;
@@ -404,6 +399,12 @@ __global__ __launch_bounds__(kBlock) void k_diag_list(SceneView<T> S, NbrList L)
     B[4] += k * d0 * d2;
     B[5] += k * d1 * d2;
   });
+}
+
+// (I - dt (D + B))^-1, or with kGC (I - dt L_i (D + B))^-1, to sp_i
+template <class T, bool kGC>
+__device__ __forceinline__ void store_diagonal(const SceneView<T> &S, int i, const T D[6],
+                                               const T B[6]) {
   T M[9];
   const T dt = S.dt;
   const T Dt[6] = {D[0] + B[0], D[1] + B[1], D[2] + B[2], D[3] + B[3], D[4] + B[4], D[5] + B[5]};
@@ -430,6 +431,60 @@ __global__ __launch_bounds__(kBlock) void k_diag_list(SceneView<T> S, NbrList L)
     M[5] = M[7] = -dt * Dt[5];
   }
   invert3(M, S.sp + 9 * static_cast<size_t>(i));
+}
+
+// with kGC: M = I - dt L_i (D + B), and the product applies L_i to the summed
+// vector (equal in real arithmetic to applying it per pair)
+template <class T, bool kGC, int kLanes>
+__global__ __launch_bounds__(kBlock) void k_diag_list(SceneView<T> S, NbrList L) {
+  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
+  const bool valid = i < S.nf;
+  const vec4_t<T> xi = valid ? S.xm[i] : make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  const T rhoi = valid ? S.rho[i] : T(1);
+  T D[6] = {0, 0, 0, 0, 0, 0};  // symmetric: xx yy zz xy xz yz
+  T B[6] = {0, 0, 0, 0, 0, 0};
+  if (valid) {
+    auto add = [&](T k, T d0, T d1, T d2) {
+      D[0] += k * d0 * d0;
+      D[1] += k * d1 * d1;
+      D[2] += k * d2 * d2;
+      D[3] += k * d0 * d1;
+      D[4] += k * d0 * d2;
+      D[5] += k * d1 * d2;
+    };
+    const T cf = T(10) * S.mu_f / rhoi;
+    struct P {
+      vec4_t<T> x;
+      T rho;
+    };
+    auto fluid = [&](const P &q) {
+      const T d0 = xi.x - q.x.x, d1 = xi.y - q.x.y, d2 = xi.z - q.x.z;
+      const T r2 = d0 * d0 + d1 * d1 + d2 * d2;
+      add(cf * q.x.w / q.rho * gradf_fast(S, r2) / (r2 + S.hh001), d0, d1, d2);
+    };
+    auto load = [&](uint32_t j) { return P{S.xm[j], S.rho[j]}; };
+    const uint32_t info = L.info[i];
+    if (!(info & kListOverflow))
+      list_gather_lanes<kLanes, 4>(L, pass_spans<kLanes>(L, S.nf, lb), static_cast<size_t>(S.nf),
+                                   i, info, sub, load, fluid);
+    else if (sub == 0)
+      nbrs_exact(S, xi, S.fcell[i], S.fstart, S.xm,
+                 [&](uint32_t j, T, T, T, T, const vec4_t<T> &) {
+                   if (j != static_cast<uint32_t>(i))
+                     fluid(load(j));
+                 });
+    boundary_matrix<kLanes>(S, i, info, sub, xi, rhoi, B);
+  }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    D[k] = lanes_sum<kLanes>(D[k]);
+    B[k] = lanes_sum<kLanes>(B[k]);
+  }
+  if (!valid || sub != 0)
+    return;
+  store_diagonal<T, kGC>(S, i, D, B);
   // B_i for the list product, (x_i, m_i / rho_i) for its gathers
   S.cb[i] = make4<vec4_t<T>>(B[0], B[1], B[2], T(0));
   S.G[i] = make4<vec4_t<T>>(B[3], B[4], B[5], T(0));
@@ -511,34 +566,45 @@ __device__ __forceinline__ void product_finish(const SceneView<T> &S, int i,
   }
 }
 
-template <class T, bool kGC>
-__device__ __forceinline__ void product_list(const SceneView<T> &S, const NbrList &L, int i,
+// the list product at particle i (valid), complete in every one of its kLanes lanes
+template <class T, bool kGC, int kLanes>
+__device__ __forceinline__ void product_list(const SceneView<T> &S, const NbrList &L, unsigned lb,
+                                             int i, bool valid, uint32_t sub,
                                              const vec4_t<T> *__restrict__ w, int ws,
                                              T out[3]) {
-  const vec4_t<T> xq = S.xq[i];  // (x_i, m_i / rho_i)
-  const vec4_t<T> wi = w[static_cast<size_t>(ws) * i];
-  const size_t n = static_cast<size_t>(S.nf);
-  const ProductPair<T> pair(S);
   T l0 = 0, l1 = 0, l2 = 0;
-  struct XW {
-    vec4_t<T> x, w;  // (x_j, m_j / rho_j) and w_j
-  };
-  auto use = [&](const XW &q) { pair(xq, wi, q.x, q.w, l0, l1, l2); };
-  const uint32_t info = L.info[i];
-  if (!(info & kListOverflow)) {
-    list_gather<4>(L, list_spans(L, i), n, i, info,
-                   [&](uint32_t j) {
-                     return XW{S.cxp[2 * static_cast<size_t>(j)], w[static_cast<size_t>(ws) * j]};
-                   },
-                   use);
-  } else {
-    nbrs_exact(S, xq, S.fcell[i], S.fstart, S.xq,
-               [&](uint32_t j, T, T, T, T, const vec4_t<T> &) {
-                 if (j != static_cast<uint32_t>(i))
-                   use(XW{S.xq[j], w[static_cast<size_t>(ws) * j]});
-               });
+  vec4_t<T> wi = make4<vec4_t<T>>(T(0), T(0), T(0), T(0)), bd = wi, bo = wi;
+  if (valid) {
+    const vec4_t<T> xq = S.xq[i];  // (x_i, m_i / rho_i)
+    wi = w[static_cast<size_t>(ws) * i];
+    const ProductPair<T> pair(S);
+    struct XW {
+      vec4_t<T> x, w;  // (x_j, m_j / rho_j) and w_j
+    };
+    auto use = [&](const XW &q) { pair(xq, wi, q.x, q.w, l0, l1, l2); };
+    const uint32_t info = L.info[i];
+    if (!(info & kListOverflow)) {
+      list_gather_lanes<kLanes, 4>(
+          L, pass_spans<kLanes>(L, S.nf, lb), static_cast<size_t>(S.nf), i, info, sub,
+          [&](uint32_t j) {
+            return XW{S.cxp[2 * static_cast<size_t>(j)], w[static_cast<size_t>(ws) * j]};
+          },
+          use);
+    } else if (sub == 0) {
+      nbrs_exact(S, xq, S.fcell[i], S.fstart, S.xq,
+                 [&](uint32_t j, T, T, T, T, const vec4_t<T> &) {
+                   if (j != static_cast<uint32_t>(i))
+                     use(XW{S.xq[j], w[static_cast<size_t>(ws) * j]});
+                 });
+    }
+    bd = S.cb[i];
+    bo = S.G[i];
   }
-  product_finish<T, kGC>(S, i, wi, l0, l1, l2, S.cb[i], S.G[i], out);
+  l0 = lanes_sum<kLanes>(l0);
+  l1 = lanes_sum<kLanes>(l1);
+  l2 = lanes_sum<kLanes>(l2);
+  if (valid)
+    product_finish<T, kGC>(S, i, wi, l0, l1, l2, bd, bo, out);
 }
 
 template <class T>
@@ -561,34 +627,43 @@ __device__ __forceinline__ vec4_t<T> precond(const T *M, const vec4_t<T> &w) {
 // setup: x = v (guess), r = A x - b with b = v (the rhs of wkbb18.hpp:296-334
 // is v - dt a_b with a_b = 0 because the boundary velocity is zero),
 // y = P r, p = -y; partials of b.b, r.r, r.y
-template <class T, bool kExact, bool kGC>
+// the CG set-up of particle i from ax = A x0; acc = b.b, r.r, r.y
+template <class T>
+__device__ __forceinline__ void cg_start(const SceneView<T> &S, int i, const vec4_t<T> &v,
+                                         const T ax[3], double acc[3]) {
+  vec4_t<T> b = v;
+  b.w = T(0);
+  vec4_t<T> r;
+  r.x = ax[0] - b.x;
+  r.y = ax[1] - b.y;
+  r.z = ax[2] - b.z;
+  r.w = T(0);
+  const vec4_t<T> y = precond(S.sp + 9 * static_cast<size_t>(i), r);
+  S.cx[i] = b;
+  S.cr[i] = r;
+  S.cy[i] = y;
+  S.cxp[2 * static_cast<size_t>(i) + 1] = make4<vec4_t<T>>(-y.x, -y.y, -y.z, T(0));
+  acc[0] = static_cast<double>(dot3r<T>(b, b));
+  acc[1] = static_cast<double>(dot3r<T>(r, r));
+  acc[2] = static_cast<double>(dot3r<T>(r, y));
+}
+
+template <class T, bool kExact, bool kGC, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_cg_setup(SceneView<T> S, NbrList L, double *part) {
   const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
+  const bool valid = i < S.nf;
   double acc[3] = {0.0, 0.0, 0.0};
-  if (i < S.nf) {
-    const vec4_t<T> v = S.v[i];
-    T ax[3];
-    if (kExact)
+  T ax[3];
+  if (kExact) {
+    if (valid)
       product_exact<T, kGC>(S, i, S.v, 1, ax);
-    else
-      product_list<T, kGC>(S, L, i, S.v, 1, ax);
-    vec4_t<T> b = v;
-    b.w = T(0);
-    vec4_t<T> r;
-    r.x = ax[0] - b.x;
-    r.y = ax[1] - b.y;
-    r.z = ax[2] - b.z;
-    r.w = T(0);
-    const vec4_t<T> y = precond(S.sp + 9 * static_cast<size_t>(i), r);
-    S.cx[i] = b;
-    S.cr[i] = r;
-    S.cy[i] = y;
-    S.cxp[2 * static_cast<size_t>(i) + 1] = make4<vec4_t<T>>(-y.x, -y.y, -y.z, T(0));
-    acc[0] = static_cast<double>(dot3r<T>(b, b));
-    acc[1] = static_cast<double>(dot3r<T>(r, r));
-    acc[2] = static_cast<double>(dot3r<T>(r, y));
+  } else {
+    product_list<T, kGC, kLanes>(S, L, lb, i, valid, sub, S.v, 1, ax);
   }
+  if (valid && sub == 0)
+    cg_start(S, i, S.v[i], ax, acc);
   store_partials<3>(part, gridDim.x, acc, lb);
 }
 
@@ -597,21 +672,23 @@ __global__ __launch_bounds__(kBlock) void k_cg_setup(SceneView<T> S, NbrList L, 
 // same order, with (x_j, m_j / rho_j) formed from x_j, m_j and rho_j as the
 // diagonal pass writes it, so the results equal those of the two kernels
 // (lb: the block's logical index, nb: the scene's block count)
-template <class T, bool kGC>
+template <class T, bool kGC, int kLanes>
 __device__ __forceinline__ void diag_setup_list_body(const SceneView<T> &S, const NbrList &L,
                                                      double *part, unsigned lb, unsigned nb) {
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
-  double acc[3] = {0.0, 0.0, 0.0};
-  if (i < S.nf) {
-    const vec4_t<T> xi = S.xm[i];
-    const T rhoi = S.rho[i];
-    const vec4_t<T> wi = S.v[i];  // the guess x0 = v
-    const vec4_t<T> xqi = make4<vec4_t<T>>(xi.x, xi.y, xi.z, xi.w / rhoi);
-    const size_t n = static_cast<size_t>(S.nf);
-    T D[6] = {0, 0, 0, 0, 0, 0};  // symmetric: xx yy zz xy xz yz
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
+  const bool valid = i < S.nf;
+  const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
+  const vec4_t<T> xi = valid ? S.xm[i] : zero4;
+  const T rhoi = valid ? S.rho[i] : T(1);
+  const vec4_t<T> wi = valid ? S.v[i] : zero4;  // the guess x0 = v
+  const vec4_t<T> xqi = make4<vec4_t<T>>(xi.x, xi.y, xi.z, xi.w / rhoi);
+  T D[6] = {0, 0, 0, 0, 0, 0};  // symmetric: xx yy zz xy xz yz
+  T B[6] = {0, 0, 0, 0, 0, 0};
+  T l0 = 0, l1 = 0, l2 = 0;
+  if (valid) {
     const T cf = T(10) * S.mu_f / rhoi;
     const ProductPair<T> pair(S);
-    T l0 = 0, l1 = 0, l2 = 0;
     struct P {
       vec4_t<T> x;  // (x_j, m_j)
       T rho;
@@ -629,107 +706,67 @@ __device__ __forceinline__ void diag_setup_list_body(const SceneView<T> &S, cons
       D[5] += k * d1 * d2;
       pair(xqi, wi, make4<vec4_t<T>>(q.x.x, q.x.y, q.x.z, q.x.w / q.rho), q.w, l0, l1, l2);
     };
+    auto load = [&](uint32_t j) { return P{S.xm[j], S.rho[j], S.v[j]}; };
     const uint32_t info = L.info[i];
-    if (!(info & kListOverflow)) {
-      list_gather<4>(L, list_spans(L, i), n, i, info,
-                     [&](uint32_t j) { return P{S.xm[j], S.rho[j], S.v[j]}; }, both);
-    } else {
+    if (!(info & kListOverflow))
+      list_gather_lanes<kLanes, 4>(L, pass_spans<kLanes>(L, S.nf, lb), static_cast<size_t>(S.nf),
+                                   i, info, sub, load, both);
+    else if (sub == 0)
       nbrs_exact(S, xi, S.fcell[i], S.fstart, S.xm,
                  [&](uint32_t j, T, T, T, T, const vec4_t<T> &) {
                    if (j != static_cast<uint32_t>(i))
-                     both(P{S.xm[j], S.rho[j], S.v[j]});
+                     both(load(j));
                  });
-    }
-    T B[6] = {0, 0, 0, 0, 0, 0};
-    const T cb = T(10) * S.mu_b / rhoi * S.rho0 / rhoi;
-    nbrs_exact(S, xi, S.fcell[i], S.bstart, S.bxV, [&](uint32_t, T d0, T d1, T d2, T r2e,
-                                                         const vec4_t<T> &pj) {
-      (void)r2e;
-      const T r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      const T k = cb * pj.w * gradf_fast(S, r2) / (r2 + S.hh001);
-      B[0] += k * d0 * d0;
-      B[1] += k * d1 * d1;
-      B[2] += k * d2 * d2;
-      B[3] += k * d0 * d1;
-      B[4] += k * d0 * d2;
-      B[5] += k * d1 * d2;
-    });
-    T M[9];
-    const T dt = S.dt;
-    const T Dt[6] = {D[0] + B[0], D[1] + B[1], D[2] + B[2],
-                     D[3] + B[3], D[4] + B[4], D[5] + B[5]};
-    if (kGC) {
-      const T Ds[9] = {Dt[0], Dt[3], Dt[4], Dt[3], Dt[1], Dt[5], Dt[4], Dt[5], Dt[2]};
-      const T *Li = S.gc + 9 * static_cast<size_t>(i);
-      T Lr[9];
+    boundary_matrix<kLanes>(S, i, info, sub, xi, rhoi, B);
+  }
 #pragma unroll
-      for (int k = 0; k < 9; ++k)
-        Lr[k] = Li[k];
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-          M[r + 3 * c] = ((r == c) ? T(1) : T(0)) -
-                         dt * (Lr[r] * Ds[3 * c] + Lr[r + 3] * Ds[1 + 3 * c] +
-                               Lr[r + 6] * Ds[2 + 3 * c]);
-    } else {
-      M[0] = T(1) - dt * Dt[0];
-      M[4] = T(1) - dt * Dt[1];
-      M[8] = T(1) - dt * Dt[2];
-      M[1] = M[3] = -dt * Dt[3];
-      M[2] = M[6] = -dt * Dt[4];
-      M[5] = M[7] = -dt * Dt[5];
-    }
-    T *spi = S.sp + 9 * static_cast<size_t>(i);
-    invert3(M, spi);
+  for (int k = 0; k < 6; ++k) {
+    D[k] = lanes_sum<kLanes>(D[k]);
+    B[k] = lanes_sum<kLanes>(B[k]);
+  }
+  l0 = lanes_sum<kLanes>(l0);
+  l1 = lanes_sum<kLanes>(l1);
+  l2 = lanes_sum<kLanes>(l2);
+  double acc[3] = {0.0, 0.0, 0.0};
+  if (valid && sub == 0) {
+    store_diagonal<T, kGC>(S, i, D, B);
     const vec4_t<T> bd = make4<vec4_t<T>>(B[0], B[1], B[2], T(0));
     const vec4_t<T> bo = make4<vec4_t<T>>(B[3], B[4], B[5], T(0));
     S.cb[i] = bd;
     S.G[i] = bo;
     S.xq[i] = xqi;
     S.cxp[2 * static_cast<size_t>(i)] = xqi;
-    // the CG set-up (k_cg_setup)
     T ax[3];
     product_finish<T, kGC>(S, i, wi, l0, l1, l2, bd, bo, ax);
-    vec4_t<T> b = wi;
-    b.w = T(0);
-    vec4_t<T> r;
-    r.x = ax[0] - b.x;
-    r.y = ax[1] - b.y;
-    r.z = ax[2] - b.z;
-    r.w = T(0);
-    const vec4_t<T> y = precond(spi, r);
-    S.cx[i] = b;
-    S.cr[i] = r;
-    S.cy[i] = y;
-    S.cxp[2 * static_cast<size_t>(i) + 1] = make4<vec4_t<T>>(-y.x, -y.y, -y.z, T(0));
-    acc[0] = static_cast<double>(dot3r<T>(b, b));
-    acc[1] = static_cast<double>(dot3r<T>(r, r));
-    acc[2] = static_cast<double>(dot3r<T>(r, y));
+    cg_start(S, i, wi, ax, acc);
   }
   store_partials<3>(part, nb, acc, lb);
 }
 
-template <class T, bool kGC>
+template <class T, bool kGC, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_diag_setup_list(SceneView<T> S, NbrList L,
                                                             double *part) {
-  diag_setup_list_body<T, kGC>(S, L, part, xcd_block(blockIdx.x, gridDim.x), gridDim.x);
+  diag_setup_list_body<T, kGC, kLanes>(S, L, part, xcd_block(blockIdx.x, gridDim.x), gridDim.x);
 }
 
 // q = A p, partial p.q
-template <class T, bool kExact, bool kGC>
+template <class T, bool kExact, bool kGC, int kLanes>
 __device__ __forceinline__ void cg_spmv_body(const SceneView<T> &S, const NbrList &L,
                                              double *part, unsigned lb, unsigned nb) {
   if (S.ctl->cg_done)
     return;
-  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
+  const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
+  const uint32_t sub = threadIdx.x % kLanes;
+  const bool valid = i < S.nf;
   double acc[1] = {0.0};
-  if (i < S.nf) {
-    T q[3];
-    if (kExact)
+  T q[3];
+  if (kExact) {
+    if (valid)
       product_exact<T, kGC>(S, i, S.cxp + 1, 2, q);
-    else
-      product_list<T, kGC>(S, L, i, S.cxp + 1, 2, q);
+  } else {
+    product_list<T, kGC, kLanes>(S, L, lb, i, valid, sub, S.cxp + 1, 2, q);
+  }
+  if (valid && sub == 0) {
     const vec4_t<T> qv = make4<vec4_t<T>>(q[0], q[1], q[2], T(0));
     S.cq[i] = qv;
     acc[0] = static_cast<double>(dot3r<T>(S.cxp[2 * static_cast<size_t>(i) + 1], qv));
@@ -737,27 +774,45 @@ __device__ __forceinline__ void cg_spmv_body(const SceneView<T> &S, const NbrLis
   store_partials<1>(part, nb, acc, lb);
 }
 
-template <class T, bool kExact, bool kGC>
+template <class T, bool kExact, bool kGC, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_cg_spmv(SceneView<T> S, NbrList L, double *part) {
-  cg_spmv_body<T, kExact, kGC>(S, L, part, xcd_block(blockIdx.x, gridDim.x), gridDim.x);
+  cg_spmv_body<T, kExact, kGC, kLanes>(S, L, part, xcd_block(blockIdx.x, gridDim.x), gridDim.x);
 }
+
+// a particle's vectors of the update, loaded ahead of the scalars (whose partial
+// sums are a chain of memory latencies of their own)
+template <class T>
+struct CgOwn {
+  vec4_t<T> p, q, x, r;
+  T M[9];
+  __device__ __forceinline__ CgOwn(const SceneView<T> &S, int i) {
+    if (i < S.nf) {
+      p = S.cxp[2 * static_cast<size_t>(i) + 1];
+      q = S.cq[i];
+      x = S.cx[i];
+      r = S.cr[i];
+#pragma unroll
+      for (int k = 0; k < 9; ++k)
+        M[k] = S.sp[9 * static_cast<size_t>(i) + k];
+    }
+  }
+};
 
 // x += alpha p, r += alpha q, y = P r; partials r.r, r.y
 template <class T>
-__device__ __forceinline__ void cg_update_body(const SceneView<T> &S, T alpha, double *part,
-                                               unsigned lb, unsigned nb) {
+__device__ __forceinline__ void cg_update_body(const SceneView<T> &S, const CgOwn<T> &o, T alpha,
+                                               double *part, unsigned lb, unsigned nb) {
   const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   double acc[2] = {0.0, 0.0};
   if (i < S.nf) {
-    const vec4_t<T> p = S.cxp[2 * static_cast<size_t>(i) + 1], q = S.cq[i];
-    vec4_t<T> x = S.cx[i], r = S.cr[i];
-    x.x += alpha * p.x;
-    x.y += alpha * p.y;
-    x.z += alpha * p.z;
-    r.x += alpha * q.x;
-    r.y += alpha * q.y;
-    r.z += alpha * q.z;
-    const vec4_t<T> y = precond(S.sp + 9 * static_cast<size_t>(i), r);
+    vec4_t<T> x = o.x, r = o.r;
+    x.x += alpha * o.p.x;
+    x.y += alpha * o.p.y;
+    x.z += alpha * o.p.z;
+    r.x += alpha * o.q.x;
+    r.y += alpha * o.q.y;
+    r.z += alpha * o.q.z;
+    const vec4_t<T> y = precond(o.M, r);
     S.cx[i] = x;
     S.cr[i] = r;
     S.cy[i] = y;
@@ -767,56 +822,70 @@ __device__ __forceinline__ void cg_update_body(const SceneView<T> &S, T alpha, d
   store_partials<2>(part, nb, acc, lb);
 }
 
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_cg_update(SceneView<T> S, double *part) {
-  if (S.ctl->cg_done)
-    return;
-  cg_update_body(S, static_cast<T>(S.ctl->cg_alpha), part, blockIdx.x, gridDim.x);
-}
-
 // p = -y + beta p
 template <class T>
-__device__ __forceinline__ void cg_direction_body(const SceneView<T> &S, T beta, unsigned lb) {
+__device__ __forceinline__ void cg_direction_body(const SceneView<T> &S, const vec4_t<T> &y,
+                                                  vec4_t<T> p, T beta, unsigned lb) {
   const int i = static_cast<int>(lb * kBlock + threadIdx.x);
   if (i >= S.nf)
     return;
-  const vec4_t<T> y = S.cy[i];
-  vec4_t<T> p = S.cxp[2 * static_cast<size_t>(i) + 1];
   p.x = -y.x + beta * p.x;
   p.y = -y.y + beta * p.y;
   p.z = -y.z + beta * p.z;
   S.cxp[2 * static_cast<size_t>(i) + 1] = p;
 }
 
+// The update and direction kernels of one scene. fold: without the two one-block
+// kernels (cg_alpha_in_block, cg_beta_in_block): the block derives alpha from the
+// npq partials of p.q (beta from the nb partials of r.r and r.y).
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_cg_direction(SceneView<T> S) {
-  if (S.ctl->cg_done)
-    return;
-  cg_direction_body(S, static_cast<T>(S.ctl->cg_beta), blockIdx.x);
-}
-
-// The iteration without its two one-block kernels (cg_alpha_in_block,
-// cg_beta_in_block): k_cg_alpha with k_cg_update, k_cg_beta with
-// k_cg_direction
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_cg_update_alpha(SceneView<T> S, const double *pq_part,
-                                                            double *part) {
+__device__ __forceinline__ void cg_update(const SceneView<T> &S, bool fold, const double *pq_part,
+                                          unsigned npq, double *part, unsigned lb, unsigned nb) {
+  const CgOwn<T> own(S, static_cast<int>(lb * kBlock + threadIdx.x));
   if (cg_done_for_block(S.ctl))
     return;
   double alpha;
-  if (!cg_alpha_in_block(S.ctl, pq_part, gridDim.x, &alpha))
-    return;
-  cg_update_body(S, static_cast<T>(alpha), part, blockIdx.x, gridDim.x);
+  if (fold) {
+    if (!cg_alpha_in_block(S.ctl, pq_part, npq, &alpha, lb))
+      return;
+  } else {
+    alpha = S.ctl->cg_alpha;
+  }
+  cg_update_body(S, own, static_cast<T>(alpha), part, lb, nb);
 }
 
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_cg_direction_beta(SceneView<T> S, const double *part) {
+__device__ __forceinline__ void cg_direction(const SceneView<T> &S, bool fold, const double *part,
+                                             unsigned lb, unsigned nb) {
+  const int i = static_cast<int>(lb * kBlock + threadIdx.x);
+  vec4_t<T> y = make4<vec4_t<T>>(T(0), T(0), T(0), T(0)), p = y;
+  if (i < S.nf) {
+    y = S.cy[i];
+    p = S.cxp[2 * static_cast<size_t>(i) + 1];
+  }
   if (cg_done_for_block(S.ctl))
     return;
   double beta;
-  if (!cg_beta_in_block(S.ctl, part, gridDim.x, &beta))
-    return;
-  cg_direction_body(S, static_cast<T>(beta), blockIdx.x);
+  if (fold) {
+    if (!cg_beta_in_block(S.ctl, part, nb, &beta, lb))
+      return;
+  } else {
+    beta = S.ctl->cg_beta;
+  }
+  cg_direction_body(S, y, p, static_cast<T>(beta), lb);
+}
+
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_cg_update(SceneView<T> S, int fold,
+                                                      const double *pq_part, unsigned npq,
+                                                      double *part) {
+  cg_update(S, fold != 0, pq_part, npq, part, blockIdx.x, gridDim.x);
+}
+
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_cg_direction(SceneView<T> S, int fold,
+                                                         const double *part) {
+  cg_direction(S, fold != 0, part, blockIdx.x, gridDim.x);
 }
 
 // apply (wkbb18.hpp:401-413): vd = (x - v) H(t - t_birth - dt_fade), a = vd / dt
@@ -839,165 +908,158 @@ __global__ __launch_bounds__(kBlock) void k_cg_apply(SceneView<T> S) {
 }
 
 // ---- batched WKBB18 (prtcl_hip_step over several scenes): the kernels above
-// over the blocks of every scene of a table (map: block map, entry of scene k
-// in bits 20.., its local block below), each block with its scene's view,
-// list, CG partials and block count, so every scene's sums and decisions are
+// over the blocks of every scene of a table (B: group 0 the scenes without, group
+// 1 those with the gradient correction), each block with its scene's view,
+// list, CG partials and block counts, so every scene's sums and decisions are
 // those of its single-scene step. A scene with cg_fold derives alpha and
 // beta in its vector kernels, otherwise its one-block kernels do.
-template <class T>
-__device__ __forceinline__ NbrList entry_list(const BatchEntry<T> &E) {
-  return NbrList{E.nidx, E.ninfo, E.nblk, E.nshift};
-}
+#define WK_BATCH_ENTRY(kF)                                                 \
+  unsigned part_;                                                          \
+  const uint32_t u = batch_block(B, kF, &part_);                           \
+  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];                      \
+  const bool split = split_scene(E.S.nf);                                  \
+  const unsigned lb = (u & kBatchLocalMask) * (split ? (kF) : 1u) + part_; \
+  const unsigned nl = list_blocks(E.S.nf);                                 \
+  const NbrList L{E.nidx, E.ninfo, E.nblk, E.nshift};                      \
+  (void)L;                                                                 \
+  if (lb >= ((kF) == 1u ? E.nblocks : nl))                                 \
+  return
 
 template <class T, bool kGC>
 __global__ __launch_bounds__(kBlock) void k_diag_setup_b(const BatchEntry<T> *tab,
-                                                         const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  diag_setup_list_body<T, kGC>(E.S, entry_list(E), E.cg_part, u & kBatchLocalMask, E.nblocks);
+                                                         BatchBlocks B) {
+  WK_BATCH_ENTRY(kListLanes);
+  if (split)
+    diag_setup_list_body<T, kGC, kListLanes>(E.S, L, E.cg_part, lb, nl);
+  else
+    diag_setup_list_body<T, kGC, 1>(E.S, L, E.cg_part, lb, nl);
 }
 
 // the gradient correction of wkbb18_gc scenes over the list
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_corr_b(const BatchEntry<T> *tab,
-                                                   const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  corr_body<T, true>(E.S, entry_list(E), u & kBatchLocalMask);
+__global__ __launch_bounds__(kBlock) void k_corr_b(const BatchEntry<T> *tab, BatchBlocks B) {
+  WK_BATCH_ENTRY(kListLanes);
+  if (split)
+    corr_body<T, true, kListLanes>(E.S, L, lb);
+  else
+    corr_body<T, true, 1>(E.S, L, lb);
 }
 
 // one block per scene
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cg_setup_fin_b(const BatchEntry<T> *tab) {
   const BatchEntry<T> &E = tab[blockIdx.x];
-  cg_setup_fin_body(E.S.ctl, E.cg_part, E.nblocks, E.cg_tol, E.cg_max_k, E.cg_seq);
+  cg_setup_fin_body(E.S.ctl, E.cg_part, list_blocks(E.S.nf), E.cg_tol, E.cg_max_k, E.cg_seq);
 }
 
 template <class T, bool kGC>
-__global__ __launch_bounds__(kBlock) void k_cg_spmv_b(const BatchEntry<T> *tab,
-                                                      const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  cg_spmv_body<T, false, kGC>(E.S, entry_list(E), E.cg_part, u & kBatchLocalMask, E.nblocks);
+__global__ __launch_bounds__(kBlock) void k_cg_spmv_b(const BatchEntry<T> *tab, BatchBlocks B) {
+  WK_BATCH_ENTRY(kListLanes);
+  if (split)
+    cg_spmv_body<T, false, kGC, kListLanes>(E.S, L, E.cg_part, lb, nl);
+  else
+    cg_spmv_body<T, false, kGC, 1>(E.S, L, E.cg_part, lb, nl);
 }
 
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cg_alpha_b(const BatchEntry<T> *tab) {
   const BatchEntry<T> &E = tab[blockIdx.x];
   if (!E.cg_fold)
-    cg_alpha_body(E.S.ctl, E.cg_part, E.nblocks);
+    cg_alpha_body(E.S.ctl, E.cg_part, list_blocks(E.S.nf));
 }
 
+// p.q partials at [0, nl), r.r and r.y at [nl, nl + 2 nb)
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cg_update_b(const BatchEntry<T> *tab,
-                                                        const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  const unsigned lb = u & kBatchLocalMask, nb = E.nblocks;
-  Ctl *c = E.S.ctl;
-  if (E.cg_fold) {  // p.q partials at [0, nb), r.r and r.y at [nb, 3 nb)
-    if (cg_done_for_block(c))
-      return;
-    double alpha;
-    if (!cg_alpha_in_block(c, E.cg_part, nb, &alpha, lb))
-      return;
-    cg_update_body(E.S, static_cast<T>(alpha), E.cg_part + nb, lb, nb);
-  } else {
-    if (c->cg_done)
-      return;
-    cg_update_body(E.S, static_cast<T>(c->cg_alpha), E.cg_part, lb, nb);
-  }
+                                                        BatchBlocks B) {
+  WK_BATCH_ENTRY(1u);
+  cg_update(E.S, E.cg_fold != 0, E.cg_part, nl, E.cg_part + nl, lb, E.nblocks);
 }
 
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cg_beta_b(const BatchEntry<T> *tab) {
   const BatchEntry<T> &E = tab[blockIdx.x];
   if (!E.cg_fold)
-    cg_beta_body(E.S.ctl, E.cg_part, E.nblocks);
+    cg_beta_body(E.S.ctl, E.cg_part + list_blocks(E.S.nf), E.nblocks);
 }
 
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cg_direction_b(const BatchEntry<T> *tab,
-                                                           const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  const unsigned lb = u & kBatchLocalMask, nb = E.nblocks;
-  Ctl *c = E.S.ctl;
-  if (E.cg_fold) {
-    if (cg_done_for_block(c))
-      return;
-    double beta;
-    if (!cg_beta_in_block(c, E.cg_part + nb, nb, &beta, lb))
-      return;
-    cg_direction_body(E.S, static_cast<T>(beta), lb);
-  } else {
-    if (c->cg_done)
-      return;
-    cg_direction_body(E.S, static_cast<T>(c->cg_beta), lb);
-  }
+                                                           BatchBlocks B) {
+  WK_BATCH_ENTRY(1u);
+  cg_direction(E.S, E.cg_fold != 0, E.cg_part + nl, lb, E.nblocks);
 }
 
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cg_apply_b(const BatchEntry<T> *tab,
-                                                       const uint32_t *map) {
-  const uint32_t u = map[blockIdx.x];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  cg_apply_body(E.S, u & kBatchLocalMask);
+                                                       BatchBlocks B) {
+  WK_BATCH_ENTRY(1u);
+  cg_apply_body(E.S, lb);
 }
 
+#undef WK_BATCH_ENTRY
+
 }  // namespace
+
+// a list kernel of one scene with its lanes per particle; the kernel's template
+// arguments before the lanes are given in parentheses
+#define WK_ARGS(...) __VA_ARGS__
+#define WK_LIST(kern, targs, ...)                                                          \
+  do {                                                                                     \
+    if (split_scene(S.nf))                                                                 \
+      hipLaunchKernelGGL((kern<WK_ARGS targs, kListLanes>), dim3(list_blocks(S.nf)),       \
+                         dim3(kBlock), 0, st, S, ##__VA_ARGS__);                           \
+    else                                                                                   \
+      hipLaunchKernelGGL((kern<WK_ARGS targs, 1>), dim3(grid_blocks(S.nf)), dim3(kBlock), 0, \
+                         st, S, ##__VA_ARGS__);                                            \
+  } while (0)
+#define WK_EXACT(kern, targs, ...)                                                           \
+  hipLaunchKernelGGL((kern<WK_ARGS targs, 1>), dim3(grid_blocks(S.nf)), dim3(kBlock), 0, st, S, \
+                     ##__VA_ARGS__)
 
 template <class T>
 void Wkbb18Ops<T>::diagonal(hipStream_t st, const SceneView<T> &S, const NbrList *L, bool gc) {
   if (S.nf <= 0)
     return;
   const dim3 gr(grid_blocks(S.nf)), bl(kBlock);
-  if (L) {
-    if (gc)
-      hipLaunchKernelGGL((k_diag_list<T, true>), gr, bl, 0, st, S, *L);
-    else
-      hipLaunchKernelGGL((k_diag_list<T, false>), gr, bl, 0, st, S, *L);
-  } else {
-    if (gc)
-      hipLaunchKernelGGL((k_diag_exact<T, true>), gr, bl, 0, st, S);
-    else
-      hipLaunchKernelGGL((k_diag_exact<T, false>), gr, bl, 0, st, S);
-  }
+  if (L && gc)
+    WK_LIST(k_diag_list, (T, true), *L);
+  else if (L)
+    WK_LIST(k_diag_list, (T, false), *L);
+  else if (gc)
+    hipLaunchKernelGGL((k_diag_exact<T, true>), gr, bl, 0, st, S);
+  else
+    hipLaunchKernelGGL((k_diag_exact<T, false>), gr, bl, 0, st, S);
 }
 
 template <class T>
 void Wkbb18Ops<T>::setup(hipStream_t st, const SceneView<T> &S, const NbrList *L, bool gc,
                          double *part, double tol, int max_k, unsigned seq) {
-  const unsigned nb = grid_blocks(S.nf);
   if (S.nf > 0) {
-    const dim3 gr(nb), bl(kBlock);
-    const NbrList Lv = L ? *L : NbrList{};
     if (L && gc)
-      hipLaunchKernelGGL((k_cg_setup<T, false, true>), gr, bl, 0, st, S, Lv, part);
+      WK_LIST(k_cg_setup, (T, false, true), *L, part);
     else if (L)
-      hipLaunchKernelGGL((k_cg_setup<T, false, false>), gr, bl, 0, st, S, Lv, part);
+      WK_LIST(k_cg_setup, (T, false, false), *L, part);
     else if (gc)
-      hipLaunchKernelGGL((k_cg_setup<T, true, true>), gr, bl, 0, st, S, Lv, part);
+      WK_EXACT(k_cg_setup, (T, true, true), NbrList{}, part);
     else
-      hipLaunchKernelGGL((k_cg_setup<T, true, false>), gr, bl, 0, st, S, Lv, part);
+      WK_EXACT(k_cg_setup, (T, true, false), NbrList{}, part);
   }
-  hipLaunchKernelGGL(k_cg_setup_fin, dim3(1), dim3(kBlock), 0, st, S.ctl, part, nb, tol, max_k,
-                     seq);
+  hipLaunchKernelGGL(k_cg_setup_fin, dim3(1), dim3(kBlock), 0, st, S.ctl, part,
+                     L ? list_blocks(S.nf) : grid_blocks(S.nf), tol, max_k, seq);
 }
 
 template <class T>
 void Wkbb18Ops<T>::diagonal_setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
                                   bool gc, double *part, double tol, int max_k, unsigned seq) {
-  const unsigned nb = grid_blocks(S.nf);
   if (S.nf > 0) {
     if (gc)
-      hipLaunchKernelGGL((k_diag_setup_list<T, true>), dim3(nb), dim3(kBlock), 0, st, S, L, part);
+      WK_LIST(k_diag_setup_list, (T, true), L, part);
     else
-      hipLaunchKernelGGL((k_diag_setup_list<T, false>), dim3(nb), dim3(kBlock), 0, st, S, L,
-                         part);
+      WK_LIST(k_diag_setup_list, (T, false), L, part);
   }
-  hipLaunchKernelGGL(k_cg_setup_fin, dim3(1), dim3(kBlock), 0, st, S.ctl, part, nb, tol, max_k,
-                     seq);
+  hipLaunchKernelGGL(k_cg_setup_fin, dim3(1), dim3(kBlock), 0, st, S.ctl, part,
+                     list_blocks(S.nf), tol, max_k, seq);
 }
 
 template <class T>
@@ -1005,46 +1067,41 @@ void Wkbb18Ops<T>::iteration_product(hipStream_t st, const SceneView<T> &S, cons
                                      bool gc, double *part) {
   if (S.nf <= 0)
     return;
-  const dim3 gr(grid_blocks(S.nf)), bl(kBlock);
-  const NbrList Lv = L ? *L : NbrList{};
   if (L && gc)
-    hipLaunchKernelGGL((k_cg_spmv<T, false, true>), gr, bl, 0, st, S, Lv, part);
+    WK_LIST(k_cg_spmv, (T, false, true), *L, part);
   else if (L)
-    hipLaunchKernelGGL((k_cg_spmv<T, false, false>), gr, bl, 0, st, S, Lv, part);
+    WK_LIST(k_cg_spmv, (T, false, false), *L, part);
   else if (gc)
-    hipLaunchKernelGGL((k_cg_spmv<T, true, true>), gr, bl, 0, st, S, Lv, part);
+    WK_EXACT(k_cg_spmv, (T, true, true), NbrList{}, part);
   else
-    hipLaunchKernelGGL((k_cg_spmv<T, true, false>), gr, bl, 0, st, S, Lv, part);
+    WK_EXACT(k_cg_spmv, (T, true, false), NbrList{}, part);
 }
 
 template <class T>
-void Wkbb18Ops<T>::iteration_vectors(hipStream_t st, const SceneView<T> &S, double *part,
-                                     bool split) {
+void Wkbb18Ops<T>::iteration_vectors(hipStream_t st, const SceneView<T> &S, const NbrList *L,
+                                     double *part, bool split) {
   if (S.nf <= 0)
     return;
-  const unsigned nb = grid_blocks(S.nf);
+  const unsigned nb = grid_blocks(S.nf), nl = L ? list_blocks(S.nf) : nb;
   const dim3 gr(nb), bl(kBlock);
-  if (!split && nb <= kFusedCgBlocks) {
-    // p.q partials at part[0, nb), r.r and r.y at part[nb, 3 nb)
-    hipLaunchKernelGGL(k_cg_update_alpha<T>, gr, bl, 0, st, S, part, part + nb);
-    hipLaunchKernelGGL(k_cg_direction_beta<T>, gr, bl, 0, st, S, part + nb);
-    return;
-  }
-  hipLaunchKernelGGL(k_cg_alpha, dim3(1), bl, 0, st, S.ctl, part, nb);
-  hipLaunchKernelGGL(k_cg_update<T>, gr, bl, 0, st, S, part);
-  hipLaunchKernelGGL(k_cg_beta, dim3(1), bl, 0, st, S.ctl, part, nb);
-  hipLaunchKernelGGL(k_cg_direction<T>, gr, bl, 0, st, S);
+  // p.q partials at part[0, nl), r.r and r.y at part[nl, nl + 2 nb)
+  const int fold = !split && nb <= kFusedCgBlocks ? 1 : 0;
+  if (!fold)
+    hipLaunchKernelGGL(k_cg_alpha, dim3(1), bl, 0, st, S.ctl, part, nl);
+  hipLaunchKernelGGL(k_cg_update<T>, gr, bl, 0, st, S, fold, part, nl, part + nl);
+  if (!fold)
+    hipLaunchKernelGGL(k_cg_beta, dim3(1), bl, 0, st, S.ctl, part + nl, nb);
+  hipLaunchKernelGGL(k_cg_direction<T>, gr, bl, 0, st, S, fold, part + nl);
 }
 
 template <class T>
 void Wkbb18Ops<T>::correction(hipStream_t st, const SceneView<T> &S, const NbrList *L) {
   if (S.nf <= 0)
     return;
-  const dim3 gr(grid_blocks(S.nf)), bl(kBlock);
   if (L)
-    hipLaunchKernelGGL((k_corr<T, true>), gr, bl, 0, st, S, *L);
+    WK_LIST(k_corr, (T, true), *L);
   else
-    hipLaunchKernelGGL((k_corr<T, false>), gr, bl, 0, st, S, NbrList{});
+    WK_EXACT(k_corr, (T, false), NbrList{});
 }
 
 template <class T>
@@ -1061,46 +1118,49 @@ void Wkbb18Ops<T>::apply(hipStream_t st, const SceneView<T> &S) {
 
 template <class T>
 void Wkbb18Ops<T>::correction_batch(hipStream_t st, const BatchEntry<T> *tab,
-                                    const BatchMaps &m) {
-  if (m.n_gc > 0)
-    hipLaunchKernelGGL(k_corr_b<T>, dim3(m.n_gc), dim3(kBlock), 0, st, tab, m.gc);
+                                    const BatchBlocks &B) {
+  const BatchBlocks G = B.group(1);
+  if (const unsigned n = G.launch(kListLanes))
+    hipLaunchKernelGGL(k_corr_b<T>, dim3(n), dim3(kBlock), 0, st, tab, G);
 }
 
 template <class T>
 void Wkbb18Ops<T>::diagonal_setup_batch(hipStream_t st, const BatchEntry<T> *tab,
-                                        const BatchMaps &m, unsigned nscenes) {
+                                        const BatchBlocks &B, unsigned nscenes) {
   if (nscenes == 0)
     return;
-  if (m.n_plain > 0)
-    hipLaunchKernelGGL((k_diag_setup_b<T, false>), dim3(m.n_plain), dim3(kBlock), 0, st, tab,
-                       m.plain);
-  if (m.n_gc > 0)
-    hipLaunchKernelGGL((k_diag_setup_b<T, true>), dim3(m.n_gc), dim3(kBlock), 0, st, tab, m.gc);
+  const BatchBlocks P = B.group(0), G = B.group(1);
+  if (const unsigned n = P.launch(kListLanes))
+    hipLaunchKernelGGL((k_diag_setup_b<T, false>), dim3(n), dim3(kBlock), 0, st, tab, P);
+  if (const unsigned n = G.launch(kListLanes))
+    hipLaunchKernelGGL((k_diag_setup_b<T, true>), dim3(n), dim3(kBlock), 0, st, tab, G);
   hipLaunchKernelGGL(k_cg_setup_fin_b<T>, dim3(nscenes), dim3(kBlock), 0, st, tab);
 }
 
 template <class T>
-void Wkbb18Ops<T>::iteration_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchMaps &m,
+void Wkbb18Ops<T>::iteration_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
                                    unsigned nscenes, bool any_split) {
-  if (m.n_all == 0)
+  const unsigned na = B.launch(1);
+  if (na == 0)
     return;
-  const dim3 gr(m.n_all), bl(kBlock);
-  if (m.n_plain > 0)
-    hipLaunchKernelGGL((k_cg_spmv_b<T, false>), dim3(m.n_plain), bl, 0, st, tab, m.plain);
-  if (m.n_gc > 0)
-    hipLaunchKernelGGL((k_cg_spmv_b<T, true>), dim3(m.n_gc), bl, 0, st, tab, m.gc);
+  const BatchBlocks P = B.group(0), G = B.group(1);
+  const dim3 bl(kBlock);
+  if (const unsigned n = P.launch(kListLanes))
+    hipLaunchKernelGGL((k_cg_spmv_b<T, false>), dim3(n), bl, 0, st, tab, P);
+  if (const unsigned n = G.launch(kListLanes))
+    hipLaunchKernelGGL((k_cg_spmv_b<T, true>), dim3(n), bl, 0, st, tab, G);
   if (any_split)
     hipLaunchKernelGGL(k_cg_alpha_b<T>, dim3(nscenes), bl, 0, st, tab);
-  hipLaunchKernelGGL(k_cg_update_b<T>, gr, bl, 0, st, tab, m.all);
+  hipLaunchKernelGGL(k_cg_update_b<T>, dim3(na), bl, 0, st, tab, B);
   if (any_split)
     hipLaunchKernelGGL(k_cg_beta_b<T>, dim3(nscenes), bl, 0, st, tab);
-  hipLaunchKernelGGL(k_cg_direction_b<T>, gr, bl, 0, st, tab, m.all);
+  hipLaunchKernelGGL(k_cg_direction_b<T>, dim3(na), bl, 0, st, tab, B);
 }
 
 template <class T>
-void Wkbb18Ops<T>::apply_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchMaps &m) {
-  if (m.n_all > 0)
-    hipLaunchKernelGGL(k_cg_apply_b<T>, dim3(m.n_all), dim3(kBlock), 0, st, tab, m.all);
+void Wkbb18Ops<T>::apply_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B) {
+  if (const unsigned n = B.launch(1))
+    hipLaunchKernelGGL(k_cg_apply_b<T>, dim3(n), dim3(kBlock), 0, st, tab, B);
 }
 
 template struct Wkbb18Ops<float>;
