@@ -91,9 +91,9 @@ def parse():
     ap.add_argument("--budget-gb", type=float, default=200.0)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--schedule", type=int, default=-1,
-                    help="force the schedule mask of the main scene (-1: autotune)")
+                    help="force the schedule mask of the main scene (-1: the default)")
     ap.add_argument("--batch-schedule", type=int, default=-1,
-                    help="force the schedule mask of batched steps (-1: autotune)")
+                    help="force the schedule mask of batched steps (-1: the default)")
     ap.add_argument("--cpu-seconds", type=float, default=15.0,
                     help="target length of the CPU baseline sample")
     ap.add_argument("--batch-scenes", type=int, default=64,
@@ -203,8 +203,8 @@ def bench_scene(ctx, sc, steps, warmup, schedules=False, traffic=False, schedule
     """Whole steps of one device-resident scene: the timed region (K steps,
     no instrumentation), a pass with per-stage HIP events, the roofline of
     the dominant stage and of the whole step. schedule >= 0 forces the
-    scene's schedule mask (bit-identical variants) instead of the tuner's
-    choice. Returns (dict, scene)."""
+    scene's schedule mask (bit-identical variants) instead of the
+    default. Returns (dict, scene)."""
     from prtcl_amd import hip
     g = hip.HipScene(ctx, sc)
     g.prepare()
@@ -248,9 +248,8 @@ def bench_scene(ctx, sc, steps, warmup, schedules=False, traffic=False, schedule
 
     sched = {}
     if schedules:
-        # per-launch stage times of both schedules of the fused passes (global
-        # gathers vs LDS-staged slabs), each forced for a few further steps
-        for name, mask in (("global", 8), ("lds", 7 | 8)):
+        # per-launch stage times of the fused passes over a few further steps
+        for name, mask in (("global", 8),):
             g.set_schedule(mask)
             g.step(1)
             ctx.profile(True)

@@ -387,11 +387,9 @@ int prtcl_hip_serve_pending(prtcl_hip_ctx *ctx, int64_t *requests, int64_t *step
 
 /* ---- schedule of the fused passes ---------------------------------------
  * No reference counterpart (tuning of this implementation; results do not
- * depend on it). The setup, pressure-acceleration and pressure passes of
- * prtcl_hip_step either gather the neighbours' fields from global memory or
- * stage them slab by slab in LDS; an autotuner times both on the first fused
- * steps of each scene (and of batched steps) and keeps the faster per pass.
- * mask: bit 0 setup, bit 1 pressure acceleration, bit 2 pressure in LDS;
+ * depend on it). mask: bits 0 to 2 once chose LDS-staged neighbour passes, which
+ * are slower at every size; they are accepted and reported back and change
+ * nothing;
  * bit 3 launches each IISPH iteration kernel by kernel instead of replaying
  * it from a captured hipGraph; bit 4 gives the alpha and beta reductions of
  * every CG iteration (WKBB18 and pt16 solves) one-block kernels of their own
@@ -400,7 +398,8 @@ int prtcl_hip_serve_pending(prtcl_hip_ctx *ctx, int64_t *requests, int64_t *step
  * WKBB18 diagonal and the CG set-up of a fused step instead of once; bit 6
  * runs IISPH iteration 1 as its own pressure-acceleration and pressure
  * passes instead of folding it into the setup pass (with every pressure 0 at
- * the start of the solve it needs no neighbours); -1 restarts the tuner.
+ * the start of the solve it needs no neighbours); -1 returns to the
+ * default (bit 3).
  * scene < 0 addresses the schedule of batched steps. */
 int prtcl_hip_set_schedule(prtcl_hip_ctx *ctx, int32_t scene, int32_t mask);
 int prtcl_hip_get_schedule(prtcl_hip_ctx *ctx, int32_t scene, int32_t *mask);

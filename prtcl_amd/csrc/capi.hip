@@ -640,8 +640,7 @@ int prtcl_hip_set_schedule(prtcl_hip_ctx *ctx, int32_t scene, int32_t mask) {
     if (mask < -1 || mask > 127)
       return fail(ctx, PRTCL_HIP_INVALID_ARGUMENT, "schedule mask must be -1 or 0..127");
     if (scene < 0) {
-      for (auto &t : ctx->res.batch_tuner)
-        t.force(mask);
+      ctx->res.batch_schedule.force(mask);
       return PRTCL_HIP_OK;
     }
     find(ctx, scene)->set_schedule(mask);
@@ -653,7 +652,7 @@ int prtcl_hip_get_schedule(prtcl_hip_ctx *ctx, int32_t scene, int32_t *mask) {
   return guarded(ctx, [&]() -> int {
     if (!mask)
       return fail(ctx, PRTCL_HIP_INVALID_ARGUMENT, "mask is NULL");
-    *mask = scene < 0 ? ctx->res.batch_tuner[0].current().mask() : find(ctx, scene)->schedule();
+    *mask = scene < 0 ? ctx->res.batch_schedule.current().mask() : find(ctx, scene)->schedule();
     return PRTCL_HIP_OK;
   });
 }

@@ -268,10 +268,7 @@ __device__ __forceinline__ double first_iteration(const SceneView<T> &S, int i,
 // thread's column of an LDS table; phase 2 runs the pair sums over the
 // compacted entries, so the lanes that reject a candidate do not wait for the
 // kernel arithmetic of the ones that accept it. The table is written to the
-// list row by row (coalesced). With kStage the block stages each slab's span
-// in LDS and runs both phases per slab against the staged copy; otherwise
-// the candidates are read from global memory (through L2) and both phases
-// run once over all 27 cells.
+// list row by row (coalesced).
 // ---------------------------------------------------------------------------
 // the pair sums of the setup pass for one particle (or one lane's share)
 template <class T, bool kWithSource>
@@ -377,20 +374,16 @@ struct SetupSums {
   }
 };
 
-template <class T, bool kStage>
 struct SetupShared {
-  vec4_t<T> sx[kStage ? slab_cap<T>() + kRunPad : 1];
   // rows kNbrCap + 1 .. kNbrCap + 8 take the writes of a lane past its cap
   uint16_t lst[kNbrCap + 9][kBlock];
   BlockRanges sR;
 };
 
-template <class T, bool kWithSource, bool kStage>
+template <class T, bool kWithSource>
 __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrList &L,
                                              vec4_t<T> *vout, unsigned lb,
-                                             SetupShared<T, kStage> &sh) {
-  constexpr uint32_t kCap = slab_cap<T>();
-  auto &sx = sh.sx;
+                                             SetupShared &sh) {
   auto &lst = sh.lst;
   BlockRanges &sR = sh.sR;
   const unsigned t = threadIdx.x;
@@ -401,9 +394,7 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
   if (t < 6)
     reinterpret_cast<uint32_t *>(L.blk + lb)[t] = t < 3 ? sR.base[t] : sR.len[t - 3];
   const Spans R = Spans::of(sR);
-  const uint32_t smax = R.max_len();
-  const bool staged = kStage && smax <= kCap;
-  const bool encodable = smax <= 0x10000u;
+  const bool encodable = R.max_len() <= 0x10000u;
 
   const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
   const vec4_t<T> xi = valid ? S.xm[i] : zero4;
@@ -412,10 +403,8 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
   q.rho = q.self();
   uint32_t cnt = 0;
   uint32_t cs[3] = {0u, 0u, 0u};  // entries per slab
-  // candidate test of the slab-s runs, positions from global memory
-  // (kLds = false) or from the staged span; accepted entries are appended
-  auto scan = [&](int s, auto lds_tag) {
-    constexpr bool kLds = decltype(lds_tag)::value;
+  // candidate test of the slab-s runs; accepted entries are appended
+  auto scan = [&](int s) {
     const uint32_t base = R.base(s);
     uint32_t rb[3], re[3];
     slab_bounds(S.grid, cell, S.fstart, s, rb, re);
@@ -435,7 +424,7 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
       // can hold the particle itself.
       auto trip = [&](uint32_t j, auto tail_tag) {
         constexpr bool kTail = decltype(tail_tag)::value;
-        const vec4_t<T> *__restrict__ src = kLds ? sx + (j - base) : S.xm + j;
+        const vec4_t<T> *__restrict__ src = S.xm + j;
         vec4_t<T> pk[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
@@ -463,33 +452,11 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
     }
   };
   bool over = !encodable;
-  if (staged) {
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-      stage_span(R, s, S.xm, sx);
-      __syncthreads();
-      if (valid && !over) {
-        const uint32_t c0 = cnt;
-        scan(s, std::true_type{});
-        if (cnt > kNbrCap) {
-          over = true;
-        } else {
-          cs[s] = cnt - c0;
-          const uint32_t base = R.base(s);
-#pragma unroll 4
-          for (uint32_t e = c0; e < cnt; ++e) {
-            const uint32_t u = lst[e][t];
-            q.pair(sx[u], q.load_v(base + u));
-          }
-        }
-      }
-      __syncthreads();
-    }
-  } else if (valid && !over) {
+  if (valid && !over) {
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
       const uint32_t c0 = cnt;
-      scan(s, std::false_type{});
+      scan(s);
       cs[s] = cnt - c0;
     }
     if (cnt > kNbrCap) {
@@ -645,11 +612,11 @@ __global__ __launch_bounds__(kBlock) void k_setup8(SceneView<T> S, NbrList L, ve
     begin_solve(S.ctl, B);
 }
 
-template <class T, bool kWithSource, bool kStage>
+template <class T, bool kWithSource>
 __global__ __launch_bounds__(kBlock) void k_setup(SceneView<T> S, NbrList L,
                                                   vec4_t<T> *vout, SolveBegin B) {
-  __shared__ SetupShared<T, kStage> sh;
-  k_setup_body<T, kWithSource, kStage>(S, L, vout, xcd_block(blockIdx.x, gridDim.x), sh);
+  __shared__ SetupShared sh;
+  k_setup_body<T, kWithSource>(S, L, vout, xcd_block(blockIdx.x, gridDim.x), sh);
   // no thread of the setup reads the control block
   if (B.seq != 0u && blockIdx.x == 0 && threadIdx.x == 0)
     begin_solve(S.ctl, B);
@@ -845,51 +812,12 @@ __global__ __launch_bounds__(kBlock) void k_source_list(SceneView<T> S, NbrList 
   k_source_list_body<T, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
-// Walk of the list entries of particle i (all threads of the block call it).
-// kStage and spans that fit LDS: per slab, stage(s) fills LDS (all threads),
-// then use(lds(u)) for the neighbour at LDS index u. Otherwise
-// use(load(j)) over the whole list with global slots, a chunk of 8 gathers
-// in flight.
-template <bool kStage, uint32_t kCap, int kLanes, int kGroup = 8, class Stage, class Lds,
-          class Load, class Use>
-__device__ __forceinline__ void list_walk(const NbrList &L, const Spans &R, size_t n, int i,
-                                          uint32_t info, uint32_t sub, Stage &&stage, Lds &&lds,
-                                          Load &&load, Use &&use) {
-  const uint32_t live = (info & kListOverflow) ? 0u : info;
-  if (kStage && R.max_len() <= kCap) {
-    uint32_t e = 0;
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-      const uint32_t c = (live >> (8 * s)) & 0xFFu;
-      stage(s);
-      __syncthreads();
-      uint32_t q = 0;
-      for (; q + 4 <= c; q += 4) {
-        const uint32_t u0 = list_entry(L, n, i, e + q), u1 = list_entry(L, n, i, e + q + 1);
-        const uint32_t u2 = list_entry(L, n, i, e + q + 2), u3 = list_entry(L, n, i, e + q + 3);
-        use(lds(u0));
-        use(lds(u1));
-        use(lds(u2));
-        use(lds(u3));
-      }
-      for (; q < c; ++q)
-        use(lds(list_entry(L, n, i, e + q)));
-      __syncthreads();
-      e += c;
-    }
-  } else {
-    list_gather_lanes<kLanes, kGroup>(L, R, n, i, live, sub, load, use);
-  }
-}
-
 // IISPH pressure acceleration over the list: a_i = p_i c_i - sum m_j pr_j gradW
-template <class T, bool kStage, int kLanes>
+template <class T, int kLanes>
 __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const NbrList &L,
                                                   unsigned lb) {
   if (S.ctl->done)
     return;
-  constexpr uint32_t kCap = slab_cap<T>();
-  __shared__ vec4_t<T> sq[kStage ? kCap : 1];
   const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
   const uint32_t sub = threadIdx.x % kLanes;
   const bool valid = i < S.nf;
@@ -909,9 +837,9 @@ __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const N
     a1 += s * d1;
     a2 += s * d2;
   };
-  list_walk<kStage, kCap, kLanes>(
-      L, R, static_cast<size_t>(S.nf), i, info, sub, [&](int s) { stage_span(R, s, S.xq, sq); },
-      [&](uint32_t u) { return sq[u]; }, [&](uint32_t j) { return S.xq[j]; }, pair);
+  if (!(info & kListOverflow))
+    list_gather_lanes<kLanes, 8>(
+        L, R, static_cast<size_t>(S.nf), i, info, sub, [&](uint32_t j) { return S.xq[j]; }, pair);
   if (valid && sub == 0 && (info & kListOverflow))
     grid_walk(S, i, xi, [&](uint32_t j) { pair(S.xq[j]); });
   a0 = lanes_sum<kLanes>(a0);
@@ -925,24 +853,21 @@ __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const N
   S.xa[S.xa_a(static_cast<size_t>(i))] = ai;
 }
 
-template <class T, bool kStage, int kLanes>
+template <class T, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_accel_list(SceneView<T> S, NbrList L) {
-  k_accel_list_body<T, kStage, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
+  k_accel_list_body<T, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // IISPH relaxed Jacobi update over the list, FP64 aprde reduction and the
 // device-side convergence decision (example.lua:409-421)
-template <class T, bool kStage, int kLanes>
+template <class T, int kLanes>
 __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, const NbrList &L,
                                                      unsigned lb) {
   if (S.ctl->done)
     return;
-  constexpr uint32_t kCap = slab_cap<T>();
   struct XA {
     vec4_t<T> x, a;  // (x, m) and (a, 0) of a neighbour
   };
-  __shared__ vec4_t<T> sx[kStage ? kCap : 1];
-  __shared__ vec4_t<T> sa[kStage ? kCap : 1];
   const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
   const uint32_t sub = threadIdx.x % kLanes;
   const bool valid = i < S.nf;
@@ -962,15 +887,10 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
     sum += q.x.w * K.gradf_unscaled(d0 * d0 + d1 * d1 + d2 * d2) *
            (q.a.x * d0 + q.a.y * d1 + q.a.z * d2);
   };
-  list_walk<kStage, kCap, kLanes, 4>(
-      L, R, static_cast<size_t>(S.nf), i, info, sub,
-      [&](int s) {
-        stage_span(R, s, S.xm, sx);
-        stage_span_fn(R, s, [&](size_t g) { return S.xa[S.xa_a(g)]; }, sa);
-      },
-      [&](uint32_t u) { return XA{sx[u], sa[u]}; },
-      [&](uint32_t j) { return XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]}; },
-      pair);
+  if (!(info & kListOverflow))
+    list_gather_lanes<kLanes, 4>(
+        L, R, static_cast<size_t>(S.nf), i, info, sub,
+        [&](uint32_t j) { return XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]}; }, pair);
   if (valid && sub == 0 && (info & kListOverflow))
     grid_walk(S, i, xi, [&](uint32_t j) {
       pair(XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]});
@@ -994,9 +914,9 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
     S.partials[lb] = bs;
 }
 
-template <class T, bool kStage, int kLanes>
+template <class T, int kLanes>
 __global__ __launch_bounds__(kBlock) void k_pressure_list(SceneView<T> S, NbrList L) {
-  k_pressure_list_body<T, kStage, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
+  k_pressure_list_body<T, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Sum of the block partials in block order (FP64, fixed tree) and the
@@ -1111,9 +1031,8 @@ __global__ __launch_bounds__(kBlock) void k_speed_finalize(Ctl *c, const double 
 // passes take the body that the block's scene takes alone (split_scene)
 // the two setup bodies share their LDS, so the large scenes' blocks keep
 // their five per CU
-template <class T, bool kStage>
 union SetupPool {
-  SetupShared<T, kStage> setup;
+  SetupShared setup;
   Scan8Shared scan;
 };
 
@@ -1133,14 +1052,14 @@ union SetupPool {
 constexpr unsigned kSetupParts = kBlock / kScanParts;  // setup blocks per block of a split scene
 constexpr unsigned kListParts = kListLanes;
 
-template <class T, bool kWithSource, bool kStage>
+template <class T, bool kWithSource>
 __global__ __launch_bounds__(kBlock) void k_setup_b(const BatchEntry<T> *tab, BatchBlocks B) {
-  __shared__ SetupPool<T, kStage> sh;
+  __shared__ SetupPool sh;
   BATCH_PASS_ENTRY(kSetupParts, setup_blocks);
   if (split)
     k_setup8_body<T, kWithSource>(E.S, L, E.vtmp, lb, sh.scan);
   else
-    k_setup_body<T, kWithSource, kStage>(E.S, L, E.vtmp, lb, sh.setup);
+    k_setup_body<T, kWithSource>(E.S, L, E.vtmp, lb, sh.setup);
 }
 
 // scenes with explicit viscosity or axial gravity: after the setup without the
@@ -1169,22 +1088,22 @@ __global__ __launch_bounds__(kBlock) void k_source_b(const BatchEntry<T> *tab, B
     k_source_list_body<T, 1>(S2, L, lb);
 }
 
-template <class T, bool kStage>
+template <class T>
 __global__ __launch_bounds__(kBlock) void k_accel_b(const BatchEntry<T> *tab, BatchBlocks B) {
   BATCH_PASS_ENTRY(kListParts, list_blocks);
   if (split)
-    k_accel_list_body<T, false, kListLanes>(E.S, L, lb);
+    k_accel_list_body<T, kListLanes>(E.S, L, lb);
   else
-    k_accel_list_body<T, kStage, 1>(E.S, L, lb);
+    k_accel_list_body<T, 1>(E.S, L, lb);
 }
 
-template <class T, bool kStage>
+template <class T>
 __global__ __launch_bounds__(kBlock) void k_pressure_b(const BatchEntry<T> *tab, BatchBlocks B) {
   BATCH_PASS_ENTRY(kListParts, list_blocks);
   if (split)
-    k_pressure_list_body<T, false, kListLanes>(E.S, L, lb);
+    k_pressure_list_body<T, kListLanes>(E.S, L, lb);
   else
-    k_pressure_list_body<T, kStage, 1>(E.S, L, lb);
+    k_pressure_list_body<T, 1>(E.S, L, lb);
 }
 
 // one block per scene
@@ -1237,8 +1156,7 @@ void FusedOps<T>::build_list(hipStream_t st, const SceneView<T> &S, const NbrLis
 
 template <class T>
 void FusedOps<T>::setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
-                        bool explicit_viscosity, vec4_t<T> *vtmp, bool lds,
-                        const SolveBegin &B) {
+                        bool explicit_viscosity, vec4_t<T> *vtmp, const SolveBegin &B) {
   if (S.nf <= 0)
     return;
   const dim3 gr(setup_blocks(S.nf)), bl(kBlock);
@@ -1249,18 +1167,14 @@ void FusedOps<T>::setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
   if (!explicit_viscosity && !S.axial) {
     if (split)
       hipLaunchKernelGGL((k_setup8<T, true>), gr, bl, 0, st, S, L, vtmp, B);
-    else if (lds)
-      hipLaunchKernelGGL((k_setup<T, true, true>), gr, bl, 0, st, S, L, vtmp, B);
     else
-      hipLaunchKernelGGL((k_setup<T, true, false>), gr, bl, 0, st, S, L, vtmp, B);
+      hipLaunchKernelGGL((k_setup<T, true>), gr, bl, 0, st, S, L, vtmp, B);
     return;
   }
   if (split)
     hipLaunchKernelGGL((k_setup8<T, false>), gr, bl, 0, st, S, L, vtmp, B);
-  else if (lds)
-    hipLaunchKernelGGL((k_setup<T, false, true>), gr, bl, 0, st, S, L, vtmp, B);
   else
-    hipLaunchKernelGGL((k_setup<T, false, false>), gr, bl, 0, st, S, L, vtmp, B);
+    hipLaunchKernelGGL((k_setup<T, false>), gr, bl, 0, st, S, L, vtmp, B);
   const dim3 gl(list_blocks(S.nf));
   if (!explicit_viscosity)
     hipLaunchKernelGGL(k_gravity_v<T>, dim3(grid_blocks(S.nf)), bl, 0, st, S, vtmp);
@@ -1278,30 +1192,25 @@ void FusedOps<T>::setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
 }
 
 template <class T>
-void FusedOps<T>::accel(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool lds) {
+void FusedOps<T>::accel(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
   if (S.nf <= 0)
     return;
   const dim3 gr(list_blocks(S.nf)), bl(kBlock);
   if (split_scene(S.nf))
-    hipLaunchKernelGGL((k_accel_list<T, false, kListLanes>), gr, bl, 0, st, S, L);
-  else if (lds)
-    hipLaunchKernelGGL((k_accel_list<T, true, 1>), gr, bl, 0, st, S, L);
+    hipLaunchKernelGGL((k_accel_list<T, kListLanes>), gr, bl, 0, st, S, L);
   else
-    hipLaunchKernelGGL((k_accel_list<T, false, 1>), gr, bl, 0, st, S, L);
+    hipLaunchKernelGGL((k_accel_list<T, 1>), gr, bl, 0, st, S, L);
 }
 
 template <class T>
-void FusedOps<T>::pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool lds) {
+void FusedOps<T>::pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
   if (S.nf <= 0)
     return;
   const unsigned nb = list_blocks(S.nf);
   if (split_scene(S.nf))
-    hipLaunchKernelGGL((k_pressure_list<T, false, kListLanes>), dim3(nb), dim3(kBlock), 0, st, S,
-                       L);
-  else if (lds)
-    hipLaunchKernelGGL((k_pressure_list<T, true, 1>), dim3(nb), dim3(kBlock), 0, st, S, L);
+    hipLaunchKernelGGL((k_pressure_list<T, kListLanes>), dim3(nb), dim3(kBlock), 0, st, S, L);
   else
-    hipLaunchKernelGGL((k_pressure_list<T, false, 1>), dim3(nb), dim3(kBlock), 0, st, S, L);
+    hipLaunchKernelGGL((k_pressure_list<T, 1>), dim3(nb), dim3(kBlock), 0, st, S, L);
   hipLaunchKernelGGL(k_pressure_finalize, dim3(1), dim3(kBlock), 0, st, S.ctl, S.partials, nb,
                      false);
 }
@@ -1349,21 +1258,13 @@ void FusedOps<T>::integrate(hipStream_t st, const SceneView<T> &S, unsigned seq)
 }
 
 template <class T>
-void FusedOps<T>::setup_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
-                              bool lds) {
+void FusedOps<T>::setup_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B) {
   const dim3 bl(kBlock);
   const BatchBlocks B1 = B.group(0), B3 = B.group(1);
-  if (const unsigned n = B1.launch(kSetupParts)) {
-    if (lds)
-      hipLaunchKernelGGL((k_setup_b<T, true, true>), dim3(n), bl, 0, st, tab, B1);
-    else
-      hipLaunchKernelGGL((k_setup_b<T, true, false>), dim3(n), bl, 0, st, tab, B1);
-  }
+  if (const unsigned n = B1.launch(kSetupParts))
+    hipLaunchKernelGGL((k_setup_b<T, true>), dim3(n), bl, 0, st, tab, B1);
   if (const unsigned n = B3.launch(kSetupParts)) {
-    if (lds)
-      hipLaunchKernelGGL((k_setup_b<T, false, true>), dim3(n), bl, 0, st, tab, B3);
-    else
-      hipLaunchKernelGGL((k_setup_b<T, false, false>), dim3(n), bl, 0, st, tab, B3);
+    hipLaunchKernelGGL((k_setup_b<T, false>), dim3(n), bl, 0, st, tab, B3);
     const dim3 gl(B3.launch(kListParts));
     hipLaunchKernelGGL(k_vstar_b<T>, gl, bl, 0, st, tab, B3);
     hipLaunchKernelGGL(k_source_b<T>, gl, bl, 0, st, tab, B3);
@@ -1371,27 +1272,18 @@ void FusedOps<T>::setup_batch(hipStream_t st, const BatchEntry<T> *tab, const Ba
 }
 
 template <class T>
-void FusedOps<T>::accel_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
-                              bool lds) {
-  const unsigned n = B.launch(kListParts);
-  if (n == 0)
-    return;
-  if (lds)
-    hipLaunchKernelGGL((k_accel_b<T, true>), dim3(n), dim3(kBlock), 0, st, tab, B);
-  else
-    hipLaunchKernelGGL((k_accel_b<T, false>), dim3(n), dim3(kBlock), 0, st, tab, B);
+void FusedOps<T>::accel_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B) {
+  if (const unsigned n = B.launch(kListParts))
+    hipLaunchKernelGGL(k_accel_b<T>, dim3(n), dim3(kBlock), 0, st, tab, B);
 }
 
 template <class T>
 void FusedOps<T>::pressure_batch(hipStream_t st, const BatchEntry<T> *tab, const BatchBlocks &B,
-                                 unsigned nscenes, bool lds) {
+                                 unsigned nscenes) {
   const unsigned n = B.launch(kListParts);
   if (n == 0)
     return;
-  if (lds)
-    hipLaunchKernelGGL((k_pressure_b<T, true>), dim3(n), dim3(kBlock), 0, st, tab, B);
-  else
-    hipLaunchKernelGGL((k_pressure_b<T, false>), dim3(n), dim3(kBlock), 0, st, tab, B);
+  hipLaunchKernelGGL(k_pressure_b<T>, dim3(n), dim3(kBlock), 0, st, tab, B);
   hipLaunchKernelGGL(k_pressure_finalize_b<T>, dim3(nscenes), dim3(kBlock), 0, st, tab);
 }
 

@@ -8,8 +8,10 @@
 // to the last run end over the block's particles (about three rows of
 // particles). A list entry is the neighbour's offset from the span start of
 // its slab (16 bits), so the list costs 2 bytes per pair; the global slot is
-// span base + entry, and a pass that stages a span in LDS reads the
-// neighbour at LDS index = entry.
+// span base + entry. (Staging the spans in LDS instead of gathering through L2 is
+// slower in full launches: 250,000 particles, setup 72.6 against 68.3 us,
+// pressure acceleration 17.3 against 14.8, pressure 29.9 against 23.7; 1M, setup
+// 321 against 229.)
 //
 // Layout: chunks of 8 entries; entry e of particle i at
 // idx[((e / 8) * n + i) * 8 + e % 8], so one 16-byte load per lane fetches 8
@@ -31,16 +33,6 @@ constexpr uint32_t kListBoundary = 1u << 24;
 __device__ __forceinline__ bool list_has_boundary(uint32_t info) {
   return (info & (kListBoundary | kListOverflow)) != 0u;
 }
-// LDS bytes of one staged field array of one span (the real4 fields of 1536
-// particles in FP32, 768 in FP64); a block whose span is larger reads the
-// neighbours' fields from global memory instead
-constexpr uint32_t kSlabBytes = 24u * 1024u;
-
-template <class T>
-constexpr uint32_t slab_cap() {
-  return kSlabBytes / static_cast<uint32_t>(sizeof(vec4_t<T>));
-}
-
 struct BlockRanges {
   uint32_t base[3];  // first slot of the span of slab s (dz = s - 1)
   uint32_t len[3];   // its length (0: no particle of the block has that layer)
@@ -77,26 +69,6 @@ __device__ __forceinline__ Spans list_spans(const NbrList &L, int i) {
   return Spans::of(L.blk[i >> L.shift]);
 }
 
-// Cooperative copy of the span of slab s into LDS: dst[u] = src[base + u]
-// (all threads of the block call it).
-template <class V>
-__device__ __forceinline__ void stage_span(const Spans &R, int s, const V *__restrict__ src,
-                                           V *dst) {
-  const V *__restrict__ p = src + R.base(s);
-  const uint32_t len = R.len(s);
-  for (uint32_t u = threadIdx.x; u < len; u += kBlock)
-    dst[u] = p[u];
-}
-
-// the same with the value of global slot g given by at(g)
-template <class V, class At>
-__device__ __forceinline__ void stage_span_fn(const Spans &R, int s, At &&at, V *dst) {
-  const size_t base = R.base(s);
-  const uint32_t len = R.len(s);
-  for (uint32_t u = threadIdx.x; u < len; u += kBlock)
-    dst[u] = at(base + u);
-}
-
 constexpr uint32_t kChunk = 8;  // list entries per 16-byte chunk
 
 // the 8 entries of chunk g of particle i
@@ -109,12 +81,6 @@ __device__ __forceinline__ uint4 list_chunk(const NbrList &L, size_t n, int i, u
 __device__ __forceinline__ uint32_t chunk_entry(const uint4 &q, int k) {
   const uint32_t w = k < 2 ? q.x : (k < 4 ? q.y : (k < 6 ? q.z : q.w));
   return (k & 1) ? (w >> 16) : (w & 0xFFFFu);
-}
-
-// entry e of particle i (single load)
-__device__ __forceinline__ uint32_t list_entry(const NbrList &L, size_t n, int i, uint32_t e) {
-  return L.idx[((static_cast<size_t>(e) / kChunk) * n + static_cast<size_t>(i)) * kChunk +
-               e % kChunk];
 }
 
 // entries of a (not overflowed) list: the sum of its three slab counts

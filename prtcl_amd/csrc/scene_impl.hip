@@ -999,7 +999,7 @@ class SceneImpl final : public SceneBase {
     // takes every decision, the host keeps one iteration queued ahead
     const unsigned seq = ++seq_;
     const int max_k = std::max(0, desc.wkbb18_maximum_iterations);
-    const bool split = tuner_.current().cg_split;
+    const bool split = schedule_.current().cg_split;
     int r;
     if (with_diagonal && pl) {
       r = pf.begin(st, kStageWkbb18DiagSetup);
@@ -1083,7 +1083,7 @@ class SceneImpl final : public SceneBase {
     const NbrList *pl = fused ? &L : nullptr;
     Profiler &pf = res_->prof;
     const T xi = static_cast<T>(pt16_xi_);
-    const bool split = tuner_.current().cg_split;
+    const bool split = schedule_.current().cg_split;
     auto solve = [&](int which) {
       const unsigned seq = ++seq_;
       const int max_k = std::max(0, pt16_max_k_);
@@ -1191,8 +1191,7 @@ class SceneImpl final : public SceneBase {
     }
   }
 
-  // IISPH iterations until the device reports convergence or the cap. With
-  // `tune`, the fused passes are also timed for the schedule tuner.
+  // IISPH iterations until the device reports convergence or the cap.
   // nprde >= 0 also sets iisph_nprde (one control launch for both)
   // first_done: the fused setup has taken iteration 1 (its pressures and
   // aprde partials are written); its convergence step is the first launch.
@@ -1203,8 +1202,7 @@ class SceneImpl final : public SceneBase {
   // begun != 0: the fused setup launch has begun solve `begun` with these
   // arguments, so no control launch is needed
   int solve_impl(double tol, int min_it, int max_it, int *iters, double *rel, bool fused,
-                 const FusedSchedule &sc = FusedSchedule{}, bool tune = false,
-                 int nprde = -1, bool first_done = false, bool integrate = false,
+                 const FusedSchedule &sc = FusedSchedule{}, int nprde = -1, bool first_done = false, bool integrate = false,
                  unsigned begun = 0u) {
     require_grid();
     hipStream_t st = res_->stream;
@@ -1220,7 +1218,6 @@ class SceneImpl final : public SceneBase {
     const NbrList L = nbr_list();
     const NbrList PL = fused || nf_ == 0 ? L : proc_list();
     Profiler &pf = res_->prof;
-    tprof_.on = tune;
     // iterations enqueued so far (the iteration taken by the setup counts)
     int enq = 0;
     if (first) {
@@ -1230,7 +1227,7 @@ class SceneImpl final : public SceneBase {
     }
     // one IISPH iteration (pressure acceleration, pressure, finalize) replayed
     // from a captured graph unless timed or eager
-    const bool graph = fused && !sc.eager && !pf.on && !tune;
+    const bool graph = fused && !sc.eager && !pf.on;
     // the iteration kernels do not read the clock: a view without it keeps
     // one graph per buffer arrangement (two, alternating step by step)
     SceneView<T> Sg = S;
@@ -1241,28 +1238,24 @@ class SceneImpl final : public SceneBase {
       if (graph) {
         for (int k = 0; k < n; ++k)
           graphs_.launch(st, key, [&] {
-            FusedOps<T>::accel(st, Sg, L, sc.accel_lds);
-            FusedOps<T>::pressure(st, Sg, L, sc.pressure_lds);
+            FusedOps<T>::accel(st, Sg, L);
+            FusedOps<T>::pressure(st, Sg, L);
           });
         enq += n;
         return;
       }
       for (int k = 0; k < n; ++k) {
         int r = pf.begin(st, kStagePressureAccel, enq + k);
-        int q = tprof_.begin(st, kStagePressureAccel, enq + k);
         if (fused)
-          FusedOps<T>::accel(st, S, L, sc.accel_lds);
+          FusedOps<T>::accel(st, S, L);
         else
           SphOps<T>::iisph_accel(st, S, PL, true);
-        tprof_.end(st, q);
         pf.end(st, r);
         r = pf.begin(st, kStagePressure, enq + k);
-        q = tprof_.begin(st, kStagePressure, enq + k);
         if (fused)
-          FusedOps<T>::pressure(st, S, L, sc.pressure_lds);
+          FusedOps<T>::pressure(st, S, L);
         else
           SphOps<T>::iisph_pressure(st, S, PL, true);
-        tprof_.end(st, q);
         pf.end(st, r);
       }
       enq += n;
@@ -1304,16 +1297,6 @@ class SceneImpl final : public SceneBase {
       PRTCL_HIP_CHECK(hipStreamSynchronize(st));
       pf.resolve(p.iters);
     }
-    if (tune) {
-      tprof_.resolve(p.iters);
-      tuner_.record(0, tprof_.ms[kStageSetup], static_cast<double>(tprof_.launches[kStageSetup]));
-      tuner_.record(1, tprof_.ms[kStagePressureAccel],
-                    static_cast<double>(tprof_.launches[kStagePressureAccel]));
-      tuner_.record(2, tprof_.ms[kStagePressure],
-                    static_cast<double>(tprof_.launches[kStagePressure]));
-      tprof_.reset();
-      tprof_.on = false;
-    }
     // an iteration predicted too many costs a no-op launch, one too few a
     // host round trip: predict the larger of the last two counts
     predicted_iters_ = std::max(1, std::max(p.iters, last_iisph_iters_));
@@ -1348,8 +1331,7 @@ class SceneImpl final : public SceneBase {
         steps_since_permute_ = 0;
       }
       const bool fused = desc.step_mode == 0;
-      const bool tune = fused && tuner_.trial();
-      const FusedSchedule sc = tuner_.current();
+      const FusedSchedule sc = schedule_.current();
       // the fused setup takes IISPH iteration 1 (no neighbours needed at p = 0)
       const bool first_iter =
           fused && !sc.first_split && nf_ > 0 && desc.iisph_max_iterations > 0;
@@ -1358,8 +1340,6 @@ class SceneImpl final : public SceneBase {
         // one neighbour pass for density + list + IISPH setup (three with
         // explicit viscosity); the integrated velocity lands in tmpV4
         r = pf.begin(st, kStageSetup);
-        tprof_.on = tune;
-        const int q = tprof_.begin(st, kStageSetup);
         SceneView<T> Sv = view();
         Sv.first_iter = first_iter ? 1 : 0;
         // the setup also begins the step's IISPH solve (solve_impl's control
@@ -1373,8 +1353,7 @@ class SceneImpl final : public SceneBase {
           sb.seq = ++seq_;
         }
         FusedOps<T>::setup(st, Sv, nbr_list(), desc.explicit_viscosity != 0, P_.tmpV4,
-                           sc.setup_lds, sb);
-        tprof_.end(st, q);
+                           sb);
         pf.end(st, r);
         std::swap(P_.v, P_.tmpV4);
       } else {
@@ -1404,13 +1383,11 @@ class SceneImpl final : public SceneBase {
       double rel = 0;
       // the integration rides behind the solve's iterations unless stages
       // are timed
-      const bool spec_integrate = fused && !desc.implicit_viscosity && !pf.on && !tune &&
+      const bool spec_integrate = fused && !desc.implicit_viscosity && !pf.on &&
                                   nf_ > 0 && desc.iisph_max_iterations > 0;
       int rc = solve_impl(desc.iisph_tolerance, desc.iisph_min_iterations,
-                          desc.iisph_max_iterations, &it, &rel, fused, sc, tune, nf_,
+                          desc.iisph_max_iterations, &it, &rel, fused, sc, nf_,
                           first_iter, spec_integrate, sb.seq);
-      if (fused)
-        tuner_.finish_step();
       if (rc != PRTCL_HIP_OK)
         status = rc;
       const SceneView<T> S = view();
@@ -1528,7 +1505,7 @@ class SceneImpl final : public SceneBase {
   // each scene's results do not depend on the rest of the batch.
   // With `fixed`, the tables go to the caller's buffers instead of the
   // context's grown ones: no allocation, no graph capture, no timing (the
-  // launches are eager and the tuner keeps its current choice).
+  // launches are eager).
   static int step_batch(const std::vector<SceneImpl *> &v, CtxResources *res,
                         const BatchTables *fixed = nullptr) {
     const unsigned ns = static_cast<unsigned>(v.size());
@@ -1650,7 +1627,7 @@ class SceneImpl final : public SceneBase {
     std::vector<unsigned> seqs(ns);
     bool any_first_step = false;  // a scene needs iteration 1's convergence step
     // the setup takes IISPH iteration 1 (batchable scenes have max_it > 0)
-    const bool fold_first = !res->batch_tuner[sizeof(T) == 8 ? 1 : 0].current().first_split;
+    const bool fold_first = !res->batch_schedule.current().first_split;
     for (unsigned k = 0; k < ns; ++k) {
       SceneImpl &s = *v[k];
       BatchEntry<T> E{};
@@ -1706,7 +1683,7 @@ class SceneImpl final : public SceneBase {
     }
     // WKBB18 after the IISPH solve (the order of run_wkbb18: the CG's
     // sequence number follows the solve's)
-    const bool cg_split = res->batch_tuner[sizeof(T) == 8 ? 1 : 0].current().cg_split;
+    const bool cg_split = res->batch_schedule.current().cg_split;
     std::vector<unsigned> cg_seqs(nvs);
     bool any_split = false;
     for (unsigned kv = 0; kv < nvs; ++kv) {
@@ -1765,17 +1742,11 @@ class SceneImpl final : public SceneBase {
     for (unsigned k = 0; k < ns; ++k)
       if (permute[k])
         v[k]->host_permute(st);
-    ScheduleTuner &tn = res->batch_tuner[sizeof(T) == 8 ? 1 : 0];
-    const bool tune = !fixed && tn.trial();
-    FusedSchedule sc = tn.current();
+    FusedSchedule sc = res->batch_schedule.current();
     if (fixed)
       sc.eager = true;
-    Profiler &tp = fixed ? idle : res->batch_prof;
-    tp.on = tune;
     r = pf.begin(st, kStageSetup);
-    int q = tp.begin(st, kStageSetup);
-    FusedOps<T>::setup_batch(st, d_setup, blocks, sc.setup_lds);
-    tp.end(st, q);
+    FusedOps<T>::setup_batch(st, d_setup, blocks);
     pf.end(st, r);
     hipLaunchKernelGGL(k_begin_solve_b<T>, dim3(grid_blocks(ns, 64)), dim3(64), 0, st, d_solve,
                        ns);
@@ -1793,7 +1764,7 @@ class SceneImpl final : public SceneBase {
       max_it = std::max(max_it, static_cast<int>(sc->desc.iisph_max_iterations));
     }
     int enq = fold_first ? 1 : 0;  // iterations enqueued (iteration 1 by the setup)
-    const bool graph = !sc.eager && !pf.on && !tune;
+    const bool graph = !sc.eager && !pf.on;
     const std::string key =
         graph ? graph_key(kGraphBatchIteration | sizeof(T), d_solve, blocks, ns, sc)
               : std::string();
@@ -1801,22 +1772,18 @@ class SceneImpl final : public SceneBase {
       if (graph) {
         for (int j = 0; j < n; ++j)
           res->batch_graphs[sizeof(T) == 8 ? 1 : 0].launch(st, key, [&] {
-            FusedOps<T>::accel_batch(st, d_solve, blocks, sc.accel_lds);
-            FusedOps<T>::pressure_batch(st, d_solve, blocks, ns, sc.pressure_lds);
+            FusedOps<T>::accel_batch(st, d_solve, blocks);
+            FusedOps<T>::pressure_batch(st, d_solve, blocks, ns);
           });
         enq += n;
         return;
       }
       for (int j = 0; j < n; ++j) {
         int q1 = pf.begin(st, kStagePressureAccel, enq + j);
-        int q2 = tp.begin(st, kStagePressureAccel, enq + j);
-        FusedOps<T>::accel_batch(st, d_solve, blocks, sc.accel_lds);
-        tp.end(st, q2);
+        FusedOps<T>::accel_batch(st, d_solve, blocks);
         pf.end(st, q1);
         q1 = pf.begin(st, kStagePressure, enq + j);
-        q2 = tp.begin(st, kStagePressure, enq + j);
-        FusedOps<T>::pressure_batch(st, d_solve, blocks, ns, sc.pressure_lds);
-        tp.end(st, q2);
+        FusedOps<T>::pressure_batch(st, d_solve, blocks, ns);
         pf.end(st, q1);
       }
       enq += n;
@@ -1826,7 +1793,7 @@ class SceneImpl final : public SceneBase {
     enqueue(std::max(0, std::min(pred, max_it) - enq));
     // the integration rides behind the iterations in its guarded form (each
     // scene integrates once its own solve is done) unless stages are timed
-    const bool spec = !tune && !pf.on;
+    const bool spec = !pf.on;
     if (spec) {
       FusedOps<T>::integrate_batch(st, d_solve, d_pmap, np, ns, true);
       for (;;) {
@@ -1864,23 +1831,6 @@ class SceneImpl final : public SceneBase {
         break;
     }
     PRTCL_HIP_CHECK(hipGetLastError());
-    if (tune) {
-      // the schedules are compared on the iterations every scene of the
-      // batch runs (below the smallest min_it): later launches skip the
-      // blocks of scenes already done, so their cost depends on the step
-      int all_run = 1 << 30;
-      for (SceneImpl *sc : v)
-        all_run = std::min(all_run, static_cast<int>(sc->desc.iisph_min_iterations));
-      tp.resolve(std::max(fold_first ? 2 : 1, all_run));
-      tn.record(0, tp.ms[kStageSetup], static_cast<double>(tp.launches[kStageSetup]));
-      tn.record(1, tp.ms[kStagePressureAccel],
-                static_cast<double>(tp.launches[kStagePressureAccel]));
-      tn.record(2, tp.ms[kStagePressure], static_cast<double>(tp.launches[kStagePressure]));
-      tp.reset();
-      tp.on = false;
-    }
-    if (!fixed)
-      tn.finish_step();
     r = pf.begin(st, kStageIntegrateX);
     if (!spec)
       FusedOps<T>::integrate_batch(st, d_solve, d_pmap, np, ns);
@@ -2128,8 +2078,8 @@ class SceneImpl final : public SceneBase {
     return need;
   }
 
-  void set_schedule(int mask) override { tuner_.force(mask); }
-  int schedule() const override { return tuner_.current().mask(); }
+  void set_schedule(int mask) override { schedule_.force(mask); }
+  int schedule() const override { return schedule_.current().mask(); }
 
   void step_info(int *it, double *rel, int *wk) override {
     if (it)
@@ -2366,8 +2316,7 @@ class SceneImpl final : public SceneBase {
   bool proc_list_valid_ = false;  // proc_list() holds for the present positions
   double clock_ = 0;
   int steps_since_permute_ = 0;
-  ScheduleTuner tuner_;
-  Profiler tprof_;     // timing of the tuner's trial steps
+  ScheduleChoice schedule_;
   GraphCache graphs_;  // captured IISPH iterations of this scene
   int predicted_iters_ = 2;
   int predicted_cg_ = 4;

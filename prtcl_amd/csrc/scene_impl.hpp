@@ -103,9 +103,8 @@ struct CtxResources {
   void *batch_dev = nullptr;
   size_t batch_bytes = 0;
   hipEvent_t batch_ev = nullptr;
-  // schedule of the batched fused passes (FP32, FP64) and its trial timing
-  ScheduleTuner batch_tuner[2];
-  Profiler batch_prof;
+  // schedule of the batched fused passes
+  ScheduleChoice batch_schedule;
   // captured batched IISPH iterations (FP32, FP64): one cache per type
   GraphCache batch_graphs[2];
   void ensure_batch(size_t bytes);
@@ -138,8 +137,7 @@ class SceneBase {
   virtual void last_permutation(int group, uint32_t *perm) = 0;
   virtual void step_info(int *iisph_iters, double *rel, int *wkbb18_iters) = 0;
   virtual uint64_t grid_bytes_for_domain() const = 0;
-  // fused-pass schedule: mask >= 0 forces it (bit 0 setup, 1 pressure
-  // acceleration, 2 pressure in LDS), -1 returns to the tuner
+  // fused-pass schedule: mask >= 0 forces it, -1 returns to the default
   virtual void set_schedule(int mask) = 0;
   virtual int schedule() const = 0;
   // residency: evict() moves the device state to host memory and frees the

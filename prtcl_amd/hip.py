@@ -310,7 +310,7 @@ class Context:
         return r.value, st.value
 
     def set_batch_schedule(self, mask: int):
-        """Force the LDS/global schedule of batched steps (-1: autotune)."""
+        """Force the launch schedule of batched steps (-1: the default)."""
         self.check(self.L.prtcl_hip_set_schedule(self.h, -1, mask), "set_schedule")
 
     def batch_schedule(self) -> int:
@@ -472,11 +472,11 @@ class HipScene:
         return bool(r.value)
 
     def set_schedule(self, mask: int):
-        """Force the schedule of the fused passes: bit 0 setup, bit 1
-        pressure acceleration, bit 2 pressure in LDS; bit 3 eager IISPH
+        """Force the schedule of the fused passes: bits 0-2 change nothing (they
+        chose LDS-staged passes once); bit 3 eager IISPH
         iterations; bit 4 separate one-block alpha/beta kernels in the CG
         solves; bit 5 separate WKBB18 diagonal and CG set-up passes; bit 6
-        IISPH iteration 1 in its own passes (-1: autotune)."""
+        IISPH iteration 1 in its own passes (-1: the default, bit 3)."""
         self.ctx.check(self.L.prtcl_hip_set_schedule(self.ctx.h, self.id, mask), "set_schedule")
 
     def schedule(self) -> int:
