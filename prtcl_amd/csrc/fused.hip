@@ -18,6 +18,7 @@
 // block's neighbourhood in LDS and gather the neighbours' fields from there.
 // A particle with more neighbours than the list holds is walked over the
 // grid instead.
+#include <limits>
 #include <type_traits>
 
 #include "fused.hpp"
@@ -86,6 +87,17 @@ struct FastSpline {
     f = r2 < eps2 ? T(0) : dw * rinv;
     if (r2 <= T(0))
       w = aw * T(4);  // W(0) = alpha/h^3 (8 - 4)
+  }
+  // the same without the factors: W / aw in w, gradW / ag3 in f
+  __device__ __forceinline__ void unscaled(T r2, T &w, T &f) const {
+    const T rinv = rsqrt_fast<T>(fmax(r2, std::numeric_limits<T>::min()));
+    const T q = r2 * rinv * inv_h;
+    const T t = fmax(T(2) - q, T(0));
+    const T u = fmax(T(2) - T(2) * q, T(0));
+    const T t2 = t * t, u2 = u * u;
+    w = t2 * t - T(0.5) * (u2 * u);
+    const T d = (u2 - t2) * rinv;
+    f = r2 < eps2 ? T(0) : d;
   }
   __device__ __forceinline__ T gradf(T r2) const { return ag3 * gradf_unscaled(r2); }
   __device__ __forceinline__ T gradf_unscaled(T r2) const {
@@ -261,14 +273,21 @@ __device__ __forceinline__ double first_iteration(const SceneView<T> &S, int i,
 // ---------------------------------------------------------------------------
 // setup pass: density + neighbour list + IISPH c, AA (+ s when the velocity
 // of every neighbour is known without another pass, i.e. no explicit
-// viscosity: v*_j = v_j + dt g H_j)
+// viscosity: the sort has stored v*_j = v_j + dt g H_j)
 //
-// Phase 1 tests the 27-cell candidates with the exact predicate and appends
-// the accepted neighbours (entries relative to the slab's span) to this
-// thread's column of an LDS table; phase 2 runs the pair sums over the
-// compacted entries, so the lanes that reject a candidate do not wait for the
-// kernel arithmetic of the ones that accept it. The table is written to the
-// list row by row (coalesced).
+// Phase 1 tests the 27-cell candidates by their 16-bit positions (fixed_sqdist)
+// and appends the accepted ones (entries relative to the slab's span) to this
+// thread's column of an LDS table; phase 2 runs the exact predicate (where the
+// 16 bits leave it open) and the pair sums over the compacted entries, so the
+// lanes that reject a candidate do not wait for the kernel arithmetic of the
+// ones that accept it. The table is written to the list row by row (coalesced).
+//
+// Bound by vector instructions and by the loads' address work, half each (216
+// candidates and 30 pairs a particle). With candidates as 16-byte positions and
+// 13 instructions, 65 a pair and five wavefronts per SIMD, 1M particles took 229
+// us, 250,000 73 us, 16 scenes of 2,000 to 200,000 together 247 us; with 8-byte
+// records and 9 instructions, 45 a pair (the kernel's factors applied to the
+// sums, the velocities integrated by the sort) and six wavefronts 188, 53 and 182.
 // ---------------------------------------------------------------------------
 // the pair sums of the setup pass for one particle (or one lane's share)
 template <class T, bool kWithSource>
@@ -276,9 +295,9 @@ struct SetupSums {
   const SceneView<T> &S;
   const FastSpline<T> K;
   vec4_t<T> xi;
-  T dtg0, dtg1, dtg2, vs0, vs1, vs2;
-  // density, G_f, sum |gradW|^2 and the velocity-divergence sum of the source
-  // term; density and G_b of the boundary
+  T vs0, vs1, vs2;
+  // density / aw, G_f / ag3, sum |gradW|^2 / ag3^2 and the velocity-divergence sum
+  // of the source term / ag3; density and G_b of the boundary
   T rho = 0, gf0 = 0, gf1 = 0, gf2 = 0, s2 = 0, dsum = 0;
   T rhob = 0, gb0 = 0, gb1 = 0, gb2 = 0;
   bool near_boundary = false;
@@ -286,29 +305,39 @@ struct SetupSums {
   __device__ __forceinline__ SetupSums(const SceneView<T> &view, const vec4_t<T> &x,
                                        const vec4_t<T> &vi)
       : S(view), K(fast_spline(view)), xi(x) {
-    const T Hi = fade_step(S, vi.w);
-    dtg0 = S.dt * S.g0, dtg1 = S.dt * S.g1, dtg2 = S.dt * S.g2;
-    vs0 = vi.x + dtg0 * Hi, vs1 = vi.y + dtg1 * Hi, vs2 = vi.z + dtg2 * Hi;
+    vs0 = vi.x, vs1 = vi.y, vs2 = vi.z;
   }
-  // density self term W(0) = 4 alpha / h^3
-  __device__ __forceinline__ T self() const { return xi.w * K.aw * T(4); }
+  // density self term W(0) = 4 alpha / h^3 (aw applied by finish)
+  __device__ __forceinline__ T self() const { return xi.w * T(4); }
   // neighbour (x_j, m_j) = pj with velocity vj (read only with kWithSource)
   __device__ __forceinline__ void pair(const vec4_t<T> &pj, const vec4_t<T> &vj) {
     const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
+    add(pj, vj, d0, d1, d2, d0 * d0 + d1 * d1 + d2 * d2);
+  }
+  // the same for a candidate that fixed_sqdist has accepted: false (and nothing
+  // added) where the exact predicate rejects it. The two forms of the squared
+  // distance differ by a few roundings, far below the 1e-6 that decide here
+  // whether the exact one is looked at; a NaN is.
+  __device__ __forceinline__ bool pair_if(const vec4_t<T> &pj, const vec4_t<T> &vj) {
+    const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
+    const T r2 = d0 * d0 + d1 * d1 + d2 * d2;
+    if (!(r2 < S.thr2 * T(0.999999)) && !(sqdist_exact(d0, d1, d2) < S.thr2))
+      return false;
+    add(pj, vj, d0, d1, d2, r2);
+    return true;
+  }
+  __device__ __forceinline__ void add(const vec4_t<T> &pj, const vec4_t<T> &vj, T d0, T d1, T d2,
+                                      T r2) {
     T w, f;
-    K.eval(d0 * d0 + d1 * d1 + d2 * d2, w, f);
+    K.unscaled(r2, w, f);
     rho += pj.w * w;
-    const T g0 = f * d0, g1 = f * d1, g2 = f * d2;
-    gf0 += pj.w * g0;
-    gf1 += pj.w * g1;
-    gf2 += pj.w * g2;
-    s2 += pj.w * (g0 * g0 + g1 * g1 + g2 * g2);
+    const T mf = pj.w * f;
+    gf0 += mf * d0;
+    gf1 += mf * d1;
+    gf2 += mf * d2;
+    s2 += mf * (f * r2);
     if (kWithSource) {
-      const T Hj = fade_step(S, vj.w);
-      const T u0 = vs0 - (vj.x + dtg0 * Hj);
-      const T u1 = vs1 - (vj.y + dtg1 * Hj);
-      const T u2 = vs2 - (vj.z + dtg2 * Hj);
-      dsum += pj.w * (u0 * g0 + u1 * g1 + u2 * g2);
+      dsum += mf * ((vs0 - vj.x) * d0 + (vs1 - vj.y) * d1 + (vs2 - vj.z) * d2);
     }
   }
   __device__ __forceinline__ vec4_t<T> load_v(uint32_t j) const {
@@ -340,9 +369,12 @@ struct SetupSums {
   }
   // the particle's fields from the complete sums; returns its aprde term of
   // IISPH iteration 1 (S.first_iter)
-  __device__ __forceinline__ double finish(int i, T birth, vec4_t<T> *vout) {
+  __device__ __forceinline__ double finish(int i) {
     const T rho0 = S.rho0;
-    rho += rho0 * rhob;
+    rho = rho * K.aw + rho0 * rhob;
+    gf0 *= K.ag3, gf1 *= K.ag3, gf2 *= K.ag3;
+    s2 *= K.ag3 * K.ag3;
+    dsum *= K.ag3;
     const T irho = T(1) / rho;
     const T irho2 = irho * irho;
     const T k14 = T(1.4) * rho0;
@@ -364,7 +396,6 @@ struct SetupSums {
       const T src = (rho0 - rho) -
                     S.dt * rho0 * irho * (dsum + rho0 * (vs0 * gb0 + vs1 * gb1 + vs2 * gb2));
       S.s[i] = src;
-      vout[i] = make4<vec4_t<T>>(vs0, vs1, vs2, birth);
       if (S.first_iter)
         return first_iteration(S, i, xi, rho, src, AA);
     } else {
@@ -374,16 +405,20 @@ struct SetupSums {
   }
 };
 
+// wavefronts per SIMD of the setup pass (FP32: 80 registers)
+template <class T>
+constexpr int kSetupWaves = sizeof(T) == 4 ? 6 : 1;
+
 struct SetupShared {
-  // rows kNbrCap + 1 .. kNbrCap + 8 take the writes of a lane past its cap
-  uint16_t lst[kNbrCap + 9][kBlock];
+  // rows kNbrCap + 1 .. kNbrCap + 3 take the writes of a lane past its cap (52
+  // rows: six blocks per CU)
+  uint16_t lst[kNbrCap + 4][kBlock];
   BlockRanges sR;
 };
 
 template <class T, bool kWithSource>
 __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrList &L,
-                                             vec4_t<T> *vout, unsigned lb,
-                                             SetupShared &sh) {
+                                             unsigned lb, SetupShared &sh) {
   auto &lst = sh.lst;
   BlockRanges &sR = sh.sR;
   const unsigned t = threadIdx.x;
@@ -399,8 +434,12 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
   const vec4_t<T> zero4 = make4<vec4_t<T>>(T(0), T(0), T(0), T(0));
   const vec4_t<T> xi = valid ? S.xm[i] : zero4;
   const vec4_t<T> vi = valid ? S.v[i] : zero4;
+  const uint2 fi = valid ? S.xf[i] : make_uint2(0u, 0u);
   SetupSums<T, kWithSource> q(S, xi, vi);
   q.rho = q.self();
+  constexpr uint32_t kRow = kBlock * sizeof(uint16_t);
+  const uint32_t at0 = t * sizeof(uint16_t), top = at0 + (kNbrCap + 1u) * kRow;
+  uint32_t at = at0;
   uint32_t cnt = 0;
   uint32_t cs[3] = {0u, 0u, 0u};  // entries per slab
   // candidate test of the slab-s runs; accepted entries are appended
@@ -413,36 +452,50 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
       const uint32_t b = rb[r], e = re[r];
       const bool own = (s == 1) & (r == 1);  // the run holding particle i
       // eight candidates per trip from consecutive slots, loads issued
-      // together. Branch-free append: every candidate is written to row cnt
-      // of this thread's column of the LDS table and cnt advances only for
-      // an accepted one. The table has 8 rows beyond kNbrCap + 1 and cnt is
-      // clamped to kNbrCap + 1 after each trip, so the writes of a trip stay
-      // in the table and a count above kNbrCap still reads as overflow. Full
+      // together. Branch-free append: every candidate is written to the next row
+      // of this thread's column of the LDS table (at byte `at`), which advances
+      // only for an accepted one. The table has 3 rows from kNbrCap + 1 on and the
+      // row is clamped to kNbrCap + 1 at least every three candidates, so the writes
+      // stay in the table and a count above kNbrCap still reads as overflow. Full
       // trips need no bound test; the last, partial trip of a run reads up
-      // to 7 slots past it (the position arrays carry kRunPad slots of
-      // padding) and rejects them. Only the run of the particle's own cell
-      // can hold the particle itself.
+      // to 7 slots past it (the positions carry kRunPad slots of padding) and
+      // rejects them. Only the run of the particle's own cell can hold the
+      // particle itself.
       auto trip = [&](uint32_t j, auto tail_tag) {
         constexpr bool kTail = decltype(tail_tag)::value;
-        const vec4_t<T> *__restrict__ src = S.xm + j;
-        vec4_t<T> pk[8];
+        struct alignas(8) Two {
+          uint32_t xy0, z0, xy1, z1;
+        };
+        Two pk[4];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          pk[u] = src[u];
+        for (int u = 0; u < 4; ++u)
+          pk[u] = *reinterpret_cast<const Two *>(S.xf + j + 2 * u);
         __builtin_amdgcn_sched_barrier(0);
         const uint32_t lim = e - j;                          // u < lim: inside the run
         const uint32_t self = static_cast<uint32_t>(i) - j;  // u == self: the particle
         const uint32_t ent = j - base;                       // entry of candidate 0
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        auto clamp = [&] { at = at < top ? at : top; };
+        auto test = [&](int u, uint32_t xy, uint32_t z) {
           const bool ok = (!kTail | (static_cast<uint32_t>(u) < lim)) &
                           (!own | (static_cast<uint32_t>(u) != self)) &
-                          (sqdist_exact(xi.x - pk[u].x, xi.y - pk[u].y, xi.z - pk[u].z) <
-                           S.thr2);
-          lst[cnt][t] = static_cast<uint16_t>(ent + u);
-          cnt += ok ? 1u : 0u;
+                          (fixed_sqdist(fi.x, fi.y, xy, z) < kFixReach);
+          *reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(lst) + at) =
+              static_cast<uint16_t>(ent + u);
+          at += ok ? kRow : 0u;
+        };
+        test(0, pk[0].xy0, pk[0].z0);
+        test(1, pk[0].xy1, pk[0].z1);
+        test(2, pk[1].xy0, pk[1].z0);
+        clamp();
+        test(3, pk[1].xy1, pk[1].z1);
+        if (!kTail || lim > 4u) {
+          test(4, pk[2].xy0, pk[2].z0);
+          test(5, pk[2].xy1, pk[2].z1);
+          clamp();
+          test(6, pk[3].xy0, pk[3].z0);
+          test(7, pk[3].xy1, pk[3].z1);
         }
-        cnt = cnt < kNbrCap + 1u ? cnt : kNbrCap + 1u;
+        clamp();
       };
       uint32_t j = b;
       for (; j + 8u <= e; j += 8u)
@@ -457,6 +510,7 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
     for (int s = 0; s < 3; ++s) {
       const uint32_t c0 = cnt;
       scan(s);
+      cnt = (at - at0) / kRow;
       cs[s] = cnt - c0;
     }
     if (cnt > kNbrCap) {
@@ -467,24 +521,36 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
       auto slot = [&](uint32_t e) {
         return R.b0 + lst[e][t] + (e >= c0 ? d1 : 0u) + (e >= c01 ? d2 : 0u);
       };
-      // groups of four: every gather of a group ahead of its arithmetic
-      uint32_t e = 0;
-      for (; e + 4 <= cnt; e += 4) {
+      // groups of four: every gather of a group ahead of its arithmetic (the
+      // last group repeats the last entry's gathers)
+      uint64_t out = 0;  // entries that the exact predicate rejects
+      for (uint32_t e = 0; e < cnt; e += 4) {
         vec4_t<T> px[4], pv[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint32_t j = slot(e + k);
+        for (uint32_t k = 0; k < 4; ++k) {
+          const uint32_t j = slot(e + k < cnt ? e + k : cnt - 1u);
           px[k] = S.xm[j];
           pv[k] = q.load_v(j);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-          q.pair(px[k], pv[k]);
+        for (uint32_t k = 0; k < 4; ++k)
+          if (e + k < cnt && !q.pair_if(px[k], pv[k]))
+            out |= 1ull << (e + k);
       }
-      for (; e < cnt; ++e) {
-        const uint32_t j = slot(e);
-        q.pair(S.xm[j], q.load_v(j));
+      if (out != 0) {  // rare: candidates at the radius to within 1 in 4000
+        uint32_t kept = 0, ks[3] = {0u, 0u, 0u};
+        for (uint32_t e = 0; e < cnt; ++e)
+          if (!((out >> e) & 1u)) {
+            lst[kept++][t] = lst[e][t];
+            ks[0] += e < c0 ? 1u : 0u;
+            ks[1] += e >= c0 && e < c01 ? 1u : 0u;
+            ks[2] += e >= c01 ? 1u : 0u;
+          }
+        cnt = kept;
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+          cs[s] = ks[s];
       }
     }
   }
@@ -517,7 +583,7 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
     }
     runs(S.grid, cell, S.bstart, [&](uint32_t b, uint32_t e) { q.boundary(b, e); });
     L.info[i] = info | (q.near_boundary && !over ? kListBoundary : 0u);
-    return q.finish(i, vi.w, vout);
+    return q.finish(i);
   };
   const double term = valid ? finish() : 0.0;
   if (kWithSource && S.first_iter) {
@@ -532,13 +598,12 @@ __device__ __forceinline__ void k_setup_body(const SceneView<T> &S, const NbrLis
 // candidates (scan8), the accepted neighbours and the boundary runs, and their
 // sums are added in a fixed tree. Bound by its chain of dependent loads: run
 // bounds, candidates of three slabs, neighbours. Measured, one lane -> eight:
-// 2,048 particles 42 -> 12.5 us, 8,000: 42 -> 13.1, 59,000: 41 -> 27, 125,000:
-// 50 -> 46, 250,000: 78 -> 82, 1M: 230 -> 294 (the lanes' idle slots cost more
-// than the shorter chain gives).
+// 2,048 particles 42 -> 13 us, 8,000: 42 -> 13, 59,000: 42 -> 31; with positions of
+// 16 bytes 125,000: 50 -> 46, 250,000: 78 -> 82, 1M: 230 -> 294 (the lanes' idle slots
+// cost more than the shorter chain gives).
 template <class T, bool kWithSource>
 __device__ __forceinline__ void k_setup8_body(const SceneView<T> &S, const NbrList &L,
-                                              vec4_t<T> *vout, unsigned lb,
-                                              Scan8Shared &sh) {
+                                              unsigned lb, Scan8Shared &sh) {
   const unsigned sub = threadIdx.x % kScanLanes, p = threadIdx.x / kScanLanes;
   const int i = static_cast<int>(lb * kScanParts + p);
   const bool valid = i < S.nf;
@@ -546,8 +611,9 @@ __device__ __forceinline__ void k_setup8_body(const SceneView<T> &S, const NbrLi
   const vec4_t<T> xi = valid ? S.xm[i] : zero4;
   const vec4_t<T> vi = valid ? S.v[i] : zero4;
   const uint32_t cell = valid ? S.fcell[i] : 0u;
-  const Scan8 c = scan8<T, false>(S, L, lb, sh, i, valid, cell, xi);
+  Scan8 c = scan8<T, false>(S, L, lb, sh, i, valid, cell, xi);
   SetupSums<T, kWithSource> q(S, xi, vi);
+  uint32_t rejected = 0;
   if (valid && !c.over) {
     const Spans R = Spans::of(sh.R);
     const uint32_t c0 = c.cs0, c01 = c.cs0 + c.cs1;
@@ -555,8 +621,8 @@ __device__ __forceinline__ void k_setup8_body(const SceneView<T> &S, const NbrLi
     for (uint32_t e0 = sub; e0 < c.cnt; e0 += 4u * kScanLanes) {
       vec4_t<T> px[4], pv[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t e = e0 + static_cast<uint32_t>(k) * kScanLanes;
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t e = e0 + k * kScanLanes;
         if (e < c.cnt) {
           const uint32_t j =
               R.b0 + sh.lst[p][e] + (e >= c0 ? d1 : 0u) + (e >= c01 ? d2 : 0u);
@@ -566,13 +632,16 @@ __device__ __forceinline__ void k_setup8_body(const SceneView<T> &S, const NbrLi
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (e0 + static_cast<uint32_t>(k) * kScanLanes < c.cnt)
-          q.pair(px[k], pv[k]);
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t e = e0 + k * kScanLanes;
+        if (e < c.cnt && !q.pair_if(px[k], pv[k]))
+          rejected |= 1u << (e / kScanLanes);
+      }
     }
   } else if (valid && sub == 0) {
     grid_walk(S, i, xi, [&](uint32_t j) { q.pair(S.xm[j], q.load_v(j)); });
   }
+  scan8_drop(sh, c, rejected);
   if (valid && S.nb > 0) {
     uint32_t b, e;
     run_bounds(S.grid, cell, S.bstart, static_cast<int>(sub), &b, &e);
@@ -592,7 +661,7 @@ __device__ __forceinline__ void k_setup8_body(const SceneView<T> &S, const NbrLi
     scan8_write(L, sh, static_cast<size_t>(S.nf), i, c, (near & 0xFFu) != 0u);
     if (sub == 0) {
       q.rho += q.self();
-      term = q.finish(i, vi.w, vout);
+      term = q.finish(i);
     }
   }
   if (kWithSource && S.first_iter) {
@@ -603,20 +672,18 @@ __device__ __forceinline__ void k_setup8_body(const SceneView<T> &S, const NbrLi
 }
 
 template <class T, bool kWithSource>
-__global__ __launch_bounds__(kBlock) void k_setup8(SceneView<T> S, NbrList L, vec4_t<T> *vout,
-                                                   SolveBegin B) {
+__global__ __launch_bounds__(kBlock) void k_setup8(SceneView<T> S, NbrList L, SolveBegin B) {
   __shared__ Scan8Shared sh;
-  k_setup8_body<T, kWithSource>(S, L, vout, xcd_block(blockIdx.x, gridDim.x), sh);
+  k_setup8_body<T, kWithSource>(S, L, xcd_block(blockIdx.x, gridDim.x), sh);
   // no thread of the setup reads the control block
   if (B.seq != 0u && blockIdx.x == 0 && threadIdx.x == 0)
     begin_solve(S.ctl, B);
 }
 
 template <class T, bool kWithSource>
-__global__ __launch_bounds__(kBlock) void k_setup(SceneView<T> S, NbrList L,
-                                                  vec4_t<T> *vout, SolveBegin B) {
+__global__ __launch_bounds__(kBlock, kSetupWaves<T>) void k_setup(SceneView<T> S, NbrList L, SolveBegin B) {
   __shared__ SetupShared sh;
-  k_setup_body<T, kWithSource>(S, L, vout, xcd_block(blockIdx.x, gridDim.x), sh);
+  k_setup_body<T, kWithSource>(S, L, xcd_block(blockIdx.x, gridDim.x), sh);
   // no thread of the setup reads the control block
   if (B.seq != 0u && blockIdx.x == 0 && threadIdx.x == 0)
     begin_solve(S.ctl, B);
@@ -1053,13 +1120,13 @@ constexpr unsigned kSetupParts = kBlock / kScanParts;  // setup blocks per block
 constexpr unsigned kListParts = kListLanes;
 
 template <class T, bool kWithSource>
-__global__ __launch_bounds__(kBlock) void k_setup_b(const BatchEntry<T> *tab, BatchBlocks B) {
+__global__ __launch_bounds__(kBlock, kSetupWaves<T>) void k_setup_b(const BatchEntry<T> *tab, BatchBlocks B) {
   __shared__ SetupPool sh;
   BATCH_PASS_ENTRY(kSetupParts, setup_blocks);
   if (split)
-    k_setup8_body<T, kWithSource>(E.S, L, E.vtmp, lb, sh.scan);
+    k_setup8_body<T, kWithSource>(E.S, L, lb, sh.scan);
   else
-    k_setup_body<T, kWithSource>(E.S, L, E.vtmp, lb, sh.setup);
+    k_setup_body<T, kWithSource>(E.S, L, lb, sh.setup);
 }
 
 // scenes with explicit viscosity or axial gravity: after the setup without the
@@ -1161,20 +1228,20 @@ void FusedOps<T>::setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
     return;
   const dim3 gr(setup_blocks(S.nf)), bl(kBlock);
   const bool split = split_scene(S.nf);
-  // the one-pass setup folds a uniform g into every neighbour's velocity;
-  // explicit viscosity or a position-dependent (axial) gravity need the
-  // integrated velocities first
+  // the one-pass setup reads velocities that the sort has integrated with a
+  // uniform g (GravityKick); explicit viscosity or a position-dependent (axial)
+  // gravity integrate them after the list is built
   if (!explicit_viscosity && !S.axial) {
     if (split)
-      hipLaunchKernelGGL((k_setup8<T, true>), gr, bl, 0, st, S, L, vtmp, B);
+      hipLaunchKernelGGL((k_setup8<T, true>), gr, bl, 0, st, S, L, B);
     else
-      hipLaunchKernelGGL((k_setup<T, true>), gr, bl, 0, st, S, L, vtmp, B);
+      hipLaunchKernelGGL((k_setup<T, true>), gr, bl, 0, st, S, L, B);
     return;
   }
   if (split)
-    hipLaunchKernelGGL((k_setup8<T, false>), gr, bl, 0, st, S, L, vtmp, B);
+    hipLaunchKernelGGL((k_setup8<T, false>), gr, bl, 0, st, S, L, B);
   else
-    hipLaunchKernelGGL((k_setup<T, false>), gr, bl, 0, st, S, L, vtmp, B);
+    hipLaunchKernelGGL((k_setup<T, false>), gr, bl, 0, st, S, L, B);
   const dim3 gl(list_blocks(S.nf));
   if (!explicit_viscosity)
     hipLaunchKernelGGL(k_gravity_v<T>, dim3(grid_blocks(S.nf)), bl, 0, st, S, vtmp);

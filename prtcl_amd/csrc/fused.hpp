@@ -51,7 +51,8 @@ struct FusedOps {
   // the neighbour list alone, for the procedures: every particle includes
   // itself, at its place in slot order
   static void build_list(hipStream_t st, const SceneView<T> &S, const NbrList &L);
-  // density, neighbour list, IISPH c / AA / s, integrated velocity into vtmp
+  // density, neighbour list, IISPH c / AA / s; with explicit viscosity or axial
+  // gravity also the integrated velocity, into vtmp (otherwise S.v holds it)
   // B.seq != 0: the first kernel also begins solve B (one launch fewer)
   static void setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
                     bool explicit_viscosity, vec4_t<T> *vtmp,

@@ -280,9 +280,10 @@ __global__ __launch_bounds__(kBlock) void k_stable_rank(GridDims g, const uint32
 
 // k_stable_rank and the reorder of the carried state in one pass: the thread
 // of unstable slot s finds the stable slot p of its particle o = perm[s] as
-// k_stable_rank does and moves x, v, id and cell of o to p (the same
+// k_stable_rank does, moves x, v, id and cell of o to p and writes p's 16-bit
+// position, the velocity with the step's kick (the same
 // permutation as gathering through k_stable_rank's result, without writing it)
-template <class V>
+template <class T, class V = vec4_t<T>>
 __device__ __forceinline__ void k_place_state_body(GridDims g, const uint32_t *__restrict__ cell,
                                                    const uint32_t *__restrict__ start,
                                                    const uint32_t *__restrict__ perm, int n,
@@ -290,7 +291,9 @@ __device__ __forceinline__ void k_place_state_body(GridDims g, const uint32_t *_
                                                    V *__restrict__ vd, const V *__restrict__ vs,
                                                    uint32_t *__restrict__ id_d,
                                                    const uint32_t *__restrict__ id_s,
-                                                   uint32_t *__restrict__ c_d, unsigned bid) {
+                                                   uint32_t *__restrict__ c_d,
+                                                   uint2 *__restrict__ xf_d,
+                                                   const GravityKick<T> &kick, unsigned bid) {
   const int s = bid * kBlock + threadIdx.x;
   if (s >= n)
     return;
@@ -304,20 +307,24 @@ __device__ __forceinline__ void k_place_state_body(GridDims g, const uint32_t *_
   for (uint32_t k = b; k < e; ++k)
     r += perm[k] < o ? 1u : 0u;
   const uint32_t p = b + r;
-  xd[p] = xs[o];
-  vd[p] = vs[o];
+  const V x = xs[o];
+  xd[p] = x;
+  xf_d[p] = fixed_record(kFixUnits / g.radius, static_cast<double>(x.x),
+                         static_cast<double>(x.y), static_cast<double>(x.z));
+  vd[p] = kick(vs[o]);
   id_d[p] = id_s[o];
   c_d[p] = c;
 }
 
-template <class V>
+template <class T, class V = vec4_t<T>>
 __global__ __launch_bounds__(kBlock) void k_place_state(GridDims g, const uint32_t *cell,
                                                         const uint32_t *start,
                                                         const uint32_t *perm, int n, V *xd,
                                                         const V *xs, V *vd, const V *vs,
                                                         uint32_t *id_d, const uint32_t *id_s,
-                                                        uint32_t *c_d) {
-  k_place_state_body<V>(g, cell, start, perm, n, xd, xs, vd, vs, id_d, id_s, c_d, blockIdx.x);
+                                                        uint32_t *c_d, uint2 *xf_d, GravityKick<T> kick) {
+  k_place_state_body<T>(g, cell, start, perm, n, xd, xs, vd, vs, id_d, id_s, c_d, xf_d, kick,
+                        blockIdx.x);
 }
 
 template <int W>
@@ -431,10 +438,10 @@ __global__ __launch_bounds__(kBlock) void k_place_state_b(const BatchEntry<T> *t
                                                           const uint32_t *pmap) {
   const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
   const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  k_place_state_body<vec4_t<T>>(E.S.grid, E.S.fcell, E.start, E.perm, E.S.nf, E.x_dst, E.S.xm,
+  k_place_state_body<T>(E.S.grid, E.S.fcell, E.start, E.perm, E.S.nf, E.x_dst, E.S.xm,
                                 E.v_dst, E.S.v, E.id_dst,
                                 reinterpret_cast<const uint32_t *>(E.S.id), E.cell_dst,
-                                u & kBatchLocalMask);
+                                E.S.xf, E.S.kick(!E.split_setup), u & kBatchLocalMask);
 }
 
 template <class T>
@@ -485,7 +492,8 @@ template <class T>
 void GridOps<T>::sort_state(hipStream_t st, const GridDims &g, const vec4_t<T> *x, int n,
                             uint32_t *cell, uint32_t *count, uint32_t *start, uint32_t *rank,
                             uint32_t *perm, uint32_t *scan_tmp, vec4_t<T> *xd, vec4_t<T> *vd,
-                            const vec4_t<T> *vs, uint32_t *id_d, const uint32_t *id_s) {
+                            const vec4_t<T> *vs, uint32_t *id_d, const uint32_t *id_s,
+                            uint2 *xf_d, const GravityKick<T> &kick) {
   if (n > 0)
     hipLaunchKernelGGL(k_cell_keys<T>, dim3(grid_blocks(n)), dim3(kBlock), 0, st, g, x, n,
                        cell, count, rank);
@@ -494,8 +502,8 @@ void GridOps<T>::sort_state(hipStream_t st, const GridDims &g, const vec4_t<T> *
     hipLaunchKernelGGL(k_scatter, dim3(grid_blocks(n)), dim3(kBlock), 0, st, g, cell, rank,
                        start, n, perm);
     // the atomic ranks are consumed: the cells go to `rank`
-    hipLaunchKernelGGL(k_place_state<vec4_t<T>>, dim3(grid_blocks(n)), dim3(kBlock), 0, st, g,
-                       cell, start, perm, n, xd, x, vd, vs, id_d, id_s, rank);
+    hipLaunchKernelGGL(k_place_state<T>, dim3(grid_blocks(n)), dim3(kBlock), 0, st, g,
+                       cell, start, perm, n, xd, x, vd, vs, id_d, id_s, rank, xf_d, kick);
   }
 }
 

@@ -6,6 +6,8 @@
 // that a single lane per particle builds.
 #pragma once
 
+#include <type_traits>
+
 #include "nbrlist.hpp"
 
 namespace prtcl_amd {
@@ -48,9 +50,18 @@ __device__ __forceinline__ void run_bounds(const GridDims &g, uint32_t cellc,
   *e = ok ? hi : 0u;
 }
 
-// The neighbours of particle i = 32 lb + threadIdx.x / 8 (every thread of the
-// block calls it; valid: i < nf) with the exact predicate, the particle itself
-// included where kSelf. Writes the block's span table.
+// makes the rows written by other lanes of the wavefront readable
+__device__ __forceinline__ void scan8_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Candidates of particle i = 32 lb + threadIdx.x / 8 (every thread of the block
+// calls it; valid: i < nf). kSelf: by the exact predicate, the particle itself
+// included; otherwise by their 16-bit positions, without the particle: the caller
+// applies the exact predicate and drops what it rejects (scan8_drop). Writes the
+// block's span table.
 template <class T, bool kSelf>
 __device__ __forceinline__ Scan8 scan8(const SceneView<T> &S, const NbrList &L, unsigned lb,
                                        Scan8Shared &sh, int i, bool valid, uint32_t cell,
@@ -96,20 +107,34 @@ __device__ __forceinline__ Scan8 scan8(const SceneView<T> &S, const NbrList &L, 
     return out;
   uint32_t cnt = 0;
   const unsigned group = lane & ~7u;
-  // candidate j (ok: it is one) against the predicate, appended in lane order
-  auto test = [&](uint32_t base, uint32_t j, bool ok, const vec4_t<T> &pj) {
-    ok = ok && (kSelf || j != static_cast<uint32_t>(i)) &&
-         sqdist_exact(xi.x - pj.x, xi.y - pj.y, xi.z - pj.z) < S.thr2;
+  // candidate j, appended in lane order where it is accepted
+  auto append = [&](uint32_t base, uint32_t j, bool ok) {
     const uint32_t m = static_cast<uint32_t>(__ballot(ok) >> group) & 0xFFu;
     const uint32_t at = cnt + static_cast<uint32_t>(__popc(m & ((1u << sub) - 1u)));
     if (ok && at < kScanRow)
       sh.lst[p][at] = static_cast<uint16_t>(j - base);
     cnt += static_cast<uint32_t>(__popc(m));
   };
+  // the positions that candidates are tested by
+  using Pos = std::conditional_t<kSelf, vec4_t<T>, uint2>;
+  const uint2 fi = !kSelf && valid ? S.xf[i] : make_uint2(0u, 0u);
+  auto load = [&](uint32_t j) {
+    if constexpr (kSelf)
+      return S.xm[j];
+    else
+      return S.xf[j];
+  };
+  auto near = [&](uint32_t j, const Pos &pj) {
+    if constexpr (kSelf)
+      return sqdist_exact(xi.x - pj.x, xi.y - pj.y, xi.z - pj.z) < S.thr2;
+    else
+      return (j != static_cast<uint32_t>(i)) &
+             (fixed_sqdist(fi.x, fi.y, pj.x, pj.y) < kFixReach);
+  };
   // The three runs of a slab as one sequence of candidates: lane l takes the
   // candidates l, l + 8, ... of it, kIn loads in flight (a lane past the end
   // reads slot 0). A fluid at rest has about 72 candidates a slab.
-  constexpr uint32_t kIn = sizeof(T) == 4 ? 10u : 5u;
+  constexpr uint32_t kIn = sizeof(Pos) <= 16 ? 10u : 5u;
   uint32_t c_end[3];
 #pragma unroll
   for (int s = 0; s < 3; ++s) {
@@ -120,20 +145,20 @@ __device__ __forceinline__ Scan8 scan8(const SceneView<T> &S, const NbrList &L, 
     const uint32_t tot = n01 + (sh.re[p][3 * s + 2] - b2);
     const uint32_t o1 = b1 - n0, o2 = b2 - n01;
     for (uint32_t q0 = sub; __ballot(q0 < tot) != 0ull; q0 += kIn * kScanLanes) {
-      vec4_t<T> pk[kIn];
+      Pos pk[kIn];
       uint32_t jk[kIn];
 #pragma unroll
       for (uint32_t u = 0; u < kIn; ++u) {
         const uint32_t q = q0 + u * kScanLanes;
         jk[u] = q < tot ? q + (q < n0 ? b0 : (q < n01 ? o1 : o2)) : 0u;
-        pk[u] = S.xm[jk[u]];
+        pk[u] = load(jk[u]);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (uint32_t u = 0; u < kIn; ++u) {
         const bool in = q0 + u * kScanLanes < tot;
         if (__ballot(in) != 0ull)
-          test(base, jk[u], in, pk[u]);
+          append(base, jk[u], in & near(jk[u], pk[u]));
       }
     }
     c_end[s] = cnt;
@@ -143,11 +168,39 @@ __device__ __forceinline__ Scan8 scan8(const SceneView<T> &S, const NbrList &L, 
   out.cs1 = c_end[1] - c_end[0];
   out.cs2 = c_end[2] - c_end[1];
   out.over = cnt > kNbrCap;
-  // the rows are read by other lanes of their wavefront
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  scan8_sync();
   return out;
+}
+
+// Drops entries of the rows: bit m of a lane's `rejected` is entry 8 m + lane of its
+// particle (every lane of the wavefront calls it; rarely is there any).
+__device__ __forceinline__ void scan8_drop(Scan8Shared &sh, Scan8 &c, uint32_t rejected) {
+  if (__ballot(rejected != 0u) == 0ull)
+    return;
+  const unsigned sub = threadIdx.x % kScanLanes, p = threadIdx.x / kScanLanes;
+  const unsigned group = (threadIdx.x % kWave) & ~7u;
+  uint64_t out = 0;
+#pragma unroll
+  for (int m = 0; m < static_cast<int>(kScanRow / kScanLanes); ++m)
+    out |= ((__ballot((rejected >> m) & 1u) >> group) & 0xFFull) << (8 * m);
+  uint32_t kept = 0, ks0 = 0, ks1 = 0;
+  if (sub == 0 && out != 0)
+    for (uint32_t e = 0; e < c.cnt; ++e)
+      if (!((out >> e) & 1u)) {
+        sh.lst[p][kept++] = sh.lst[p][e];
+        ks0 += e < c.cs0 ? 1u : 0u;
+        ks1 += e >= c.cs0 && e < c.cs0 + c.cs1 ? 1u : 0u;
+      }
+  scan8_sync();
+  kept = __shfl(kept, static_cast<int>(group), kWave);
+  ks0 = __shfl(ks0, static_cast<int>(group), kWave);
+  ks1 = __shfl(ks1, static_cast<int>(group), kWave);
+  if (out != 0) {
+    c.cnt = kept;
+    c.cs0 = ks0;
+    c.cs1 = ks1;
+    c.cs2 = kept - ks0 - ks1;
+  }
 }
 
 // the list of particle i to memory: lane l writes chunk l

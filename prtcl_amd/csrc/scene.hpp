@@ -154,6 +154,49 @@ struct GridDims {
   double radius;      // cell edge = neighbourhood radius
 };
 
+// ---- positions in 16 bits for the candidate test of the neighbour search
+//
+// A component is floor(x * kFixUnits / radius), x and y modulo 2^16. The difference
+// of two components, modulo 2^16, is within one unit of the exact difference where
+// that is below 4 radii, so two particles within the radius are at less than
+// kFixUnits + sqrt(3) units: candidates at kFixUnits + 2 units or more are no
+// neighbours, and the exact predicate decides about the others that are close to
+// the radius (or beyond it: farther candidates can alias; they are accepted here at
+// most, never rejected).
+constexpr int kFixUnits = 8192;
+constexpr uint32_t kFixReach = (kFixUnits + 2) * (kFixUnits + 2);
+__device__ __forceinline__ uint2 fixed_record(double scale, double x, double y, double z) {
+  const uint32_t qx = static_cast<uint32_t>(static_cast<int>(floor(x * scale)));
+  const uint32_t qy = static_cast<uint32_t>(static_cast<int>(floor(y * scale)));
+  const uint32_t qz = static_cast<uint32_t>(static_cast<int>(floor(z * scale)));
+  return make_uint2((qx & 0xFFFFu) | (qy << 16), qz);
+}
+// squared distance in units of two records, modulo 2^32 (z to 24 bits)
+using fix2_t = short __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t fixed_sqdist(uint32_t axy, uint32_t az, uint32_t bxy,
+                                                 uint32_t bz) {
+  const fix2_t d = __builtin_bit_cast(fix2_t, axy) - __builtin_bit_cast(fix2_t, bxy);
+  const int e = static_cast<int>(az - bz);
+  return static_cast<uint32_t>(__builtin_amdgcn_sdot2(d, d, __mul24(e, e), false));
+}
+
+// v + dt g H(t - t_birth - fade) for the sort of a step whose setup pass needs the
+// velocities after a uniform gravity (kicked once, here, instead of for every
+// pair); on = 0: v as it is
+template <class T>
+struct GravityKick {
+  T d0 = 0, d1 = 0, d2 = 0, t = 0, fade = 0;
+  int on = 0;
+  __device__ __forceinline__ vec4_t<T> operator()(vec4_t<T> v) const {
+    if (on != 0 && T(0) < (t - v.w) - fade) {
+      v.x += d0;
+      v.y += d1;
+      v.z += d2;
+    }
+    return v;
+  }
+};
+
 template <class T>
 struct SceneView {
   using V4 = vec4_t<T>;
@@ -180,11 +223,21 @@ struct SceneView {
   // whole 64-byte segments per pass): the pressure pass gains more from the
   // adjacent pair than the acceleration pass loses on half-segment writes.
   V4 *xa;
+  __host__ __device__ GravityKick<T> kick(bool on) const {
+#pragma clang fp contract(off)  // dt g is rounded before it is added
+    GravityKick<T> k;
+    k.d0 = dt * g0, k.d1 = dt * g1, k.d2 = dt * g2;
+    k.t = t, k.fade = fade, k.on = on ? 1 : 0;
+    return k;
+  }
   static constexpr size_t kXaGroup = 1;
   __host__ __device__ static size_t xa_x(size_t j) {
     return (j / kXaGroup) * (2 * kXaGroup) + j % kXaGroup;
   }
   __host__ __device__ static size_t xa_a(size_t j) { return xa_x(j) + kXaGroup; }
+  // positions in units of radius / kFixUnits modulo 2^16 (fixed_record), written
+  // by the sort of a fused step and read by its neighbour search
+  uint2 *xf;
   T *rho, *p, *pr, *s, *AA, *Ap, *sp;
   T *gc;  // gradient correction L (3x3 column-major per fluid particle)
   // pt16 (scenes with implicit viscosity 3; empty otherwise): vorticity, the
@@ -341,7 +394,8 @@ struct GridOps {
   static void sort_state(hipStream_t st, const GridDims &g, const vec4_t<T> *x, int n,
                          uint32_t *cell, uint32_t *count, uint32_t *start, uint32_t *rank,
                          uint32_t *perm, uint32_t *scan_tmp, vec4_t<T> *xd, vec4_t<T> *vd,
-                         const vec4_t<T> *vs, uint32_t *id_d, const uint32_t *id_s);
+                         const vec4_t<T> *vs, uint32_t *id_d, const uint32_t *id_s, uint2 *xf_d,
+                         const GravityKick<T> &kick);
   static void gather4(hipStream_t st, void *dst, const void *src, const uint32_t *perm, int n);
   static void gather_elems(hipStream_t st, void *dst, const void *src,
                            const uint32_t *perm, int n, int elem_bytes);

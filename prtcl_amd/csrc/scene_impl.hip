@@ -715,7 +715,9 @@ class SceneImpl final : public SceneBase {
       GridOps<T>::sort_state(st, gd_, P_.xm, nf_, P_.fcell, G_.count, G_.fstart, P_.frank,
                              P_.fperm, G_.scan_tmp, P_.xq, P_.tmpV4, P_.v,
                              reinterpret_cast<uint32_t *>(P_.tmpI),
-                             reinterpret_cast<const uint32_t *>(P_.id));
+                             reinterpret_cast<const uint32_t *>(P_.id),
+                             reinterpret_cast<uint2 *>(P_.tmpSp),
+                             view().kick(desc.step_mode == 0 && !split_setup()));
       if (nf_ > 0) {
         std::swap(P_.xm, P_.xq);
         std::swap(P_.v, P_.tmpV4);
@@ -853,6 +855,7 @@ class SceneImpl final : public SceneBase {
     S.vd = P_.vd;
     S.xq = P_.xq;
     S.xa = P_.xa;
+    S.xf = reinterpret_cast<uint2 *>(P_.tmpSp);
     S.rho = P_.rho;
     S.p = P_.p;
     S.pr = P_.pr;
@@ -1338,7 +1341,8 @@ class SceneImpl final : public SceneBase {
       SolveBegin sb;
       if (fused) {
         // one neighbour pass for density + list + IISPH setup (three with
-        // explicit viscosity); the integrated velocity lands in tmpV4
+        // explicit viscosity or axial gravity, whose integrated velocity lands in
+        // tmpV4; otherwise the sort has integrated it)
         r = pf.begin(st, kStageSetup);
         SceneView<T> Sv = view();
         Sv.first_iter = first_iter ? 1 : 0;
@@ -1355,7 +1359,8 @@ class SceneImpl final : public SceneBase {
         FusedOps<T>::setup(st, Sv, nbr_list(), desc.explicit_viscosity != 0, P_.tmpV4,
                            sb);
         pf.end(st, r);
-        std::swap(P_.v, P_.tmpV4);
+        if (split_setup())
+          std::swap(P_.v, P_.tmpV4);
       } else {
         const SceneView<T> S = view();
         r = pf.begin(st, kStageDensity);
@@ -1647,6 +1652,7 @@ class SceneImpl final : public SceneBase {
       E.cell_dst = s.P_.frank;  // the atomic ranks are consumed by then
       E.nblocks = grid_blocks(s.nf_);
       E.ntiles = scan_tiles(s.gd_.ncells);
+      E.split_setup = s.split_setup() ? 1 : 0;
       t_sort[k] = E;
       std::swap(s.P_.xm, s.P_.xq);
       std::swap(s.P_.v, s.P_.tmpV4);
@@ -1663,10 +1669,10 @@ class SceneImpl final : public SceneBase {
       E.S = s.view();
       E.S.first_iter = fold_first ? 1 : 0;
       E.vtmp = s.P_.tmpV4;
-      E.split_setup = s.split_setup() ? 1 : 0;
       E.explicit_visc = s.desc.explicit_viscosity ? 1 : 0;
       t_setup[k] = E;
-      std::swap(s.P_.v, s.P_.tmpV4);
+      if (s.split_setup())
+        std::swap(s.P_.v, s.P_.tmpV4);
       E.S = s.view();
       E.vtmp = nullptr;
       seqs[k] = ++s.seq_;
@@ -2171,7 +2177,8 @@ class SceneImpl final : public SceneBase {
     for (T **q : {&P.rho, &P.p, &P.pr, &P.s, &P.AA, &P.Ap, &P.tmpT})
       A.take(*q, f);
     A.take(P.sp, 9 * f);
-    A.take(P.tmpSp, 9 * f);
+    // also the 16-bit positions of a fused step, with the run padding
+    A.take(P.tmpSp, std::max(9 * f, (f + kRunPad) * sizeof(uint2) / sizeof(T)));
     A.take(P.gc, 9 * f);
     A.take(P.id, f);
     A.take(P.tmpI, f);

@@ -156,6 +156,16 @@ void launch(const char *name, void (*k)(P...), dim3 g, dim3 b, size_t, hipStream
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
 // used on values that are uniform over the wavefront
 #define __builtin_amdgcn_readfirstlane(x) (x)
+using emu_short2 = short __attribute__((ext_vector_type(2)));
+inline int emu_sdot2(emu_short2 a, emu_short2 b, int c) {
+  return static_cast<int>(static_cast<unsigned>(c) + static_cast<unsigned>(a.x * b.x) +
+                          static_cast<unsigned>(a.y * b.y));
+}
+#define __builtin_amdgcn_sdot2(a, b, c, clamp) emu_sdot2(a, b, c)
+inline int __mul24(int a, int b) {
+  auto low = [](int v) { return static_cast<long long>(static_cast<int>(static_cast<unsigned>(v) << 8) >> 8); };
+  return static_cast<int>(static_cast<unsigned>(low(a) * low(b)));
+}
 #define __builtin_amdgcn_rsqf(x) (1.0f / std::sqrt(static_cast<float>(x)))
 #define __builtin_amdgcn_rcpf(x) (1.0f / static_cast<float>(x))
 
