@@ -84,6 +84,8 @@ __device__ __forceinline__ bool integrate_now(const Ctl *c, unsigned seq) {
 // host_mirror words: [0] IISPH progress, [1] its aprde / nprde, [2] CG
 // progress, [3] end-of-step report, [4] see kMirrorCg3
 constexpr int kMirrorStep = 3;
+constexpr int kMirrorBox = 8;      // six doubles: the bounding box of a position upload
+constexpr int kMirrorWords = 16;
 constexpr int kMirrorCg3 = 4;  // iterations of the third component of a pt16 solve
 
 // Counts the finished step (one thread; after the integration kernel of the

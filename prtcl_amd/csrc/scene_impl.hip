@@ -192,6 +192,71 @@ __global__ __launch_bounds__(kBlock) void k_upload(T *dst, int stride, int off,
     dst[static_cast<long>(s) * stride + off + k] = src[h * ncomp + k];
 }
 
+// Bounding box of the finite coordinates of n uploaded positions (src: 3 n values):
+// each block's box at box[6 b .. 6 b + 5] (lo, hi), then one block folds them
+// into out. Bound by the read (3 us for 1M particles); the loop over the host's
+// copy that small uploads take costs 0.3 ns a coordinate: 0.9 ms for 1M particles,
+// 7 us for kHostBoxMax, about what the two launches cost.
+constexpr int kHostBoxMax = 8192;
+constexpr unsigned kBoxBlocks = 256;
+
+template <class T>
+__device__ __forceinline__ void box_reduce(T (&lo)[3], T (&hi)[3]) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    hi[k] = block_max<kBlock>(hi[k]);
+    lo[k] = -block_max<kBlock>(-lo[k]);
+  }
+}
+
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_box(T *box, const T *src, int n) {
+  T lo[3], hi[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    lo[k] = std::numeric_limits<T>::infinity();
+    hi[k] = -std::numeric_limits<T>::infinity();
+  }
+  for (int i = static_cast<int>(blockIdx.x * kBlock + threadIdx.x); i < n;
+       i += static_cast<int>(gridDim.x * kBlock)) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const T x = src[3 * static_cast<size_t>(i) + k];
+      if (isfinite(x)) {
+        lo[k] = x < lo[k] ? x : lo[k];
+        hi[k] = x > hi[k] ? x : hi[k];
+      }
+    }
+  }
+  box_reduce(lo, hi);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      box[6 * blockIdx.x + k] = lo[k];
+      box[6 * blockIdx.x + 3 + k] = hi[k];
+    }
+}
+
+// out: page-locked host memory
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_box_fold(double *out, const T *box, unsigned nblocks) {
+  static_assert(kBoxBlocks <= kBlock, "a box per thread");
+  T lo[3], hi[3];
+  const unsigned b = threadIdx.x < nblocks ? threadIdx.x : 0u;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    lo[k] = box[6 * b + k];
+    hi[k] = box[6 * b + 3 + k];
+  }
+  box_reduce(lo, hi);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      out[k] = static_cast<double>(lo[k]);
+      out[3 + k] = static_cast<double>(hi[k]);
+    }
+}
+
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_download(T *dst, int ncomp, const T *src,
                                                      int stride, int off, const int32_t *id,
@@ -412,21 +477,41 @@ class SceneImpl final : public SceneBase {
     const int32_t *ids = group == PRTCL_HIP_FLUID ? P_.id : P_.bid;
     hipLaunchKernelGGL(k_upload<T>, dim3(grid_blocks(n)), dim3(kBlock), 0, st, L.base, L.stride,
                        L.off, static_cast<const T *>(stg), L.ncomp, ids, n);
+    const bool device_box = field == PRTCL_HIP_F_POSITION && n > kHostBoxMax;
+    if (device_box) {
+      // the blocks' boxes go to a scratch vector of the group, in stream order
+      T *box = reinterpret_cast<T *>(group == PRTCL_HIP_FLUID ? P_.tmpV4 : P_.btmpV4);
+      const unsigned nb = std::min(grid_blocks(n), kBoxBlocks);
+      static_assert(6 * kBoxBlocks <= 4 * kHostBoxMax, "the boxes fit the scratch vector");
+      hipLaunchKernelGGL(k_box<T>, dim3(nb), dim3(kBlock), 0, st, box,
+                         static_cast<const T *>(stg), n);
+      hipLaunchKernelGGL(k_box_fold<T>, dim3(1), dim3(kBlock), 0, st,
+                         reinterpret_cast<double *>(mirror_dev_ + kMirrorBox), box, nb);
+    }
     PRTCL_HIP_CHECK(hipGetLastError());
     PRTCL_HIP_CHECK(hipStreamSynchronize(st));
     if (field == PRTCL_HIP_F_POSITION) {
       proc_list_valid_ = false;
-      // host-side bounding box for the grid domain
-      const T *hp = static_cast<const T *>(host);
+      // bounding box for the grid domain
       double lo[3] = {HUGE_VAL, HUGE_VAL, HUGE_VAL}, hi[3] = {-HUGE_VAL, -HUGE_VAL, -HUGE_VAL};
-      for (int i = 0; i < n; ++i)
+      if (device_box) {
+        const double *m =
+            const_cast<const double *>(reinterpret_cast<volatile double *>(mirror_host_ + kMirrorBox));
         for (int k = 0; k < 3; ++k) {
-          double x = static_cast<double>(hp[3 * i + k]);
-          if (std::isfinite(x)) {
-            lo[k] = std::min(lo[k], x);
-            hi[k] = std::max(hi[k], x);
-          }
+          lo[k] = m[k];
+          hi[k] = m[3 + k];
         }
+      } else {
+        const T *hp = static_cast<const T *>(host);
+        for (int i = 0; i < n; ++i)
+          for (int k = 0; k < 3; ++k) {
+            double x = static_cast<double>(hp[3 * i + k]);
+            if (std::isfinite(x)) {
+              lo[k] = std::min(lo[k], x);
+              hi[k] = std::max(hi[k], x);
+            }
+          }
+      }
       auto &B = group == PRTCL_HIP_FLUID ? bb_f_ : bb_b_;
       for (int k = 0; k < 3; ++k) {
         B.lo[k] = lo[k];
@@ -2290,7 +2375,7 @@ class SceneImpl final : public SceneBase {
     if (nb_ > 0)
       hipLaunchKernelGGL(k_iota, dim3(grid_blocks(nb_)), dim3(kBlock), 0, st, P_.bid, nb_);
     // pinned, mapped, coherent progress words of the IISPH solve
-    PRTCL_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&mirror_host_), 64,
+    PRTCL_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&mirror_host_), 8 * kMirrorWords,
                                   hipHostMallocMapped | hipHostMallocCoherent));
     // page-locked home of the last host-visible permutation (fluid, then
     // boundary), so the permutes inside steps allocate nothing

@@ -1,4 +1,4 @@
-"""The passes that give a particle several lanes (scenes of up to 16,384
+"""The passes that give a particle several lanes (scenes of up to 65,536
 particles) and the procedures' list, at the sizes where they change: groups of
 32 and 64 particles with remainders, and the line between one lane and several.
 Bars: density is one pair sum in another order (2e-5 of the field's scale, as for
@@ -11,15 +11,15 @@ from prtcl_amd import scenes
 
 pytestmark = pytest.mark.gpu
 
-SPLIT = 16384  # kSplitMax
+SPLIT = 65536  # kSplitMax
 
 
-def _block(n, seed=4, **kw):
+def _block(n, seed=4, jitter=1e-3, **kw):
     """n particles of a jittered block in a box, moving."""
     s = 0.025
     side = int(np.ceil(n ** (1 / 3)))
     box = scenes.box_boundary(side + 4, side + 4, side + 4, s)
-    fx = scenes.fluid_block((side, side, side), (1, 1, 1), s, 1e-3, scenes.stream_base(seed, n))
+    fx = scenes.fluid_block((side, side, side), (1, 1, 1), s, jitter, scenes.stream_base(seed, n))
     v = np.random.default_rng(n).uniform(-0.2, 0.2, (n, 3))
     sc = scenes._finish(f"block{n}", s, fx[:n], box, 1, v=v, **kw)
     sc.permute_every = 0
@@ -32,10 +32,14 @@ def _close(gpu, ref, rtol, what):
     assert err <= rtol, f"{what}: {err:.3e} > {rtol:.1e}"
 
 
-@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 65, 255, 257, 1025, SPLIT, SPLIT + 1])
-def test_step_sizes_vs_oracle(hip_ctx, oracle_lib, n):
+@pytest.mark.parametrize("n,jitter", [(n, 1e-3) for n in (1, 31, 32, 33, 64, 65, 255, 257, 1025,
+                                                         SPLIT, SPLIT + 1)] +
+                         [(n, 0.0) for n in (343, SPLIT + 1)])
+def test_step_sizes_vs_oracle(hip_ctx, oracle_lib, n, jitter):
+    """Without jitter most particles have six neighbours at exactly the radius, which
+    the 16-bit candidate test leaves to the exact predicate."""
     from prtcl_amd import hip
-    sc = _block(n)
+    sc = _block(n, jitter=jitter)
     o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
     g = hip.HipScene(hip_ctx, sc)
     o.prepare()
@@ -91,6 +95,45 @@ def test_batch_of_both_kinds_equals_alone(hip_ctx):
         assert ia == ib
         np.testing.assert_array_equal(va, vb)
         np.testing.assert_array_equal(pa, pb)
+
+
+@pytest.mark.parametrize("group", ["fluid", "boundary"])
+@pytest.mark.parametrize("n", [8192, 8193, 70001])
+def test_grid_follows_uploaded_box(hip_ctx, oracle_lib, n, group):
+    """The bounding box of an upload, on the host up to 8,192 particles and on the
+    device beyond: after an upload far from the first one every neighbour is found, and
+    a particle without a finite position does not move the box."""
+    from prtcl_amd import hip
+    rng = np.random.default_rng(n)
+    sc = scenes.tiny(4)
+    fx = rng.uniform(0.0, 0.6, (n if group == "fluid" else 500, 3)).astype(np.float32)
+    bx = rng.uniform(0.0, 0.6, (n if group == "boundary" else 500, 3)).astype(np.float32)
+    sc = scenes._finish("cloud", 0.025, fx, bx, 1)
+    sc.permute_every = 0
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    g = hip.HipScene(hip_ctx, sc)
+    o.prepare()
+    g.prepare()
+    moved = (fx if group == "fluid" else bx) * np.float32([1.0, -2.0, 0.5]) + np.float32(3.0)
+    q = 1 if group == "fluid" else 0
+    for x in (o, g):
+        (x.set if x is o else x.upload)(group, "position", moved)
+        x.update() if x is o else x.run("neighborhood.update")
+    oo, oi = o.neighbors(q, q)
+    go, gi = g.neighbors(q, q)
+    np.testing.assert_array_equal(oo, go)
+    np.testing.assert_array_equal(oi, gi)
+    bad = moved.copy()
+    bad[n // 2] = [np.nan, np.inf, -np.inf]
+    g.upload(group, "position", bad)
+    g.run("neighborhood.update")
+    go, gi = g.neighbors(q, q)
+    keep = [np.delete(gi[go[i]:go[i + 1]], np.flatnonzero(gi[go[i]:go[i + 1]] == n // 2))
+            for i in (0, n // 2 - 1, n - 1)]
+    for i, k in zip((0, n // 2 - 1, n - 1), keep):
+        ref = oi[oo[i]:oo[i + 1]]
+        np.testing.assert_array_equal(k, ref[ref != n // 2])
+    g.destroy()
 
 
 @pytest.mark.parametrize("spacing", [1.0, 0.6], ids=["list", "overflow"])
