@@ -169,11 +169,11 @@ __device__ __forceinline__ void list_gather(const NbrList &L, const Spans &R, si
 // particles 5.9 -> 3.7 us, 8,000: 6.3 -> 3.9, 59,000: 5.5 -> 5.2, 125,000: 7.2 ->
 // 7.3, 250,000: 13.6 -> 13.6; pressure pass 8.1 -> 4.7, 8.3 -> 4.9, 8.0 -> 7.1,
 // 10.0 -> 10.4, 20.7 -> 21.3. The rule depends on the scene alone, so that a
-// scene's results are the same alone and in a batch; a batch fills the chip, and
-// there the lanes' idle slots cost: with the line at 65,536, 16 scenes of
-// 2,000 to 200,000 particles took 11.83 ms instead of 11.60 ms for 10 steps. Below
-// 16,384 a batch's share of the work is too small to show.
-constexpr int kSplitMax = 16384;
+// scene's results are the same alone and in a batch. At the line a scene of 59,000
+// particles still gains (10 steps 1.71 -> 1.51 ms, FP64 27,000 1.90 -> 1.39); a batch,
+// which fills the chip anyway, pays for the search's idle lanes (16 scenes of 2,000
+// to 200,000 particles: setup 182 -> 221 us, pressure passes 59.3 -> 56.6).
+constexpr int kSplitMax = 65536;
 constexpr int kListLanes = 4;
 __host__ __device__ inline bool split_scene(int nf) { return nf <= kSplitMax; }
 // threads of a list pass
