@@ -879,11 +879,61 @@ __global__ __launch_bounds__(kBlock) void k_source_list(SceneView<T> S, NbrList 
   k_source_list_body<T, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
 }
 
+// The end of IISPH iteration `it` with the sum aprde (example.lua:418-419): stop when
+// it >= min_it and aprde / nprde < tol, or at max_it. store: this thread writes
+// and reports it.
+__device__ __forceinline__ bool iteration_decision(Ctl *c, double aprde, int it, bool store) {
+  const double rel = aprde / static_cast<double>(c->nprde);
+  const bool converged = it >= c->min_it && rel < c->tol;
+  const bool done = converged || it >= c->max_it;
+  if (store) {
+    c->aprde = aprde;
+    c->iters = it;
+    c->rel = rel;
+    if (done) {
+      c->done = 1;
+      c->converged = converged ? 1 : 0;
+    }
+    publish_progress(c);
+  }
+  return done;
+}
+
+// The same decision in the first pass of the next iteration: every block sums the
+// partials of the pressure pass before it (the sum of k_pressure_finalize_body, bit
+// for bit) and derives the decision, block 0 stores it. One launch fewer per
+// iteration, 2.5 us and the gap before it, for about 1 us in the pass; the blocks
+// read all partials, so it is for launches of up to kFoldBlocks blocks (1,000 blocks
+// read 8 MB from L2; 4,000 would read 128 MB), and not for batches, which fill the
+// chip: there the pass went from 20 to 32 us. A block reads `done` once: block 0 of
+// this launch may set it meanwhile, and a block that sees it set would decide the
+// same. iters_next, staged by the pressure pass, is not written here.
+// False: the solve is done.
+constexpr unsigned kFoldBlocks = 1024;
+__host__ __device__ inline bool fold_scene(int nf) { return list_blocks(nf) <= kFoldBlocks; }
+__device__ __forceinline__ bool fold_iteration(const Ctl *c, const double *partials,
+                                               unsigned nparts, bool store) {
+  __shared__ double ws[kBlock / kWave];
+  __shared__ int flag;
+  static_assert(kBlock / kWave == 4, "four wave sums");
+  const double part = wave_sum(strided_sum<kBlock>(partials, nparts));
+  if (threadIdx.x % kWave == 0)
+    ws[threadIdx.x / kWave] = part;
+  if (threadIdx.x == 0)
+    flag = c->done;
+  __syncthreads();
+  if (flag != 0)
+    return false;
+  // block_sum's order
+  return !iteration_decision(const_cast<Ctl *>(c), (ws[0] + ws[2]) + (ws[1] + ws[3]),
+                             c->iters_next, store && threadIdx.x == 0);
+}
+
 // IISPH pressure acceleration over the list: a_i = p_i c_i - sum m_j pr_j gradW
 template <class T, int kLanes>
 __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const NbrList &L,
-                                                  unsigned lb) {
-  if (S.ctl->done)
+                                                  unsigned lb, bool fold) {
+  if (!fold && S.ctl->done)
     return;
   const int i = static_cast<int>((lb * kBlock + threadIdx.x) / kLanes);
   const uint32_t sub = threadIdx.x % kLanes;
@@ -896,6 +946,8 @@ __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const N
   // own fields loaded ahead of the walk so their latency overlaps it
   const vec4_t<T> ci = valid ? S.c[i] : zero4;
   const T pi = valid ? S.p[i] : T(0);
+  if (fold && !fold_iteration(S.ctl, S.partials, list_blocks(S.nf), lb == 0))
+    return;
   T a0 = 0, a1 = 0, a2 = 0;
   auto pair = [&](const vec4_t<T> &qj) {  // (x_j, m_j p_j / rho_j^2)
     const T d0 = xi.x - qj.x, d1 = xi.y - qj.y, d2 = xi.z - qj.z;
@@ -921,8 +973,8 @@ __device__ __forceinline__ void k_accel_list_body(const SceneView<T> &S, const N
 }
 
 template <class T, int kLanes>
-__global__ __launch_bounds__(kBlock) void k_accel_list(SceneView<T> S, NbrList L) {
-  k_accel_list_body<T, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x));
+__global__ __launch_bounds__(kBlock) void k_accel_list(SceneView<T> S, NbrList L, int fold) {
+  k_accel_list_body<T, kLanes>(S, L, xcd_block(blockIdx.x, gridDim.x), fold != 0);
 }
 
 // IISPH relaxed Jacobi update over the list, FP64 aprde reduction and the
@@ -932,6 +984,8 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
                                                      unsigned lb) {
   if (S.ctl->done)
     return;
+  if (lb == 0 && threadIdx.x == 0)
+    S.ctl->iters_next = S.ctl->iters + 1;
   struct XA {
     vec4_t<T> x, a;  // (x, m) and (a, 0) of a neighbour
   };
@@ -987,9 +1041,8 @@ __global__ __launch_bounds__(kBlock) void k_pressure_list(SceneView<T> S, NbrLis
 }
 
 // Sum of the block partials in block order (FP64, fixed tree) and the
-// convergence decision of example.lua:418-419: stop when it >= min_it and
-// aprde / nprde < tol, or at max_it. half: the partials are of half the
-// particles of a list pass's block (k_setup8) and are added in pairs first.
+// convergence decision, in a kernel of its own. half: the partials are of half
+// the particles of a list pass's block (k_setup8) and are added in pairs first.
 __device__ __forceinline__ void k_pressure_finalize_body(Ctl *c, const double *partials,
                                                         unsigned nparts, bool half = false) {
   if (c->done)
@@ -1002,18 +1055,8 @@ __device__ __forceinline__ void k_pressure_finalize_body(Ctl *c, const double *p
     part = strided_sum<kBlock>(partials, nparts);
   }
   const double acc = block_sum<kBlock>(part);
-  if (threadIdx.x == 0) {
-    c->aprde = acc;
-    const int it = c->iters + 1;
-    c->iters = it;
-    const double rel = acc / static_cast<double>(c->nprde);
-    c->rel = rel;
-    if ((it >= c->min_it && rel < c->tol) || it >= c->max_it) {
-      c->done = 1;
-      c->converged = (it >= c->min_it && rel < c->tol) ? 1 : 0;
-    }
-    publish_progress(c);
-  }
+  if (threadIdx.x == 0)
+    iteration_decision(c, acc, c->iters + 1, true);
 }
 
 __global__ __launch_bounds__(kBlock) void k_pressure_finalize(Ctl *c, const double *partials,
@@ -1159,9 +1202,9 @@ template <class T>
 __global__ __launch_bounds__(kBlock) void k_accel_b(const BatchEntry<T> *tab, BatchBlocks B) {
   BATCH_PASS_ENTRY(kListParts, list_blocks);
   if (split)
-    k_accel_list_body<T, kListLanes>(E.S, L, lb);
+    k_accel_list_body<T, kListLanes>(E.S, L, lb, false);
   else
-    k_accel_list_body<T, 1>(E.S, L, lb);
+    k_accel_list_body<T, 1>(E.S, L, lb, false);
 }
 
 template <class T>
@@ -1259,18 +1302,18 @@ void FusedOps<T>::setup(hipStream_t st, const SceneView<T> &S, const NbrList &L,
 }
 
 template <class T>
-void FusedOps<T>::accel(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
+void FusedOps<T>::accel(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool fold) {
   if (S.nf <= 0)
     return;
   const dim3 gr(list_blocks(S.nf)), bl(kBlock);
   if (split_scene(S.nf))
-    hipLaunchKernelGGL((k_accel_list<T, kListLanes>), gr, bl, 0, st, S, L);
+    hipLaunchKernelGGL((k_accel_list<T, kListLanes>), gr, bl, 0, st, S, L, fold ? 1 : 0);
   else
-    hipLaunchKernelGGL((k_accel_list<T, 1>), gr, bl, 0, st, S, L);
+    hipLaunchKernelGGL((k_accel_list<T, 1>), gr, bl, 0, st, S, L, fold ? 1 : 0);
 }
 
 template <class T>
-void FusedOps<T>::pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L) {
+void FusedOps<T>::pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool last) {
   if (S.nf <= 0)
     return;
   const unsigned nb = list_blocks(S.nf);
@@ -1278,8 +1321,14 @@ void FusedOps<T>::pressure(hipStream_t st, const SceneView<T> &S, const NbrList 
     hipLaunchKernelGGL((k_pressure_list<T, kListLanes>), dim3(nb), dim3(kBlock), 0, st, S, L);
   else
     hipLaunchKernelGGL((k_pressure_list<T, 1>), dim3(nb), dim3(kBlock), 0, st, S, L);
-  hipLaunchKernelGGL(k_pressure_finalize, dim3(1), dim3(kBlock), 0, st, S.ctl, S.partials, nb,
-                     false);
+  if (last)
+    hipLaunchKernelGGL(k_pressure_finalize, dim3(1), dim3(kBlock), 0, st, S.ctl, S.partials, nb,
+                       false);
+}
+
+template <class T>
+bool FusedOps<T>::folds(int nf) {
+  return fold_scene(nf);
 }
 
 // a = the acceleration of the last pressure-acceleration pass

@@ -58,8 +58,11 @@ struct FusedOps {
                     bool explicit_viscosity, vec4_t<T> *vtmp,
                     const SolveBegin &B = SolveBegin{});
   // the pressure acceleration goes to the second half of S.xa only
-  static void accel(hipStream_t st, const SceneView<T> &S, const NbrList &L);
-  static void pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L);
+  // fold: the pass first ends the iteration before it, whose pressure pass had
+  // last = false (only where folds(nf)); last: with the iteration's end
+  static void accel(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool fold = false);
+  static void pressure(hipStream_t st, const SceneView<T> &S, const NbrList &L, bool last = true);
+  static bool folds(int nf);
   // the convergence step of IISPH iteration 1, whose pressures and aprde
   // partials the setup (with S.first_iter) has written (batched: for the
   // scenes without first_preset)

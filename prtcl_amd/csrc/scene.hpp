@@ -43,6 +43,7 @@ struct Ctl {
   unsigned ticket2;  // last-block counter of the other reductions
   int nprde;         // iisph_nprde
   int iters;         // iterations done in the current solve
+  int iters_next;  // iters + 1, staged for the iteration that folds the sums (accel pass)
   int done;          // solve finished (converged or capped)
   int converged;
   int min_it, max_it;

@@ -1332,16 +1332,18 @@ class SceneImpl final : public SceneBase {
         enq += n;
         return;
       }
+      // within one call each iteration's end is folded into the next one
+      const bool folds = fused && FusedOps<T>::folds(nf_);
       for (int k = 0; k < n; ++k) {
         int r = pf.begin(st, kStagePressureAccel, enq + k);
         if (fused)
-          FusedOps<T>::accel(st, S, L);
+          FusedOps<T>::accel(st, S, L, folds && k > 0);
         else
           SphOps<T>::iisph_accel(st, S, PL, true);
         pf.end(st, r);
         r = pf.begin(st, kStagePressure, enq + k);
         if (fused)
-          FusedOps<T>::pressure(st, S, L);
+          FusedOps<T>::pressure(st, S, L, !folds || k + 1 == n);
         else
           SphOps<T>::iisph_pressure(st, S, PL, true);
         pf.end(st, r);
