@@ -1008,10 +1008,11 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
     sum += q.x.w * K.gradf_unscaled(d0 * d0 + d1 * d1 + d2 * d2) *
            (q.a.x * d0 + q.a.y * d1 + q.a.z * d2);
   };
-  if (!(info & kListOverflow))
-    list_gather_lanes<kLanes, 4>(
-        L, R, static_cast<size_t>(S.nf), i, info, sub,
-        [&](uint32_t j) { return XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]}; }, pair);
+  static_assert(SceneView<T>::kXaGroup == 1, "x and a of a particle side by side");
+  list_gather_records<kLanes, 4>(
+      L, R, static_cast<size_t>(S.nf), i, (info & kListOverflow) ? 0u : info, sub,
+      static_cast<uint32_t>(valid ? i : 0), S.xa,
+      [&](const vec4_t<T> &x, const vec4_t<T> &a) { pair(XA{x, a}); });
   if (valid && sub == 0 && (info & kListOverflow))
     grid_walk(S, i, xi, [&](uint32_t j) {
       pair(XA{S.xa[S.xa_x(j)], S.xa[S.xa_a(j)]});

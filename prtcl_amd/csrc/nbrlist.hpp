@@ -274,6 +274,85 @@ __device__ __forceinline__ void list_gather_lanes(const NbrList &L, const Spans 
   }
 }
 
+// the value of the lane beside (lane ^ 1; every lane of the wavefront calls it)
+template <class V>
+__device__ __forceinline__ V pair_swap(const V &v) {
+  static_assert(sizeof(V) % sizeof(int) == 0, "whole words");
+  int w[sizeof(V) / sizeof(int)];
+  __builtin_memcpy(w, &v, sizeof(V));
+#pragma unroll
+  for (unsigned k = 0; k < sizeof(V) / sizeof(int); ++k)
+    w[k] = __builtin_amdgcn_update_dpp(0, w[k], 0xB1, 0xF, 0xF, true);  // quad_perm 1 0 3 2
+  V r;
+  __builtin_memcpy(&r, w, sizeof(V));
+  return r;
+}
+
+// list_gather_lanes for records of two adjacent values: use(rec[2 j], rec[2 j + 1])
+// for the entries j of the lane. A gather is bound by the cache lines that its
+// lanes touch, and the two values of a record lie in one line: so two lanes load
+// the two values of the even lane's record together, then those of the odd lane's,
+// and exchange what is the other's. Every lane of the wavefront calls it (info 0: no
+// entries); a lane without an entry left loads record `idle`. Pressure pass of 1M
+// particles 87 -> 79 us, of a batch 37.5 -> 34.5, CG product of 250,000 22.2 -> 20.5.
+// With four lanes per particle it pays only for 32-byte values (FP64, 27,000: 7.4 ->
+// 6.5 us; FP32, 2,048: 4.2 -> 4.7, 59,000: 6.8 -> 6.9): launches of latency rather than
+// of cache lines.
+template <int kLanes, int kGroup, class V, class Use>
+__device__ __forceinline__ void list_gather_records(const NbrList &L, const Spans &R, size_t n,
+                                                    int i, uint32_t info, uint32_t sub,
+                                                    uint32_t idle, const V *__restrict__ rec,
+                                                    Use &&use) {
+  if constexpr (kLanes > 1 && sizeof(V) == 16) {
+    struct Two {
+      V a, b;
+    };
+    list_gather_lanes<kLanes, kGroup>(
+        L, R, n, i, info, sub,
+        [&](uint32_t j) {
+          return Two{rec[2 * static_cast<size_t>(j)], rec[2 * static_cast<size_t>(j) + 1]};
+        },
+        [&](const Two &q) { use(q.a, q.b); });
+    return;
+  }
+  const uint32_t c0 = info & 0xFFu;
+  const uint32_t c01 = c0 + ((info >> 8) & 0xFFu);
+  const uint32_t c = c01 + ((info >> 16) & 0xFFu);
+  const uint32_t d1 = R.b1 - R.b0, d2 = R.b2 - R.b1;
+  const bool odd = (threadIdx.x & 1u) != 0u;
+  const V *__restrict__ half = rec + (odd ? 1 : 0);
+  const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+  uint4 q = sub * kChunk < c ? list_chunk(L, n, i, sub) : none;
+  for (uint32_t g = sub; __ballot(g * kChunk < c) != 0ull; g += kLanes) {
+    const uint4 cur = q;
+    if ((g + kLanes) * kChunk < c)
+      q = list_chunk(L, n, i, g + kLanes);
+#pragma unroll
+    for (int h = 0; h < static_cast<int>(kChunk); h += kGroup) {
+      V r1[kGroup], r2[kGroup];
+      if (__ballot(g * kChunk + h < c) == 0ull)
+        break;
+#pragma unroll
+      for (int k = 0; k < kGroup; ++k) {
+        const uint32_t e = g * kChunk + h + k;
+        const uint32_t j =
+            e < c ? R.b0 + chunk_entry(cur, h + k) + (e >= c0 ? d1 : 0u) + (e >= c01 ? d2 : 0u)
+                  : idle;
+        const uint32_t p = pair_swap(j);
+        r1[k] = half[2 * static_cast<size_t>(odd ? p : j)];  // the even lane's neighbour
+        r2[k] = half[2 * static_cast<size_t>(odd ? j : p)];  // the odd lane's
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < kGroup; ++k) {
+        const V s1 = pair_swap(r1[k]), s2 = pair_swap(r2[k]);
+        if (g * kChunk + h + k < c)
+          use(odd ? s2 : r1[k], odd ? r2[k] : s1);
+      }
+    }
+  }
+}
+
 // the sum over a particle's kLanes lanes, in every one of them (all lanes of
 // the wavefront call it)
 template <int kLanes, class T>

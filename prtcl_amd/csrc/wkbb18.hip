@@ -567,36 +567,43 @@ __device__ __forceinline__ void product_finish(const SceneView<T> &S, int i,
 }
 
 // the list product at particle i (valid), complete in every one of its kLanes lanes
-template <class T, bool kGC, int kLanes>
+// with w at stride kStride: S.v, or the second half of the records S.cxp
+template <class T, bool kGC, int kLanes, int kStride>
 __device__ __forceinline__ void product_list(const SceneView<T> &S, const NbrList &L, unsigned lb,
                                              int i, bool valid, uint32_t sub,
-                                             const vec4_t<T> *__restrict__ w, int ws,
+                                             const vec4_t<T> *__restrict__ w,
                                              T out[3]) {
   T l0 = 0, l1 = 0, l2 = 0;
   vec4_t<T> wi = make4<vec4_t<T>>(T(0), T(0), T(0), T(0)), bd = wi, bo = wi;
-  if (valid) {
-    const vec4_t<T> xq = S.xq[i];  // (x_i, m_i / rho_i)
-    wi = w[static_cast<size_t>(ws) * i];
-    const ProductPair<T> pair(S);
+  const vec4_t<T> xq = valid ? S.xq[i] : wi;  // (x_i, m_i / rho_i)
+  const uint32_t info = valid ? L.info[i] : kListOverflow;
+  if (valid)
+    wi = w[kStride * static_cast<size_t>(i)];
+  const ProductPair<T> pair(S);
+  // (x_j, m_j / rho_j) and w_j
+  auto use = [&](const vec4_t<T> &xj, const vec4_t<T> &wj) { pair(xq, wi, xj, wj, l0, l1, l2); };
+  const Spans R = pass_spans<kLanes>(L, S.nf, lb);
+  const size_t n = static_cast<size_t>(S.nf);
+  const uint32_t live = (info & kListOverflow) ? 0u : info;
+  if constexpr (kStride == 2) {
+    list_gather_records<kLanes, 4>(L, R, n, i, live, sub, static_cast<uint32_t>(valid ? i : 0),
+                                   S.cxp, use);
+  } else {
     struct XW {
-      vec4_t<T> x, w;  // (x_j, m_j / rho_j) and w_j
+      vec4_t<T> x, w;
     };
-    auto use = [&](const XW &q) { pair(xq, wi, q.x, q.w, l0, l1, l2); };
-    const uint32_t info = L.info[i];
-    if (!(info & kListOverflow)) {
-      list_gather_lanes<kLanes, 4>(
-          L, pass_spans<kLanes>(L, S.nf, lb), static_cast<size_t>(S.nf), i, info, sub,
-          [&](uint32_t j) {
-            return XW{S.cxp[2 * static_cast<size_t>(j)], w[static_cast<size_t>(ws) * j]};
-          },
-          use);
-    } else if (sub == 0) {
+    list_gather_lanes<kLanes, 4>(
+        L, R, n, i, live, sub,
+        [&](uint32_t j) { return XW{S.cxp[2 * static_cast<size_t>(j)], w[j]}; },
+        [&](const XW &q) { use(q.x, q.w); });
+  }
+  if (valid) {
+    if (sub == 0 && (info & kListOverflow))
       nbrs_exact(S, xq, S.fcell[i], S.fstart, S.xq,
                  [&](uint32_t j, T, T, T, T, const vec4_t<T> &) {
                    if (j != static_cast<uint32_t>(i))
-                     use(XW{S.xq[j], w[static_cast<size_t>(ws) * j]});
+                     use(S.xq[j], w[kStride * static_cast<size_t>(j)]);
                  });
-    }
     bd = S.cb[i];
     bo = S.G[i];
   }
@@ -660,7 +667,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_setup(SceneView<T> S, NbrList L, 
     if (valid)
       product_exact<T, kGC>(S, i, S.v, 1, ax);
   } else {
-    product_list<T, kGC, kLanes>(S, L, lb, i, valid, sub, S.v, 1, ax);
+    product_list<T, kGC, kLanes, 1>(S, L, lb, i, valid, sub, S.v, ax);
   }
   if (valid && sub == 0)
     cg_start(S, i, S.v[i], ax, acc);
@@ -764,7 +771,7 @@ __device__ __forceinline__ void cg_spmv_body(const SceneView<T> &S, const NbrLis
     if (valid)
       product_exact<T, kGC>(S, i, S.cxp + 1, 2, q);
   } else {
-    product_list<T, kGC, kLanes>(S, L, lb, i, valid, sub, S.cxp + 1, 2, q);
+    product_list<T, kGC, kLanes, 2>(S, L, lb, i, valid, sub, S.cxp + 1, q);
   }
   if (valid && sub == 0) {
     const vec4_t<T> qv = make4<vec4_t<T>>(q[0], q[1], q[2], T(0));
