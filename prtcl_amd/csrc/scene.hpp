@@ -413,9 +413,8 @@ struct GridOps {
                            const vec4_t<T> *vs, uint32_t *id_d, const uint32_t *id_s,
                            uint32_t *c_d, const uint32_t *c_s, const uint32_t *perm, int n);
 };
-// exclusive scan of n uint32 counts into start[0..n] (start[n] = total); the
-// counts are cleared to zero for the next build
-void scan_counts(hipStream_t st, uint32_t *count, uint32_t *start, uint32_t n,
+// exclusive scan of n uint32 counts into start[0..n] (start[n] = total)
+void scan_counts(hipStream_t st, const uint32_t *count, uint32_t *start, uint32_t n,
                  uint32_t *tmp);
 size_t scan_tmp_words(uint32_t n);
 unsigned scan_tiles(uint32_t ncells);

@@ -136,6 +136,36 @@ def test_grid_follows_uploaded_box(hip_ctx, oracle_lib, n, group):
     g.destroy()
 
 
+@pytest.mark.parametrize("dims", [(4, 3, 3), (16, 16, 16), (16, 16, 17), (40, 40, 40), (32, 32, 64),
+                                  (40, 40, 41), (61, 40, 40)])
+def test_sort_over_scan_tiles(hip_ctx, oracle_lib, dims):
+    """The cell scan in one launch up to 16 tiles of 4,096 cells and in two beyond, with
+    whole and partial last tiles; sorted three times, so counts left over would show."""
+    from prtcl_amd import hip
+    r = 0.05
+    rng = np.random.default_rng(dims[2])
+    hi = (np.array(dims) - 3 + 0.5) * r
+    fx = rng.uniform(0.5 * r, hi, (700, 3)).astype(np.float32)
+    bx = np.array([[0.5 * r] * 3, hi], np.float32)
+    sc = scenes._finish("tiles", r / 2, fx, bx, 1)
+    sc.permute_every = 0
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    g = hip.HipScene(hip_ctx, sc)
+    o.prepare()
+    g.prepare()
+    for _ in range(3):
+        fx = rng.uniform(0.5 * r, hi, (700, 3)).astype(np.float32)
+        o.set("fluid", "position", fx)
+        o.update()
+        g.upload("fluid", "position", fx)
+        g.run("neighborhood.update")
+        oo, oi = o.neighbors(1, 1)
+        go, gi = g.neighbors(1, 1)
+        np.testing.assert_array_equal(oo, go)
+        np.testing.assert_array_equal(oi, gi)
+    g.destroy()
+
+
 @pytest.mark.parametrize("spacing", [1.0, 0.6], ids=["list", "overflow"])
 def test_procedures_follow_the_positions(hip_ctx, oracle_lib, spacing):
     """A procedure between two changes of the positions reads a list that an
