@@ -12,10 +12,9 @@
 //   Ap_i = dt^2 rho0/rho_i (a_i . (G_f + rho0 G_b) - sum_f m_j a_j.gradW_ij)
 // so boundary particles are visited once per step (in the setup pass) and
 // each IISPH iteration is two passes over fluid neighbours only. The setup
-// pass tests the 27-cell candidates with the exact predicate and records the
-// accepted fluid neighbours (self excluded) in a per-step list of 16-bit
-// slab indices (nbrlist.hpp); the IISPH passes stage each slab of their
-// block's neighbourhood in LDS and gather the neighbours' fields from there.
+// pass records the fluid neighbours (self excluded, exact predicate) in a
+// per-step list of 16-bit offsets (nbrlist.hpp), from which the IISPH passes
+// gather the neighbours' fields through L2.
 // A particle with more neighbours than the list holds is walked over the
 // grid instead.
 #include <limits>
@@ -1141,7 +1140,7 @@ __global__ __launch_bounds__(kBlock) void k_speed_finalize(Ctl *c, const double 
 // ---- batched wrappers (prtcl_hip_step over several scenes): the setup and list
 // passes take the body that the block's scene takes alone (split_scene)
 // the two setup bodies share their LDS, so the large scenes' blocks keep
-// their five per CU
+// their six per CU
 union SetupPool {
   SetupShared setup;
   Scan8Shared scan;

@@ -16,8 +16,8 @@
 // Layout: chunks of 8 entries; entry e of particle i at
 // idx[((e / 8) * n + i) * 8 + e % 8], so one 16-byte load per lane fetches 8
 // entries and a wavefront's load is 1 KB contiguous. Entries are ordered by
-// slab; info[i] holds the entry
-// count of each slab (8 bits each) and kListOverflow when the particle has
+// slab; info[i] holds the entry count of each slab (8 bits each),
+// kListBoundary where a boundary particle is in reach, and kListOverflow when the particle has
 // more than kNbrCap neighbours or a span of its block exceeds 16 bits (its
 // passes then walk the grid with the exact predicate instead).
 #pragma once
