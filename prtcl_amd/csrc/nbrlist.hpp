@@ -88,38 +88,11 @@ __device__ __forceinline__ uint32_t list_count(uint32_t info) {
   return (info & 0xFFu) + ((info >> 8) & 0xFFu) + ((info >> 16) & 0xFFu);
 }
 
-// Visits the list entries of particle i (not overflowed) in list order:
-// fn(e, j) with e the entry's index and j its global slot. R is the span
-// table of i's block. The slot is b0 + entry + [e >= c0] (b1 - b0) +
-// [e >= c01] (b2 - b1) (two selects against register values).
-template <class Fn>
-__device__ __forceinline__ void list_visit_indexed(const NbrList &L, const Spans &R, size_t n,
-                                                   int i, uint32_t info, Fn &&fn) {
-  const uint32_t c0 = info & 0xFFu;
-  const uint32_t c01 = c0 + ((info >> 8) & 0xFFu);
-  const uint32_t c = c01 + ((info >> 16) & 0xFFu);
-  const uint32_t d1 = R.b1 - R.b0, d2 = R.b2 - R.b1;
-  for (uint32_t g = 0; g * kChunk < c; ++g) {
-    const uint4 q = list_chunk(L, n, i, g);
-#pragma unroll
-    for (int k = 0; k < static_cast<int>(kChunk); ++k) {
-      const uint32_t e = g * kChunk + k;
-      if (e < c)
-        fn(e, R.b0 + chunk_entry(q, k) + (e >= c0 ? d1 : 0u) + (e >= c01 ? d2 : 0u));
-    }
-  }
-}
-
-// the same with the slot only: fn(j)
-template <class Fn>
-__device__ __forceinline__ void list_visit(const NbrList &L, const Spans &R, size_t n, int i,
-                                           uint32_t info, Fn &&fn) {
-  list_visit_indexed(L, R, n, i, info, [&](uint32_t, uint32_t j) { fn(j); });
-}
-
-// The same walk one chunk (8 entries) at a time with the memory traffic of
-// a chunk issued before its arithmetic: the chunk, then the gathers
-// (v[k] = load(j_k)) of kGroup entries, then use(v[k]) in order; the next
+// Walks the list entries of particle i (not overflowed) in list order, one chunk
+// (8 entries) at a time, with the memory traffic of a chunk issued before its
+// arithmetic: the chunk, then the gathers (v[k] = load(j_k)) of kGroup entries,
+// then use(v[k]) in order. R is the span table of i's list: the slot of entry e is
+// b0 + entry + [e >= c0] (b1 - b0) + [e >= c01] (b2 - b1). The next
 // chunk is fetched while the current one is in flight. kGroup < 8 keeps fewer
 // gathered values live (more waves per SIMD) for wide records.
 template <int kGroup = 8, class Load, class Use>

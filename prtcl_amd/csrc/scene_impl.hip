@@ -2257,9 +2257,8 @@ class SceneImpl final : public SceneBase {
     const size_t b = static_cast<size_t>(std::max(nb, 1));
     for (V4 **q : {&P.v, &P.a, &P.c, &P.G, &P.vd, &P.tmpV4})
       A.take(*q, f);
-    // xm and xq swap roles every step; both carry the run padding
     for (V4 **q : {&P.xm, &P.xq})
-      A.take(*q, f + kRunPad);
+      A.take(*q, f);
     A.take(P.xa, SceneView<T>::xa_x(f - 1) + 1 + SceneView<T>::kXaGroup);
     for (T **q : {&P.rho, &P.p, &P.pr, &P.s, &P.AA, &P.Ap, &P.tmpT})
       A.take(*q, f);
