@@ -75,28 +75,14 @@ template <class T>
 struct FastSpline {
   T inv_h, aw, ag, ag3, eps2;
   __device__ __forceinline__ void eval(T r2, T &w, T &f) const {
-    const T rinv = rsqrt_fast<T>(r2 > T(0) ? r2 : T(1));
+    const T rinv = rsqrt_fast<T>(fmax(r2, std::numeric_limits<T>::min()));
     const T r = r2 * rinv;
     const T q = r * inv_h;
-    const T b2 = q < T(2) ? T(2) - q : T(0);
-    const T b1 = T(1) - q;
-    const T b1p = b1 > T(0) ? b1 : T(0);
+    const T b2 = fmax(T(2) - q, T(0));
+    const T b1p = fmax(T(1) - q, T(0));
     w = aw * (b2 * b2 * b2 - T(4) * b1p * b1p * b1p);
     const T dw = ag * (T(12) * b1p * b1p - T(3) * b2 * b2);
     f = r2 < eps2 ? T(0) : dw * rinv;
-    if (r2 <= T(0))
-      w = aw * T(4);  // W(0) = alpha/h^3 (8 - 4)
-  }
-  // the same without the factors: W / aw in w, gradW / ag3 in f
-  __device__ __forceinline__ void unscaled(T r2, T &w, T &f) const {
-    const T rinv = rsqrt_fast<T>(fmax(r2, std::numeric_limits<T>::min()));
-    const T q = r2 * rinv * inv_h;
-    const T t = fmax(T(2) - q, T(0));
-    const T u = fmax(T(2) - T(2) * q, T(0));
-    const T t2 = t * t, u2 = u * u;
-    w = t2 * t - T(0.5) * (u2 * u);
-    const T d = (u2 - t2) * rinv;
-    f = r2 < eps2 ? T(0) : d;
   }
   __device__ __forceinline__ T gradf(T r2) const { return ag3 * gradf_unscaled(r2); }
   __device__ __forceinline__ T gradf_unscaled(T r2) const {
@@ -285,8 +271,9 @@ __device__ __forceinline__ double first_iteration(const SceneView<T> &S, int i,
 // candidates and 30 pairs a particle). With candidates as 16-byte positions and
 // 13 instructions, 65 a pair and five wavefronts per SIMD, 1M particles took 229
 // us, 250,000 73 us, 16 scenes of 2,000 to 200,000 together 247 us; with 8-byte
-// records and 9 instructions, 45 a pair (the kernel's factors applied to the
-// sums, the velocities integrated by the sort) and six wavefronts 188, 53 and 182.
+// records and 9 instructions, the velocities integrated by the sort and six
+// wavefronts 182, 54 and 223 (batches pay for the 8-lane search of their small
+// scenes, nbrlist.hpp: 182 with one lane for each).
 // ---------------------------------------------------------------------------
 // the pair sums of the setup pass for one particle (or one lane's share)
 template <class T, bool kWithSource>
@@ -295,8 +282,8 @@ struct SetupSums {
   const FastSpline<T> K;
   vec4_t<T> xi;
   T vs0, vs1, vs2;
-  // density / aw, G_f / ag3, sum |gradW|^2 / ag3^2 and the velocity-divergence sum
-  // of the source term / ag3; density and G_b of the boundary
+  // density, G_f, sum |gradW|^2 and the velocity-divergence sum of the source
+  // term; density and G_b of the boundary
   T rho = 0, gf0 = 0, gf1 = 0, gf2 = 0, s2 = 0, dsum = 0;
   T rhob = 0, gb0 = 0, gb1 = 0, gb2 = 0;
   bool near_boundary = false;
@@ -306,8 +293,8 @@ struct SetupSums {
       : S(view), K(fast_spline(view)), xi(x) {
     vs0 = vi.x, vs1 = vi.y, vs2 = vi.z;
   }
-  // density self term W(0) = 4 alpha / h^3 (aw applied by finish)
-  __device__ __forceinline__ T self() const { return xi.w * T(4); }
+  // density self term W(0) = 4 alpha / h^3
+  __device__ __forceinline__ T self() const { return xi.w * K.aw * T(4); }
   // neighbour (x_j, m_j) = pj with velocity vj (read only with kWithSource)
   __device__ __forceinline__ void pair(const vec4_t<T> &pj, const vec4_t<T> &vj) {
     const T d0 = xi.x - pj.x, d1 = xi.y - pj.y, d2 = xi.z - pj.z;
@@ -325,18 +312,23 @@ struct SetupSums {
     add(pj, vj, d0, d1, d2, r2);
     return true;
   }
+  // The kernel's factors are in every term: applied to the sums they save 1 % of the
+  // pass (1M particles 182 -> 180 us), but the square of the gradient's leaves the FP32
+  // range by itself, and the association shows, as 1e-4 of the pressure: the solve starts
+  // from rho0 - rho, a difference of nearly equal numbers.
   __device__ __forceinline__ void add(const vec4_t<T> &pj, const vec4_t<T> &vj, T d0, T d1, T d2,
                                       T r2) {
     T w, f;
-    K.unscaled(r2, w, f);
+    K.eval(r2, w, f);
     rho += pj.w * w;
-    const T mf = pj.w * f;
-    gf0 += mf * d0;
-    gf1 += mf * d1;
-    gf2 += mf * d2;
-    s2 += mf * (f * r2);
+    const T g0 = f * d0, g1 = f * d1, g2 = f * d2;
+    gf0 += pj.w * g0;
+    gf1 += pj.w * g1;
+    gf2 += pj.w * g2;
+    s2 += pj.w * (g0 * g0 + g1 * g1 + g2 * g2);
     if (kWithSource) {
-      dsum += mf * ((vs0 - vj.x) * d0 + (vs1 - vj.y) * d1 + (vs2 - vj.z) * d2);
+      const T u0 = vs0 - vj.x, u1 = vs1 - vj.y, u2 = vs2 - vj.z;
+      dsum += pj.w * (u0 * g0 + u1 * g1 + u2 * g2);
     }
   }
   __device__ __forceinline__ vec4_t<T> load_v(uint32_t j) const {
@@ -370,10 +362,7 @@ struct SetupSums {
   // IISPH iteration 1 (S.first_iter)
   __device__ __forceinline__ double finish(int i) {
     const T rho0 = S.rho0;
-    rho = rho * K.aw + rho0 * rhob;
-    gf0 *= K.ag3, gf1 *= K.ag3, gf2 *= K.ag3;
-    s2 *= K.ag3 * K.ag3;
-    dsum *= K.ag3;
+    rho += rho0 * rhob;
     const T irho = T(1) / rho;
     const T irho2 = irho * irho;
     const T k14 = T(1.4) * rho0;
