@@ -327,8 +327,8 @@ __device__ __forceinline__ void k_place_state_body(GridDims g, const uint32_t *_
   const uint32_t p = b + r;
   const V x = xs[o];
   xd[p] = x;
-  xf_d[p] = fixed_record(kFixUnits / g.radius, static_cast<double>(x.x),
-                         static_cast<double>(x.y), static_cast<double>(x.z));
+  xf_d[p] = fixed_record(g, static_cast<double>(x.x), static_cast<double>(x.y),
+                         static_cast<double>(x.z));
   vd[p] = kick(vs[o]);
   id_d[p] = id_s[o];
   c_d[p] = c;

@@ -159,20 +159,29 @@ struct GridDims {
 
 // ---- positions in 16 bits for the candidate test of the neighbour search
 //
-// A component is floor(x * kFixUnits / radius), x and y modulo 2^16. The difference
-// of two components, modulo 2^16, is within one unit of the exact difference where
-// that is below 4 radii, so two particles within the radius are at less than
-// kFixUnits + sqrt(3) units: candidates at kFixUnits + 2 units or more are no
-// neighbours, and the exact predicate decides about the others that are close to
-// the radius (or beyond it: farther candidates can alias; they are accepted here at
-// most, never rejected).
+// A component is floor(x * kFixUnits / radius) counted from the corner of the cell
+// box, x and y modulo 2^16. The difference of two components, modulo 2^16, is within
+// one unit of the exact difference where that is below 4 radii, so two particles
+// within the radius are at less than kFixUnits + sqrt(3) units: candidates at
+// kFixUnits + 2 units or more are no neighbours, and the exact predicate decides about
+// the others that are close to the radius (or beyond it: farther candidates can alias;
+// they are accepted here at most, never rejected). Counted from the box, a scene far
+// from the origin has the differences that it has at the origin; a particle that left
+// the box by more than 2^17 radii (or has no finite position) is held there, which
+// brings records together and parts none.
 constexpr int kFixUnits = 8192;
 constexpr uint32_t kFixReach = (kFixUnits + 2) * (kFixUnits + 2);
-__device__ __forceinline__ uint2 fixed_record(double scale, double x, double y, double z) {
-  const uint32_t qx = static_cast<uint32_t>(static_cast<int>(floor(x * scale)));
-  const uint32_t qy = static_cast<uint32_t>(static_cast<int>(floor(y * scale)));
-  const uint32_t qz = static_cast<uint32_t>(static_cast<int>(floor(z * scale)));
-  return make_uint2((qx & 0xFFFFu) | (qy << 16), qz);
+constexpr double kFixFar = 1073741824.0;
+__device__ __forceinline__ uint32_t fixed_component(double scale, double x, int origin) {
+  const double u = fma(x, scale, -static_cast<double>(origin) * kFixUnits);
+  // (fmax gives -kFixFar for a NaN)
+  return static_cast<uint32_t>(static_cast<int>(floor(fmin(fmax(u, -kFixFar), kFixFar))));
+}
+__device__ __forceinline__ uint2 fixed_record(const GridDims &g, double x, double y, double z) {
+  const double scale = kFixUnits / g.radius;
+  const uint32_t qx = fixed_component(scale, x, g.ox);
+  const uint32_t qy = fixed_component(scale, y, g.oy);
+  return make_uint2((qx & 0xFFFFu) | (qy << 16), fixed_component(scale, z, g.oz));
 }
 // squared distance in units of two records, modulo 2^32 (z to 24 bits)
 using fix2_t = short __attribute__((ext_vector_type(2)));

@@ -249,3 +249,61 @@ def test_diagonal_of_a_lone_particle_at_small_scale(hip_ctx):
     g.step(1)
     np.testing.assert_array_equal(g.download("fluid", "iisph_diagonal_element"), [0, 0])
     g.destroy()
+
+
+def test_step_far_from_the_origin(hip_ctx):
+    """A scene of 64-bit positions 786,432 radii from the origin has the lists, and so
+    the bits, that it has at the origin. (All lengths are multiples of 2^-22 and the
+    shift is one of the cell edge, 2^-4, so that every difference is exact; beyond 2^18
+    radii a candidate position counted from the origin leaves 32 bits, every candidate
+    is accepted, and the overflowed lists walk the grid in another order.)"""
+    from prtcl_amd import hip
+    s = 2.0 ** -5
+    rng = np.random.default_rng(8)
+    fx = scenes.fluid_block((9, 9, 9), (1, 1, 1), s, 0.0, None).astype(np.float64)
+    fx = np.round((fx + rng.uniform(-1e-3, 1e-3, fx.shape)) * 2.0 ** 22) / 2.0 ** 22
+    bx = scenes.box_boundary(12, 12, 12, s).astype(np.float64)
+    out = []
+    for shift in (0.0, 3.0 * 2.0 ** 14, -3.0 * 2.0 ** 14):
+        sc = scenes._finish("far", s, fx + shift, bx + shift, 1,
+                            v=rng.uniform(-0.2, 0.2, fx.shape) if not out else v)
+        v = sc.fluid_v
+        sc.permute_every = 0
+        g = hip.HipScene(hip_ctx, sc, real_type=1)
+        g.prepare()
+        g.step(1)
+        out.append([g.download("fluid", f) for f in ("density", "iisph_diagonal_element",
+                                                     "pressure", "velocity")])
+        g.destroy()
+    for far in out[1:]:
+        for a, b in zip(out[0], far):
+            np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [343, SPLIT + 1])
+@pytest.mark.parametrize("far", [5.0, -5.0, 1e4])
+def test_step_outside_the_planned_box(hip_ctx, oracle_lib, n, far):
+    """Particles that have left the cell box are candidates of each other in its border
+    cells. Eight radii apart their 16-bit positions agree, which the exact predicate has
+    to see, also where they are more than a list holds; those within the radius are found."""
+    from prtcl_amd import hip
+    sc = _block(n, seed=6)
+    r = sc.radius
+    g = hip.HipScene(hip_ctx, sc)
+    g.prepare()  # plans the box
+    x = sc.fluid_x.copy()
+    k = np.arange(70)
+    x[:70] = far
+    x[:60, 0] += (8 * r * k[:60]).astype(np.float32)       # a row, all alike in 16 bits
+    x[60:70, 1] += (0.9 * r * k[:10]).astype(np.float32)   # a chain of neighbours
+    x[60:70, 2] += np.float32(20 * r)
+    sc.fluid_x = x
+    g.upload("fluid", "position", x)
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    o.prepare()
+    o.step()
+    g.step(1)
+    rho, ref = g.download("fluid", "density"), o.get("fluid", "density")
+    np.testing.assert_allclose(rho[:70], ref[:70], rtol=2e-5)
+    _close(rho, ref, 2e-5, "density")
+    g.destroy()
