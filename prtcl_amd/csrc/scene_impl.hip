@@ -2262,10 +2262,12 @@ class SceneImpl final : public SceneBase {
     A.take(P.xa, SceneView<T>::xa_x(f - 1) + 1 + SceneView<T>::kXaGroup);
     for (T **q : {&P.rho, &P.p, &P.pr, &P.s, &P.AA, &P.Ap, &P.tmpT})
       A.take(*q, f);
-    A.take(P.sp, 9 * f);
-    // also the 16-bit positions of a fused step, with the run padding
-    A.take(P.tmpSp, std::max(9 * f, (f + kRunPad) * sizeof(uint2) / sizeof(T)));
-    A.take(P.gc, 9 * f);
+    // tmpSp also takes the 16-bit positions of a fused step, with the run padding,
+    // and changes places with sp, gc and (pt16) tvg in an update of all fields: each
+    // holds either
+    const size_t f9 = std::max(9 * f, (f + kRunPad) * sizeof(uint2) / sizeof(T));
+    for (T **q : {&P.sp, &P.tmpSp, &P.gc})
+      A.take(*q, f9);
     A.take(P.id, f);
     A.take(P.tmpI, f);
     A.take(P.fcell, f);
@@ -2297,7 +2299,7 @@ class SceneImpl final : public SceneBase {
     const size_t np = pt16 ? f : 1;
     for (V4 **q : {&P.om, &P.orhs, &P.vrhs})
       A.take(*q, np);
-    A.take(P.tvg, 9 * np);
+    A.take(P.tvg, pt16 ? f9 : 9);
     A.take(P.pcoef, pt16 ? static_cast<size_t>(kNbrCap) * f : 1);
     for (T **q : {&P.prho, &P.psrho, &P.pone, &P.odiag, &P.vdiag})
       A.take(*q, np);

@@ -307,3 +307,26 @@ def test_step_outside_the_planned_box(hip_ctx, oracle_lib, n, far):
     np.testing.assert_allclose(rho[:70], ref[:70], rtol=2e-5)
     _close(rho, ref, 2e-5, "density")
     g.destroy()
+
+
+@pytest.mark.parametrize("iv,n", [(0, n) for n in (1, 2, 3, 257, SPLIT + 1)] +
+                         [(3, n) for n in (2, 3, 257, SPLIT + 1)])
+def test_step_after_updates_vs_oracle(hip_ctx, oracle_lib, iv, n):
+    """An update of all fields exchanges the vector that holds the 16-bit positions with
+    the nine-component fields; after one, two and three of them a step finds room. (The
+    preconditioner of pt16 divides a lone particle by 0.)"""
+    from prtcl_amd import hip
+    kw = dict(KINDS["pt16"], pt16_vorticity_maximum_error=1e-4,
+              pt16_velocity_maximum_error=1e-4) if iv else {}
+    sc = _block(n, **kw)
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    g = hip.HipScene(hip_ctx, sc)
+    o.prepare()
+    g.prepare()
+    for _ in range(3):
+        o.step()
+        g.run("neighborhood.update")
+        g.step(1)
+    _close(g.download("fluid", "density"), o.get("fluid", "density"), 6e-5, "density")
+    _close(g.download("fluid", "position"), o.get("fluid", "position"), 3e-5, "position")
+    g.destroy()
