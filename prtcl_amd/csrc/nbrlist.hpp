@@ -22,6 +22,8 @@
 // passes then walk the grid with the exact predicate instead).
 #pragma once
 
+#include <type_traits>
+
 #include "scene.hpp"
 
 namespace prtcl_amd {
@@ -48,7 +50,9 @@ struct NbrList {
   uint32_t *info;
   BlockRanges *blk;  // one per 1 << shift slots
   uint32_t shift;
+  uint32_t zero = 0;  // no byte left unset: the list is part of a graph's key
 };
+static_assert(std::has_unique_object_representations_v<NbrList>, "no padding");
 
 // The span table of one block in registers (selected by slab without
 // indexing, so it never lives in scratch memory).
@@ -177,6 +181,7 @@ struct BatchBlocks {
                        {g ? 0u : n[0], g ? 0u : n[1], g ? n[2] : 0u, g ? n[3] : 0u}};
   }
 };
+static_assert(std::has_unique_object_representations_v<BatchBlocks>, "no padding (graph keys)");
 // the word of this block and its part (0 .. factor - 1) of a split scene's block
 __device__ __forceinline__ uint32_t batch_block(const BatchBlocks &B, unsigned factor,
                                                 unsigned *part) {
