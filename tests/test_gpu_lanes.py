@@ -1,6 +1,6 @@
 """The passes that give a particle several lanes (scenes of up to 65,536
-particles) and the procedures' list, at the sizes where they change: groups of
-32 and 64 particles with remainders, and the line between one lane and several.
+particles), those that give it one, and the procedures' list, at the sizes where they
+change: groups of 32 and 64 particles with remainders, and the line between them.
 Bars: density is one pair sum in another order (2e-5 of the field's scale, as for
 the single procedures), position after one step as for whole steps (1e-5)."""
 
@@ -330,3 +330,72 @@ def test_step_after_updates_vs_oracle(hip_ctx, oracle_lib, iv, n):
     _close(g.download("fluid", "density"), o.get("fluid", "density"), 6e-5, "density")
     _close(g.download("fluid", "position"), o.get("fluid", "position"), 3e-5, "position")
     g.destroy()
+
+
+def _tight(kind):
+    """The kind with solves that stop at 1e-4, as in test_viscous_step_sizes_vs_oracle."""
+    return dict(KINDS[kind], wkbb18_maximum_error=1e-4, pt16_vorticity_maximum_error=1e-4,
+                pt16_velocity_maximum_error=1e-4)
+
+
+def _one_step_vs_oracle(hip_ctx, oracle_lib, sc, bars, real_type=0):
+    from prtcl_amd import hip
+    o = oracle_lib.OracleScene(sc, fp64_reductions=True, permute_every=0)
+    g = hip.HipScene(hip_ctx, sc, real_type=real_type)
+    o.prepare()
+    g.prepare()
+    o.step()
+    g.step(1)
+    for f, bar in bars.items():
+        _close(g.download("fluid", f), o.get("fluid", f), bar, f)
+    g.destroy()
+
+
+BARS = {"density": 2e-5, "position": 1e-5, "velocity": 1e-3}
+
+
+@pytest.mark.parametrize("kind", [k for k in KINDS if k != "plain"])
+def test_one_lane_kinds_vs_oracle(hip_ctx, oracle_lib, kind):
+    """Every kind of step just above the line, where its passes give a particle one lane."""
+    print(f"case: {SPLIT + 1} particles, {kind}", flush=True)
+    _one_step_vs_oracle(hip_ctx, oracle_lib, _block(SPLIT + 1, **_tight(kind)), BARS)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_one_lane_overflow_vs_oracle(hip_ctx, oracle_lib, kind):
+    """A block at 0.6 spacings (about 200 neighbours) beside an ordinary one, above the
+    line: its particles run past the rows of the setup's table and walk the grid in
+    every pass, beside lanes that do not. Bars of the same block alone
+    (test_dense_block_list_overflow and its viscous form, in test_gpu_parity), and its
+    two iterations: further ones diverge in it, the pressure grows from 1e8 to 1e10 by
+    the twentieth, and a difference of 1e-6 grows with it to 1e-4, in the oracle's FP32
+    as well."""
+    s, side = 0.025, 41
+    fx = np.concatenate([
+        scenes.fluid_block((side, side, side), (1, 1, 1), s, 1e-4,
+                           scenes.stream_base(3, 0))[:SPLIT + 1 - 1000],
+        scenes.fluid_block((10, 10, 10), (10, 10, (side + 6) / 0.6), 0.6 * s, 1e-4,
+                           scenes.stream_base(9, 0))])
+    v = np.random.default_rng(5).uniform(-0.2, 0.2, fx.shape)
+    sc = scenes._finish("dense", s, fx, scenes.box_boundary(side + 4, side + 4, side + 20, s), 1,
+                        v=v, **_tight(kind))
+    sc.permute_every = 0
+    sc.iisph_max_iterations = 2
+    print(f"case: {len(fx)} particles, 1000 of them dense, {kind}", flush=True)
+    bars = {"density": 2e-5, "position": 1e-5}
+    if "implicit_viscosity" in KINDS[kind]:
+        bars = {"density": 1e-3, "position": 1e-5, "velocity": 5e-3}
+    if kind == "pt16":
+        # the velocity itself is what its solves stop at 1e-4 of, an iteration apart if
+        # need be: ten times that of the block's speed, which moves it by 0.28 m of the
+        # 1.5 m that the position is measured by, is 2e-4 there
+        bars["position"] = 2e-4
+    _one_step_vs_oracle(hip_ctx, oracle_lib, sc, bars)
+
+
+@pytest.mark.parametrize("kind", ["plain", "wkbb18"])
+@pytest.mark.parametrize("n", [2, 31, 32, 33, 64, 65, 257, SPLIT, SPLIT + 1])
+def test_fp64_step_sizes_vs_oracle(hip_ctx, oracle_lib, n, kind):
+    """The 64-bit forms (32-byte records, gathered by lane pairs with several lanes too)
+    against the oracle, whose FP32 sums set the bars."""
+    _one_step_vs_oracle(hip_ctx, oracle_lib, _block(n, **_tight(kind)), BARS, real_type=1)
