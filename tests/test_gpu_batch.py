@@ -166,22 +166,31 @@ def test_batch_rejects_duplicate(hip_ctx):
 
 @pytest.mark.parametrize("real_type", [0, 1], ids=["fp32", "fp64"])
 def test_schedules_bit_identical(hip_ctx, real_type):
-    """The global-memory and the LDS-staged schedule of each fused pass visit
-    the same neighbours in the same order: forced schedules give identical
-    fields, alone and batched."""
+    """Every launch schedule gives identical fields, alone and batched: iterations
+    launched one by one (bit 3, the default) or replayed from a graph, the CG's scalars
+    in kernels of their own (bit 4), the WKBB18 diagonal and the CG set-up in two walks
+    (bit 5), IISPH iteration 1 in passes of its own (bit 6). Bits 0-2 choose nothing:
+    they are accepted and reported back. The scenes: two inviscid ones, on both sides
+    of the line between several lanes per particle and one, WKBB18 without and with
+    the gradient correction, and pt16."""
     from prtcl_amd import hip
-    mix = small_mix(3, seed=7)
+    mix = small_mix(4, seed=7) + [scenes.random_scene(7, 9, 66000, 70000, 4)]
+    for sc, iv in zip(mix[1:], (1, 2, 3)):
+        sc.implicit_viscosity = iv
+        sc.fluid_viscosity = sc.boundary_viscosity = 10.0
+    assert mix[0].n_fluid <= 65536 < mix[4].n_fluid
     out = {}
-    for mask in (0, 7, 5):
+    masks = (8, 0, 7, 8 | 16, 8 | 32, 8 | 64, 127)
+    for mask in masks:
         hs = [hip.HipScene(hip_ctx, sc, real_type=real_type) for sc in mix]
         for h in hs:
             h.prepare()
             h.set_schedule(mask)
-        for _ in range(3):
+        for _ in range(2):
             for h in hs:
                 h.step(1)
         hip_ctx.set_batch_schedule(mask)
-        for _ in range(3):
+        for _ in range(2):
             hip_ctx.step(hs, 1)
         assert all(h.schedule() == mask for h in hs)
         assert hip_ctx.batch_schedule() == mask
@@ -189,10 +198,10 @@ def test_schedules_bit_identical(hip_ctx, real_type):
         for h in hs:
             h.destroy()
     hip_ctx.set_batch_schedule(-1)
-    for mask in (7, 5):
-        for a, b in zip(out[0], out[mask]):
+    for mask in masks[1:]:
+        for j, (a, b) in enumerate(zip(out[8], out[mask])):
             for f in FIELDS:
-                assert np.array_equal(a[f], b[f]), (mask, f)
+                assert np.array_equal(a[f], b[f]), (mask, j, f)
 
 
 def test_fp32_and_fp64_batch_graphs_stay_apart(hip_ctx):
@@ -280,8 +289,8 @@ def test_first_iteration_fold_bit_identical(hip_ctx, real_type):
 
 
 def test_graph_replay_equals_eager(hip_ctx):
-    """The IISPH iteration replayed from captured hipGraphs (default) and
-    launched kernel by kernel (schedule bit 3) give identical fields, alone
+    """The IISPH iteration replayed from captured hipGraphs and launched kernel
+    by kernel (schedule bit 3, the default) give identical fields, alone
     and batched; several steps, so the cached graphs are replayed with the
     step-to-step buffer swaps and the per-step tables."""
     from prtcl_amd import hip
