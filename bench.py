@@ -244,24 +244,10 @@ def bench_scene(ctx, sc, steps, warmup, schedules=False, traffic=False, schedule
     ctx.synchronize()
     prof = ctx.profile_read()
     ctx.profile(False)
-    tuned = g.schedule()
-
-    sched = {}
-    if schedules:
-        # per-launch stage times of the fused passes over a few further steps
-        for name, mask in (("global", 8),):
-            g.set_schedule(mask)
-            g.step(1)
-            ctx.profile(True)
-            for _ in range(min(prof_steps, 10)):
-                g.step(1)
-            ctx.synchronize()
-            pr = ctx.profile_read()
-            ctx.profile(False)
-            sched[name] = {k: round(v[0] / v[1], 5) for k, v in pr.items()
-                           if v[1] > 0 and k in ("iisph_setup", "iisph_pressure_acceleration",
-                                                 "iisph_pressure")}
-        g.set_schedule(tuned)
+    # per-launch stage times of the fused passes
+    sched = {k: round(v[0] / v[1], 5) for k, v in prof.items()
+             if v[1] > 0 and k in ("iisph_setup", "iisph_pressure_acceleration",
+                                   "iisph_pressure")}
 
     nf = sc.n_fluid
     viscous = sc.implicit_viscosity == 1
@@ -313,7 +299,7 @@ def bench_scene(ctx, sc, steps, warmup, schedules=False, traffic=False, schedule
                              wkbb18_tolerance=sc.wkbb18_maximum_error,
                              wkbb18_max_iterations=sc.wkbb18_maximum_iterations)
     if schedules:
-        out["schedule"] = {"tuned_mask": tuned, "ms_per_launch": sched}
+        out["schedule"] = {"mask": g.schedule(), "ms_per_launch": sched}
     return out, g
 
 

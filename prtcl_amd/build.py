@@ -5,7 +5,7 @@ FP32 instructions disabled (-Xclang -target-feature -Xclang -packed-fp32-ops).
 The procedure kernels of sph.hip and wkbb18.hip are built without FMA
 contraction so their pair terms round exactly like the FP32 CPU code; the
 fused step kernels contract within single expressions only, so every
-schedule of a pass rounds alike.
+form of a pass rounds alike.
 """
 
 from __future__ import annotations
@@ -32,8 +32,9 @@ COMMON = [
 SOURCES = {
     "nsearch.hip": [],
     "sph.hip": ["-ffp-contract=off"],
-    # contraction only within one expression: the LDS and global-memory
-    # schedules of a pass share the pair arithmetic and must round alike
+    # contraction only within one expression: the single-scene and the batched
+    # form of a pass, and its forms with one and several lanes per particle, share
+    # the pair arithmetic and must round alike
     "fused.hip": ["-ffp-contract=on"],
     "wkbb18.hip": ["-ffp-contract=off"],
     "pt16.hip": ["-ffp-contract=off"],

@@ -1012,7 +1012,6 @@ __device__ __forceinline__ void k_pressure_list_body(const SceneView<T> &S, cons
     sum += q.x.w * K.gradf_unscaled(d0 * d0 + d1 * d1 + d2 * d2) *
            (q.a.x * d0 + q.a.y * d1 + q.a.z * d2);
   };
-  static_assert(SceneView<T>::kXaGroup == 1, "x and a of a particle side by side");
   list_gather_records<kLanes, 4>(
       L, R, static_cast<size_t>(S.nf), i, (info & kListOverflow) ? 0u : info, sub,
       static_cast<uint32_t>(valid ? i : 0), S.xa,

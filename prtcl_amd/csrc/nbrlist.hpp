@@ -62,7 +62,6 @@ struct Spans {
     return Spans{R.base[0], R.base[1], R.base[2], R.len[0], R.len[1], R.len[2]};
   }
   __device__ __forceinline__ uint32_t base(int s) const { return s == 0 ? b0 : (s == 1 ? b1 : b2); }
-  __device__ __forceinline__ uint32_t len(int s) const { return s == 0 ? l0 : (s == 1 ? l1 : l2); }
   __device__ __forceinline__ uint32_t max_len() const {
     return l0 > l1 ? (l0 > l2 ? l0 : l2) : (l1 > l2 ? l1 : l2);
   }

@@ -442,15 +442,6 @@ __global__ __launch_bounds__(kBlock) void k_scatter_b(const BatchEntry<T> *tab,
                  u & kBatchLocalMask);
 }
 
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_stable_rank_b(const BatchEntry<T> *tab,
-                                                          const uint32_t *pmap) {
-  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  k_stable_rank_body(E.S.grid, E.S.fcell, E.start, E.perm, E.S.nf, E.rank,
-                     u & kBatchLocalMask);
-}
-
 // cell_dst must not be the perm buffer: perm is read by every thread
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_place_state_b(const BatchEntry<T> *tab,
@@ -461,16 +452,6 @@ __global__ __launch_bounds__(kBlock) void k_place_state_b(const BatchEntry<T> *t
                                 E.v_dst, E.S.v, E.id_dst,
                                 reinterpret_cast<const uint32_t *>(E.S.id), E.cell_dst,
                                 E.S.xf, E.S.kick(!E.split_setup), u & kBatchLocalMask);
-}
-
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_gather_state_b(const BatchEntry<T> *tab,
-                                                           const uint32_t *pmap) {
-  const uint32_t u = pmap[xcd_block(blockIdx.x, gridDim.x)];
-  const BatchEntry<T> &E = tab[u >> kBatchLocalBits];
-  k_gather_state_body<vec4_t<T>>(E.x_dst, E.S.xm, E.v_dst, E.S.v, E.id_dst,
-                                 reinterpret_cast<const uint32_t *>(E.S.id), E.cell_dst,
-                                 E.S.fcell, E.rank, E.S.nf, u & kBatchLocalMask);
 }
 
 }  // namespace

@@ -227,13 +227,12 @@ struct SceneView {
   const uint32_t *bstart;
   V4 *xm, *v, *a, *c, *G, *vd;
   V4 *xq;  // (x, y, z, m p / rho^2): the one gather of the pressure-acceleration pass
-  // (x, y, z, m) and (a, 0) records of the pressure pass's gathers, in
-  // groups of kXaGroup particles (their x-records, then their a-records), so
-  // both records of a particle share one cache line: xa_x() / xa_a() give
-  // the index of a record. One particle per group (x and a side by side,
-  // 32 bytes for FP32) measured faster than 4 per group (128-byte groups,
-  // whole 64-byte segments per pass): the pressure pass gains more from the
-  // adjacent pair than the acceleration pass loses on half-segment writes.
+  // (x, y, z, m) and (a, 0) records of the pressure pass's gathers, side by side
+  // (32 bytes for FP32), so both records of a particle share one cache line:
+  // xa_x() / xa_a() give the index of a record. Groups of four x-records and
+  // their a-records (whole 64-byte segments per pass) measured slower: the
+  // pressure pass gains more from the adjacent pair than the acceleration pass
+  // loses on half-segment writes.
   V4 *xa;
   __host__ __device__ GravityKick<T> kick(bool on) const {
 #pragma clang fp contract(off)  // dt g is rounded before it is added
@@ -242,11 +241,8 @@ struct SceneView {
     k.t = t, k.fade = fade, k.on = on ? 1 : 0;
     return k;
   }
-  static constexpr size_t kXaGroup = 1;
-  __host__ __device__ static size_t xa_x(size_t j) {
-    return (j / kXaGroup) * (2 * kXaGroup) + j % kXaGroup;
-  }
-  __host__ __device__ static size_t xa_a(size_t j) { return xa_x(j) + kXaGroup; }
+  __host__ __device__ static size_t xa_x(size_t j) { return 2 * j; }
+  __host__ __device__ static size_t xa_a(size_t j) { return 2 * j + 1; }
   // positions in units of radius / kFixUnits modulo 2^16 (fixed_record), written
   // by the sort of a fused step and read by its neighbour search
   uint2 *xf;

@@ -2259,7 +2259,7 @@ class SceneImpl final : public SceneBase {
       A.take(*q, f);
     for (V4 **q : {&P.xm, &P.xq})
       A.take(*q, f);
-    A.take(P.xa, SceneView<T>::xa_x(f - 1) + 1 + SceneView<T>::kXaGroup);
+    A.take(P.xa, 2 * f);
     for (T **q : {&P.rho, &P.p, &P.pr, &P.s, &P.AA, &P.Ap, &P.tmpT})
       A.take(*q, f);
     // tmpSp also takes the 16-bit positions of a fused step, with the run padding,

@@ -161,9 +161,9 @@ inline int emu_sdot2(emu_short2 a, emu_short2 b, int c) {
   return static_cast<int>(static_cast<unsigned>(c) + static_cast<unsigned>(a.x * b.x) +
                           static_cast<unsigned>(a.y * b.y));
 }
-// the moves used: quad_perm 1 0 3 2 and 2 3 0 1, row_half_mirror (lane ^ 1, 2, 7)
+// the one move used: quad_perm 1 0 3 2 (lane ^ 1); another does not compile
 #define __builtin_amdgcn_update_dpp(old, src, ctrl, rows, banks, bound) \
-  __shfl_xor(src, (ctrl) == 0xB1 ? 1 : (ctrl) == 0x4E ? 2 : 7, 64)
+  (static_cast<void>(sizeof(char[(ctrl) == 0xB1 ? 1 : -1])), __shfl_xor(src, 1, 64))
 #define __builtin_amdgcn_sdot2(a, b, c, clamp) emu_sdot2(a, b, c)
 inline int __mul24(int a, int b) {
   auto low = [](int v) { return static_cast<long long>(static_cast<int>(static_cast<unsigned>(v) << 8) >> 8); };
