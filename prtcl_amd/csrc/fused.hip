@@ -290,8 +290,8 @@ __device__ __forceinline__ double first_iteration(const SceneView<T> &S, int i,
 // lanes that reject a candidate do not wait for the kernel arithmetic of the
 // ones that accept it. The table is written to the list row by row (coalesced).
 //
-// Bound by vector instructions and by the loads' address work, half each (216
-// candidates and 30 pairs a particle). With candidates as 16-byte positions and
+// Bound by vector instructions (82 % busy; the loads' address work 62 %: 216 candidates
+// and 30 pairs a particle). With candidates as 16-byte positions and
 // 13 instructions, 65 a pair and five wavefronts per SIMD, 1M particles took 229
 // us, 250,000 73 us, 16 scenes of 2,000 to 200,000 together 247 us; with 8-byte
 // records and 9 instructions, the velocities integrated by the sort and six
